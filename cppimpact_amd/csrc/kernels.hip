@@ -76,6 +76,19 @@ __device__ __forceinline__ RowPre row_prefetch(const Params &p, int base) {
   return RowPre{r[EP_WINT], r[EP_WPL], r[EP_BAD], r[EP_WGRAV]};
 }
 
+// Scalar loads issued at the kernel's start (the energy row, dt) must not
+// sink: the compiler moves them down to their first use, past the loads of
+// the node records, where the whole workgroup then waits for another round
+// trip before its first barrier.  A use here, in the block that issues them,
+// keeps them where they are written.
+__device__ __forceinline__ void keep_here(double &v) { asm volatile("" : "+s"(v)); }
+__device__ __forceinline__ void keep_here(RowPre &r) {
+  keep_here(r.wint);
+  keep_here(r.wpl);
+  keep_here(r.bad);
+  keep_here(r.wgrav);
+}
+
 // One wave's energy terms into its row: the cumulative ones added to what
 // the row held (pre), and with ALL the instantaneous ones (kinetic,
 // penalty, contact force, stable dt) stored.
@@ -159,21 +172,65 @@ __device__ __forceinline__ void node_update(const Params &p, int g, const double
   ea.wgrav += m * wg;
 }
 
+// N consecutive corner forces of local node j, ranks k..k+N-1 (k a multiple
+// of N, N of 4, or below 4 read one by one), added to s in rank order.  All N
+// slots are read before the first add, so their LDS latencies overlap.
+template <int N, typename R>
+__device__ __forceinline__ void node_force_batch(const R *lf, const uint16_t *joff, int j, int k,
+                                                 R s[3]) {
+  unsigned o[N];
+  if constexpr (N >= 4) {
+    const uint2 *w = reinterpret_cast<const uint2 *>(joff + k);
+#pragma unroll
+    for (int i = 0; i < N / 4; i++) {
+      const uint2 u = w[i];
+      o[4 * i] = u.x & 0xffffu;
+      o[4 * i + 1] = u.x >> 16;
+      o[4 * i + 2] = u.y & 0xffffu;
+      o[4 * i + 3] = u.y >> 16;
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < N; i++) o[i] = joff[k + i];
+  }
+  R v[N][3];
+#pragma unroll
+  for (int i = 0; i < N; i++) {
+    const R *q = lf + 3 * (int)(o[i] + (unsigned)j);
+#pragma unroll
+    for (int c = 0; c < 3; c++) v[i][c] = q[c];
+  }
+#pragma unroll
+  for (int i = 0; i < N; i++)
+#pragma unroll
+    for (int c = 0; c < 3; c++) s[c] += v[i][c];
+}
+
 // A local node's force from its deg corner-force slots in the block's LDS
 // (jagged-diagonal: the k-th at off[k] + j), summed in slot order in the
 // element precision R: FP64 for FP64 elements, FP32 for FP32 ones, whose
 // element forces carry FP32 rounding already (the nodal update that
-// follows is FP64 either way).
+// follows is FP64 either way).  Eight slots at a time, then four, two and
+// one by the bits of deg: a remainder taken slot by slot costs two dependent
+// LDS reads per slot, up to seven times over.  With the scalar loads kept at
+// the kernel's start (keep_here) the 1.57M-tet4 step went from 48.5 to 46.4
+// us (FP64) and from 33.1 to 32.1 us (FP32), the 1.2M-tet10 one from 157.0
+// to 153.8 us (FP32; FP64 within noise).
 template <typename R>
 __device__ __forceinline__ void node_force_sum(const R *lf, const uint16_t *joff, int j, int deg,
                                                double f[3]) {
   R s[3] = {R(0), R(0), R(0)};
-  for (int k = 0; k < deg; k++) {
-    const int q = joff[k] + j;
-    s[0] += lf[3 * q + 0];
-    s[1] += lf[3 * q + 1];
-    s[2] += lf[3 * q + 2];
+  int k = 0;
+  for (; k + 8 <= deg; k += 8) node_force_batch<8, R>(lf, joff, j, k, s);
+  if (deg & 4) {
+    node_force_batch<4, R>(lf, joff, j, k, s);
+    k += 4;
   }
+  if (deg & 2) {
+    node_force_batch<2, R>(lf, joff, j, k, s);
+    k += 2;
+  }
+  if (deg & 1) node_force_batch<1, R>(lf, joff, j, k, s);
   f[0] = double(s[0]);
   f[1] = double(s[1]);
   f[2] = double(s[2]);
@@ -314,13 +371,13 @@ k_elem_block10(Params p) {
   extern __shared__ double smem[];
   const int b = xcd_remap(blockIdx.x, gridDim.x);
   const int t = threadIdx.x, q = t & 3;
-  const RowPre row = row_prefetch(p, p.epart_base + b * (NT / 64));
+  RowPre row = row_prefetch(p, p.epart_base + b * (NT / 64));
   const int32_t *mt = p.meta + 8 * b;
   const int es = mt[0], nel = mt[1];
   const LNodes ln{smem, p.ml};
   R *lf = (R *)((char *)smem + lds_node_bytes(p.ml));
   uint16_t *joff = (uint16_t *)((char *)lf + lds_force_bytes(sizeof(R), 10, p.max_el));
-  const double dt = p.ctl->dt;
+  double dt = p.ctl->dt;
   // yielded bits, one per lane (point) of the wave: a point's ep is read
   // only when it has yielded before
   const int wv = __builtin_amdgcn_readfirstlane(t >> 6);
@@ -354,6 +411,8 @@ k_elem_block10(Params p) {
   if constexpr (PHYS != PHYS_COMPAT)
     load_state_sel<R, STREAM>(p, ec, q, (yw >> (t & 63)) & 1ull, pre);
   __builtin_amdgcn_sched_barrier(0);
+  keep_here(dt);
+  keep_here(row);
   if (has_n) ln.stage(t, xr, mr, vr);
   if (t <= p.kmax) joff[t] = jo;
   __syncthreads();
@@ -440,13 +499,13 @@ __device__ __forceinline__ void block4(const Params &p, const int b, const unsig
                                        int *wcnt, unsigned *misc) {
   extern __shared__ double smem[];
   const int t = threadIdx.x, w = t >> 6, lane = t & 63;
-  const RowPre row = row_prefetch(p, p.epart_base + b * (NT / 64));
+  RowPre row = row_prefetch(p, p.epart_base + b * (NT / 64));
   const int32_t *mt = p.meta + 8 * b;
   const int es = mt[0], nel = mt[1];
   const LNodes ln{smem, p.ml};
   R *lf = (R *)((char *)smem + lds_node_bytes(p.ml));
   uint16_t *joff = (uint16_t *)((char *)lf + lds_force_bytes(sizeof(R), 4, p.max_el));
-  const double dt = p.ctl->dt;
+  double dt = p.ctl->dt;
 
   // yielded bits of this wave's elements: a block has ywords words, one
   // per 64 elements of the largest block, and a wave past them (a block
@@ -482,6 +541,8 @@ __device__ __forceinline__ void block4(const Params &p, const int b, const unsig
   if constexpr (PHYS != PHYS_COMPAT)
     load_state_sel<R, STREAM>(p, ec, 0, (yw >> (t & 63)) & 1ull, pre);
   __builtin_amdgcn_sched_barrier(0);
+  keep_here(dt);
+  keep_here(row);
   if (has_n) ln.stage(t, xr, mr, vr);
   if (t <= p.kmax) joff[t] = jo;
   if constexpr (WALK)
