@@ -38,6 +38,8 @@ struct cpi_ctx {
   int ncol = 0;
   std::vector<int32_t> eperm, nperm, ninv;  // device->user elem, device->user node, user->device
   std::vector<int32_t> color_off;           // colour scatter launch ranges (device order)
+  std::vector<int32_t> loose;               // user nodes of no element
+  int32_t *d_last = nullptr;                // per user node: last element holding it (device id)
   BlockPlan plan;
   std::vector<void *> allocs;
   double *d_tmp = nullptr;
@@ -220,6 +222,13 @@ int capture_graphs(cpi_ctx *c) {
 
 int ensure_tmp(cpi_ctx *c, size_t n) {
   if (c->tmp_len >= n) return CPI_OK;
+  if (c->d_tmp) {
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    c->allocs.erase(std::find(c->allocs.begin(), c->allocs.end(), (void *)c->d_tmp));
+    (void)hipFree(c->d_tmp);
+    c->d_tmp = nullptr;
+    c->tmp_len = 0;
+  }
   double *p = nullptr;
   int rc = dalloc(c, &p, n);
   if (rc) return rc;
@@ -532,6 +541,16 @@ static int create_impl(cpi_ctx *c, const cpi_mesh_desc *m, const cpi_material *m
     int32_t *d = nullptr;
     if ((rc = dalloc(c, &d, cd.size())) || (rc = upload(c, d, cd))) return rc;
     P.conn = d;
+  }
+  // the element whose strain and stress a node reports
+  {
+    std::vector<int32_t> einv(ne), last(nn, -1);
+    for (int e = 0; e < ne; e++) einv[c->eperm[e]] = e;
+    for (int e = 0; e < ne; e++)
+      for (int j = 0; j < npe; j++) last[c->conn_u[(size_t)npe * e + j]] = einv[e];
+    for (int i = 0; i < nn; i++)
+      if (last[i] < 0) c->loose.push_back(i);
+    if ((rc = dalloc(c, &c->d_last, last.size())) || (rc = upload(c, c->d_last, last))) return rc;
   }
   // per-node flags in device node order from a list of user node ids
   auto node_mask = [&](int n, const int32_t *ids, const char *what, const uint8_t **out) {
@@ -987,24 +1006,29 @@ extern "C" int cpi_get_element_state(cpi_ctx *c, double *sig, double *ep) {
 extern "C" int cpi_get_stress_strain(cpi_ctx *c, double *strain, double *stress) {
   if (!c) return CPI_ERR_INVALID;
   if (!c->inited) return fail(c, CPI_ERR_STATE, "cpi_get_stress_strain before cpi_init");
-  int rc = ensure_tmp(c, 12 * (size_t)c->ne);
+  const size_t n6 = 6 * (size_t)c->nn;
+  int rc = ensure_tmp(c, 2 * n6);
   if (rc) return rc;
-  hipError_t e = launch_stress_elem(c->P, c->d_tmp, c->stream);
+  hipError_t e = launch_stress_node(c->P, c->d_last, c->d_tmp, c->d_tmp + n6, c->stream);
   if (e != hipSuccess) return fail(c, CPI_ERR_HIP, hipGetErrorString(e));
-  std::vector<double> h(12 * (size_t)c->ne), byuser(12 * (size_t)c->ne);
-  HIPCHK(c, hipMemcpyAsync(h.data(), c->d_tmp, sizeof(double) * h.size(), hipMemcpyDeviceToHost, c->stream));
+  // nodes of no element keep what the caller's arrays hold
+  double *out[2] = {strain, stress};
+  std::vector<double> keep;
+  for (double *o : out)
+    if (o)
+      for (int32_t n : c->loose) keep.insert(keep.end(), o + 6L * n, o + 6L * n + 6);
+  for (int k = 0; k < 2; k++)
+    if (out[k])
+      HIPCHK(c, hipMemcpyAsync(out[k], c->d_tmp + k * n6, sizeof(double) * n6,
+                               hipMemcpyDeviceToHost, c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));
-  for (int e2 = 0; e2 < c->ne; e2++)
-    std::memcpy(&byuser[12 * (size_t)c->eperm[e2]], &h[12 * (size_t)e2], 12 * sizeof(double));
-  // element order, last element containing the node wins (dynamics_kernels.h:141-147)
-  for (int e2 = 0; e2 < c->ne; e2++)
-    for (int j = 0; j < c->npe; j++) {
-      int n = c->conn_u[(size_t)c->npe * e2 + j];
-      for (int k = 0; k < 6; k++) {
-        if (strain) strain[6L * n + k] = byuser[12 * (size_t)e2 + k];
-        if (stress) stress[6L * n + k] = byuser[12 * (size_t)e2 + 6 + k];
+  const double *was = keep.data();
+  for (double *o : out)
+    if (o)
+      for (int32_t n : c->loose) {
+        std::memcpy(o + 6L * n, was, 6 * sizeof(double));
+        was += 6;
       }
-    }
   return CPI_OK;
 }
 

@@ -34,7 +34,10 @@ int energy_reduce_blocks();  // rows of p.ered (EP_N doubles each)
 hipError_t launch_mass(const Params &p, int rule, int scatter, int kind, double rho,
                        int nblocks, hipStream_t s);
 hipError_t launch_elem_dt(const Params &p, double *out, hipStream_t s);
-hipError_t launch_stress_elem(const Params &p, double *out, hipStream_t s);
+// strain and stress [nn][6] in user node order; last: per user node, the
+// device id of the highest-numbered element holding it (-1: none, not written)
+hipError_t launch_stress_node(const Params &p, const int32_t *last, double *strain,
+                              double *stress, hipStream_t s);
 hipError_t launch_debug_strain(const Params &p, int rule, double alpha, int dcase, double nu,
                                double *out, hipStream_t s);
 // the surrogate network on queue rows [0, n) (rows hold ceil(n/16)*16 rows
