@@ -37,7 +37,6 @@ struct cpi_ctx {
   std::vector<int32_t> conn_u, color, slave_u;
   int ncol = 0;
   std::vector<int32_t> eperm, nperm, ninv;  // device->user elem, device->user node, user->device
-  std::vector<int32_t> color_off;           // colour scatter launch ranges (device order)
   std::vector<int32_t> loose;               // user nodes of no element
   int32_t *d_last = nullptr;                // per user node: last element holding it (device id)
   BlockPlan plan;
@@ -46,7 +45,6 @@ struct cpi_ctx {
   size_t tmp_len = 0;
   Params P{};
   int nblocks = 0, n_elem_rows = 0, n_node_rows = 0, n_rows = 0;
-  std::vector<int> color_rows;  // first energy row of each colour launch
   size_t smem = 0;
   // captured steps: one plain step, the energy/output step, and kGraphRuns[k]
   // plain steps in one graph each
@@ -161,17 +159,11 @@ int enqueue_step(cpi_ctx *c, bool aux) {
       e = launch_node_bnd(p, c->prec, aux, c->stream);
     }
   } else {
-    const bool atomic = c->scatter == CPI_SCATTER_ATOMIC;
-    const int nc = atomic ? 1 : c->ncol;
-    for (int k = 0; k < nc && e == hipSuccess; k++) {
-      p.elem_base = atomic ? 0 : c->color_off[k];
-      p.elem_count = atomic ? c->ne : c->color_off[k + 1] - c->color_off[k];
-      p.epart_base = c->color_rows[k];
-      e = launch_elem_direct(p, c->rule, c->prec, c->phys, atomic, c->stream);
-    }
+    p.epart_base = 0;
+    e = launch_elem_direct(p, c->rule, c->prec, c->phys, c->scatter == CPI_SCATTER_ATOMIC, c->stream);
     if (e == hipSuccess) {
       p.epart_base = c->n_elem_rows;
-      e = launch_node_all(p, aux, c->stream);
+      e = launch_node_all(p, c->prec, aux, c->stream);
     }
   }
   if (e == hipSuccess && aux) e = launch_energy_reduce(p, c->stream);
@@ -242,19 +234,8 @@ int compute_mass(cpi_ctx *c) {
   HIPCHK(c, hipMemsetAsync((void *)p.m, 0, sizeof(double) * c->nn, c->stream));
   const double rho = c->mat.rho;
   hipError_t e = hipSuccess;
-  if (c->scatter == CPI_SCATTER_BLOCK) {
-    e = launch_mass(p, c->rule, 0, c->mass_kind, rho, c->nblocks, c->stream);
-  } else if (c->scatter == CPI_SCATTER_ATOMIC) {
-    p.elem_base = 0;
-    p.elem_count = c->ne;
-    e = launch_mass(p, c->rule, 2, c->mass_kind, rho, 0, c->stream);
-  } else {
-    for (int k = 0; k < c->ncol && e == hipSuccess; k++) {
-      p.elem_base = c->color_off[k];
-      p.elem_count = c->color_off[k + 1] - c->color_off[k];
-      e = launch_mass(p, c->rule, 1, c->mass_kind, rho, 0, c->stream);
-    }
-  }
+  // CPI_SCATTER_* in launch_mass's numbering
+  e = launch_mass(p, c->rule, c->scatter, c->mass_kind, rho, c->nblocks, c->stream);
   if (e != hipSuccess) return fail(c, CPI_ERR_HIP, std::string("mass kernel: ") + hipGetErrorString(e));
   HIPCHK(c, hipStreamSynchronize(c->stream));
   c->mass_ready = true;
@@ -488,12 +469,8 @@ static int create_impl(cpi_ctx *c, const cpi_mesh_desc *m, const cpi_material *m
     c->nperm.resize(c->nn);
     c->ninv.resize(c->nn);
     for (int i = 0; i < c->nn; i++) c->nperm[i] = c->ninv[i] = i;
-    if (c->scatter == CPI_SCATTER_COLOR) {
-      color_order(c->ne, c->color.data(), c->ncol, c->eperm, c->color_off);
-    } else {
-      c->eperm.resize(c->ne);
-      for (int e = 0; e < c->ne; e++) c->eperm[e] = e;
-    }
+    c->eperm.resize(c->ne);
+    for (int e = 0; e < c->ne; e++) c->eperm[e] = e;
   }
   Params &P = c->P;
   P.nn = c->nn;
@@ -675,16 +652,25 @@ static int create_impl(cpi_ctx *c, const cpi_mesh_desc *m, const cpi_material *m
     c->n_node_rows = 4 * std::max(1, (B.n_boundary + 255) / 256);
   } else {
     const int nt = elem_direct_threads(npe);
-    c->color_rows.clear();
-    int rows = 0;
+    const int rows = (nt / 64) * ((ne + nt - 1) / nt);
     if (c->scatter == CPI_SCATTER_COLOR) {
-      for (int kk = 0; kk < c->ncol; kk++) {
-        c->color_rows.push_back(rows);
-        rows += (nt / 64) * ((c->color_off[kk + 1] - c->color_off[kk] + nt - 1) / nt);
-      }
-    } else {
-      c->color_rows.push_back(0);
-      rows = (nt / 64) * ((ne + nt - 1) / nt);
+      if ((size_t)npe * ne > UINT32_MAX)
+        return fail(c, CPI_ERR_INVALID, "the colour scatter holds at most 2^32 element corners");
+      std::vector<uint32_t> slot, ptr;
+      std::vector<int32_t> order;
+      color_slots(ne, npe, c->conn_u.data(), nn, c->color.data(), c->ncol, slot, ptr, order);
+      uint32_t *ds, *dp;
+      int32_t *dor;
+      char *cf;  // the records; before the first step, FP64 corner masses
+      if ((rc = dalloc(c, &ds, slot.size())) || (rc = upload(c, ds, slot)) ||
+          (rc = dalloc(c, &dp, ptr.size())) || (rc = upload(c, dp, ptr)) ||
+          (rc = dalloc(c, &dor, order.size())) || (rc = upload(c, dor, order)) ||
+          (rc = dalloc(c, &cf, slot.size() * (c->prec == CPI_PREC_F32 ? sizeof(Vec3f) : sizeof(Vec3)))))
+        return rc;
+      P.fslot = ds;
+      P.node_slot = dp;
+      P.sample_id = dor;
+      P.cforce = cf;
     }
     c->n_elem_rows = rows;
     c->n_node_rows = 4 * ((nn + 255) / 256);
@@ -1184,15 +1170,9 @@ extern "C" int cpi_profile_kernels(cpi_ctx *c, int32_t nsteps, cpi_kernel_time *
       launches[0] += 1;
     } else {
       HIPCHK(c, hipEventRecord(ev[0], c->stream));
-      const bool atomic = c->scatter == CPI_SCATTER_ATOMIC;
-      const int nc = atomic ? 1 : c->ncol;
-      for (int k = 0; k < nc && e == hipSuccess; k++) {
-        p.elem_base = atomic ? 0 : c->color_off[k];
-        p.elem_count = atomic ? c->ne : c->color_off[k + 1] - c->color_off[k];
-        p.epart_base = c->color_rows[k];
-        e = launch_elem_direct(p, c->rule, c->prec, c->phys, atomic, c->stream);
-        launches[0] += 1;
-      }
+      e = launch_elem_direct(p, c->rule, c->prec, c->phys, c->scatter == CPI_SCATTER_ATOMIC,
+                             c->stream);
+      launches[0] += 1;
       HIPCHK(c, hipEventRecord(ev[1], c->stream));
     }
     p.epart_base = c->n_elem_rows;
@@ -1203,7 +1183,7 @@ extern "C" int cpi_profile_kernels(cpi_ctx *c, int32_t nsteps, cpi_kernel_time *
         set_launch_events(nullptr, nullptr);
       } else {
         HIPCHK(c, hipEventRecord(ev[2], c->stream));
-        e = launch_node_all(p, false, c->stream);
+        e = launch_node_all(p, c->prec, false, c->stream);
         HIPCHK(c, hipEventRecord(ev[3], c->stream));
       }
     }

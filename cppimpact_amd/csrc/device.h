@@ -73,7 +73,15 @@ struct Params {
   Vec3 *pos;             // x
   Vec3 *vv;              // v_{n+1/2}
   double *m;             // lumped mass (read by the node's owner only)
-  double *f[3];          // assembled force (colour / atomic scatter)
+  double *f[3];          // assembled force (atomic scatter)
+  // colour scatter: one corner force (Vec3, Vec3f in FP32) per node and
+  // element in cforce, a node's slots node_slot[n] .. node_slot[n+1] in
+  // ascending colour; corner k of element e at fslot[k * ne + e].
+  // sample_id: the element's number for the sample recorder's hash, its place
+  // in the elements sorted by colour (null: the device element id)
+  void *cforce;
+  const uint32_t *fslot, *node_slot;
+  const int32_t *sample_id;
   Node4 *acc;            // a_n                   written when store_aux
   Node4 *du;             // du of the step        written when store_aux
   Node4 *xprev;          // x_n before the step   written when store_aux
@@ -122,8 +130,6 @@ struct Params {
   double *hist;          // [hist_cap][8]
   int hist_cap;
   int store_aux;
-  int elem_base;         // colour / atomic: first device element of launch
-  int elem_count;
   const MlpParams *mlp;  // null unless the surrogate is enabled
   double mlp_tol;        // fallback threshold on |f_yield| / sy0
   unsigned long long *mlp_stats;  // [nblocks][2] surrogate accepted / fell back

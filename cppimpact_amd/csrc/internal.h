@@ -65,9 +65,13 @@ bool build_block_plan(int ne, int npe, const int32_t *conn, int nn,
                       const double *xloc, int max_elems, int max_nodes,
                       BlockPlan &plan, std::string &err);
 
-// Element order sorted by colour (stable), and colour offsets.
-void color_order(int ne, const int32_t *color, int ncol,
-                 std::vector<int32_t> &perm, std::vector<int32_t> &offsets);
+// Corner-force slots of the colour scatter: node n's slots are node_slot[n]
+// .. node_slot[n+1], one per element that holds it, in ascending colour, and
+// corner k of element e writes slot[k * ne + e].  order[e]: the element's
+// place in the elements sorted by colour (stable).
+void color_slots(int ne, int npe, const int32_t *conn, int nn, const int32_t *color, int ncol,
+                 std::vector<uint32_t> &slot, std::vector<uint32_t> &node_slot,
+                 std::vector<int32_t> &order);
 
 // Hilbert index of a point with 21-bit integer coordinates.
 uint64_t hilbert3(uint32_t x, uint32_t y, uint32_t z);

@@ -26,11 +26,12 @@ hipError_t launch_elem_direct(const Params &p, int rule, int prec, int phys, boo
                               hipStream_t s);
 // prec: the element kernel's precision (its partials are stored in it)
 hipError_t launch_node_bnd(const Params &p, int prec, bool aux, hipStream_t s);
-hipError_t launch_node_all(const Params &p, bool aux, hipStream_t s);
+// prec: the corner-force slots' precision (colour scatter)
+hipError_t launch_node_all(const Params &p, int prec, bool aux, hipStream_t s);
 hipError_t launch_node_init(const Params &p, hipStream_t s);
 hipError_t launch_energy_reduce(const Params &p, hipStream_t s);
 int energy_reduce_blocks();  // rows of p.ered (EP_N doubles each)
-// lumped mass into p.m (scatter: 0 block, 1 colour range, 2 atomic)
+// lumped mass into p.m (scatter: 0 block, 1 colour, 2 atomic)
 hipError_t launch_mass(const Params &p, int rule, int scatter, int kind, double rho,
                        int nblocks, hipStream_t s);
 hipError_t launch_elem_dt(const Params &p, double *out, hipStream_t s);

@@ -12,10 +12,10 @@
 //                 partial force per shared node
 //   k_node_bnd    one thread per shared node: sum its partials in block
 //                 order, then wall, gravity and leapfrog
-// With the colour scatter the element pass is one k_elem_direct launch per
-// colour (plain read-modify-write, no two elements of a colour share a
-// node); with the atomic scatter it is one launch using FP64 atomics; both
-// are followed by k_node_all.
+// With the colour scatter k_elem_direct stores every corner force into the
+// node's slot of the element's colour (no two elements of a colour share a
+// node) and k_node_all sums a node's slots in colour order; with the atomic
+// scatter it adds them with FP64 atomics, and k_node_all reads the sums.
 //
 // Nodal state: 24-byte records pos = x and vv = v, and the lumped mass m
 // (read only by the nodes' owners: a step never writes it).
@@ -756,6 +756,30 @@ __global__ void __launch_bounds__(NT) k_mlp_queue(const MlpParams *P, uint16_t *
   }
 }
 
+// force records [s, s1) added to f in order, loaded four at a time
+template <typename PR, typename I>
+__device__ __forceinline__ void sum_records(const PR *rec, I s, I s1, double f[3]) {
+  auto add = [&](const PR &q) {
+    f[0] += double(q.x);
+    f[1] += double(q.y);
+    f[2] += double(q.z);
+  };
+  for (; s + 4 <= s1; s += 4) {
+    const PR q0 = rec[s], q1 = rec[s + 1], q2 = rec[s + 2], q3 = rec[s + 3];
+    add(q0);
+    add(q1);
+    add(q2);
+    add(q3);
+  }
+  if (s + 2 <= s1) {
+    const PR q0 = rec[s], q1 = rec[s + 1];
+    add(q0);
+    add(q1);
+    s += 2;
+  }
+  if (s < s1) add(rec[s]);
+}
+
 template <bool AUX, typename R>
 __global__ void __launch_bounds__(256) k_node_bnd(Params p) {
   using PR = typename std::conditional<std::is_same<R, float>::value, Vec3f, Vec3>::type;
@@ -768,29 +792,9 @@ __global__ void __launch_bounds__(256) k_node_bnd(Params p) {
     const int g = p.n_interior + i;
     const Vec3 xr = p.pos[g], vv = p.vv[g];
     const double m = p.m[g];
-    // partials in slot order, loaded four at a time
+    // partials in slot order
     double f[3] = {0.0, 0.0, 0.0};
-    const int s1 = p.slot_ptr[i + 1];
-    int s = p.slot_ptr[i];
-    auto add = [&](const PR &q) {
-      f[0] += double(q.x);
-      f[1] += double(q.y);
-      f[2] += double(q.z);
-    };
-    for (; s + 4 <= s1; s += 4) {
-      const PR q0 = part[s], q1 = part[s + 1], q2 = part[s + 2], q3 = part[s + 3];
-      add(q0);
-      add(q1);
-      add(q2);
-      add(q3);
-    }
-    if (s + 2 <= s1) {
-      const PR q0 = part[s], q1 = part[s + 1];
-      add(q0);
-      add(q1);
-      s += 2;
-    }
-    if (s < s1) add(part[s]);
+    sum_records(part, p.slot_ptr[i], p.slot_ptr[i + 1], f);
     const double x[3] = {xr.x, xr.y, xr.z}, v[3] = {vv.x, vv.y, vv.z};
     node_update<AUX>(p, g, f, x, v, m, dt, ea);
   }
@@ -805,15 +809,23 @@ __global__ void __launch_bounds__(256) k_node_bnd(Params p) {
 
 // ---------------------------------------------------------------------------
 // colour / atomic element pass: one thread per element, nodes from HBM
+//
+// Colour: the forces go to per-node slots, summed by k_node_all in ascending
+// colour, the order in which one launch per colour would add them, so the
+// sums have the same bits.  One launch per colour (30 of them on a box mesh)
+// costs a launch and a chain of dependent loads each, for a few thousand
+// elements; the slots cost 24 (FP32: 12) bytes written and read per corner.
+// Per step: 6,000 tet4 148 -> 10.0 us, 48,000 tet10 684 -> 35 us, 1.57M
+// tet4 484 -> 204 us (there bound by the scattered 24-byte records).
 // ---------------------------------------------------------------------------
 template <int NPE, int RULE, typename R, int PHYS, bool ATOMIC, int NT>
 __global__ void __launch_bounds__(NT) k_elem_direct(Params p) {
-  const int t = blockIdx.x * NT + threadIdx.x;
+  using FR = typename std::conditional<std::is_same<R, float>::value, Vec3f, Vec3>::type;
+  const int e = blockIdx.x * NT + threadIdx.x;
   const RowPre row = row_prefetch(p, p.epart_base + blockIdx.x * (NT / 64));
   const double dt = p.ctl->dt;
   EAcc ea;
-  if (t < p.elem_count) {
-    const int e = p.elem_base + t;
+  if (e < p.ne) {
     int nd[NPE];
 #pragma unroll
     for (int k = 0; k < NPE; k++) nd[k] = p.conn[(long)k * p.ne + e];
@@ -827,12 +839,11 @@ __global__ void __launch_bounds__(NT) k_elem_direct(Params p) {
       vk[2] = b.z;
     };
     auto put = [&](int k, const R fk[3]) {
+      if constexpr (ATOMIC) {
 #pragma unroll
-      for (int c = 0; c < 3; c++) {
-        if (ATOMIC)
-          unsafeAtomicAdd(&p.f[c][nd[k]], double(fk[c]));
-        else
-          p.f[c][nd[k]] += double(fk[c]);
+        for (int c = 0; c < 3; c++) unsafeAtomicAdd(&p.f[c][nd[k]], double(fk[c]));
+      } else {
+        static_cast<FR *>(p.cforce)[p.fslot[(long)k * p.ne + e]] = FR{fk[0], fk[1], fk[2]};
       }
     };
     elem_core<NPE, RULE, R, PHYS>(p, get, dt, e, put, ea);
@@ -840,22 +851,29 @@ __global__ void __launch_bounds__(NT) k_elem_direct(Params p) {
   wave_flush<true>(p, p.epart_base + blockIdx.x * (NT / 64), ea, row);
 }
 
-template <bool AUX>
+// FR: the record of a corner-force slot (colour scatter), or void for the
+// sums of the atomic scatter, which are cleared for the next step
+template <bool AUX, typename FR>
 __global__ void __launch_bounds__(256) k_node_all(Params p) {
   const int g = blockIdx.x * 256 + threadIdx.x;
   const RowPre row = row_prefetch(p, p.epart_base + blockIdx.x * 4);
   const double dt = p.ctl->dt;
   EAcc ea;
   if (g < p.nn) {
-    double f[3];
-#pragma unroll
-    for (int c = 0; c < 3; c++) {
-      f[c] = p.f[c][g];
-      p.f[c][g] = 0.0;
-    }
     const Vec3 xr = p.pos[g], vv = p.vv[g];
+    const double m = p.m[g];
+    double f[3] = {0.0, 0.0, 0.0};
+    if constexpr (std::is_void<FR>::value) {
+#pragma unroll
+      for (int c = 0; c < 3; c++) {
+        f[c] = p.f[c][g];
+        p.f[c][g] = 0.0;
+      }
+    } else {
+      sum_records(static_cast<const FR *>(p.cforce), p.node_slot[g], p.node_slot[g + 1], f);
+    }
     const double x[3] = {xr.x, xr.y, xr.z}, v[3] = {vv.x, vv.y, vv.z};
-    node_update<AUX>(p, g, f, x, v, p.m[g], dt, ea);
+    node_update<AUX>(p, g, f, x, v, m, dt, ea);
   }
   wave_flush<AUX>(p, p.epart_base + blockIdx.x * 4, ea, row);
   if (blockIdx.x == 0 && threadIdx.x == 0) p.ctl->step += 1;
@@ -1038,11 +1056,12 @@ __global__ void __launch_bounds__(256) k_mass_bnd(Params p) {
   p.m[p.n_interior + i] = s;
 }
 
+// colour scatter: corner masses into the x of the corner-force slots (FP64
+// words, whatever the slots' record), summed in colour order by k_mass_slots
 template <int NPE, int RULE, bool ATOMIC>
 __global__ void __launch_bounds__(256) k_mass_direct(Params p, int kind, double rho) {
-  const int t = blockIdx.x * 256 + threadIdx.x;
-  if (t >= p.elem_count) return;
-  const int e = p.elem_base + t;
+  const int e = blockIdx.x * 256 + threadIdx.x;
+  if (e >= p.ne) return;
   int nd[NPE];
   double xs[NPE][3], me[NPE];
 #pragma unroll
@@ -1059,8 +1078,17 @@ __global__ void __launch_bounds__(256) k_mass_direct(Params p, int kind, double 
     if (ATOMIC)
       unsafeAtomicAdd(&p.m[nd[k]], me[k]);
     else
-      p.m[nd[k]] += me[k];
+      static_cast<double *>(p.cforce)[p.fslot[(long)k * p.ne + e]] = me[k];
   }
+}
+
+__global__ void __launch_bounds__(256) k_mass_slots(Params p) {
+  const int g = blockIdx.x * 256 + threadIdx.x;
+  if (g >= p.nn) return;
+  double s = 0.0;
+  for (uint32_t q = p.node_slot[g]; q < p.node_slot[g + 1]; q++)
+    s += static_cast<const double *>(p.cforce)[q];
+  p.m[g] = s;
 }
 
 // ---------------------------------------------------------------------------
@@ -1434,8 +1462,7 @@ static hipError_t elem_block_t(const Params &p, bool aux, int nblocks, size_t sm
 template <int NPE, int RULE, typename R, int PHYS>
 static hipError_t elem_direct_t(const Params &p, bool atomic, hipStream_t s) {
   constexpr int NT = NPE == 4 ? 256 : 128;
-  const int grid = (p.elem_count + NT - 1) / NT;
-  if (grid == 0) return hipSuccess;
+  const int grid = (p.ne + NT - 1) / NT;
   if (atomic) CPI_LAUNCH((k_elem_direct<NPE, RULE, R, PHYS, true, NT>), grid, NT, 0, s, p);
   CPI_LAUNCH((k_elem_direct<NPE, RULE, R, PHYS, false, NT>), grid, NT, 0, s, p);
 }
@@ -1546,10 +1573,18 @@ hipError_t launch_node_bnd(const Params &p, int prec, bool aux, hipStream_t s) {
   CPI_LAUNCH((k_node_bnd<false, double>), grid, 256, 0, s, p);
 }
 
-hipError_t launch_node_all(const Params &p, bool aux, hipStream_t s) {
+hipError_t launch_node_all(const Params &p, int prec, bool aux, hipStream_t s) {
   const int grid = (p.nn + 255) / 256;
-  if (aux) CPI_LAUNCH(k_node_all<true>, grid, 256, 0, s, p);
-  CPI_LAUNCH(k_node_all<false>, grid, 256, 0, s, p);
+  if (!p.cforce) {
+    if (aux) CPI_LAUNCH((k_node_all<true, void>), grid, 256, 0, s, p);
+    CPI_LAUNCH((k_node_all<false, void>), grid, 256, 0, s, p);
+  }
+  if (prec == 1) {
+    if (aux) CPI_LAUNCH((k_node_all<true, Vec3f>), grid, 256, 0, s, p);
+    CPI_LAUNCH((k_node_all<false, Vec3f>), grid, 256, 0, s, p);
+  }
+  if (aux) CPI_LAUNCH((k_node_all<true, Vec3>), grid, 256, 0, s, p);
+  CPI_LAUNCH((k_node_all<false, Vec3>), grid, 256, 0, s, p);
 }
 
 hipError_t launch_node_init(const Params &p, hipStream_t s) {
@@ -1578,10 +1613,12 @@ static hipError_t mass_rule_t(const Params &p, int scatter, int kind, double rho
     if (e != hipSuccess || p.n_boundary == 0) return e;
     CPI_LAUNCH(k_mass_bnd, (p.n_boundary + 255) / 256, 256, 0, s, p);
   }
-  const int grid = (p.elem_count + 255) / 256;
-  if (grid == 0) return hipSuccess;
+  const int grid = (p.ne + 255) / 256;
   if (scatter == 2) CPI_LAUNCH((k_mass_direct<NPE, RULE, true>), grid, 256, 0, s, p, kind, rho);
-  CPI_LAUNCH((k_mass_direct<NPE, RULE, false>), grid, 256, 0, s, p, kind, rho);
+  hipLaunchKernelGGL((k_mass_direct<NPE, RULE, false>), dim3(grid), dim3(256), 0, s, p, kind, rho);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  CPI_LAUNCH(k_mass_slots, (p.nn + 255) / 256, 256, 0, s, p);
 }
 
 hipError_t launch_mass(const Params &p, int rule, int scatter, int kind, double rho, int nblocks,

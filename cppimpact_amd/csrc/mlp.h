@@ -152,6 +152,7 @@ __device__ __forceinline__ void record_sample(const Params &p, int e, int q, con
                                               const R so[6], R ep0, const R s[6], R ep1) {
   if (p.sample_keep < (1ull << 32)) {
     const uint64_t step = (uint64_t)p.ctl->step;
+    if (p.sample_id) e = p.sample_id[e];
     const uint64_t h = mix64(p.sample_seed + 0x9E3779B97F4A7C15ull * (step * 8 + q + 1) +
                              (uint64_t)(uint32_t)e * 0xD1B54A32D192ED03ull);
     if ((h >> 32) >= p.sample_keep) return;
