@@ -115,6 +115,7 @@ SIGNATURES = {
     "cpi_step": (C.c_int, [C.c_void_p, C.c_int32]),
     "cpi_synchronize": (C.c_int, [C.c_void_p]),
     "cpi_get_state": (C.c_int, [C.c_void_p, _dp, _dp, _dp, _dp, _dp]),
+    "cpi_get_state_mass3": (C.c_int, [C.c_void_p, _dp, _dp, _dp, _dp, _dp, _dp]),
     "cpi_get_increment": (C.c_int, [C.c_void_p, _dp]),
     "cpi_get_element_state": (C.c_int, [C.c_void_p, _dp, _dp]),
     "cpi_get_stress_strain": (C.c_int, [C.c_void_p, _dp, _dp]),

@@ -5,11 +5,16 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <memory>
 #include <mutex>
+#include <new>
 #include <string>
+#include <system_error>
+#include <thread>
 #include <vector>
 
 #include "../../include/cppimpact_hip.h"
@@ -33,16 +38,21 @@ struct cpi_ctx {
   cpi_options opt{};
   cpi_material mat{};
   cpi_wall wall{};
-  std::vector<double> X0u, V0u;  // user order [N][3]
   std::vector<int32_t> conn_u, color, slave_u;
   int ncol = 0;
   std::vector<int32_t> eperm, nperm, ninv;  // device->user elem, device->user node, user->device
   std::vector<int32_t> loose;               // user nodes of no element
   int32_t *d_last = nullptr;                // per user node: last element holding it (device id)
+  int32_t *d_ninv = nullptr, *d_einv = nullptr;  // user node / element -> device id
+  Vec3 *d_V0 = nullptr;                     // initial velocities, device order
   BlockPlan plan;
   std::vector<void *> allocs;
   double *d_tmp = nullptr;
   size_t tmp_len = 0;
+  // pinned host words results come back through, and one event per chunk of
+  // a large context's ring
+  double *pin = nullptr;
+  std::vector<hipEvent_t> ring;
   Params P{};
   int nblocks = 0, n_elem_rows = 0, n_node_rows = 0, n_rows = 0;
   size_t smem = 0;
@@ -58,7 +68,38 @@ struct cpi_ctx {
   MlpHost mlp;  // surrogate weights and sample buffer
 };
 
+// one workgroup: the minimum of the element partials and the smallest
+// positive nodal mass (the wall spring's limit needs it)
+__global__ void __launch_bounds__(256) k_dt_finish(const double *part, int nb, const double *m,
+                                                   int nn, double *out) {
+  __shared__ double r0[256], r1[256];
+  double a = 1e300, b = 1e300;
+  for (int i = threadIdx.x; i < nb; i += 256) a = fmin(a, part[i]);
+  for (int i = threadIdx.x; i < nn; i += 256)
+    if (m[i] > 0.0) b = fmin(b, m[i]);
+  r0[threadIdx.x] = a;
+  r1[threadIdx.x] = b;
+  __syncthreads();
+  for (int h = 128; h > 0; h >>= 1) {
+    if ((int)threadIdx.x < h) {
+      r0[threadIdx.x] = fmin(r0[threadIdx.x], r0[threadIdx.x + h]);
+      r1[threadIdx.x] = fmin(r1[threadIdx.x], r1[threadIdx.x + h]);
+    }
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) {
+    out[0] = r0[0];
+    out[1] = r1[0];
+  }
+}
+
 namespace {
+
+hipError_t launch_dt_finish(const double *part, int nb, const double *m, int nn, double *out,
+                            hipStream_t s) {
+  hipLaunchKernelGGL(k_dt_finish, dim3(1), dim3(256), 0, s, part, nb, m, nn, out);
+  return hipGetLastError();
+}
 
 #define HIPCHK(ctx, expr)                                                                  \
   do {                                                                                    \
@@ -116,35 +157,145 @@ double rule_weight_sum(int rule) {
   }
 }
 
-// user AoS [N][3] <-> device nodal records in device node order (Node4
-// with w = 0, or Vec3)
-template <typename T>
-int put_nodes(cpi_ctx *c, T *d, const double *aos) {
-  std::vector<T> tmp(c->nn);
-  for (int i = 0; i < c->nn; i++) {
-    const double *s = aos + 3L * c->nperm[i];
-    tmp[i] = T{};
-    tmp[i].x = s[0];
-    tmp[i].y = s[1];
-    tmp[i].z = s[2];
+// pinned words of a context: results up to kSmall come back in one transfer;
+// a context whose nodal state is larger holds a ring of 1 MiB chunks, at most
+// kRing of them (see bring_back_ring)
+constexpr size_t kSmall = 512u << 10;
+constexpr size_t kRing = 32;
+constexpr int kCopyThreads = 6;
+constexpr size_t kStateWords = (sizeof(Ctl) + 7) / 8;  // ahead of the exported arrays
+
+int ensure_tmp(cpi_ctx *c, size_t n);
+
+// user-order [N][3] on the host -> nodal records in device node order
+int put_nodes(cpi_ctx *c, const double *aos, Vec3 *d3, Node4 *d4) {
+  const size_t n = 3 * (size_t)c->nn;
+  int rc = ensure_tmp(c, n);
+  if (rc) return rc;
+  HIPCHK(c, hipMemcpyAsync(c->d_tmp, aos, sizeof(double) * n, hipMemcpyHostToDevice, c->stream));
+  HIPCHK(c, launch_import_nodes(c->d_tmp, c->d_ninv, c->nn, d3, d4, c->stream));
+  HIPCHK(c, hipStreamSynchronize(c->stream));  // d_tmp and the caller's array are free again
+  return CPI_OK;
+}
+
+// Results that lie one after the other in d_tmp, to the caller's arrays.
+// Waits for the stream.
+struct Piece {
+  void *host;
+  size_t words;
+};
+
+// bytes [at, at + n) of the pieces' concatenation, from src
+void spread(const Piece *p, size_t at, size_t n, const char *src) {
+  for (; n; p++) {
+    const size_t len = 8 * p->words;
+    if (at >= len) {
+      at -= len;
+      continue;
+    }
+    const size_t k = std::min(n, len - at);
+    std::memcpy((char *)p->host + at, src, k);
+    src += k;
+    n -= k;
+    at = 0;
   }
-  HIPCHK(c, hipMemcpyAsync(d, tmp.data(), sizeof(T) * c->nn, hipMemcpyHostToDevice, c->stream));
+}
+
+// Results too large for one transfer: the chunks go through the pinned ring
+// while a few threads copy those that have arrived to the caller's pages,
+// which are fresh as a rule.  One thread (the runtime's staged copy) is bound
+// by its page faults: the 239 MB of the 1.87M-node cylinder took 26 ms, this
+// takes 8.4 (88 ms when the host also permuted them).
+// false: no thread could be started and nothing was moved.
+constexpr size_t kChunk = 1u << 20;
+bool bring_back_ring(cpi_ctx *c, const Piece *p, size_t bytes, int *rc) {
+  const size_t chunks = (bytes + kChunk - 1) / kChunk, ring = c->ring.size();
+  std::atomic<size_t> issued{0}, next{0};
+  std::unique_ptr<std::atomic<bool>[]> copied(new (std::nothrow) std::atomic<bool>[chunks]);
+  if (!copied) return false;
+  for (size_t i = 0; i < chunks; i++) copied[i] = false;
+  std::atomic<int> err{(int)hipSuccess};
+  auto work = [&] {
+    (void)hipSetDevice(c->dev);
+    for (;;) {
+      const size_t i = next.fetch_add(1);
+      if (i >= chunks) return;
+      while (issued.load(std::memory_order_acquire) <= i) {
+        if (err.load()) return;
+        std::this_thread::yield();
+      }
+      const hipError_t e = hipEventSynchronize(c->ring[i % ring]);
+      if (e != hipSuccess) {
+        err = (int)e;
+        return;
+      }
+      const size_t at = i * kChunk;
+      spread(p, at, std::min(kChunk, bytes - at), (const char *)c->pin + (i % ring) * kChunk);
+      copied[i].store(true, std::memory_order_release);
+    }
+  };
+  std::vector<std::thread> team;
+  const size_t want = std::min<size_t>(kCopyThreads, chunks);
+  try {
+    team.reserve(want);
+    while (team.size() < want) team.emplace_back(work);
+  } catch (const std::system_error &) {
+  } catch (const std::bad_alloc &) {
+  }
+  if (team.empty()) return false;
+  for (size_t i = 0; i < chunks && !err.load(); i++) {
+    while (i >= ring && !copied[i - ring].load(std::memory_order_acquire) && !err.load())
+      std::this_thread::yield();
+    const size_t at = i * kChunk;
+    hipError_t e = hipMemcpyAsync((char *)c->pin + (i % ring) * kChunk, (const char *)c->d_tmp + at,
+                                  std::min(kChunk, bytes - at), hipMemcpyDeviceToHost, c->stream);
+    if (e == hipSuccess) e = hipEventRecord(c->ring[i % ring], c->stream);
+    if (e != hipSuccess)
+      err = (int)e;
+    else
+      issued.store(i + 1, std::memory_order_release);
+  }
+  for (auto &t : team) t.join();
+  const hipError_t e = (hipError_t)err.load(), f = hipStreamSynchronize(c->stream);
+  *rc = CPI_OK;
+  if (e != hipSuccess || f != hipSuccess)
+    *rc = fail(c, CPI_ERR_HIP, std::string("download: ") + hipGetErrorString(e != hipSuccess ? e : f));
+  return true;
+}
+
+int bring_back(cpi_ctx *c, const Piece *p, int n) {
+  size_t bytes = 0;
+  for (int i = 0; i < n; i++) bytes += 8 * p[i].words;
+  if (bytes <= kSmall) {
+    HIPCHK(c, hipMemcpyAsync(c->pin, c->d_tmp, bytes, hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    spread(p, 0, bytes, (const char *)c->pin);
+    return CPI_OK;
+  }
+  int rc;
+  if (!c->ring.empty() && bring_back_ring(c, p, bytes, &rc)) return rc;
+  const double *src = c->d_tmp;
+  for (int i = 0; i < n; src += p[i].words, i++)
+    HIPCHK(c, hipMemcpyAsync(p[i].host, src, 8 * p[i].words, hipMemcpyDeviceToHost, c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));
   return CPI_OK;
 }
 
-template <typename T>
-int get_nodes(cpi_ctx *c, const T *d, double *aos) {
-  std::vector<T> tmp(c->nn);
-  HIPCHK(c, hipMemcpyAsync(tmp.data(), d, sizeof(T) * c->nn, hipMemcpyDeviceToHost, c->stream));
+// the control block
+int get_ctl(cpi_ctx *c, Ctl *h) {
+  HIPCHK(c, hipMemcpyAsync(c->pin, c->P.ctl, sizeof(Ctl), hipMemcpyDeviceToHost, c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));
-  for (int i = 0; i < c->nn; i++) {
-    double *o = aos + 3L * c->nperm[i];
-    o[0] = tmp[i].x;
-    o[1] = tmp[i].y;
-    o[2] = tmp[i].z;
-  }
+  std::memcpy(h, c->pin, sizeof(Ctl));
   return CPI_OK;
+}
+
+bool all_finite(const double *v, size_t n) {
+  double s[4] = {0.0, 0.0, 0.0, 0.0};  // v * 0 is NaN for an infinity or NaN
+  size_t i = 0;
+  for (; i + 4 <= n; i += 4)
+    for (int k = 0; k < 4; k++) s[k] += v[i + k] * 0.0;
+  for (; i < n; i++) s[0] += v[i] * 0.0;
+  return s[0] + s[1] + s[2] + s[3] == 0.0;
 }
 
 int enqueue_step(cpi_ctx *c, bool aux) {
@@ -244,14 +395,7 @@ int compute_mass(cpi_ctx *c) {
 
 // x = X0, v = v0, forces/aux/state zeroed (the mass, once assembled, stays)
 int reset_state(cpi_ctx *c) {
-  int rc = put_nodes(c, c->P.pos, c->X0u.data());
-  if (!rc) rc = put_nodes(c, c->P.vv, c->V0u.data());
-  if (!rc) rc = put_nodes(c, c->P.xprev, c->X0u.data());
-  if (rc) return rc;
-  for (int k = 0; k < 3; k++)
-    HIPCHK(c, hipMemsetAsync(c->P.f[k], 0, sizeof(double) * c->nn, c->stream));
-  HIPCHK(c, hipMemsetAsync(c->P.acc, 0, sizeof(Node4) * c->nn, c->stream));
-  HIPCHK(c, hipMemsetAsync(c->P.du, 0, sizeof(Node4) * c->nn, c->stream));
+  HIPCHK(c, launch_reset_nodes(c->P, c->d_V0, c->stream));
   const size_t rs = c->prec == CPI_PREC_F32 ? 4 : 8;
   if (c->phys != CPI_PHYSICS_COMPAT) {
     HIPCHK(c, hipMemsetAsync(c->P.sig, 0, rs * 6 * c->nq * (size_t)c->ne, c->stream));
@@ -267,32 +411,25 @@ int reset_state(cpi_ctx *c) {
 
 // stable dt of the current device positions: element limit and the wall
 // spring limit 2 sqrt(m_min / k)
+constexpr int kMassMinBlocks = 256;
 int stable_dt(cpi_ctx *c, double *dte, double *dtc) {
   const int nb = (c->ne + 255) / 256;
-  int rc = ensure_tmp(c, std::max(nb, c->nn));
+  int rc = ensure_tmp(c, (size_t)nb + kMassMinBlocks + 2);
   if (rc) return rc;
-  hipError_t e = launch_elem_dt(c->P, c->d_tmp, c->stream);
-  if (e != hipSuccess) return fail(c, CPI_ERR_HIP, hipGetErrorString(e));
-  std::vector<double> h(std::max(nb, c->nn));
-  HIPCHK(c, hipMemcpyAsync(h.data(), c->d_tmp, sizeof(double) * nb, hipMemcpyDeviceToHost, c->stream));
+  double *mm = c->d_tmp + nb, *out = mm + kMassMinBlocks;
+  HIPCHK(c, launch_elem_dt(c->P, c->d_tmp, c->stream));
+  HIPCHK(c, launch_mass_min(c->P, mm, kMassMinBlocks, c->stream));
+  HIPCHK(c, launch_dt_finish(c->d_tmp, nb, mm, kMassMinBlocks, out, c->stream));
+  HIPCHK(c, hipMemcpyAsync(c->pin, out, 2 * sizeof(double), hipMemcpyDeviceToHost, c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));
-  double m1 = 1e300;
-  for (int i = 0; i < nb; i++) m1 = std::min(m1, h[i]);
-  *dte = m1;
-  HIPCHK(c, hipMemcpyAsync(h.data(), c->P.m, sizeof(double) * c->nn, hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
-  double mmin = 1e300;
-  for (int i = 0; i < c->nn; i++)
-    if (h[i] > 0.0) mmin = std::min(mmin, h[i]);
-  *dtc = (c->wall.enabled && c->wall.stiffness > 0.0) ? 2.0 * std::sqrt(mmin / c->wall.stiffness)
-                                                      : INFINITY;
+  *dte = c->pin[0];
+  *dtc = (c->wall.enabled && c->wall.stiffness > 0.0)
+             ? 2.0 * std::sqrt(c->pin[1] / c->wall.stiffness)
+             : INFINITY;
   return CPI_OK;
 }
 
-int check_flags(cpi_ctx *c) {
-  Ctl h;
-  HIPCHK(c, hipMemcpyAsync(&h, c->P.ctl, sizeof(Ctl), hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
+int report_flags(cpi_ctx *c, const Ctl &h) {
   if (h.flags & 2u) return fail(c, CPI_ERR_NUMERIC, "inverted or degenerate element (detJ <= 0) during the step");
   if (h.flags & 1u) return fail(c, CPI_ERR_NUMERIC, "non-finite value in the energy terms (NaN/Inf state)");
   if (h.flags & 4u)
@@ -301,6 +438,12 @@ int check_flags(cpi_ctx *c) {
                     std::to_string(std::min(h.row[7], h.dt_contact)) +
                     " of the configuration (element CFL / wall spring)");
   return CPI_OK;
+}
+
+int check_flags(cpi_ctx *c) {
+  Ctl h;
+  int rc = get_ctl(c, &h);
+  return rc ? rc : report_flags(c, h);
 }
 
 }  // namespace
@@ -341,6 +484,9 @@ extern "C" void cpi_destroy(cpi_ctx *c) {
   if (c->stream) (void)hipStreamSynchronize(c->stream);
   drop_graphs(c);
   for (void *p : c->allocs) (void)hipFree(p);
+  if (c->pin) (void)hipHostFree(c->pin);
+  for (hipEvent_t e : c->ring)
+    if (e) (void)hipEventDestroy(e);
   mlp_free(c->mlp);
   if (c->stream) (void)hipStreamDestroy(c->stream);
   delete c;
@@ -389,21 +535,19 @@ static int create_impl(cpi_ctx *c, const cpi_mesh_desc *m, const cpi_material *m
                                  : (opt->physics == CPI_PHYSICS_COMPAT ? CPI_MASS_ROWSUM : CPI_MASS_HRZ);
   c->nq = (npe == 4) ? 1 : (c->rule == CPI_QUAD_REF5 ? 5 : 4);
   // host copies and validation
-  c->X0u.assign(m->xloc, m->xloc + 3L * c->nn);
-  c->V0u.assign(3L * c->nn, 0.0);
   c->conn_u.assign(m->element_nodes, m->element_nodes + (long)npe * c->ne);
   for (int32_t v : c->conn_u)
     if (v < 0 || v >= c->nn) return fail(c, CPI_ERR_MESH, "element_nodes references a node out of range");
-  for (double v : c->X0u)
-    if (!std::isfinite(v)) return fail(c, CPI_ERR_MESH, "non-finite node coordinate");
+  const double *X0u = m->xloc;
+  if (!all_finite(X0u, 3 * (size_t)c->nn)) return fail(c, CPI_ERR_MESH, "non-finite node coordinate");
   for (int e = 0; e < c->ne; e++) {
     const int32_t *ce = &c->conn_u[(long)npe * e];
     const int o = npe == 4 ? 0 : 2, i1 = npe == 4 ? 1 : 0, i2 = npe == 4 ? 2 : 1;
     double a[3], b[3], d[3];
     for (int k = 0; k < 3; k++) {
-      a[k] = c->X0u[3L * ce[i1] + k] - c->X0u[3L * ce[o] + k];
-      b[k] = c->X0u[3L * ce[i2] + k] - c->X0u[3L * ce[o] + k];
-      d[k] = c->X0u[3L * ce[3] + k] - c->X0u[3L * ce[o] + k];
+      a[k] = X0u[3L * ce[i1] + k] - X0u[3L * ce[o] + k];
+      b[k] = X0u[3L * ce[i2] + k] - X0u[3L * ce[o] + k];
+      d[k] = X0u[3L * ce[3] + k] - X0u[3L * ce[o] + k];
     }
     double v6 = a[0] * (b[1] * d[2] - b[2] * d[1]) - a[1] * (b[0] * d[2] - b[2] * d[0]) +
                 a[2] * (b[0] * d[1] - b[1] * d[0]);
@@ -425,6 +569,16 @@ static int create_impl(cpi_ctx *c, const cpi_mesh_desc *m, const cpi_material *m
                                           ", this library is built for gfx950 only");
   c->dev = opt->device;
   HIPCHK(c, hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
+  {
+    const size_t all = 8 * (kStateWords + 16 * (size_t)c->nn);
+    size_t pinned = kSmall;
+    if (all > kSmall) {
+      c->ring.resize(std::min(kRing, (all + kChunk - 1) / kChunk), nullptr);
+      pinned = std::max(pinned, c->ring.size() * kChunk);
+      for (hipEvent_t &e : c->ring) HIPCHK(c, hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    }
+    HIPCHK(c, hipHostMalloc((void **)&c->pin, pinned, hipHostMallocDefault));
+  }
   // device orders
   if (c->scatter == CPI_SCATTER_BLOCK) {
     const int nt = elem_block_threads(npe, c->rule);
@@ -452,7 +606,7 @@ static int create_impl(cpi_ctx *c, const cpi_mesh_desc *m, const cpi_material *m
     // node; the five-point tet10 kernel loops over its nodes
     int mn = (int)std::min<long>(mnl, (npe == 4 || c->nq == 4) ? nt : 1024);
     std::string e;
-    if (!build_block_plan(c->ne, npe, c->conn_u.data(), c->nn, c->X0u.data(), me, mn, c->plan, e))
+    if (!build_block_plan(c->ne, npe, c->conn_u.data(), c->nn, X0u, me, mn, c->plan, e))
       return fail(c, CPI_ERR_INVALID, "partition: " + e);
     if (c->plan.max_local_nodes > mn)
       return fail(c, CPI_ERR_INVALID, "partition: a block holds more nodes than its kernel");
@@ -527,7 +681,12 @@ static int create_impl(cpi_ctx *c, const cpi_mesh_desc *m, const cpi_material *m
       for (int j = 0; j < npe; j++) last[c->conn_u[(size_t)npe * e + j]] = einv[e];
     for (int i = 0; i < nn; i++)
       if (last[i] < 0) c->loose.push_back(i);
-    if ((rc = dalloc(c, &c->d_last, last.size())) || (rc = upload(c, c->d_last, last))) return rc;
+    if ((rc = dalloc(c, &c->d_last, last.size())) || (rc = upload(c, c->d_last, last)) ||
+        (rc = dalloc(c, &c->d_einv, einv.size())) || (rc = upload(c, c->d_einv, einv)) ||
+        (rc = dalloc(c, &c->d_ninv, c->ninv.size())) || (rc = upload(c, c->d_ninv, c->ninv)) ||
+        (rc = dalloc(c, &c->d_V0, nn)))
+      return rc;
+    HIPCHK(c, hipMemsetAsync(c->d_V0, 0, sizeof(Vec3) * nn, c->stream));
   }
   // per-node flags in device node order from a list of user node ids
   auto node_mask = [&](int n, const int32_t *ids, const char *what, const uint8_t **out) {
@@ -695,8 +854,10 @@ static int create_impl(cpi_ctx *c, const cpi_mesh_desc *m, const cpi_material *m
     P.mlp = c->mlp.d_params;
     P.mlp_stats = c->mlp.d_stats;
   }
-  // reference positions on the device (stress output)
-  if ((rc = put_nodes(c, c->P.X0, c->X0u.data()))) return rc;
+  // the words cpi_get_state brings back, allocated once
+  if ((rc = ensure_tmp(c, kStateWords + 16 * (size_t)nn))) return rc;
+  // reference positions on the device
+  if ((rc = put_nodes(c, X0u, nullptr, c->P.X0))) return rc;
   return reset_state(c);
 }
 
@@ -736,22 +897,14 @@ extern "C" int cpi_create(const cpi_mesh_desc *m, const cpi_material *mat, const
 
 extern "C" int cpi_set_state(cpi_ctx *c, const double *x0, const double *v0) {
   if (!c) return CPI_ERR_INVALID;
-  if (x0) {
-    for (long i = 0; i < 3L * c->nn; i++)
-      if (!std::isfinite(x0[i])) return fail(c, CPI_ERR_INVALID, "non-finite position");
-    c->X0u.assign(x0, x0 + 3L * c->nn);
-    c->mass_ready = false;
-  }
-  if (v0) {
-    for (long i = 0; i < 3L * c->nn; i++)
-      if (!std::isfinite(v0[i])) return fail(c, CPI_ERR_INVALID, "non-finite velocity");
-    c->V0u.assign(v0, v0 + 3L * c->nn);
-  }
+  const size_t n = 3 * (size_t)c->nn;
+  if (x0 && !all_finite(x0, n)) return fail(c, CPI_ERR_INVALID, "non-finite position");
+  if (v0 && !all_finite(v0, n)) return fail(c, CPI_ERR_INVALID, "non-finite velocity");
+  if (x0) c->mass_ready = false;
   c->inited = false;
-  drop_graphs(c);
-  int rc = put_nodes(c, c->P.X0, c->X0u.data());
-  if (rc) return rc;
-  return reset_state(c);
+  int rc = x0 ? put_nodes(c, x0, nullptr, c->P.X0) : CPI_OK;
+  if (!rc && v0) rc = put_nodes(c, v0, c->d_V0, nullptr);
+  return rc ? rc : reset_state(c);
 }
 
 extern "C" int cpi_stable_dt(cpi_ctx *c, double *dte, double *dtc) {
@@ -774,31 +927,6 @@ extern "C" int cpi_stable_dt(cpi_ctx *c, double *dte, double *dtc) {
 constexpr int kNoallocPartials = 65536;  // 16,777,216 elements at most
 constexpr int kNoallocOut = 2;
 static __device__ __align__(256) double scratch[kNoallocPartials + kNoallocOut];
-
-// one workgroup: the minimum of the element partials and the smallest
-// positive nodal mass (the wall spring's limit needs it)
-__global__ void __launch_bounds__(256) k_dt_finish(const double *part, int nb, const double *m,
-                                                   int nn, double *out) {
-  __shared__ double r0[256], r1[256];
-  double a = 1e300, b = 1e300;
-  for (int i = threadIdx.x; i < nb; i += 256) a = fmin(a, part[i]);
-  for (int i = threadIdx.x; i < nn; i += 256)
-    if (m[i] > 0.0) b = fmin(b, m[i]);
-  r0[threadIdx.x] = a;
-  r1[threadIdx.x] = b;
-  __syncthreads();
-  for (int h = 128; h > 0; h >>= 1) {
-    if ((int)threadIdx.x < h) {
-      r0[threadIdx.x] = fmin(r0[threadIdx.x], r0[threadIdx.x + h]);
-      r1[threadIdx.x] = fmin(r1[threadIdx.x], r1[threadIdx.x + h]);
-    }
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) {
-    out[0] = r0[0];
-    out[1] = r1[0];
-  }
-}
 
 namespace {
 
@@ -836,9 +964,7 @@ extern "C" int cpi_stable_dt_noalloc(cpi_ctx *c, double *dte, double *dtc) {
   int rc = scratch_of(c, &sp);
   if (rc) return rc;
   HIPCHK(c, launch_elem_dt(c->P, sp, c->stream));
-  hipLaunchKernelGGL(k_dt_finish, dim3(1), dim3(256), 0, c->stream, (const double *)sp, nb,
-                     (const double *)c->P.m, c->nn, sp + kNoallocPartials);
-  HIPCHK(c, hipGetLastError());
+  HIPCHK(c, launch_dt_finish(sp, nb, c->P.m, c->nn, sp + kNoallocPartials, c->stream));
   double r[kNoallocOut];
   HIPCHK(c, hipMemcpyAsync(r, sp + kNoallocPartials, sizeof(r), hipMemcpyDeviceToHost, c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));
@@ -853,7 +979,6 @@ extern "C" int cpi_init(cpi_ctx *c, double dt) {
   if (!std::isfinite(dt)) return fail(c, CPI_ERR_INVALID, "cpi_init: dt must be finite");
   if (c->phys == 2 && !c->mlp.ready)
     return fail(c, CPI_ERR_STATE, "cpi_init: CPI_RETURN_MLP needs cpi_set_surrogate first");
-  drop_graphs(c);
   c->inited = false;
   int rc = reset_state(c);
   if (!rc) rc = compute_mass(c);
@@ -880,7 +1005,12 @@ extern "C" int cpi_init(cpi_ctx *c, double dt) {
   if (e != hipSuccess) return fail(c, CPI_ERR_HIP, std::string("init kernels: ") + hipGetErrorString(e));
   HIPCHK(c, hipMemsetAsync(c->P.epart, 0, sizeof(double) * EP_N * c->n_rows, c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));
-  if (c->opt.use_graph && (rc = capture_graphs(c))) return rc;
+  // the step graphs hold the context's buffers, which a new initial state
+  // does not change; what does change the launches drops them
+  if (c->opt.use_graph && !c->gs.run[1]) {
+    drop_graphs(c);
+    if ((rc = capture_graphs(c))) return rc;
+  }
   c->inited = true;
   return CPI_OK;
 }
@@ -918,75 +1048,71 @@ extern "C" int cpi_synchronize(cpi_ctx *c) {
 }
 
 extern "C" int cpi_get_state(cpi_ctx *c, double *x, double *v, double *a, double *m, double *vi) {
+  return cpi_get_state_mass3(c, x, v, a, m, vi, nullptr);
+}
+
+extern "C" int cpi_get_state_mass3(cpi_ctx *c, double *x, double *v, double *a, double *m,
+                                   double *vi, double *m3) {
   if (!c) return CPI_ERR_INVALID;
-  HIPCHK(c, hipStreamSynchronize(c->stream));
-  int rc = CPI_OK;
-  if (x && (rc = get_nodes(c, c->P.pos, x))) return rc;
-  std::vector<double> hv, ha;
-  if (v || vi) {
-    hv.resize(3L * c->nn);
-    if ((rc = get_nodes(c, c->P.vv, hv.data()))) return rc;
-    if (v) std::memcpy(v, hv.data(), sizeof(double) * hv.size());
-  }
-  if (a || vi) {
-    ha.resize(3L * c->nn);
-    if ((rc = get_nodes(c, c->P.acc, ha.data()))) return rc;
-    if (a) std::memcpy(a, ha.data(), sizeof(double) * ha.size());
-  }
-  if (vi)
-    for (long i = 0; i < 3L * c->nn; i++) vi[i] = hv[i] - 0.5 * c->dt * ha[i];
-  if (m) {
-    std::vector<double> hm(c->nn);
-    HIPCHK(c, hipMemcpyAsync(hm.data(), c->P.m, sizeof(double) * c->nn, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    for (int i = 0; i < c->nn; i++) m[c->nperm[i]] = hm[i];
-  }
-  return c->inited ? check_flags(c) : CPI_OK;
+  const size_t n3 = 3 * (size_t)c->nn;
+  int rc = ensure_tmp(c, kStateWords + 5 * n3 + c->nn);
+  if (rc) return rc;
+  Ctl h;
+  Piece p[7] = {{&h, sizeof(Ctl) / 8}};
+  int k = 1;
+  double *d = c->d_tmp + kStateWords;
+  auto place = [&](double *host, size_t n) -> double * {
+    if (!host) return nullptr;
+    p[k++] = Piece{host, n};
+    d += n;
+    return d - n;
+  };
+  NodeExport o{};
+  o.ctl = reinterpret_cast<Ctl *>(c->d_tmp);
+  o.x = place(x, n3);
+  o.v = place(v, n3);
+  o.a = place(a, n3);
+  o.m = place(m, c->nn);
+  o.vi = place(vi, n3);
+  o.m3 = place(m3, n3);
+  o.half_dt = 0.5 * c->dt;
+  HIPCHK(c, launch_export_nodes(c->P, c->d_ninv, o, c->stream));
+  if ((rc = bring_back(c, p, k))) return rc;
+  return c->inited ? report_flags(c, h) : CPI_OK;
 }
 
 extern "C" int cpi_get_increment(cpi_ctx *c, double *du) {
   if (!c || !du) return CPI_ERR_INVALID;
-  HIPCHK(c, hipStreamSynchronize(c->stream));
-  return get_nodes(c, c->P.du, du);
+  const size_t n3 = 3 * (size_t)c->nn;
+  int rc = ensure_tmp(c, n3);
+  if (rc) return rc;
+  Params p = c->P;
+  p.acc = c->P.du;
+  NodeExport o{};
+  o.a = c->d_tmp;
+  HIPCHK(c, launch_export_nodes(p, c->d_ninv, o, c->stream));
+  const Piece q{du, n3};
+  return bring_back(c, &q, 1);
 }
 
 extern "C" int cpi_get_element_state(cpi_ctx *c, double *sig, double *ep) {
   if (!c) return CPI_ERR_INVALID;
-  if (c->phys == CPI_PHYSICS_COMPAT) {
-    if (sig) std::memset(sig, 0, sizeof(double) * 6 * c->nq * (size_t)c->ne);
-    if (ep) std::memset(ep, 0, sizeof(double) * c->nq * (size_t)c->ne);
-    return CPI_OK;
-  }
-  HIPCHK(c, hipStreamSynchronize(c->stream));
   const size_t n = (size_t)c->nq * c->ne;
-  auto fetch = [&](const void *d, size_t cnt, std::vector<double> &out) -> int {
-    out.resize(cnt);
-    if (c->prec == CPI_PREC_F32) {
-      std::vector<float> t(cnt);
-      HIPCHK(c, hipMemcpyAsync(t.data(), d, 4 * cnt, hipMemcpyDeviceToHost, c->stream));
-      HIPCHK(c, hipStreamSynchronize(c->stream));
-      for (size_t i = 0; i < cnt; i++) out[i] = t[i];
-    } else {
-      HIPCHK(c, hipMemcpyAsync(out.data(), d, 8 * cnt, hipMemcpyDeviceToHost, c->stream));
-      HIPCHK(c, hipStreamSynchronize(c->stream));
-    }
+  if (c->phys == CPI_PHYSICS_COMPAT) {
+    if (sig) std::memset(sig, 0, sizeof(double) * 6 * n);
+    if (ep) std::memset(ep, 0, sizeof(double) * n);
     return CPI_OK;
-  };
-  std::vector<double> hs, he;
-  int rc;
-  if (sig) {
-    if ((rc = fetch(c->P.sig, 6 * n, hs))) return rc;
-    for (int e = 0; e < c->ne; e++)
-      for (int q = 0; q < c->nq; q++)
-        for (int k = 0; k < 6; k++)
-          sig[((size_t)c->eperm[e] * c->nq + q) * 6 + k] = hs[(size_t)(q * 6 + k) * c->ne + e];
   }
-  if (ep) {
-    if ((rc = fetch(c->P.epbar, n, he))) return rc;
-    for (int e = 0; e < c->ne; e++)
-      for (int q = 0; q < c->nq; q++) ep[(size_t)c->eperm[e] * c->nq + q] = he[(size_t)q * c->ne + e];
-  }
-  return CPI_OK;
+  int rc = ensure_tmp(c, (sig ? 6 * n : 0) + (ep ? n : 0));
+  if (rc) return rc;
+  Piece p[2];
+  int k = 0;
+  if (sig) p[k++] = Piece{sig, 6 * n};
+  if (ep) p[k++] = Piece{ep, n};
+  if (k)
+    HIPCHK(c, launch_export_elems(c->P, c->prec, c->d_einv, sig ? c->d_tmp : nullptr,
+                                  ep ? c->d_tmp + (sig ? 6 * n : 0) : nullptr, c->stream));
+  return bring_back(c, p, k);
 }
 
 extern "C" int cpi_get_stress_strain(cpi_ctx *c, double *strain, double *stress) {
@@ -995,7 +1121,8 @@ extern "C" int cpi_get_stress_strain(cpi_ctx *c, double *strain, double *stress)
   const size_t n6 = 6 * (size_t)c->nn;
   int rc = ensure_tmp(c, 2 * n6);
   if (rc) return rc;
-  hipError_t e = launch_stress_node(c->P, c->d_last, c->d_tmp, c->d_tmp + n6, c->stream);
+  hipError_t e = launch_stress_node(c->P, c->d_last, strain ? c->d_tmp : nullptr,
+                                    stress ? c->d_tmp + (strain ? n6 : 0) : nullptr, c->stream);
   if (e != hipSuccess) return fail(c, CPI_ERR_HIP, hipGetErrorString(e));
   // nodes of no element keep what the caller's arrays hold
   double *out[2] = {strain, stress};
@@ -1003,11 +1130,11 @@ extern "C" int cpi_get_stress_strain(cpi_ctx *c, double *strain, double *stress)
   for (double *o : out)
     if (o)
       for (int32_t n : c->loose) keep.insert(keep.end(), o + 6L * n, o + 6L * n + 6);
-  for (int k = 0; k < 2; k++)
-    if (out[k])
-      HIPCHK(c, hipMemcpyAsync(out[k], c->d_tmp + k * n6, sizeof(double) * n6,
-                               hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
+  Piece p[2];
+  int k = 0;
+  if (strain) p[k++] = Piece{strain, n6};
+  if (stress) p[k++] = Piece{stress, n6};
+  if ((rc = bring_back(c, p, k))) return rc;
   const double *was = keep.data();
   for (double *o : out)
     if (o)
@@ -1021,8 +1148,8 @@ extern "C" int cpi_get_stress_strain(cpi_ctx *c, double *strain, double *stress)
 extern "C" int cpi_get_energy(cpi_ctx *c, double *row, int64_t *step) {
   if (!c || !row) return CPI_ERR_INVALID;
   Ctl h;
-  HIPCHK(c, hipMemcpyAsync(&h, c->P.ctl, sizeof(Ctl), hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
+  int rc = get_ctl(c, &h);
+  if (rc) return rc;
   std::memcpy(row, h.row, sizeof(double) * CPI_NENERGY);
   if (step) *step = h.step;
   return CPI_OK;
@@ -1031,8 +1158,8 @@ extern "C" int cpi_get_energy(cpi_ctx *c, double *row, int64_t *step) {
 extern "C" int cpi_get_energy_history(cpi_ctx *c, double *rows, int32_t cap, int32_t *count) {
   if (!c || !count || cap < 0) return CPI_ERR_INVALID;
   Ctl h;
-  HIPCHK(c, hipMemcpyAsync(&h, c->P.ctl, sizeof(Ctl), hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
+  int rc = get_ctl(c, &h);
+  if (rc) return rc;
   const int64_t have = std::min<int64_t>(h.nrows, c->P.hist_cap);
   const int64_t n = std::min<int64_t>(have, cap);
   std::vector<double> all(8 * (size_t)c->P.hist_cap);

@@ -1189,10 +1189,13 @@ __global__ void __launch_bounds__(256) k_stress_node(Params p, const int32_t *la
     de[4] += dn[2] * u[i][1] + dn[1] * u[i][2];
     de[5] += dn[2] * u[i][0] + dn[0] * u[i][2];
   }
-  double *o = strain + 6L * node;
+  if (strain) {
+    double *o = strain + 6L * node;
 #pragma unroll
-  for (int c = 0; c < 6; c++) o[c] = de[c];
-  o = stress + 6L * node;
+    for (int c = 0; c < 6; c++) o[c] = de[c];
+  }
+  if (!stress) return;
+  double *o = stress + 6L * node;
   o[0] = p.c11 * de[0] + p.c12 * (de[1] + de[2]);
   o[1] = p.c11 * de[1] + p.c12 * (de[0] + de[2]);
   o[2] = p.c11 * de[2] + p.c12 * (de[0] + de[1]);
@@ -1280,6 +1283,93 @@ __global__ void __launch_bounds__(256) k_debug_strain(Params p, double alpha, in
     out[2 * blockIdx.x] = red[0] + red[2] + red[4] + red[6];
     out[2 * blockIdx.x + 1] = red[1] + red[3] + red[5] + red[7];
   }
+}
+
+// ---------------------------------------------------------------------------
+// host layouts: user-order [N][3] arrays to and from the device's node
+// records, user-order element state from the device's structure of arrays.
+// One thread per double of the host array, so the host side is contiguous
+// across a wave and the records are gathered 24 bytes at a time; permuting on
+// the host cost several passes over fresh host pages per array.
+// ---------------------------------------------------------------------------
+__global__ void __launch_bounds__(256) k_import_nodes(const double *src, const int32_t *ninv,
+                                                      int nn, Vec3 *d3, Node4 *d4) {
+  const long i = (long)blockIdx.x * 256 + threadIdx.x;
+  if (i >= 3L * nn) return;
+  const int n = (int)(i / 3), c = (int)(i - 3L * n);
+  const long g = ninv[n];
+  const double v = src[i];
+  if (d3) reinterpret_cast<double *>(d3)[3 * g + c] = v;
+  if (d4) {
+    reinterpret_cast<double *>(d4)[4 * g + c] = v;
+    if (c == 0) d4[g].w = 0.0;
+  }
+}
+
+// ctl: a copy of the control block, so one transfer brings it along
+__global__ void __launch_bounds__(256) k_export_nodes(Params p, const int32_t *ninv, NodeExport o) {
+  const long i = (long)blockIdx.x * 256 + threadIdx.x;
+  constexpr int words = sizeof(Ctl) / 8;
+  if (blockIdx.x == 0 && threadIdx.x < words && o.ctl)
+    reinterpret_cast<uint64_t *>(o.ctl)[threadIdx.x] =
+        reinterpret_cast<const uint64_t *>(p.ctl)[threadIdx.x];
+  if (i >= 3L * p.nn) return;
+  const int n = (int)(i / 3), c = (int)(i - 3L * n);
+  const long g = ninv[n];
+  if (o.x) o.x[i] = reinterpret_cast<const double *>(p.pos)[3 * g + c];
+  double v = 0.0, a = 0.0;
+  if (o.v || o.vi) v = reinterpret_cast<const double *>(p.vv)[3 * g + c];
+  if (o.a || o.vi) a = reinterpret_cast<const double *>(p.acc)[4 * g + c];
+  if (o.v) o.v[i] = v;
+  if (o.a) o.a[i] = a;
+  if (o.vi) {
+    // v_n = v_{n+1/2} - dt/2 a_n, product and difference rounded apart
+    const double h = o.half_dt * a;
+    o.vi[i] = v - h;
+  }
+  if (o.m && c == 0) o.m[n] = p.m[g];
+  if (o.m3) o.m3[i] = p.m[g];
+}
+
+template <typename R>
+__global__ void __launch_bounds__(256) k_export_elems(Params p, const int32_t *einv, double *sig,
+                                                      double *ep) {
+  const long i = (long)blockIdx.x * 256 + threadIdx.x, ne = p.ne;
+  const int w = 6 * p.nq;
+  if (sig && i < ne * w) {
+    const long e = i / w;
+    sig[i] = double(static_cast<const R *>(p.sig)[(i - e * w) * ne + einv[e]]);
+  }
+  if (ep && i < ne * p.nq) {
+    const long e = i / p.nq;
+    ep[i] = double(static_cast<const R *>(p.epbar)[(i - e * p.nq) * ne + einv[e]]);
+  }
+}
+
+// x = X0, v = v0, forces, du and a zeroed
+__global__ void __launch_bounds__(256) k_reset_nodes(Params p, const Vec3 *v0) {
+  const int g = blockIdx.x * 256 + threadIdx.x;
+  if (g >= p.nn) return;
+  const Node4 x = p.X0[g];
+  p.pos[g] = Vec3{x.x, x.y, x.z};
+  p.vv[g] = v0[g];
+  p.xprev[g] = Node4{x.x, x.y, x.z, 0.0};
+  p.acc[g] = Node4{0.0, 0.0, 0.0, 0.0};
+  p.du[g] = Node4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+  for (int c = 0; c < 3; c++) p.f[c][g] = 0.0;
+}
+
+// the smallest positive mass, one value per workgroup (1e300: none)
+__global__ void __launch_bounds__(256) k_mass_min(const double *m, int nn, double *out) {
+  __shared__ double red[4];
+  double v = 1e300;
+  for (int i = blockIdx.x * 256 + threadIdx.x; i < nn; i += (int)gridDim.x * 256)
+    if (m[i] > 0.0) v = fmin(v, m[i]);
+  v = wave_min(v);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+  __syncthreads();
+  if (threadIdx.x == 0) out[blockIdx.x] = fmin(fmin(red[0], red[1]), fmin(red[2], red[3]));
 }
 
 // ---------------------------------------------------------------------------
@@ -1642,6 +1732,31 @@ hipError_t launch_elem_dt(const Params &p, double *out, hipStream_t s) {
   const int grid = (p.ne + 255) / 256;
   if (p.npe == 4) CPI_LAUNCH(k_elem_dt<4>, grid, 256, 0, s, p, out);
   CPI_LAUNCH(k_elem_dt<10>, grid, 256, 0, s, p, out);
+}
+
+hipError_t launch_import_nodes(const double *src, const int32_t *ninv, int nn, Vec3 *d3, Node4 *d4,
+                               hipStream_t s) {
+  CPI_LAUNCH(k_import_nodes, (unsigned)((3L * nn + 255) / 256), 256, 0, s, src, ninv, nn, d3, d4);
+}
+
+hipError_t launch_export_nodes(const Params &p, const int32_t *ninv, const NodeExport &o,
+                               hipStream_t s) {
+  CPI_LAUNCH(k_export_nodes, (unsigned)((3L * p.nn + 255) / 256), 256, 0, s, p, ninv, o);
+}
+
+hipError_t launch_export_elems(const Params &p, int prec, const int32_t *einv, double *sig,
+                               double *ep, hipStream_t s) {
+  const unsigned grid = (unsigned)(((long)p.ne * p.nq * (sig ? 6 : 1) + 255) / 256);
+  if (prec == 1) CPI_LAUNCH(k_export_elems<float>, grid, 256, 0, s, p, einv, sig, ep);
+  CPI_LAUNCH(k_export_elems<double>, grid, 256, 0, s, p, einv, sig, ep);
+}
+
+hipError_t launch_reset_nodes(const Params &p, const Vec3 *v0, hipStream_t s) {
+  CPI_LAUNCH(k_reset_nodes, (p.nn + 255) / 256, 256, 0, s, p, v0);
+}
+
+hipError_t launch_mass_min(const Params &p, double *out, int blocks, hipStream_t s) {
+  CPI_LAUNCH(k_mass_min, blocks, 256, 0, s, (const double *)p.m, p.nn, out);
 }
 
 hipError_t launch_stress_node(const Params &p, const int32_t *last, double *strain,

@@ -242,12 +242,12 @@ class Dynamics:
     def fetch(self):
         """Downloads x, v (v_{n+1/2}), a_n, mass and v_n into the host arrays."""
         n = self.mesh.num_nodes
-        x, v, a, vi = (np.zeros((n, 3)) for _ in range(4))
-        m = np.zeros(n)
-        L.check(L.lib().cpi_get_state(self.ctx, L.dptr(x), L.dptr(v), L.dptr(a), L.dptr(m),
-                                      L.dptr(vi)), self.ctx)
+        x, v, a, vi, m3 = (np.empty((n, 3)) for _ in range(5))
+        m = np.empty(n)
+        L.check(L.lib().cpi_get_state_mass3(self.ctx, L.dptr(x), L.dptr(v), L.dptr(a), L.dptr(m),
+                                            L.dptr(vi), L.dptr(m3)), self.ctx)
         self.global_xloc, self.vel, self.global_acc, self.vel_i = x, v, a, vi
-        self.global_mass = np.repeat(m[:, None], 3, axis=1)
+        self.global_mass = m3
         return x, v, a, m, vi
 
     def stress_strain(self):

@@ -59,7 +59,8 @@ typedef enum cpi_status {
 
 /* nodal force assembly */
 #define CPI_SCATTER_BLOCK 0  /* workgroup-local LDS assembly, deterministic */
-#define CPI_SCATTER_COLOR 1  /* greedy element colouring, one pass per colour */
+#define CPI_SCATTER_COLOR 1  /* greedy element colouring: forces summed in colour
+                                order, reproducible */
 #define CPI_SCATTER_ATOMIC 2 /* FP64 global atomics (order not reproducible) */
 
 /* quadrature (tetrahedral.h:7-74) */
@@ -243,6 +244,11 @@ int cpi_synchronize(cpi_ctx *ctx);
    global_mass (one value per node) and vel_i (v_n).  Any pointer may be NULL. */
 int cpi_get_state(cpi_ctx *ctx, double *x, double *v, double *a, double *m,
                   double *v_i);
+
+/* cpi_get_state and the mass of every node once per component, m3
+   [num_nodes][3], as Dynamics::global_mass holds it. */
+int cpi_get_state_mass3(cpi_ctx *ctx, double *x, double *v, double *a, double *m,
+                        double *v_i, double *m3);
 
 /* du of the last completed step [num_nodes][3] (Dynamics::global_dof,
    dynamics.h:473-476); zeros before the first step. */

@@ -38,3 +38,38 @@ def test_nodal_stress_takes_the_last_element_and_leaves_loose_nodes(quad, scatte
     L.check(L.lib().cpi_get_stress_strain(d.ctx, L.dptr(only), None), d.ctx)
     assert np.array_equal(only[:-1], st[:-1])
     d.close()
+
+
+@pytest.mark.parametrize("n,scatter", [(3, L.SCATTER_BLOCK), (3, L.SCATTER_COLOR),
+                                       (24, L.SCATTER_BLOCK), (66, L.SCATTER_ATOMIC)])
+def test_state_goes_in_and_comes_out_in_user_order(n, scatter):
+    """Without wall and gravity nothing moves the initial state, so x, v and
+    v_n come back exactly as set, over the sizes of the one transfer (n = 3),
+    of a ring larger (24) and smaller (66: 38 MB) than the result; the state
+    of a second initial condition replaces the first."""
+    x, conn = cube(n)
+    d = ci.Dynamics(ci.Mesh.from_arrays(x, conn), ci.Elastoplastic(E, RHO, NU, 1.0, 7e8, 2.76e8),
+                    None, physics=L.PHYSICS_EP, scatter=scatter, gravity=(0.0, 0.0, 0.0))
+    for seed in (1, 2):
+        rng = np.random.default_rng(seed)
+        x0 = x + rng.uniform(-1, 1, x.shape) * 1e-3 * 0.25 / n
+        v0 = rng.standard_normal(x.shape)
+        d._x0, d.vel = x0, v0.copy()
+        d.init(1e-9)
+        gx, gv, ga, gm, gvi = d.fetch()
+        assert np.array_equal(gx, x0) and np.array_equal(gv, v0) and np.array_equal(gvi, v0)
+        assert not ga.any() and (gm > 0).all()
+        assert np.array_equal(d.global_mass, np.repeat(gm[:, None], 3, axis=1))
+        du = np.full_like(x, 3.0)
+        L.check(L.lib().cpi_get_increment(d.ctx, L.dptr(du)), d.ctx)
+        assert not du.any()
+        sig, ep = d.element_state()
+        assert not sig.any() and not ep.any()
+    # a refused state leaves the one that was set
+    bad = v0.copy()
+    bad[-1, 2] = np.inf
+    with pytest.raises(L.CpiError) as err:
+        L.check(L.lib().cpi_set_state(d.ctx, L.dptr(x), L.dptr(bad)), d.ctx)
+    assert err.value.code == -1
+    assert np.array_equal(d.fetch()[0], x0)
+    d.close()
