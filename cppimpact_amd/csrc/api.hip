@@ -62,6 +62,11 @@ struct cpi_ctx {
     hipGraphExec_t plain = nullptr, aux = nullptr;
     hipGraphExec_t run[2] = {nullptr, nullptr};
   } gs;
+  // resident steps (k_resident): usable, and the steps taken that way
+  Resident res{};
+  size_t res_smem = 0;
+  bool resident = false;
+  bool res_pending = false;  // launched since the control block was last read
   bool mass_ready = false, inited = false;
   double dt = 0.0;
   int64_t step = 0;
@@ -327,6 +332,10 @@ int enqueue_step(cpi_ctx *c, bool aux) {
 // steps (measured at c2: ≈ 4 µs less per step than one graph per step)
 constexpr int kGraphRuns[2] = {32, 4};
 
+// fewest plain steps of a call that go through the resident kernel: its
+// cooperative launch and first loads cost as much as a few steps
+constexpr int kMinResident = 4;
+
 int capture(cpi_ctx *c, bool aux, hipGraphExec_t *out, int nrep = 1) {
   hipGraph_t g = nullptr;
   HIPCHK(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
@@ -440,9 +449,42 @@ int report_flags(cpi_ctx *c, const Ctl &h) {
   return CPI_OK;
 }
 
+int steps_one_by_one(cpi_ctx *c, int64_t nsteps);
+
+// Steps that resident launches missed are taken now, one launch per kernel of
+// a step: the state does not depend on how its steps were launched, only on
+// their number.  h: the control block as read after the launches.
+int settle(cpi_ctx *c, const Ctl &h) {
+  c->res_pending = false;
+  if (!(h.decision & 1u)) return CPI_OK;
+  c->resident = false;
+  int rc = steps_one_by_one(c, h.missed);
+  if (rc) return rc;
+  // no launch reads these again; a later call must not settle twice
+  HIPCHK(c, hipMemsetAsync(&c->P.ctl->decision, 0, sizeof(uint32_t), c->stream));
+  HIPCHK(c, hipMemsetAsync(&c->P.ctl->missed, 0, sizeof(int64_t), c->stream));
+  HIPCHK(c, hipStreamSynchronize(c->stream));
+  return CPI_OK;
+}
+
+// the control block after all steps asked for
+int settled_ctl(cpi_ctx *c, Ctl *h) {
+  int rc = get_ctl(c, h);
+  if (rc || !c->res_pending) return rc;
+  const bool missed = h->decision & 1u;
+  if ((rc = settle(c, *h))) return rc;
+  return missed ? get_ctl(c, h) : CPI_OK;
+}
+
+// before results are read by other ways than the control block
+int settled(cpi_ctx *c) {
+  Ctl h;
+  return c->res_pending ? settled_ctl(c, &h) : CPI_OK;
+}
+
 int check_flags(cpi_ctx *c) {
   Ctl h;
-  int rc = get_ctl(c, &h);
+  int rc = settled_ctl(c, &h);
   return rc ? rc : report_flags(c, h);
 }
 
@@ -806,6 +848,29 @@ static int create_impl(cpi_ctx *c, const cpi_mesh_desc *m, const cpi_material *m
     if (pe != hipSuccess)
       return fail(c, CPI_ERR_HIP, std::string("LDS opt-in for the element kernel: ") +
                                       hipGetErrorString(pe));
+    // resident steps when every block fits the chip at once
+    if (opt->use_graph && c->phys != 2 && words && prop.cooperativeLaunch) {
+      const MailPlan M = build_mail(B);
+      const size_t n = M.dest.size(), bytes = mail_bytes(c->prec, n);
+      const size_t smem = resident_smem(c->smem, c->prec, M.most);
+      if (bytes <= (size_t)INT32_MAX && M.most <= 65535 && smem <= (size_t)prop.sharedMemPerBlock &&
+          B.nblocks <= resident_capacity(npe, c->rule, c->prec, c->phys, smem,
+                                         prop.multiProcessorCount)) {
+        char *mail = nullptr;
+        int32_t *mf, *mlo, *md;
+        uint16_t *ms, *mi;
+        if ((rc = dalloc(c, &mail, bytes)) || (rc = dalloc(c, &mf, M.first.size())) ||
+            (rc = upload(c, mf, M.first)) || (rc = dalloc(c, &mlo, M.lo.size())) ||
+            (rc = upload(c, mlo, M.lo)) || (rc = dalloc(c, &md, n)) || (rc = upload(c, md, M.dest)) ||
+            (rc = dalloc(c, &ms, n)) || (rc = upload(c, ms, M.src)) || (rc = dalloc(c, &mi, n)) ||
+            (rc = upload(c, mi, M.idx)))
+          return rc;
+        c->res = Resident{mail, (int)n, M.most, mf, md, ms, mlo, mi, 0, 0, 0,
+                          opt->debug_fill_nan & 2 ? 1u : 1u << 20};
+        c->res_smem = smem;
+        c->resident = true;
+      }
+    }
     // one energy row per wave
     c->n_elem_rows = c->nblocks * (elem_block_threads(npe, c->rule) / 64);
     c->n_node_rows = 4 * std::max(1, (B.n_boundary + 255) / 256);
@@ -902,6 +967,7 @@ extern "C" int cpi_set_state(cpi_ctx *c, const double *x0, const double *v0) {
   if (v0 && !all_finite(v0, n)) return fail(c, CPI_ERR_INVALID, "non-finite velocity");
   if (x0) c->mass_ready = false;
   c->inited = false;
+  c->res_pending = false;
   int rc = x0 ? put_nodes(c, x0, nullptr, c->P.X0) : CPI_OK;
   if (!rc && v0) rc = put_nodes(c, v0, c->d_V0, nullptr);
   return rc ? rc : reset_state(c);
@@ -914,7 +980,8 @@ extern "C" int cpi_stable_dt(cpi_ctx *c, double *dte, double *dtc) {
     if (!rc && !c->mass_ready) rc = compute_mass(c);
     if (rc) return rc;
   }
-  return stable_dt(c, dte, dtc);
+  int rc = settled(c);
+  return rc ? rc : stable_dt(c, dte, dtc);
 }
 
 // ---------------------------------------------------------------------------
@@ -961,7 +1028,8 @@ extern "C" int cpi_stable_dt_noalloc(cpi_ctx *c, double *dte, double *dtc) {
                 "cpi_stable_dt_noalloc: at most " + std::to_string(256L * kNoallocPartials) +
                     " elements (the mesh has " + std::to_string(c->ne) + ")");
   double *sp = nullptr;
-  int rc = scratch_of(c, &sp);
+  int rc = settled(c);
+  if (!rc) rc = scratch_of(c, &sp);
   if (rc) return rc;
   HIPCHK(c, launch_elem_dt(c->P, sp, c->stream));
   HIPCHK(c, launch_dt_finish(sp, nb, c->P.m, c->nn, sp + kNoallocPartials, c->stream));
@@ -980,6 +1048,7 @@ extern "C" int cpi_init(cpi_ctx *c, double dt) {
   if (c->phys == 2 && !c->mlp.ready)
     return fail(c, CPI_ERR_STATE, "cpi_init: CPI_RETURN_MLP needs cpi_set_surrogate first");
   c->inited = false;
+  c->res_pending = false;  // steps of a state that is given up
   int rc = reset_state(c);
   if (!rc) rc = compute_mass(c);
   if (rc) return rc;
@@ -1004,6 +1073,11 @@ extern "C" int cpi_init(cpi_ctx *c, double dt) {
   if (e == hipSuccess) e = launch_energy_reduce(c->P, c->stream);
   if (e != hipSuccess) return fail(c, CPI_ERR_HIP, std::string("init kernels: ") + hipGetErrorString(e));
   HIPCHK(c, hipMemsetAsync(c->P.epart, 0, sizeof(double) * EP_N * c->n_rows, c->stream));
+  if (c->resident) {
+    c->res.base = 0;
+    c->res.launch = 0;
+    HIPCHK(c, launch_mail_clear(c->res, c->prec, c->stream));
+  }
   HIPCHK(c, hipStreamSynchronize(c->stream));
   // the step graphs hold the context's buffers, which a new initial state
   // does not change; what does change the launches drops them
@@ -1019,7 +1093,35 @@ extern "C" int cpi_step(cpi_ctx *c, int32_t nsteps) {
   if (!c) return CPI_ERR_INVALID;
   if (!c->inited) return fail(c, CPI_ERR_STATE, "cpi_step before cpi_init");
   if (nsteps < 0) return fail(c, CPI_ERR_INVALID, "nsteps < 0");
-  for (int i = 0; i < nsteps;) {
+  int64_t rest = nsteps;
+  // the plain steps in one launch (the last step of a call is the one with
+  // the energies and outputs)
+  if (c->resident && c->gs.plain && !c->P.samples && nsteps - 1 >= kMinResident) {
+    c->res.steps = nsteps - 1;
+    c->res.launch++;
+    Params p = c->P;
+    p.epart_base = 0;
+    const hipError_t e = launch_resident(p, c->rule, c->prec, c->phys, c->res, c->nblocks,
+                                         c->res_smem, c->stream);
+    if (e == hipSuccess) {
+      c->res.base ^= c->res.steps & 1;
+      c->res_pending = true;
+      rest = 1;
+    } else {
+      (void)hipGetLastError();
+      c->resident = false;  // the per-step launches from here on
+    }
+  }
+  int rc = steps_one_by_one(c, rest);
+  if (rc) return rc;
+  c->step += nsteps;
+  return CPI_OK;
+}
+
+namespace {
+// nsteps steps in the stream, from the step graphs or kernel by kernel
+int steps_one_by_one(cpi_ctx *c, int64_t nsteps) {
+  for (int64_t i = 0; i < nsteps;) {
     const bool aux = (i == nsteps - 1);
     const auto &G = c->gs;
     if (G.plain) {
@@ -1037,9 +1139,9 @@ extern "C" int cpi_step(cpi_ctx *c, int32_t nsteps) {
     }
     i++;
   }
-  c->step += nsteps;
   return CPI_OK;
 }
+}  // namespace
 
 extern "C" int cpi_synchronize(cpi_ctx *c) {
   if (!c) return CPI_ERR_INVALID;
@@ -1078,13 +1180,20 @@ extern "C" int cpi_get_state_mass3(cpi_ctx *c, double *x, double *v, double *a, 
   o.half_dt = 0.5 * c->dt;
   HIPCHK(c, launch_export_nodes(c->P, c->d_ninv, o, c->stream));
   if ((rc = bring_back(c, p, k))) return rc;
+  if (c->res_pending && (h.decision & 1u)) {
+    if ((rc = settle(c, h))) return rc;
+    HIPCHK(c, launch_export_nodes(c->P, c->d_ninv, o, c->stream));
+    if ((rc = bring_back(c, p, k))) return rc;
+  }
+  c->res_pending = false;
   return c->inited ? report_flags(c, h) : CPI_OK;
 }
 
 extern "C" int cpi_get_increment(cpi_ctx *c, double *du) {
   if (!c || !du) return CPI_ERR_INVALID;
   const size_t n3 = 3 * (size_t)c->nn;
-  int rc = ensure_tmp(c, n3);
+  int rc = settled(c);
+  if (!rc) rc = ensure_tmp(c, n3);
   if (rc) return rc;
   Params p = c->P;
   p.acc = c->P.du;
@@ -1103,7 +1212,8 @@ extern "C" int cpi_get_element_state(cpi_ctx *c, double *sig, double *ep) {
     if (ep) std::memset(ep, 0, sizeof(double) * n);
     return CPI_OK;
   }
-  int rc = ensure_tmp(c, (sig ? 6 * n : 0) + (ep ? n : 0));
+  int rc = settled(c);
+  if (!rc) rc = ensure_tmp(c, (sig ? 6 * n : 0) + (ep ? n : 0));
   if (rc) return rc;
   Piece p[2];
   int k = 0;
@@ -1119,7 +1229,8 @@ extern "C" int cpi_get_stress_strain(cpi_ctx *c, double *strain, double *stress)
   if (!c) return CPI_ERR_INVALID;
   if (!c->inited) return fail(c, CPI_ERR_STATE, "cpi_get_stress_strain before cpi_init");
   const size_t n6 = 6 * (size_t)c->nn;
-  int rc = ensure_tmp(c, 2 * n6);
+  int rc = settled(c);
+  if (!rc) rc = ensure_tmp(c, 2 * n6);
   if (rc) return rc;
   hipError_t e = launch_stress_node(c->P, c->d_last, strain ? c->d_tmp : nullptr,
                                     stress ? c->d_tmp + (strain ? n6 : 0) : nullptr, c->stream);
@@ -1148,7 +1259,7 @@ extern "C" int cpi_get_stress_strain(cpi_ctx *c, double *strain, double *stress)
 extern "C" int cpi_get_energy(cpi_ctx *c, double *row, int64_t *step) {
   if (!c || !row) return CPI_ERR_INVALID;
   Ctl h;
-  int rc = get_ctl(c, &h);
+  int rc = settled_ctl(c, &h);
   if (rc) return rc;
   std::memcpy(row, h.row, sizeof(double) * CPI_NENERGY);
   if (step) *step = h.step;
@@ -1158,7 +1269,7 @@ extern "C" int cpi_get_energy(cpi_ctx *c, double *row, int64_t *step) {
 extern "C" int cpi_get_energy_history(cpi_ctx *c, double *rows, int32_t cap, int32_t *count) {
   if (!c || !count || cap < 0) return CPI_ERR_INVALID;
   Ctl h;
-  int rc = get_ctl(c, &h);
+  int rc = settled_ctl(c, &h);
   if (rc) return rc;
   const int64_t have = std::min<int64_t>(h.nrows, c->P.hist_cap);
   const int64_t n = std::min<int64_t>(have, cap);
@@ -1507,7 +1618,9 @@ extern "C" int cpi_samples_enable(cpi_ctx *c, int32_t cap) {
     return fail(c, CPI_ERR_STATE, "cpi_samples_enable: needs CPI_PHYSICS_EP with the exact return");
   HIPCHK(c, hipSetDevice(c->dev));
   HIPCHK(c, hipStreamSynchronize(c->stream));
-  int rc = mlp_samples_alloc(c->mlp, cap, c->stream, c->err);
+  int rc = settled(c);
+  if (rc) return rc;
+  rc = mlp_samples_alloc(c->mlp, cap, c->stream, c->err);
   if (rc) return rc;
   c->P.samples = c->mlp.d_samples;
   c->P.sample_count = c->mlp.d_sample_count;

@@ -31,7 +31,13 @@ struct Ctl {
   int64_t nrows;   // energy rows written to the history ring
   uint32_t flags;  // bit 0: non-finite energy, bit 1: inverted element,
                    // bit 2: dt above the stable limit of the configuration
-  uint32_t pad;
+  // resident launches, numbered from 1: decision is 2 L once launch L has
+  // stored its steps, 2 L + 1 if it gave up, and then no later one runs;
+  // finished counts the workgroups that reached the end, missed the steps of
+  // the launches that did not run
+  uint32_t decision;
+  uint64_t finished;
+  int64_t missed;
   double e0;       // KE + Epen of the initial state
   double row[8];   // latest energy row (CPI_E_* order)
   double dt_contact;  // wall-spring limit 2 sqrt(m_min / k) (fixed: mass is)
@@ -148,6 +154,21 @@ struct Params {
   // element, point) is below sample_keep (2^32: every point)
   unsigned long long sample_keep;
   unsigned long long sample_seed;
+};
+
+// arguments of the resident steps besides Params (see k_resident); the
+// message tables are build_mail's
+struct Resident {
+  void *mail;           // [2][messages] records (MailRec)
+  int messages, most;   // all, and the most of one block
+  const int32_t *first; // per block, nblocks + 1: its first message
+  const int32_t *dest;  // per message: the receiver's message it is posted to
+  const uint16_t *src;  // per message: the local node it is of
+  const int32_t *lo;    // [nblocks][ml]: start of a shared node's list in idx
+  const uint16_t *idx;  // lists of the block's messages per node, in slot order
+  int base, steps;      // inbox of the first step, steps to take
+  unsigned launch;      // number of the launch (Ctl::decision)
+  unsigned spin_limit;  // polls of one wait before it gives up
 };
 
 // ---------------------------------------------------------------------------

@@ -464,6 +464,80 @@ bool build_block_plan(int ne, int npe, const int32_t *conn, int nn,
   return true;
 }
 
+MailPlan build_mail(const BlockPlan &P) {
+  MailPlan M;
+  const int nb = P.nblocks, ml = P.max_local_nodes, ns = P.n_slots;
+  // the block and local node of every partial slot, messages per block
+  std::vector<int32_t> blk(ns), loc(ns);
+  for (int b = 0; b < nb; b++)
+    for (int l = 0; l < ml; l++) {
+      const int s = P.slot_pad[(size_t)b * ml + l];
+      if (s < 0) continue;
+      blk[s] = b;
+      loc[s] = l;
+    }
+  M.first.assign((size_t)nb + 1, 0);
+  std::vector<int32_t> count(nb, 0), shared_ptr(nb + 1, 0);
+  std::vector<size_t> pair(P.n_boundary + 1, 0);  // a node's (slot, other slot) pairs
+  for (int i = 0; i < P.n_boundary; i++) {
+    const int s0 = P.slot_ptr[i], s1 = P.slot_ptr[i + 1];
+    pair[i + 1] = pair[i] + (size_t)(s1 - s0) * (s1 - s0);
+    for (int s = s0; s < s1; s++) {
+      count[blk[s]] += s1 - s0 - 1;
+      shared_ptr[blk[s] + 1]++;
+    }
+  }
+  for (int b = 0; b < nb; b++) {
+    M.first[b + 1] = M.first[b] + count[b];
+    M.most = std::max(M.most, count[b]);
+    shared_ptr[b + 1] += shared_ptr[b];
+  }
+  // the shared nodes of every block, ascending
+  std::vector<int32_t> shared(ns), own(ns), fill(shared_ptr.begin(), shared_ptr.end() - 1);
+  for (int i = 0; i < P.n_boundary; i++)
+    for (int s = P.slot_ptr[i]; s < P.slot_ptr[i + 1]; s++) {
+      own[fill[blk[s]]] = s;
+      shared[fill[blk[s]]++] = i;
+    }
+  // With the other blocks c taken in order and their nodes in order, every
+  // block's messages come out grouped by c and in node order.
+  const size_t n = M.first[nb];
+  M.dest.resize(n);
+  M.src.resize(n);
+  M.idx.resize(n);
+  M.lo.assign((size_t)nb * ml, 0);
+  std::vector<int32_t> at(pair[P.n_boundary]), next(M.first.begin(), M.first.end() - 1);
+  for (int c = 0; c < nb; c++)
+    for (int k = shared_ptr[c]; k < shared_ptr[c + 1]; k++) {
+      const int i = shared[k], r = own[k], s0 = P.slot_ptr[i], s1 = P.slot_ptr[i + 1];
+      for (int s = s0; s < s1; s++)
+        if (s != r) {
+          const int m = next[blk[s]]++;
+          M.src[m] = (uint16_t)loc[s];
+          at[pair[i] + (size_t)(s - s0) * (s1 - s0) + (r - s0)] = m;
+        }
+    }
+  // a message lands where the other block lists the same pair; a node's
+  // messages in slot order
+  for (int b = 0; b < nb; b++) {
+    int off = 0;
+    for (int l = 0; l < ml; l++) {
+      const int s = P.slot_pad[(size_t)b * ml + l];
+      if (s < 0) continue;
+      const int i = P.nid_pad[(size_t)b * ml + l] - P.n_interior;
+      const int s0 = P.slot_ptr[i], k = P.slot_ptr[i + 1] - s0;
+      M.lo[(size_t)b * ml + l] = off;
+      for (int r = 0; r < k; r++) {
+        if (s0 + r == s) continue;
+        const int32_t m = at[pair[i] + (size_t)(s - s0) * k + r];
+        M.dest[m] = at[pair[i] + (size_t)r * k + (s - s0)];
+        M.idx[M.first[b] + off++] = (uint16_t)(m - M.first[b]);
+      }
+    }
+  }
+  return M;
+}
+
 }  // namespace cpi
 
 using namespace cpi;

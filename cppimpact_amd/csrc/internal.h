@@ -65,6 +65,21 @@ bool build_block_plan(int ne, int npe, const int32_t *conn, int nn,
                       const double *xloc, int max_elems, int max_nodes,
                       BlockPlan &plan, std::string &err);
 
+// Messages of the resident steps.  Every two blocks that share a node send
+// each other their partial force on it.  Block b has messages first[b] ..
+// first[b+1], which are at once the ones it posts and its inbox, grouped by the
+// other block and in node order inside a group.  Message m is local node
+// src[m]'s and is posted to the inbox message dest[m]; dest runs on inside a
+// group.  The messages (counted from first[b]) a shared local node l receives,
+// in slot order, are idx[first[b] + lo[b*ml + l]] and on, one per other block
+// holding it.
+struct MailPlan {
+  std::vector<int32_t> first, dest, lo;
+  std::vector<uint16_t> src, idx;
+  int most = 0;  // messages of one block
+};
+MailPlan build_mail(const BlockPlan &plan);
+
 // Corner-force slots of the colour scatter: node n's slots are node_slot[n]
 // .. node_slot[n+1], one per element that holds it, in ascending colour, and
 // corner k of element e writes slot[k * ne + e].  order[e]: the element's

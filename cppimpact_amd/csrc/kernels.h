@@ -24,6 +24,15 @@ hipError_t prepare_elem_block(int npe, int rule, int prec, int phys, size_t smem
 void set_launch_events(hipEvent_t start, hipEvent_t stop);
 hipError_t launch_elem_direct(const Params &p, int rule, int prec, int phys, bool atomic,
                               hipStream_t s);
+// workgroups of the resident kernel the device can hold at once (0: there is
+// none for this combination)
+int resident_capacity(int npe, int rule, int prec, int phys, size_t smem, int cus);
+hipError_t launch_resident(const Params &p, int rule, int prec, int phys, const Resident &rs,
+                           int nblocks, size_t smem, hipStream_t s);
+hipError_t launch_mail_clear(const Resident &rs, int prec, hipStream_t s);
+// LDS of a resident workgroup and bytes of the mail records
+size_t resident_smem(size_t block_smem, int prec, int most);
+size_t mail_bytes(int prec, size_t messages);
 // prec: the element kernel's precision (its partials are stored in it)
 hipError_t launch_node_bnd(const Params &p, int prec, bool aux, hipStream_t s);
 // prec: the corner-force slots' precision (colour scatter)

@@ -125,51 +125,70 @@ __device__ __forceinline__ void wave_flush(const Params &p, int base, const EAcc
 // A held node (fixed set, when enabled) has a = 0 and no contact; its
 // velocity is zero from the start, so it stays where it is.
 // ---------------------------------------------------------------------------
-template <bool AUX>
-__device__ __forceinline__ void node_update(const Params &p, int g, const double f[3],
-                                            const double x[3], const double v[3], double m,
-                                            double dt, EAcc &ea) {
-  double du[3], a[3];
-  const double minv = 1.0 / m;
+struct NodeStep {
+  double x[3], v[3];    // x_{n+1}, v_{n+3/2}
+  double a[3], du[3];
+};
+
+// minv = 1 / m; contact: the wall acts on the node
+__device__ __forceinline__ void node_advance(const Params &p, bool held, bool contact,
+                                             const double f[3], const double x[3],
+                                             const double v[3], double m, double minv, double dt,
+                                             NodeStep &s, EAcc &ea) {
 #pragma unroll
   for (int c = 0; c < 3; c++) {
-    du[c] = dt * v[c];
-    a[c] = (m != 0.0) ? minv * (-f[c]) : 0.0;
+    s.du[c] = dt * v[c];
+    s.a[c] = (m != 0.0) ? minv * (-f[c]) : 0.0;
   }
-  const bool held = p.fixed_mask && p.fixed_mask[g];
-  if (p.wall_on && !held && (!p.contact_mask || p.contact_mask[g])) {
+  if (contact) {
 #pragma unroll
     for (int c = 0; c < 3; c++) {
       if (c == p.wall_dim) {
-        double pos = x[c] + du[c];
+        double pos = x[c] + s.du[c];
         double d = (pos - p.wall_loc) * p.wall_normal;
         if (d < 0.0) {
-          a[c] += -1 * minv * d * p.wall_nk;
+          s.a[c] += -1 * minv * d * p.wall_nk;
           ea.pen += 0.5 * p.wall_k * d * d;
           ea.fc += -p.wall_k * d;
         }
       }
     }
   }
-  double ke = 0.0, wg = 0.0, xn[3], vn[3];
+  double ke = 0.0, wg = 0.0;
 #pragma unroll
   for (int c = 0; c < 3; c++) {
-    a[c] = held ? 0.0 : a[c] + p.grav[c];
-    vn[c] = v[c] + dt * a[c];
-    double vi = vn[c] - 0.5 * dt * a[c];
+    s.a[c] = held ? 0.0 : s.a[c] + p.grav[c];
+    s.v[c] = v[c] + dt * s.a[c];
+    double vi = s.v[c] - 0.5 * dt * s.a[c];
     ke += vi * vi;
-    wg += p.grav[c] * du[c];
-    xn[c] = x[c] + du[c];
-  }
-  p.pos[g] = Vec3{xn[0], xn[1], xn[2]};
-  p.vv[g] = Vec3{vn[0], vn[1], vn[2]};
-  if (AUX) {
-    p.acc[g] = Node4{a[0], a[1], a[2], 0.0};
-    p.du[g] = Node4{du[0], du[1], du[2], 0.0};
-    p.xprev[g] = Node4{x[0], x[1], x[2], m};
+    wg += p.grav[c] * s.du[c];
+    s.x[c] = x[c] + s.du[c];
   }
   ea.ke += 0.5 * m * ke;
   ea.wgrav += m * wg;
+}
+
+__device__ __forceinline__ bool node_held(const Params &p, int g) {
+  return p.fixed_mask && p.fixed_mask[g];
+}
+__device__ __forceinline__ bool node_contact(const Params &p, int g, bool held) {
+  return p.wall_on && !held && (!p.contact_mask || p.contact_mask[g]);
+}
+
+template <bool AUX>
+__device__ __forceinline__ void node_update(const Params &p, int g, const double f[3],
+                                            const double x[3], const double v[3], double m,
+                                            double dt, EAcc &ea) {
+  const bool held = node_held(p, g);
+  NodeStep s;
+  node_advance(p, held, node_contact(p, g, held), f, x, v, m, 1.0 / m, dt, s, ea);
+  p.pos[g] = Vec3{s.x[0], s.x[1], s.x[2]};
+  p.vv[g] = Vec3{s.v[0], s.v[1], s.v[2]};
+  if (AUX) {
+    p.acc[g] = Node4{s.a[0], s.a[1], s.a[2], 0.0};
+    p.du[g] = Node4{s.du[0], s.du[1], s.du[2], 0.0};
+    p.xprev[g] = Node4{x[0], x[1], x[2], m};
+  }
 }
 
 // N consecutive corner forces of local node j, ranks k..k+N-1 (k a multiple
@@ -805,6 +824,366 @@ __global__ void __launch_bounds__(256) k_node_bnd(Params p) {
     p.ctl->step += 1;
     if (p.mlp_ctr) *p.mlp_ctr = 0ull;
   }
+}
+
+// ---------------------------------------------------------------------------
+// Resident steps: many steps of a mesh whose element blocks all fit the chip
+// at once, in one launch.
+//
+// A small mesh spends its step on two launches and on the loads behind them
+// (a 16-block mesh: 5.6 + 4.5 us for 0.7 MB that sits in the caches).  Here
+// every block keeps its elements' stress state in registers and its node
+// records in LDS from the first step to the last, and only the partial forces
+// of shared nodes travel between blocks.
+//
+// Exchange.  A block posts its partial force on a shared node to every other
+// block that holds the node, one message each, into the receiver's inbox
+// (build_mail); each receiver adds the node's partials in slot order
+// (k_node_bnd's order) and updates its own copy of the node, so all copies
+// stay the same bits and no second launch, flag or grid barrier is needed.
+// The messages between two blocks lie together, in the same order on both
+// sides, and message m is posted and read by thread m of its block, so posts
+// and inbox reads coalesce into whole lines: they are written and read past
+// the XCDs' L2s (agent scope, sc1), where every transaction counts.  An empty
+// message holds a NaN with a payload no arithmetic makes (MailRec::empty) in
+// every word: the data is its own flag, word by word.  The reader empties a
+// message as soon as it has it.  Steps alternate between two inboxes: the
+// writer fills one again two steps later, after it has received the reader's
+// message for the same node of the step between, which the reader posted
+// after the emptying store completed (every thread waits for its stores
+// before the barrier ahead of the posts).  A launch starts at the inbox after
+// the last one's (base).
+//
+// All blocks have to run at once: a cooperative launch sized by
+// resident_capacity.  Should some not get to run all the same (another
+// process's kernels hold the chip), nothing hangs and nothing is lost: past
+// spin_limit polls a thread decides that the launch gives up
+// (Ctl::decision), and every block leaves without storing anything.  The
+// blocks store their state only after the last of them to finish has decided
+// that the launch counts, so a launch takes all its steps or none; the host
+// takes missed steps with the per-step kernels (settled_ctl).
+//
+// Same arithmetic in the same order as the per-step kernels: same state
+// bits.  The cumulative energies are summed over the steps per lane and over
+// the lanes once at the end, shared nodes' by the block of their first slot.
+//
+// Per step (MI355X; before: the two launches): 6,000 tet4 8.9 -> 5.0 us
+// (FP64), 8.7 -> 4.6 (FP32); 196,608 tet4 12.2 -> 7.9, 10.6 -> 6.5; 48,000 tet10
+// 17.2 -> 13, 13.8 -> 8.5.  What is left is the element pass and node sums
+// (3.9 us for 16 blocks, 4.8 for 512) and one trip of the mail.
+// ---------------------------------------------------------------------------
+typedef unsigned mail4 __attribute__((ext_vector_type(4)));
+typedef unsigned mail2 __attribute__((ext_vector_type(2)));
+constexpr int kSc1 = 16;  // cache policy bit of the buffer builtins
+
+// Message records, n of them: 16 bytes (x, y, z, unused) for FP32 partials;
+// for FP64 ones (x, y) in 16 bytes and, past the n of those, z in 8.  Each word
+// is an aligned 4- or 8-byte part of one store.
+template <typename R> struct MailRec;
+template <> struct MailRec<float> {
+  static constexpr int bytes = 16;
+  static constexpr unsigned empty = 0xffc0deadu, nan = 0x7fc00000u;
+  __device__ static unsigned bits(float v) {
+    const unsigned w = __float_as_uint(v);
+    return w == empty ? nan : w;
+  }
+  __device__ static void put(__amdgpu_buffer_rsrc_t m, int, int i, const float f[3]) {
+    const mail4 w = {bits(f[0]), bits(f[1]), bits(f[2]), 0u};
+    __builtin_amdgcn_raw_buffer_store_b128(w, m, 16 * i, 0, kSc1);
+  }
+  __device__ static void clear(__amdgpu_buffer_rsrc_t m, int, int i) {
+    const mail4 w = {empty, empty, empty, empty};
+    __builtin_amdgcn_raw_buffer_store_b128(w, m, 16 * i, 0, kSc1);
+  }
+  __device__ static bool get(__amdgpu_buffer_rsrc_t m, int, int i, float f[3]) {
+    const mail4 w = __builtin_amdgcn_raw_buffer_load_b128(m, 16 * i, 0, kSc1);
+    f[0] = __uint_as_float(w.x);
+    f[1] = __uint_as_float(w.y);
+    f[2] = __uint_as_float(w.z);
+    return w.x != empty && w.y != empty && w.z != empty;
+  }
+};
+template <> struct MailRec<double> {
+  static constexpr int bytes = 24;
+  static constexpr unsigned long long empty = 0xfff8dead5107e000ull, nan = 0x7ff8000000000000ull;
+  __device__ static unsigned long long bits(double v) {
+    const unsigned long long w = (unsigned long long)__double_as_longlong(v);
+    return w == empty ? nan : w;
+  }
+  __device__ static void store(__amdgpu_buffer_rsrc_t m, int n, int i, unsigned long long x,
+                               unsigned long long y, unsigned long long z) {
+    const mail4 a = {(unsigned)x, (unsigned)(x >> 32), (unsigned)y, (unsigned)(y >> 32)};
+    const mail2 b = {(unsigned)z, (unsigned)(z >> 32)};
+    __builtin_amdgcn_raw_buffer_store_b128(a, m, 16 * i, 0, kSc1);
+    __builtin_amdgcn_raw_buffer_store_b64(b, m, 8 * i, 16 * n, kSc1);
+  }
+  __device__ static void put(__amdgpu_buffer_rsrc_t m, int n, int i, const double f[3]) {
+    store(m, n, i, bits(f[0]), bits(f[1]), bits(f[2]));
+  }
+  __device__ static void clear(__amdgpu_buffer_rsrc_t m, int n, int i) {
+    store(m, n, i, empty, empty, empty);
+  }
+  __device__ static bool get(__amdgpu_buffer_rsrc_t m, int n, int i, double f[3]) {
+    const mail4 a = __builtin_amdgcn_raw_buffer_load_b128(m, 16 * i, 0, kSc1);
+    const mail2 b = __builtin_amdgcn_raw_buffer_load_b64(m, 8 * i, 16 * n, kSc1);
+    const unsigned long long x = a.x | (unsigned long long)a.y << 32,
+                             y = a.z | (unsigned long long)a.w << 32,
+                             z = b.x | (unsigned long long)b.y << 32;
+    f[0] = __longlong_as_double((long long)x);
+    f[1] = __longlong_as_double((long long)y);
+    f[2] = __longlong_as_double((long long)z);
+    return x != empty && y != empty && z != empty;
+  }
+};
+
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t mail_rsrc(void *mail, int bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(mail, 0, bytes, 0x00027000);
+}
+
+template <typename R>
+__global__ void __launch_bounds__(256) k_mail_clear(void *mail, int records) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i < records) MailRec<R>::clear(mail_rsrc(mail, records * MailRec<R>::bytes), records, i);
+}
+
+// LDS past the element kernel's: the messages received, then per message its
+// destination, its local node and the nodes' message lists
+__host__ __device__ constexpr int lds_mail_bytes(int rsz, int most) {
+  return lds_round16(3L * rsz * most) + lds_round16(8L * most);
+}
+
+// NPE 4: thread t has element t and node t of the block, as k_elem_block4.
+// NPE 10: thread t has point t & 3 of element t / 4, as k_elem_block10.
+__device__ __forceinline__ uint32_t decision(const Params &p) {
+  return __hip_atomic_load(&p.ctl->decision, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// launch L's decision, taken once: 0 it counts, 1 it gives up
+__device__ __forceinline__ void decide(const Params &p, unsigned L, unsigned how, int steps) {
+  if (atomicCAS(&p.ctl->decision, 2u * (L - 1u), 2u * L + how) == 2u * (L - 1u) && how)
+    p.ctl->missed = steps;
+}
+
+template <int NPE, int RULE, typename R, int PHYS, int NT, int WPE>
+__global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WPE)))
+k_resident(Params p, Resident rs) {
+  using Rec = MailRec<R>;
+  extern __shared__ double smem[];
+  __shared__ int gave_up;
+  // after a launch that gave up, whose mail lies about, none runs
+  if (threadIdx.x == 0) {
+    const uint32_t past = decision(p);
+    gave_up = past & 1u;
+    if (blockIdx.x == 0 && gave_up && past >> 1 != rs.launch) p.ctl->missed += rs.steps;
+  }
+  __syncthreads();
+  if (gave_up) return;
+  const int b = xcd_remap(blockIdx.x, gridDim.x);
+  const int t = threadIdx.x, q = NPE == 4 ? 0 : t & 3, el = NPE == 4 ? t : t >> 2;
+  const int32_t *mt = p.meta + 8 * b;
+  const int es = mt[0], nel = mt[1];
+  const LNodes ln{smem, p.ml};
+  R *lf = (R *)((char *)smem + lds_node_bytes(p.ml));
+  uint16_t *joff = (uint16_t *)((char *)lf + lds_force_bytes(sizeof(R), NPE, p.max_el));
+  R *lm = (R *)((char *)joff + lds_off_bytes(p.kmax));
+  int32_t *ldest = (int32_t *)((char *)lm + lds_round16(3L * sizeof(R) * rs.most));
+  uint16_t *lsrc = (uint16_t *)(ldest + rs.most), *lidx = lsrc + rs.most;
+  const double dt = p.ctl->dt;
+  const int wv = __builtin_amdgcn_readfirstlane(t >> 6);
+  const bool has_word = PHYS == PHYS_EP && wv < p.ywords;
+  const long yi = (long)b * p.ywords + wv;
+
+  // Node t: its record, and in two registers its contribution count, its
+  // place among the blocks holding it, its messages (kNotShared: none, and
+  // this block alone moves it) and their start in the list.
+  constexpr unsigned kNotShared = 0xffffu;
+  const long o = (long)b * p.ml + t;
+  const int g = t < p.ml ? p.nid_pad[o] : -1;
+  const bool has_n = g >= 0;
+  unsigned deg_lo = 0u, own_cnt = kNotShared << 16;
+  bool held = false, contact = false;
+  if (has_n) {
+    held = node_held(p, g);
+    contact = node_contact(p, g, held);
+    const int slot = p.slot_pad[o];
+    deg_lo = p.deg_pad[o];
+    if (slot >= 0) {
+      const int s0 = p.slot_ptr[g - p.n_interior], s1 = p.slot_ptr[g - p.n_interior + 1];
+      deg_lo |= (unsigned)rs.lo[o] << 16;
+      own_cnt = (unsigned)(slot - s0) | (unsigned)(s1 - s0 - 1) << 16;
+    }
+    ln.stage(t, p.pos[g], p.m[g], p.vv[g]);
+  }
+  const int m0 = rs.first[b], nm = rs.first[b + 1] - m0;
+  for (int m = t; m < nm; m += NT) {
+    ldest[m] = rs.dest[m0 + m];
+    lsrc[m] = rs.src[m0 + m];
+    lidx[m] = rs.idx[m0 + m];
+  }
+  const __amdgpu_buffer_rsrc_t mail = mail_rsrc(rs.mail, (int)(2 * rs.messages * Rec::bytes));
+  for (int k = t; k <= p.kmax; k += NT) joff[k] = p.off_pad[(long)b * (p.kmax + 1) + k];
+  // element el: corner words and the point's state
+  const bool has_e = el < nel;
+  uint32_t cw[NPE / 2];
+  PreState<R> pre{};
+  if (has_e) {
+    const uint32_t *cp = reinterpret_cast<const uint32_t *>(p.corner + (long)NPE * (es + el));
+#pragma unroll
+    for (int k = 0; k < NPE / 2; k++) cw[k] = cp[k];
+    if constexpr (PHYS == PHYS_EP) {
+      const unsigned long long yw = has_word ? p.yielded[yi] : 0ull;
+      load_state_if<R>(p, es + el, q, (yw >> (t & 63)) & 1ull, pre);
+    }
+  }
+  __syncthreads();
+
+  EAcc ea;
+  bool changed = false;
+  auto half = [&](int k) { return (int)((cw[k >> 1] >> (16 * (k & 1))) & 0xffffu); };
+  auto get = [&](int k, double xk[3], double vk[3]) { ln.get(half(k) & 511, xk, vk); };
+  auto slot_of = [&](int h) { return (int)joff[h >> 9] + (h & 511); };
+  int box = rs.base;  // the step's inbox, 0 or 1
+  int qs = q, ts = t;
+  typedef const __attribute__((address_space(4))) Params *Args;
+  Args args = (Args)__builtin_amdgcn_kernarg_segment_ptr();
+  for (int left = rs.steps; left > 0; left--, box ^= 1) {
+    // What follows from the lane's point, node and corners (basis values, LDS
+    // addresses) is cheap to form and must not be held over the step: hoisted
+    // out of the loop it costs 30 to 90 spilled registers.
+    // So are the kernel arguments (scalar loads from the argument segment,
+    // Params first): held, they spill a hundred scalar registers.
+    asm volatile("" : "+v"(qs), "+v"(ts), "+v"(deg_lo), "+v"(own_cnt), "+s"(args));
+#pragma unroll
+    for (int k = 0; k < NPE / 2; k++) asm volatile("" : "+v"(cw[k]));
+#ifdef __HIP_DEVICE_COMPILE__
+    Params pl = *args;
+#else
+    Params pl = p;  // the host pass knows no copy out of that address space
+#endif
+    pl.samples = nullptr;  // the recorder's steps are not resident
+    if (has_e) {
+      if constexpr (NPE == 4) {
+        auto put = [&](int k, const R fk[3]) {
+          R *dst = lf + 3 * slot_of(half(k));
+#pragma unroll
+          for (int c = 0; c < 3; c++) dst[c] = fk[c];
+        };
+        tet4_core<R, PHYS, true, false, true>(pl, get, dt, es + el, put, ea, &pre);
+      } else {
+        // lane q stores corners q, q + 4 and q + 8
+        int sl[3];
+#pragma unroll
+        for (int j = 0; j < 3; j++) {
+          const uint32_t wj = (qs >> 1) ? cw[j == 2 ? 4 : 2 * j + 1] : cw[2 * j];
+          sl[j] = slot_of((int)((wj >> (16 * (qs & 1))) & 0xffffu));
+        }
+        auto put = [&](int k, const R f[3]) {
+          if ((k & 3) == qs) {
+            R *dst = lf + 3 * sl[k >> 2];
+            dst[0] = f[0];
+            dst[1] = f[1];
+            dst[2] = f[2];
+          }
+        };
+        tet10_point_lane<RULE, R, PHYS, false, true>(pl, get, dt, es + el, qs, pre, put, ea);
+      }
+      if constexpr (PHYS == PHYS_EP) changed = changed || pre.changed;
+    }
+    // the emptying stores of the last step have completed
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    double f[3];
+    if (has_n) {
+      node_force_sum<R>(lf, joff, ts, (int)(deg_lo & 0xffffu), f);
+      // the partial for the posts, in the node's own first slot (off[0] = 0)
+      if ((own_cnt >> 16) != kNotShared) {
+#pragma unroll
+        for (int c = 0; c < 3; c++) lf[3 * ts + c] = R(f[c]);
+      }
+    }
+    __syncthreads();
+    const int inbox = box * rs.messages;
+    for (int m = ts; m < nm; m += NT) {
+      const R *fs = lf + 3 * lsrc[m];
+      const R fr[3] = {fs[0], fs[1], fs[2]};
+      Rec::put(mail, 2 * rs.messages, inbox + ldest[m], fr);
+    }
+    for (int m = ts; m < nm; m += NT) {
+      R w[3];
+      unsigned spins = 0;
+      while (!Rec::get(mail, 2 * rs.messages, inbox + m0 + m, w)) {
+        if (++spins >= rs.spin_limit || ((spins & 255u) == 0u && (decision(pl) & 1u))) {
+          gave_up = 1;
+          decide(pl, rs.launch, 1u, rs.steps);
+          break;
+        }
+        asm volatile("" ::: "memory");
+      }
+      Rec::clear(mail, 2 * rs.messages, inbox + m0 + m);
+#pragma unroll
+      for (int c = 0; c < 3; c++) lm[3 * m + c] = w[c];
+    }
+    __syncthreads();
+    if (gave_up) return;
+    if (has_n) {
+      const int own = (int)(own_cnt & 0xffffu), cnt = (int)(own_cnt >> 16);
+      if (cnt != (int)kNotShared) {
+        const int lo = (int)(deg_lo >> 16);
+        double s[3] = {0.0, 0.0, 0.0};
+        auto add = [&](int k) {
+          const R *msg = lm + 3 * lidx[lo + k];
+#pragma unroll
+          for (int c = 0; c < 3; c++) s[c] += double(msg[c]);
+        };
+        for (int k = 0; k < own; k++) add(k);
+#pragma unroll
+        for (int c = 0; c < 3; c++) s[c] += f[c];
+        for (int k = own; k < cnt; k++) add(k);
+#pragma unroll
+        for (int c = 0; c < 3; c++) f[c] = s[c];
+      }
+      double x[3], v[3];
+      ln.get(ts, x, v);
+      const double m = ln.mass(ts);
+      NodeStep s;
+      EAcc en;
+      node_advance(pl, held, contact, f, x, v, m, 1.0 / m, dt, s, en);
+      if (own == 0) ea.wgrav += en.wgrav;
+      ln.stage(ts, Vec3{s.x[0], s.x[1], s.x[2]}, m, Vec3{s.v[0], s.v[1], s.v[2]});
+    }
+    __syncthreads();
+  }
+
+  // all blocks or none
+  if (gridDim.x > 1) {
+    if (t == 0) {
+      const uint64_t all = (uint64_t)rs.launch * gridDim.x;
+      if (atomicAdd((unsigned long long *)&p.ctl->finished, 1ull) + 1ull == all)
+        decide(p, rs.launch, 0u, 0);
+      uint32_t d = decision(p);
+      for (unsigned spins = 0; d == 2u * (rs.launch - 1u); d = decision(p))
+        if (++spins == rs.spin_limit) decide(p, rs.launch, 1u, rs.steps);
+      gave_up = d & 1u;
+    }
+    __syncthreads();
+    if (gave_up) return;
+  } else if (t == 0) {
+    decide(p, rs.launch, 0u, 0);
+  }
+  if (has_n && (own_cnt & 0xffffu) == 0u) {
+    const int n = p.nid_pad[o];
+    double x[3], v[3];
+    ln.get(t, x, v);
+    p.pos[n] = Vec3{x[0], x[1], x[2]};
+    p.vv[n] = Vec3{v[0], v[1], v[2]};
+  }
+  if constexpr (PHYS == PHYS_EP) {
+    if (has_e) store_state<R>(p, es + el, q, pre.s, pre.ep, changed);
+    const unsigned long long nb = __ballot(has_e && pre.ep > R(0));
+    if (has_word && (t & 63) == 0) p.yielded[yi] = nb;
+  }
+  const int row_base = p.epart_base + b * (NT / 64);
+  wave_flush<false>(p, row_base, ea, row_prefetch(p, row_base));
+  if (blockIdx.x == 0 && t == 0) p.ctl->step += rs.steps;
 }
 
 // ---------------------------------------------------------------------------
@@ -1651,6 +2030,74 @@ hipError_t prepare_elem_block(int npe, int rule, int prec, int phys, size_t smem
 hipError_t launch_elem_direct(const Params &p, int rule, int prec, int phys, bool atomic,
                               hipStream_t s) {
   return dispatch<ElemDirectF>(p.npe, rule, prec, phys, p, atomic, s);
+}
+
+// minimum waves per SIMD of the resident kernels
+template <int NPE, typename R> constexpr int resident_waves() {
+  return 4;
+}
+
+template <int NPE, int RULE, typename R, int PHYS> struct ResidentF {
+  static constexpr bool has() {
+    return PHYS != PHYS_EP_MLP && (NPE == 4 || Quad<RULE>::n == 4);
+  }
+  // the kernel, its threads per workgroup
+  static hipError_t run(const void **kernel, int *threads) {
+    if constexpr (!has()) {
+      return hipErrorInvalidValue;
+    } else {
+      *kernel = reinterpret_cast<const void *>(
+          k_resident<NPE, RULE, R, PHYS, block_threads<NPE, RULE>(), resident_waves<NPE, R>()>);
+      *threads = block_threads<NPE, RULE>();
+      return hipSuccess;
+    }
+  }
+};
+
+int resident_capacity(int npe, int rule, int prec, int phys, size_t smem, int cus) {
+  const void *k = nullptr;
+  int nt = 0, per = 0;
+  if (dispatch<ResidentF>(npe, rule, prec, phys, &k, &nt) != hipSuccess) return 0;
+  if (smem > 65536 &&
+      hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess)
+    return 0;
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, k, nt, smem) != hipSuccess) return 0;
+  // The query counts waves over the whole CU; a workgroup of six waves lands
+  // as 2, 2, 1, 1 on the four SIMDs, and nothing makes the next one fill the
+  // gaps.  Count ceil(waves / 4) on every SIMD, so that all really fit.
+  hipFuncAttributes at{};
+  if (hipFuncGetAttributes(&at, k) != hipSuccess || at.numRegs <= 0) return 0;
+  const int simd = std::min(8, 512 / ((at.numRegs + 7) / 8 * 8)), wg = (nt / 64 + 3) / 4;
+  return std::min(per, simd / wg) * cus;
+}
+
+hipError_t launch_resident(const Params &p, int rule, int prec, int phys, const Resident &rs,
+                           int nblocks, size_t smem, hipStream_t s) {
+  const void *k = nullptr;
+  int nt = 0;
+  hipError_t e = dispatch<ResidentF>(p.npe, rule, prec, phys, &k, &nt);
+  if (e != hipSuccess) return e;
+  Params pa = p;
+  Resident ra = rs;
+  void *args[2] = {&pa, &ra};
+  // one block waits for nobody
+  if (nblocks == 1) return hipLaunchKernel(k, dim3(1), dim3(nt), args, smem, s);
+  return hipLaunchCooperativeKernel(k, dim3(nblocks), dim3(nt), args, (unsigned)smem, s);
+}
+
+hipError_t launch_mail_clear(const Resident &rs, int prec, hipStream_t s) {
+  const int records = 2 * rs.messages;
+  if (records == 0) return hipSuccess;
+  if (prec == 1) CPI_LAUNCH(k_mail_clear<float>, (records + 255) / 256, 256, 0, s, rs.mail, records);
+  CPI_LAUNCH(k_mail_clear<double>, (records + 255) / 256, 256, 0, s, rs.mail, records);
+}
+
+size_t resident_smem(size_t block_smem, int prec, int most) {
+  return block_smem + lds_mail_bytes(prec == 1 ? 4 : 8, most);
+}
+
+size_t mail_bytes(int prec, size_t messages) {
+  return 2 * messages * (prec == 1 ? MailRec<float>::bytes : MailRec<double>::bytes);
 }
 
 hipError_t launch_node_bnd(const Params &p, int prec, bool aux, hipStream_t s) {

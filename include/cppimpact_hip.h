@@ -149,7 +149,10 @@ typedef struct cpi_options {
                                all-ones bytes (NaN as a float or double, -1 as
                                an integer) when it is allocated, so a read of
                                memory the context never wrote shows as a
-                               non-finite state (diagnostics; default 0) */
+                               non-finite state (diagnostics; default 0).
+                                 3: also every wait of a resident step gives
+                                 up at once, so the steps are taken one by
+                                 one */
   int32_t stream_state;     /* the block kernels' stress-state accesses
                                (tet4 and the 4-point tet10 kernel):
                                0 = non-temporal when a step's working set
