@@ -43,7 +43,9 @@ struct cpi_ctx {
   std::vector<int32_t> eperm, nperm, ninv;  // device->user elem, device->user node, user->device
   std::vector<int32_t> loose;               // user nodes of no element
   int32_t *d_last = nullptr;                // per user node: last element holding it (device id)
-  int32_t *d_ninv = nullptr, *d_einv = nullptr;  // user node / element -> device id
+  int32_t *d_ninv = nullptr;                // user node -> device id
+  uint32_t *d_spos = nullptr;               // per user element: its state (k_export_elems)
+  size_t state_points = 0;                  // points the state arrays hold
   Vec3 *d_V0 = nullptr;                     // initial velocities, device order
   BlockPlan plan;
   std::vector<void *> allocs;
@@ -407,8 +409,8 @@ int reset_state(cpi_ctx *c) {
   HIPCHK(c, launch_reset_nodes(c->P, c->d_V0, c->stream));
   const size_t rs = c->prec == CPI_PREC_F32 ? 4 : 8;
   if (c->phys != CPI_PHYSICS_COMPAT) {
-    HIPCHK(c, hipMemsetAsync(c->P.sig, 0, rs * 6 * c->nq * (size_t)c->ne, c->stream));
-    HIPCHK(c, hipMemsetAsync(c->P.epbar, 0, rs * c->nq * (size_t)c->ne, c->stream));
+    HIPCHK(c, hipMemsetAsync(c->P.sig, 0, rs * 6 * c->state_points, c->stream));
+    HIPCHK(c, hipMemsetAsync(c->P.epbar, 0, rs * c->state_points, c->stream));
     if (c->P.yielded)
       HIPCHK(c, hipMemsetAsync(c->P.yielded, 0, 8 * (size_t)c->P.ywords * c->nblocks, c->stream));
     if (c->P.mlp_ctr) HIPCHK(c, hipMemsetAsync(c->P.mlp_ctr, 0, sizeof(unsigned long long), c->stream));
@@ -724,7 +726,6 @@ static int create_impl(cpi_ctx *c, const cpi_mesh_desc *m, const cpi_material *m
     for (int i = 0; i < nn; i++)
       if (last[i] < 0) c->loose.push_back(i);
     if ((rc = dalloc(c, &c->d_last, last.size())) || (rc = upload(c, c->d_last, last)) ||
-        (rc = dalloc(c, &c->d_einv, einv.size())) || (rc = upload(c, c->d_einv, einv)) ||
         (rc = dalloc(c, &c->d_ninv, c->ninv.size())) || (rc = upload(c, c->d_ninv, c->ninv)) ||
         (rc = dalloc(c, &c->d_V0, nn)))
       return rc;
@@ -752,7 +753,26 @@ static int create_impl(cpi_ctx *c, const cpi_mesh_desc *m, const cpi_material *m
   if (c->phys != CPI_PHYSICS_COMPAT) {
     const size_t rs = c->prec == CPI_PREC_F32 ? 4 : 8;
     char *s = nullptr, *q = nullptr;
-    if ((rc = dalloc(c, &s, rs * 6 * c->nq * (size_t)ne)) || (rc = dalloc(c, &q, rs * c->nq * (size_t)ne)))
+    std::vector<uint32_t> spos(ne);
+    c->state_points = c->nq * (size_t)ne;
+    if (c->scatter == CPI_SCATTER_BLOCK && (npe == 4 || c->nq == 4)) {
+      // rows of whole 128-byte lines in FP32; of blocks smaller than that,
+      // the next power of two (a row is never twice its block)
+      const BlockPlan &B = c->plan;
+      int row = c->nq;
+      while (row < 32 && row < c->nq * B.max_block_elems) row *= 2;
+      P.state_ld = (c->nq * B.max_block_elems + row - 1) / row * row;
+      c->state_points = (size_t)B.nblocks * P.state_ld;
+      if (c->state_points / c->nq > UINT32_MAX)
+        return fail(c, CPI_ERR_INVALID, "the stress state's rows pass 2^32 elements");
+      for (int b = 0; b < B.nblocks; b++)
+        for (int k = 0; k < B.meta[8 * (size_t)b + 1]; k++)
+          spos[c->eperm[B.meta[8 * (size_t)b] + k]] = (uint32_t)((size_t)b * (P.state_ld / c->nq) + k);
+    } else {
+      for (int e = 0; e < ne; e++) spos[c->eperm[e]] = (uint32_t)e;
+    }
+    if ((rc = dalloc(c, &s, rs * 6 * c->state_points)) || (rc = dalloc(c, &q, rs * c->state_points)) ||
+        (rc = dalloc(c, &c->d_spos, spos.size())) || (rc = upload(c, c->d_spos, spos)))
       return rc;
     P.sig = s;
     P.epbar = q;
@@ -1220,7 +1240,7 @@ extern "C" int cpi_get_element_state(cpi_ctx *c, double *sig, double *ep) {
   if (sig) p[k++] = Piece{sig, 6 * n};
   if (ep) p[k++] = Piece{ep, n};
   if (k)
-    HIPCHK(c, launch_export_elems(c->P, c->prec, c->d_einv, sig ? c->d_tmp : nullptr,
+    HIPCHK(c, launch_export_elems(c->P, c->prec, c->d_spos, sig ? c->d_tmp : nullptr,
                                   ep ? c->d_tmp + (sig ? 6 * n : 0) : nullptr, c->stream));
   return bring_back(c, p, k);
 }

@@ -93,8 +93,12 @@ struct Params {
   Node4 *xprev;          // x_n before the step   written when store_aux
   Node4 *X0;             // reference positions
   const int32_t *conn;   // [npe][ne] device node ids (colour / atomic)
-  void *sig;             // [nq][6][ne] stress state (ep)
-  void *epbar;           // [nq][ne]
+  // stress state (EP), [nblocks][6][state_ld] and ep [nblocks][state_ld] in
+  // the kernels with a thread per point, [nq][6][ne] and [nq][ne] in the
+  // others (state_ld 0); see StateBlock
+  void *sig;
+  void *epbar;
+  int state_ld;
   // tet4 and per-point tet10 block kernels, exact return: one bit per
   // stress point, set once it has yielded (ep > 0), ywords 64-bit words per
   // block (the point of thread t of block b at word b*ywords + t/64, bit

@@ -45,46 +45,86 @@ template <> struct Quad<RULE_CENTROID> {
   __device__ static constexpr double pt(int, int) { return 0.25; }
 };
 
-// Stress-state words are read and written once per step.  STREAM = true
-// marks those accesses non-temporal: for a state larger than the
-// last-level cache, caching it only evicts the node records and partial
-// forces that other blocks and the boundary-node kernel read again.
-template <bool STREAM, typename T>
-__device__ __forceinline__ T state_ld(const T *a) {
-  if constexpr (STREAM)
-    return __builtin_nontemporal_load(a);
-  else
-    return *a;
-}
-template <bool STREAM, typename T>
-__device__ __forceinline__ void state_st(T *a, T v) {
-  if constexpr (STREAM)
-    __builtin_nontemporal_store(v, a);
-  else
-    *a = v;
+// Where a point's stress state lies.  The kernels with a thread per point
+// (k_elem_block4, k_elem_block10, the resident steps) keep a block's state
+// together, [block][6][state_ld] with thread t's point at t (StateBlock): a
+// wave reads whole aligned lines, and a block one contiguous piece of memory
+// per step, through a buffer descriptor with one 32-bit offset per thread
+// (64-bit addresses, shared by a component's load and store, stay live across
+// the stress update and spill: 59 us per 64^3 step instead of 46).  The other
+// kernels keep planes of the whole mesh, [nq][6][ne] (StatePlane), as all did:
+// the 1.2M-tet10 kernel's waves then read four short runs of each of 24 planes,
+// and its traffic alone (no arithmetic) took 204 of its 217 us in FP64.  With
+// the block layout the whole kernel takes 165 us (FP32 137 -> 117), the 64^3
+// tet4 kernel 41 -> 39 (FP32 27.5 -> 26.5).
+//
+// State words are read and written once per step.  STREAM = true marks those
+// accesses non-temporal: for a state larger than the last-level cache,
+// caching it only evicts the node records and partial forces that other
+// blocks and the boundary-node kernel read again.
+template <typename R> struct StatePlane {
+  R *s, *ep;
+  long ne;
+  template <bool STREAM> __device__ __forceinline__ R get(int c) const { return s[c * ne]; }
+  template <bool STREAM> __device__ __forceinline__ void set(int c, R v) const { s[c * ne] = v; }
+  // has: the point has yielded before (ep of the others is 0)
+  template <bool STREAM> __device__ __forceinline__ R get_ep(bool has) const {
+    return has ? *ep : R(0);
+  }
+  template <bool STREAM> __device__ __forceinline__ void set_ep(R v) const { *ep = v; }
+};
+template <typename R>
+__device__ __forceinline__ StatePlane<R> state_plane(const Params &p, int e, int q) {
+  return StatePlane<R>{(R *)p.sig + ((long)q * 6 * p.ne + e), (R *)p.epbar + ((long)q * p.ne + e),
+                       p.ne};
 }
 
-template <typename R, bool STREAM = false>
-__device__ __forceinline__ void load_state(const Params &p, int e, int q, R s[6], R &ep) {
-  const R *S = (const R *)p.sig;
-  const R *P = (const R *)p.epbar;
-  const long ne = p.ne;
-#pragma unroll
-  for (int c = 0; c < 6; c++) s[c] = state_ld<STREAM>(&S[(long)(q * 6 + c) * ne + e]);
-  ep = state_ld<STREAM>(&P[(long)q * ne + e]);
-}
-
-// ep is written only when it changed (a plastic step): elastic steps store
-// the stress alone
-template <typename R, bool STREAM = false>
-__device__ __forceinline__ void store_state(const Params &p, int e, int q, const R s[6], R ep,
-                                            bool ep_changed = true) {
-  R *S = (R *)p.sig;
-  R *P = (R *)p.epbar;
-  const long ne = p.ne;
-#pragma unroll
-  for (int c = 0; c < 6; c++) state_st<STREAM>(&S[(long)(q * 6 + c) * ne + e], s[c]);
-  if (ep_changed) state_st<STREAM>(&P[(long)q * ne + e], ep);
+template <typename R> struct StateBlock {
+  __amdgpu_buffer_rsrc_t s, ep;
+  unsigned off;  // bytes into a component's row
+  int row;       // bytes of a row
+  template <bool STREAM>
+  __device__ __forceinline__ static R ld(__amdgpu_buffer_rsrc_t r, unsigned o, int at) {
+    constexpr int aux = STREAM ? 2 : 0;  // nt
+    if constexpr (std::is_same<R, double>::value)
+      return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, o, at, aux));
+    else
+      return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, o, at, aux));
+  }
+  template <bool STREAM>
+  __device__ __forceinline__ static void st(__amdgpu_buffer_rsrc_t r, unsigned o, int at, R v) {
+    constexpr int aux = STREAM ? 2 : 0;
+    if constexpr (std::is_same<R, double>::value) {
+      typedef unsigned w2 __attribute__((ext_vector_type(2)));
+      __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(w2, v), r, o, at, aux);
+    } else {
+      __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), r, o, at, aux);
+    }
+  }
+  template <bool STREAM> __device__ __forceinline__ R get(int c) const {
+    return ld<STREAM>(s, off, c * row);
+  }
+  template <bool STREAM> __device__ __forceinline__ void set(int c, R v) const {
+    st<STREAM>(s, off, c * row, v);
+  }
+  // without a branch: an offset past the descriptor's range reads as 0, so
+  // every lane issues the same loads and the kernel can wait by count for those
+  // issued before them while these stay in flight
+  template <bool STREAM> __device__ __forceinline__ R get_ep(bool has) const {
+    return ld<STREAM>(ep, has ? off : ~7u, 0);
+  }
+  template <bool STREAM> __device__ __forceinline__ void set_ep(R v) const {
+    st<STREAM>(ep, off, 0, v);
+  }
+};
+// b: uniform; threads past the block's row take its last place
+template <typename R>
+__device__ __forceinline__ StateBlock<R> state_block(const Params &p, int b, int t) {
+  const int row = p.state_ld * (int)sizeof(R);
+  R *s = (R *)p.sig + (long)b * 6 * p.state_ld, *ep = (R *)p.epbar + (long)b * p.state_ld;
+  return StateBlock<R>{__builtin_amdgcn_make_buffer_rsrc(s, 0, 6 * row, 0x00027000),
+                       __builtin_amdgcn_make_buffer_rsrc(ep, 0, row, 0x00027000),
+                       (unsigned)(t < p.state_ld ? t : p.state_ld - 1) * (unsigned)sizeof(R), row};
 }
 
 // State of one point loaded ahead of use (the tet4 workgroup kernel issues
@@ -98,47 +138,33 @@ template <typename R> struct PreState {
 };
 
 // The stress of one point, and its ep only when the point has yielded
-// before (ep of the others is 0).
-template <typename R, bool STREAM = false>
-__device__ __forceinline__ void load_state_if(const Params &p, int e, int q, bool has_ep,
-                                              PreState<R> &st) {
-  const R *S = (const R *)p.sig;
-  const long ne = p.ne;
+// before.
+template <bool STREAM, typename R, class At>
+__device__ __forceinline__ void load_state(const At &at, bool has_ep, PreState<R> &st) {
 #pragma unroll
-  for (int c = 0; c < 6; c++) st.s[c] = state_ld<STREAM>(&S[(long)(q * 6 + c) * ne + e]);
-  st.ep = has_ep ? state_ld<STREAM>(&((const R *)p.epbar)[(long)q * ne + e]) : R(0);
+  for (int c = 0; c < 6; c++) st.s[c] = at.template get<STREAM>(c);
+  st.ep = at.template get_ep<STREAM>(has_ep);
 }
 
-// A zero word in global memory (the bits of 0.0 in FP64 and in FP32); no
-// kernel writes it.  Not const: a constant-memory address selected against
-// a global one makes the load a flat load, which the compiler waits for in
-// full before the next barrier.
-__device__ double kZeroWord[1] = {0.0};
-
-// load_state_if without a branch, for the block kernels' load phase: a
-// point that has not yielded loads its ep from kZeroWord, so every lane
-// issues the same seven loads, nothing waits for them before their first
-// use, and the kernel can wait for the loads issued before them by count
-// while these stay in flight.
-template <typename R, bool STREAM = false>
-__device__ __forceinline__ void load_state_sel(const Params &p, int e, int q, bool has_ep,
-                                               PreState<R> &st) {
-  const R *S = (const R *)p.sig;
-  const R *P = (const R *)p.epbar;
-  const long ne = p.ne;
+// ep is written only when it changed (a plastic step): elastic steps store
+// the stress alone
+template <bool STREAM, typename R, class At>
+__device__ __forceinline__ void store_state(const At &at, const R s[6], R ep, bool ep_changed) {
 #pragma unroll
-  for (int c = 0; c < 6; c++) st.s[c] = state_ld<STREAM>(&S[(long)(q * 6 + c) * ne + e]);
-  st.ep = state_ld<STREAM>(has_ep ? &P[(long)q * ne + e] : (const R *)kZeroWord);
+  for (int c = 0; c < 6; c++) at.template set<STREAM>(c, s[c]);
+  if (ep_changed) at.template set_ep<STREAM>(ep);
 }
 
 // Stress at one point from the strain increment de.  compat: sigma = D de
 // with no memory (dynamics_kernels.h:101-114 evaluates K_e du); ep: trial
 // sigma_n + D de, then the return map (exact or surrogate).  Adds the
-// point's internal work and plastic dissipation (times wd) to ea.  (The
+// point's internal work and plastic dissipation (times wd) to ea.  at: where
+// the point's state lies; e, q: its element and number, for the recorder.  (The
 // surrogate's return map is applied by the tet4 block kernel's walk.)
-template <typename R, int PHYS, bool PRE = false, bool STREAM = false, bool DEFER = false>
-__device__ __forceinline__ void point_stress(const Params &p, int e, int q, const R de[6],
-                                             R wd, R s[6], EAcc &ea,
+template <typename R, int PHYS, bool PRE = false, bool STREAM = false, bool DEFER = false,
+          class At>
+__device__ __forceinline__ void point_stress(const Params &p, const At &at, int e, int q,
+                                             const R de[6], R wd, R s[6], EAcc &ea,
                                              PreState<R> *pre = nullptr) {
   const R c11 = R(p.c11), c12 = R(p.c12), c44 = R(p.c44);
   R ds[6];
@@ -163,7 +189,11 @@ __device__ __forceinline__ void point_stress(const Params &p, int e, int q, cons
       for (int c = 0; c < 6; c++) so[c] = pre->s[c];
       ep = pre->ep;
     } else {
-      load_state<R>(p, e, q, so, ep);
+      PreState<R> st;
+      load_state<STREAM, R>(at, true, st);
+#pragma unroll
+      for (int c = 0; c < 6; c++) so[c] = st.s[c];
+      ep = st.ep;
     }
     // midpoint internal work 1/2 (sigma_n + sigma_{n+1}) : de, split so that
     // sigma_n need not stay live through the return map
@@ -186,7 +216,7 @@ __device__ __forceinline__ void point_stress(const Params &p, int e, int q, cons
       for (int c = 0; c < 6; c++) pre->s[c] = s[c];
       pre->changed = dg > R(0);
     } else {
-      store_state<R, STREAM>(p, e, q, s, ep, dg > R(0));
+      store_state<STREAM, R>(at, s, ep, dg > R(0));
     }
     if constexpr (PRE) pre->ep = ep;
   }
@@ -321,15 +351,15 @@ __device__ __forceinline__ void tet4_forces(const R Ji[9], const R s[6], R wd, c
 // STREAM: the state is read and written non-temporal.  DEFER: the updated
 // state is left in pre, as in tet10_point_lane.
 // ---------------------------------------------------------------------------
-template <typename R, int PHYS, bool PRE, bool STREAM = false, bool DEFER = false, class Get,
-          class Put>
-__device__ __forceinline__ void tet4_core(const Params &p, const Get &get, double dt, int e,
-                                          const Put &put, EAcc &ea,
+template <typename R, int PHYS, bool PRE, bool STREAM = false, bool DEFER = false, class At,
+          class Get, class Put>
+__device__ __forceinline__ void tet4_core(const Params &p, const At &at, const Get &get, double dt,
+                                          int e, const Put &put, EAcc &ea,
                                           PreState<R> *pre = nullptr) {
   R Ji[9], de[6], wd;
   tet4_kin<R, PHYS>(p, get, dt, Ji, de, wd, ea);
   R s[6];
-  point_stress<R, PHYS, PRE, STREAM, DEFER>(p, e, 0, de, wd, s, ea, pre);
+  point_stress<R, PHYS, PRE, STREAM, DEFER>(p, at, e, 0, de, wd, s, ea, pre);
   tet4_forces<R>(Ji, s, wd, put);
 }
 
@@ -419,7 +449,7 @@ __device__ __forceinline__ void tet10_points(const Params &p, const Get &get, do
     }
     R wd = R(Q::w(q)) * detJ;
     R s[6];
-    point_stress<R, PHYS>(p, e, q, de, wd, s, ea);
+    point_stress<R, PHYS>(p, state_plane<R>(p, e, q), e, q, de, wd, s, ea);
 #pragma unroll
     for (int i = 0; i < 10; i++) {
       R dn[3];
@@ -469,9 +499,9 @@ __device__ __forceinline__ void tet10_points(const Params &p, const Get &get, do
 // else it is stored here (STREAM: non-temporal): registers that a store
 // reads must not be reused before the store has completed, so a store
 // issued here makes the rest of the kernel wait for it.
-template <int RULE, typename R, int PHYS, bool STREAM, bool DEFER, class Get, class Put>
-__device__ __forceinline__ void tet10_point_lane(const Params &p, const Get &get, double dt,
-                                                 int e, int q, PreState<R> &pre, const Put &put,
+template <int RULE, typename R, int PHYS, bool STREAM, bool DEFER, class At, class Get, class Put>
+__device__ __forceinline__ void tet10_point_lane(const Params &p, const At &at, const Get &get,
+                                                 double dt, int e, int q, PreState<R> &pre, const Put &put,
                                                  EAcc &ea) {
   using Q = Quad<RULE>;
   static_assert(Q::n == 4, "one lane per point of a 4-point rule");
@@ -636,7 +666,7 @@ __device__ __forceinline__ void tet10_point_lane(const Params &p, const Get &get
   for (int k = 0; k < 6; k++) de[k] *= R(dt);
   const R wd = R(Q::w(q)) * detJ;
   R s[6];
-  point_stress<R, PHYS, true, STREAM, DEFER>(p, e, q, de, wd, s, ea, &pre);
+  point_stress<R, PHYS, true, STREAM, DEFER>(p, at, e, q, de, wd, s, ea, &pre);
   // M[r][k] = sum_t (w detJ sigma)[r][t] Ji[k][t], sigma rows (s0 s3 s5),
   // (s3 s1 s4), (s5 s4 s2)
   R M[9], S[3];
@@ -688,7 +718,7 @@ template <int NPE, int RULE, typename R, int PHYS, class Get, class Put>
 __device__ __forceinline__ void elem_core(const Params &p, const Get &get, double dt, int e,
                                           const Put &put, EAcc &ea) {
   if constexpr (NPE == 4)
-    tet4_core<R, PHYS, false>(p, get, dt, e, put, ea);
+    tet4_core<R, PHYS, false>(p, state_plane<R>(p, e, 0), get, dt, e, put, ea);
   else
     tet10_core<RULE, R, PHYS>(p, get, dt, e, put, ea);
 }

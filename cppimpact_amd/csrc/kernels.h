@@ -44,7 +44,8 @@ int energy_reduce_blocks();  // rows of p.ered (EP_N doubles each)
 hipError_t launch_mass(const Params &p, int rule, int scatter, int kind, double rho,
                        int nblocks, hipStream_t s);
 hipError_t launch_elem_dt(const Params &p, double *out, hipStream_t s);
-// user-order host layouts (ninv, einv: user node / element -> device id).
+// user-order host layouts (ninv: user node -> device id; spos: see
+// k_export_elems).
 // Import: [nn][3] into Vec3 and / or Node4 records (w = 0), null skipped.
 hipError_t launch_import_nodes(const double *src, const int32_t *ninv, int nn, Vec3 *d3, Node4 *d4,
                                hipStream_t s);
@@ -59,7 +60,7 @@ struct NodeExport {
 hipError_t launch_export_nodes(const Params &p, const int32_t *ninv, const NodeExport &o,
                                hipStream_t s);
 // sig [ne][nq][6], ep [ne][nq] as doubles (null skipped)
-hipError_t launch_export_elems(const Params &p, int prec, const int32_t *einv, double *sig,
+hipError_t launch_export_elems(const Params &p, int prec, const uint32_t *spos, double *sig,
                                double *ep, hipStream_t s);
 // positions X0, velocities v0 (device order), forces, a and du zeroed
 hipError_t launch_reset_nodes(const Params &p, const Vec3 *v0, hipStream_t s);

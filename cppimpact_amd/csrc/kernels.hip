@@ -89,6 +89,24 @@ __device__ __forceinline__ void keep_here(RowPre &r) {
   keep_here(r.wgrav);
 }
 
+// The kernel's Params (its first argument) read again from the argument
+// segment: for the body of a loop, where arguments held from before it spill
+// a hundred scalar registers.  at: set once with params_at(), and made unknown
+// to the compiler on every pass so that the loads stay in the body.
+typedef const __attribute__((address_space(4))) Params *ParamsAt;
+__device__ __forceinline__ ParamsAt params_at() {
+  return (ParamsAt)__builtin_amdgcn_kernarg_segment_ptr();
+}
+__device__ __forceinline__ Params params_again(ParamsAt &at, const Params &p) {
+  asm volatile("" : "+s"(at));
+#ifdef __HIP_DEVICE_COMPILE__
+  (void)p;
+  return *at;
+#else
+  return p;  // the host pass knows no copy out of that address space
+#endif
+}
+
 // One wave's energy terms into its row: the cumulative ones added to what
 // the row held (pre), and with ALL the instantaneous ones (kinetic,
 // penalty, contact force, stable dt) stored.
@@ -418,6 +436,7 @@ k_elem_block10(Params p) {
   __builtin_amdgcn_sched_barrier(0);
   const bool has_e = (t >> 2) < nel;
   const int e = es + (t >> 2), ec = has_e ? e : es + nel - 1;
+  const StateBlock<R> at = state_block<R>(p, b, t);
   // the element's ten corner words (local node | rank << 9), two per word
   // (the rows of 20 bytes are 4-byte aligned)
   uint32_t cw[5];
@@ -428,7 +447,7 @@ k_elem_block10(Params p) {
   }
   PreState<R> pre;
   if constexpr (PHYS != PHYS_COMPAT)
-    load_state_sel<R, STREAM>(p, ec, q, (yw >> (t & 63)) & 1ull, pre);
+    load_state<STREAM, R>(at, (yw >> (t & 63)) & 1ull, pre);
   __builtin_amdgcn_sched_barrier(0);
   keep_here(dt);
   keep_here(row);
@@ -460,7 +479,7 @@ k_elem_block10(Params p) {
         dst[2] = f[2];
       }
     };
-    tet10_point_lane<RULE, R, PHYS, STREAM, !AUX>(p, get, dt, e, q, pre, put, ea);
+    tet10_point_lane<RULE, R, PHYS, STREAM, !AUX>(p, at, get, dt, e, q, pre, put, ea);
     yielded = pre.ep > R(0);
   }
   if constexpr (PHYS == PHYS_EP) {
@@ -484,7 +503,7 @@ k_elem_block10(Params p) {
   // the point's state last (tet10_point_lane leaves it in pre), except in
   // the once-per-batch variant, whose outputs leave no registers for it
   if constexpr (PHYS != PHYS_COMPAT && !AUX)
-    if (has_e) store_state<R, STREAM>(p, e, q, pre.s, pre.ep, pre.changed);
+    if (has_e) store_state<STREAM, R>(at, pre.s, pre.ep, pre.changed);
 }
 
 // tet4: the plan gives every workgroup at most NT elements and NT local
@@ -553,12 +572,13 @@ __device__ __forceinline__ void block4(const Params &p, const int b, const unsig
   __builtin_amdgcn_sched_barrier(0);
   const bool has_e = t < nel;
   const int e = es + t, ec = has_e ? e : es + nel - 1;
+  const StateBlock<R> at = state_block<R>(p, b, t);
   const uint2 lc4 = *(const uint2 *)((CW ? p.corner : p.conn_local) + 4L * ec);
   uint2 ps4 = make_uint2(0u, 0u);
   if constexpr (!CW) ps4 = *(const uint2 *)(p.csr_pos + 4L * ec);
   PreState<R> pre;
   if constexpr (PHYS != PHYS_COMPAT)
-    load_state_sel<R, STREAM>(p, ec, 0, (yw >> (t & 63)) & 1ull, pre);
+    load_state<STREAM, R>(at, (yw >> (t & 63)) & 1ull, pre);
   __builtin_amdgcn_sched_barrier(0);
   keep_here(dt);
   keep_here(row);
@@ -623,7 +643,7 @@ __device__ __forceinline__ void block4(const Params &p, const int b, const unsig
         yielding = true;
       }
     } else {
-      tet4_core<R, PHYS, true, STREAM>(p, get, dt, e, put, ea, &pre);
+      tet4_core<R, PHYS, true, STREAM>(p, at, get, dt, e, put, ea, &pre);
       if constexpr (PHYS == PHYS_EP) has_ep = pre.ep > R(0);
     }
   }
@@ -664,7 +684,7 @@ __device__ __forceinline__ void block4(const Params &p, const int b, const unsig
       }
       // stored here, not last: held through the node pass, the stress
       // would not fit the elastic pass's 64 VGPRs
-      if (has_e) store_state<R, STREAM>(p, e, 0, snew, pre.ep, false);
+      if (has_e) store_state<STREAM, R>(at, snew, pre.ep, false);
     } else {
       int how = MLP_ELASTIC;
       if (yielding) {
@@ -719,7 +739,7 @@ __device__ __forceinline__ void block4(const Params &p, const int b, const unsig
   // earlier would hold up the node pass (the exact-return body stores it
   // in point_stress: held to the end, the FP64 kernel ran 1-2% slower)
   if constexpr (PHYS == PHYS_EP_MLP && WALK) {
-    if (has_e) store_state<R, STREAM>(p, e, 0, snew, pre.ep, ep_changed);
+    if (has_e) store_state<STREAM, R>(at, snew, pre.ep, ep_changed);
   }
 }
 
@@ -745,7 +765,8 @@ k_elem_block4_walk(Params p) {
   __shared__ unsigned misc[2];
   if (blockIdx.x >= (unsigned)(*p.mlp_ctr >> 32)) return;
   const int2 ent = p.mlp_list[blockIdx.x];
-  block4<float, PHYS_EP_MLP, AUX, NT, true, STREAM, CW>(p, ent.x, (unsigned)ent.y, wcnt, misc);
+  block4<float, PHYS_EP_MLP, AUX, NT, true, STREAM, CW>(
+      p, __builtin_amdgcn_readfirstlane(ent.x), (unsigned)ent.y, wcnt, misc);
 }
 
 // The network on queue rows [0, n): n from the step's counter (ctr) or
@@ -1031,7 +1052,7 @@ k_resident(Params p, Resident rs) {
     for (int k = 0; k < NPE / 2; k++) cw[k] = cp[k];
     if constexpr (PHYS == PHYS_EP) {
       const unsigned long long yw = has_word ? p.yielded[yi] : 0ull;
-      load_state_if<R>(p, es + el, q, (yw >> (t & 63)) & 1ull, pre);
+      load_state<false, R>(state_block<R>(p, b, t), (yw >> (t & 63)) & 1ull, pre);
     }
   }
   __syncthreads();
@@ -1043,22 +1064,15 @@ k_resident(Params p, Resident rs) {
   auto slot_of = [&](int h) { return (int)joff[h >> 9] + (h & 511); };
   int box = rs.base;  // the step's inbox, 0 or 1
   int qs = q, ts = t;
-  typedef const __attribute__((address_space(4))) Params *Args;
-  Args args = (Args)__builtin_amdgcn_kernarg_segment_ptr();
+  ParamsAt args = params_at();
   for (int left = rs.steps; left > 0; left--, box ^= 1) {
     // What follows from the lane's point, node and corners (basis values, LDS
     // addresses) is cheap to form and must not be held over the step: hoisted
     // out of the loop it costs 30 to 90 spilled registers.
-    // So are the kernel arguments (scalar loads from the argument segment,
-    // Params first): held, they spill a hundred scalar registers.
-    asm volatile("" : "+v"(qs), "+v"(ts), "+v"(deg_lo), "+v"(own_cnt), "+s"(args));
+    asm volatile("" : "+v"(qs), "+v"(ts), "+v"(deg_lo), "+v"(own_cnt));
 #pragma unroll
     for (int k = 0; k < NPE / 2; k++) asm volatile("" : "+v"(cw[k]));
-#ifdef __HIP_DEVICE_COMPILE__
-    Params pl = *args;
-#else
-    Params pl = p;  // the host pass knows no copy out of that address space
-#endif
+    Params pl = params_again(args, p);
     pl.samples = nullptr;  // the recorder's steps are not resident
     if (has_e) {
       if constexpr (NPE == 4) {
@@ -1067,7 +1081,7 @@ k_resident(Params p, Resident rs) {
 #pragma unroll
           for (int c = 0; c < 3; c++) dst[c] = fk[c];
         };
-        tet4_core<R, PHYS, true, false, true>(pl, get, dt, es + el, put, ea, &pre);
+        tet4_core<R, PHYS, true, false, true>(pl, StatePlane<R>{}, get, dt, es + el, put, ea, &pre);
       } else {
         // lane q stores corners q, q + 4 and q + 8
         int sl[3];
@@ -1084,7 +1098,8 @@ k_resident(Params p, Resident rs) {
             dst[2] = f[2];
           }
         };
-        tet10_point_lane<RULE, R, PHYS, false, true>(pl, get, dt, es + el, qs, pre, put, ea);
+        tet10_point_lane<RULE, R, PHYS, false, true>(pl, StatePlane<R>{}, get, dt, es + el, qs, pre, put,
+                                                     ea);
       }
       if constexpr (PHYS == PHYS_EP) changed = changed || pre.changed;
     }
@@ -1177,7 +1192,7 @@ k_resident(Params p, Resident rs) {
     p.vv[n] = Vec3{v[0], v[1], v[2]};
   }
   if constexpr (PHYS == PHYS_EP) {
-    if (has_e) store_state<R>(p, es + el, q, pre.s, pre.ep, changed);
+    if (has_e) store_state<false, R>(state_block<R>(p, b, t), pre.s, pre.ep, changed);
     const unsigned long long nb = __ballot(has_e && pre.ep > R(0));
     if (has_word && (t & 63) == 0) p.yielded[yi] = nb;
   }
@@ -1710,18 +1725,24 @@ __global__ void __launch_bounds__(256) k_export_nodes(Params p, const int32_t *n
   if (o.m3) o.m3[i] = p.m[g];
 }
 
+// spos: per user element, its place in ep, in elements (nq points each, next
+// to each other) of the block layout; in the planes the device element
 template <typename R>
-__global__ void __launch_bounds__(256) k_export_elems(Params p, const int32_t *einv, double *sig,
+__global__ void __launch_bounds__(256) k_export_elems(Params p, const uint32_t *spos, double *sig,
                                                       double *ep) {
-  const long i = (long)blockIdx.x * 256 + threadIdx.x, ne = p.ne;
+  const long i = (long)blockIdx.x * 256 + threadIdx.x, ne = p.ne, ld = p.state_ld;
   const int w = 6 * p.nq;
   if (sig && i < ne * w) {
     const long e = i / w;
-    sig[i] = double(static_cast<const R *>(p.sig)[(i - e * w) * ne + einv[e]]);
+    const int q = (int)(i - e * w) / 6, c = (int)(i - e * w) - 6 * q;
+    const long at = ld ? (long)spos[e] * p.nq + q : spos[e];
+    sig[i] = double(static_cast<const R *>(
+        p.sig)[ld ? (at / ld) * 6 * ld + c * ld + at % ld : (6L * q + c) * ne + at]);
   }
   if (ep && i < ne * p.nq) {
     const long e = i / p.nq;
-    ep[i] = double(static_cast<const R *>(p.epbar)[(i - e * p.nq) * ne + einv[e]]);
+    const int q = (int)(i - e * p.nq);
+    ep[i] = double(static_cast<const R *>(p.epbar)[ld ? (long)spos[e] * p.nq + q : spos[e] + q * ne]);
   }
 }
 
@@ -2191,11 +2212,11 @@ hipError_t launch_export_nodes(const Params &p, const int32_t *ninv, const NodeE
   CPI_LAUNCH(k_export_nodes, (unsigned)((3L * p.nn + 255) / 256), 256, 0, s, p, ninv, o);
 }
 
-hipError_t launch_export_elems(const Params &p, int prec, const int32_t *einv, double *sig,
+hipError_t launch_export_elems(const Params &p, int prec, const uint32_t *spos, double *sig,
                                double *ep, hipStream_t s) {
   const unsigned grid = (unsigned)(((long)p.ne * p.nq * (sig ? 6 : 1) + 255) / 256);
-  if (prec == 1) CPI_LAUNCH(k_export_elems<float>, grid, 256, 0, s, p, einv, sig, ep);
-  CPI_LAUNCH(k_export_elems<double>, grid, 256, 0, s, p, einv, sig, ep);
+  if (prec == 1) CPI_LAUNCH(k_export_elems<float>, grid, 256, 0, s, p, spos, sig, ep);
+  CPI_LAUNCH(k_export_elems<double>, grid, 256, 0, s, p, spos, sig, ep);
 }
 
 hipError_t launch_reset_nodes(const Params &p, const Vec3 *v0, hipStream_t s) {
