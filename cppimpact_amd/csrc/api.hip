@@ -625,7 +625,7 @@ static int create_impl(cpi_ctx *c, const cpi_mesh_desc *m, const cpi_material *m
   }
   // device orders
   if (c->scatter == CPI_SCATTER_BLOCK) {
-    const int nt = elem_block_threads(npe, c->rule);
+    const int nt = elem_block_threads(npe, c->rule, c->prec, c->phys, 0);
     const int dflt = elem_block_default_elements(npe);
     int me = opt->block_elements > 0 ? opt->block_elements : dflt;
     // the tet4 kernel gives each thread one element and at most one node,
@@ -755,9 +755,10 @@ static int create_impl(cpi_ctx *c, const cpi_mesh_desc *m, const cpi_material *m
     char *s = nullptr, *q = nullptr;
     std::vector<uint32_t> spos(ne);
     c->state_points = c->nq * (size_t)ne;
-    if (c->scatter == CPI_SCATTER_BLOCK && (npe == 4 || c->nq == 4)) {
-      // rows of whole 128-byte lines in FP32; of blocks smaller than that,
-      // the next power of two (a row is never twice its block)
+    if (c->scatter == CPI_SCATTER_BLOCK) {
+      // rows of a multiple of 32 points (five-point rule: 40); of a block
+      // smaller than that, its points to the next power of two (times five),
+      // so a row is never twice its block
       const BlockPlan &B = c->plan;
       int row = c->nq;
       while (row < 32 && row < c->nq * B.max_block_elems) row *= 2;
@@ -795,9 +796,9 @@ static int create_impl(cpi_ctx *c, const cpi_mesh_desc *m, const cpi_material *m
   }
   if (c->scatter == CPI_SCATTER_BLOCK) {
     BlockPlan &B = c->plan;
-    if (npe == 4 && B.max_local_nodes > elem_block_threads(4, c->rule))
+    if (npe == 4 && B.max_local_nodes > elem_block_threads(4, c->rule, c->prec, c->phys, B.nblocks))
       return fail(c, CPI_ERR_INVALID, "partition: a tet4 block has more nodes than threads");
-    if (npe == 10 && c->nq == 4 && 4 * B.max_block_elems > elem_block_threads(10, c->rule))
+    if (npe == 10 && c->nq == 4 && 4 * B.max_block_elems > elem_block_threads(10, c->rule, c->prec, c->phys, B.nblocks))
       return fail(c, CPI_ERR_INVALID, "partition: a tet10 block has more points than threads");
     int32_t *meta, *bn, *bs, *sp, *dn, *ds;
     uint16_t *cl, *ci, *cw = nullptr, *dg, *dof;
@@ -892,7 +893,7 @@ static int create_impl(cpi_ctx *c, const cpi_mesh_desc *m, const cpi_material *m
       }
     }
     // one energy row per wave
-    c->n_elem_rows = c->nblocks * (elem_block_threads(npe, c->rule) / 64);
+    c->n_elem_rows = c->nblocks * (elem_block_threads(npe, c->rule, c->prec, c->phys, c->nblocks) / 64);
     c->n_node_rows = 4 * std::max(1, (B.n_boundary + 255) / 256);
   } else {
     const int nt = elem_direct_threads(npe);

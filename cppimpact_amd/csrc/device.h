@@ -207,7 +207,13 @@ __device__ __forceinline__ int xcd_remap(int hw, int n) {
 // DPP lane moves (the source lane must be active).  CTRL: 0xB1 lane ^ 1 and
 // 0x4E lane ^ 2 (quad_perm), 0x141 the mirror lane within each 8 lanes,
 // 0x140 the mirror lane within each row of 16.
-enum : int { kDppXor1 = 0xB1, kDppXor2 = 0x4E, kDppHalfMirror = 0x141, kDppMirror = 0x140 };
+enum : int {
+  kDppXor1 = 0xB1,
+  kDppXor2 = 0x4E,
+  kDppHalfMirror = 0x141,
+  kDppMirror = 0x140,
+  kDppBefore = 0x138  // the lane before (wave_shr:1)
+};
 template <int CTRL>
 __device__ __forceinline__ float dpp_mov(float v) {
   return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xF, 0xF, false));

@@ -400,85 +400,85 @@ __device__ __forceinline__ void tet10_dn(const R Ji[9], const G Gd[30], int i, R
 }
 
 // ---------------------------------------------------------------------------
-// tet10: loop over the rule's points with coordinates relative to corner 2
-// (the origin of the reference's quadratic parametrisation); nodes are
-// re-read through get() at every pass instead of being held in registers.
-// Corner forces accumulate through add(i, dN_i, sigma, w detJ), which adds
-// w detJ sigma . dN_i to node i's force, one point at a time in rule order.
+// tet10, one point of a rule, with coordinates relative to corner 2 (the
+// origin of the reference's quadratic parametrisation); nodes are re-read
+// through get() at every pass instead of being held in registers.  Node i's
+// sigma . dN_i and w detJ go to put(i, g, w detJ).  pre: the point's stress
+// state, loaded ahead (PRE).
 // ---------------------------------------------------------------------------
-template <int RULE, typename R, int PHYS, class Get, class Add>
-__device__ __forceinline__ void tet10_points(const Params &p, const Get &get, double dt, int e,
-                                             const Add &add, EAcc &ea) {
+template <int RULE, typename R, int PHYS, bool PRE, class At, class Get, class Put>
+__device__ __forceinline__ void tet10_point(const Params &p, const At &at, const Get &get,
+                                            double dt, int e, int q, const Put &put, EAcc &ea,
+                                            PreState<R> *pre = nullptr) {
+  using Q = Quad<RULE>;
   double o[3];
   {
     double ov[3];
     get(2, o, ov);
   }
-  using Q = Quad<RULE>;
-  // a rolled loop: unrolled, the compiler hoists every point's state loads
-  // and the kernel no longer fits the register file
-#pragma unroll 1
-  for (int q = 0; q < Q::n; q++) {
-    double Gd[30];
-    tet10_grad(Q::pt(q, 0), Q::pt(q, 1), Q::pt(q, 2), Gd);
-    R J[9] = {R(0), R(0), R(0), R(0), R(0), R(0), R(0), R(0), R(0)};
+  double Gd[30];
+  tet10_grad(Q::pt(q, 0), Q::pt(q, 1), Q::pt(q, 2), Gd);
+  R J[9] = {R(0), R(0), R(0), R(0), R(0), R(0), R(0), R(0), R(0)};
 #pragma unroll
-    for (int i = 0; i < 10; i++) {
-      double xi[3], vi[3];
-      get(i, xi, vi);
-      const R d[3] = {R(xi[0] - o[0]), R(xi[1] - o[1]), R(xi[2] - o[2])};
-      tet10_jac_add<R>(J, Gd, i, d);
-    }
-    R Ji[9];
-    R detJ = inv3<R>(J, Ji);
-    if (!(detJ > R(0))) ea.bad += 1.0;
-    R de[6] = {R(0), R(0), R(0), R(0), R(0), R(0)};
-#pragma unroll
-    for (int i = 0; i < 10; i++) {
-      double xi[3], vi[3];
-      get(i, xi, vi);
-      R u[3] = {R(dt * vi[0]), R(dt * vi[1]), R(dt * vi[2])};
-      R dn[3];
-      tet10_dn<R>(Ji, Gd, i, dn);
-      de[0] += dn[0] * u[0];
-      de[1] += dn[1] * u[1];
-      de[2] += dn[2] * u[2];
-      de[3] += dn[1] * u[0] + dn[0] * u[1];
-      de[4] += dn[2] * u[1] + dn[1] * u[2];
-      de[5] += dn[2] * u[0] + dn[0] * u[2];
-    }
-    R wd = R(Q::w(q)) * detJ;
-    R s[6];
-    point_stress<R, PHYS>(p, state_plane<R>(p, e, q), e, q, de, wd, s, ea);
-#pragma unroll
-    for (int i = 0; i < 10; i++) {
-      R dn[3];
-      tet10_dn<R>(Ji, Gd, i, dn);
-      add(i, dn, s, wd);
-    }
+  for (int i = 0; i < 10; i++) {
+    double xi[3], vi[3];
+    get(i, xi, vi);
+    const R d[3] = {R(xi[0] - o[0]), R(xi[1] - o[1]), R(xi[2] - o[2])};
+    tet10_jac_add<R>(J, Gd, i, d);
   }
-  if constexpr (PHYS != PHYS_COMPAT) {
-    // corners in the linear ordering: (2, 0, 1, 3) is an even permutation
-    R e1[3], e2[3], e3[3];
-    double xa[3], va[3];
-    get(0, xa, va);
+  R Ji[9];
+  R detJ = inv3<R>(J, Ji);
+  if (!(detJ > R(0))) ea.bad += 1.0;
+  R de[6] = {R(0), R(0), R(0), R(0), R(0), R(0)};
 #pragma unroll
-    for (int c = 0; c < 3; c++) e1[c] = R(xa[c] - o[c]);
-    get(1, xa, va);
+  for (int i = 0; i < 10; i++) {
+    double xi[3], vi[3];
+    get(i, xi, vi);
+    R u[3] = {R(dt * vi[0]), R(dt * vi[1]), R(dt * vi[2])};
+    R dn[3];
+    tet10_dn<R>(Ji, Gd, i, dn);
+    de[0] += dn[0] * u[0];
+    de[1] += dn[1] * u[1];
+    de[2] += dn[2] * u[2];
+    de[3] += dn[1] * u[0] + dn[0] * u[1];
+    de[4] += dn[2] * u[1] + dn[1] * u[2];
+    de[5] += dn[2] * u[0] + dn[0] * u[2];
+  }
+  R wd = R(Q::w(q)) * detJ;
+  R s[6];
+  point_stress<R, PHYS, PRE>(p, at, e, q, de, wd, s, ea, pre);
 #pragma unroll
-    for (int c = 0; c < 3; c++) e2[c] = R(xa[c] - o[c]);
-    get(3, xa, va);
-#pragma unroll
-    for (int c = 0; c < 3; c++) e3[c] = R(xa[c] - o[c]);
-    R v6 = e1[0] * (e2[1] * e3[2] - e2[2] * e3[1]) - e1[1] * (e2[0] * e3[2] - e2[2] * e3[0]) +
-           e1[2] * (e2[0] * e3[1] - e2[1] * e3[0]);
-    ea.mindt = fmin(ea.mindt, corner_dt<R>(e1, e2, e3, v6, p.wave_speed, kTet10LengthFactor));
+  for (int i = 0; i < 10; i++) {
+    R dn[3], g[3];
+    tet10_dn<R>(Ji, Gd, i, dn);
+    sig_dn<R>(dn, s, g);
+    put(i, g, wd);
   }
 }
 
-// tet10 on a 4-point rule with one lane per point: lanes 4k..4k+3 hold the
-// same element e, lane q = (lane & 3) point q.  All four lanes of a quad
-// must be active.  pre: the point's stress state, loaded ahead (EP models).
+// the stable dt of the corner tetrahedron
+template <typename R, class Get>
+__device__ __forceinline__ void tet10_stable_dt(const Params &p, const Get &get, EAcc &ea) {
+  // corners in the linear ordering: (2, 0, 1, 3) is an even permutation
+  R e1[3], e2[3], e3[3];
+  double o[3], xa[3], va[3];
+  get(2, o, va);
+  get(0, xa, va);
+#pragma unroll
+  for (int c = 0; c < 3; c++) e1[c] = R(xa[c] - o[c]);
+  get(1, xa, va);
+#pragma unroll
+  for (int c = 0; c < 3; c++) e2[c] = R(xa[c] - o[c]);
+  get(3, xa, va);
+#pragma unroll
+  for (int c = 0; c < 3; c++) e3[c] = R(xa[c] - o[c]);
+  R v6 = e1[0] * (e2[1] * e3[2] - e2[2] * e3[1]) - e1[1] * (e2[0] * e3[2] - e2[2] * e3[0]) +
+         e1[2] * (e2[0] * e3[1] - e2[1] * e3[0]);
+  ea.mindt = fmin(ea.mindt, corner_dt<R>(e1, e2, e3, v6, p.wave_speed, kTet10LengthFactor));
+}
+
+// tet10 with one lane per point: the lane's point q of element e.  pre: the
+// point's stress state, loaded ahead (EP models).
 //
 // The basis gradients of tet10_grad at a point, with a = 4 xi, b = 4 eta,
 // c = 4 zeta and l = 4 (1 - xi - eta - zeta), are
@@ -491,10 +491,9 @@ __device__ __forceinline__ void tet10_points(const Params &p, const Get &get, do
 //   Lv = sum_i v_i (x) G_i, grad v = Lv J^-1, de = dt sym(grad v)
 //   M  = w detJ sigma J^-T, f_i = M G_i      (= w detJ sigma . dN_i)
 // so a node's force is one or two products per component instead of the
-// gradient dN_i = J^-T G_i and sigma . dN_i.  Each corner force is then
-// summed over the quad's lanes as (q0 + q1) + (q2 + q3) (quad_sum, DPP
-// inside the quad), so every lane holds corner i's element force and hands
-// it to put(i, f).  DEFER: the updated state is left in pre (ep changed
+// gradient dN_i = J^-T G_i and sigma . dN_i.  The point's part of corner i's
+// force goes to put(i, f), which sums it over the element's lanes.  DEFER:
+// the updated state is left in pre (ep changed
 // in pre.changed) for the caller to store after everything else it does,
 // else it is stored here (STREAM: non-temporal): registers that a store
 // reads must not be reused before the store has completed, so a store
@@ -504,7 +503,6 @@ __device__ __forceinline__ void tet10_point_lane(const Params &p, const At &at, 
                                                  double dt, int e, int q, PreState<R> &pre, const Put &put,
                                                  EAcc &ea) {
   using Q = Quad<RULE>;
-  static_assert(Q::n == 4, "one lane per point of a 4-point rule");
   const double px = Q::pt(q, 0), py = Q::pt(q, 1), pz = Q::pt(q, 2);
   const R a = R(4.0 * px), b = R(4.0 * py), c = R(4.0 * pz);
   const R l = R(4.0 - 4.0 * px - 4.0 * py - 4.0 * pz);
@@ -683,10 +681,9 @@ __device__ __forceinline__ void tet10_point_lane(const Params &p, const At &at, 
 #pragma unroll
     for (int r = 0; r < 3; r++) S[r] = M[3 * r] + M[3 * r + 1] + M[3 * r + 2];
   }
-  // f_i = M G_i (f_5, f_6, f_9 through S = M (1, 1, 1)), summed over the
-  // element's points
+  // f_i = M G_i (f_5, f_6, f_9 through S = M (1, 1, 1))
   auto emit = [&](int i, R f0, R f1, R f2) {
-    const R f[3] = {quad_sum(f0), quad_sum(f1), quad_sum(f2)};
+    const R f[3] = {f0, f1, f2};
     put(i, f);
   };
   emit(0, am1() * M[0], am1() * M[3], am1() * M[6]);
@@ -701,15 +698,25 @@ __device__ __forceinline__ void tet10_point_lane(const Params &p, const At &at, 
   emit(9, l * M[2] - c * S[0], l * M[5] - c * S[1], l * M[8] - c * S[2]);
 }
 
-// tet10 with the corner forces summed in registers, handed to put() at the end
+// tet10, an element's points one after another, its corner forces summed in
+// registers and handed to put() at the end
 template <int RULE, typename R, int PHYS, class Get, class Put>
 __device__ __forceinline__ void tet10_core(const Params &p, const Get &get, double dt, int e,
                                            const Put &put, EAcc &ea) {
   R f[10][3];
 #pragma unroll
   for (int i = 0; i < 10; i++) f[i][0] = f[i][1] = f[i][2] = R(0);
-  auto add = [&](int i, const R dn[3], const R s[6], R wd) { add_bts<R>(f[i], dn, s, wd); };
-  tet10_points<RULE, R, PHYS>(p, get, dt, e, add, ea);
+  // a rolled loop: unrolled, the compiler hoists every point's state loads
+  // and the kernel no longer fits the register file
+#pragma unroll 1
+  for (int q = 0; q < Quad<RULE>::n; q++) {
+    auto add = [&](int i, const R g[3], R wd) {
+#pragma unroll
+      for (int c = 0; c < 3; c++) f[i][c] = fma(wd, g[c], f[i][c]);
+    };
+    tet10_point<RULE, R, PHYS, false>(p, state_plane<R>(p, e, q), get, dt, e, q, add, ea);
+  }
+  if constexpr (PHYS != PHYS_COMPAT) tet10_stable_dt<R>(p, get, ea);
 #pragma unroll
   for (int i = 0; i < 10; i++) put(i, f[i]);
 }

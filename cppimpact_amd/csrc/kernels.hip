@@ -321,63 +321,114 @@ __host__ __device__ constexpr int lds_force_bytes(int rsz, int npe, int max_el) 
 __host__ __device__ constexpr int lds_off_bytes(int kmax) { return lds_round16(2L * (kmax + 1)); }
 
 // ---------------------------------------------------------------------------
-// LDS-assembled element pass, tet10: loops over elements and nodes.  LDS:
-// node records (LNodes), corner forces [max_el*NPE][3] R in jagged-diagonal
-// slots (local node j's k-th contribution at off[k] + j), off[k].
+// LDS-assembled element pass, tet10 on the 5-point rule: five lanes per
+// element, one per point, twelve elements per wave (four lanes idle).  A
+// corner's force is the chain f = w_q detJ_q g_q + f over the points in rule
+// order, which every lane runs on the value of the lane before it: after
+// four steps the last point's lane has it, with the bits of one thread going
+// through the points.  FP64 takes tet10_point_lane's arithmetic (f_q = M G
+// summed in the same order); FP32 keeps tet10_point's, whose bits the direct
+// kernels share.  VALU-bound for a full chip.  Against one thread per element
+// looping over the points (128 threads): 13k elements FP64 compat 18.9 -> 9.4
+// us, FP32 15.6 -> 9.3, FP64 EP 23.2 -> 10.9; 663k elements 214 -> 141, FP32
+// 127 -> 114, FP64 EP 319 -> 230, FP32 EP 180 -> 154 us.
+// LDS: node records (LNodes), corner forces [max_el*10][3] R in jagged-
+// diagonal slots (local node j's k-th contribution at off[k] + j), off[k].
 // ---------------------------------------------------------------------------
-template <int NPE, int RULE, typename R, int PHYS, bool AUX, int NT>
-__global__ void __launch_bounds__(NT) k_elem_block(Params p) {
+template <int RULE, typename R, int PHYS, bool AUX, int NT, int WPE>
+__global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WPE)))
+k_elem_block5(Params p) {
   extern __shared__ double smem[];
+  constexpr int NQ = Quad<RULE>::n, EW = 64 / NQ, EB = NT / 64 * EW;
   const int b = xcd_remap(blockIdx.x, gridDim.x);
-  const RowPre row = row_prefetch(p, p.epart_base + b * (NT / 64));
+  RowPre row = row_prefetch(p, p.epart_base + b * (NT / 64));
   const int32_t *mt = p.meta + 8 * b;
   const int es = mt[0], nel = mt[1];
   const int ml = p.ml;
   const int32_t *nid = p.nid_pad + (long)b * ml;
   const LNodes ln{smem, ml};
   R *lf = (R *)((char *)smem + lds_node_bytes(ml));
-  uint16_t *joff = (uint16_t *)((char *)lf + lds_force_bytes(sizeof(R), NPE, p.max_el));
+  uint16_t *joff = (uint16_t *)((char *)lf + lds_force_bytes(sizeof(R), 10, p.max_el));
   const double dt = p.ctl->dt;
+  const int lane = threadIdx.x & 63, q = lane % NQ, te = (threadIdx.x >> 6) * EW + lane / NQ;
 
+  // a thread's element words, local ids and slots two per word (rows of 20
+  // bytes), and its point's state: the first element's before the nodes are
+  // waited for, and the first node's places in the assembly too
+  uint32_t lw[5], pw[5];
+  PreState<R> pre;
+  auto ahead = [&](int t) {
+    const long e = es + (t < nel ? t : nel - 1);
+#pragma unroll
+    for (int k = 0; k < 5; k++) {
+      lw[k] = reinterpret_cast<const uint32_t *>(p.conn_local + 10L * e)[k];
+      pw[k] = reinterpret_cast<const uint32_t *>(p.csr_pos + 10L * e)[k];
+    }
+    if constexpr (PHYS != PHYS_COMPAT)
+      load_state<false, R>(state_block<R>(p, b, NQ * t + q), true, pre);
+  };
+  const long o = (long)b * ml;
+  const int j0 = threadIdx.x < ml ? threadIdx.x : ml - 1;
+  const int g0 = nid[j0], slot0 = p.slot_pad[o + j0], deg0 = p.deg_pad[o + j0];
+  ahead(te);
   for (int j = threadIdx.x; j < ml; j += NT) {
-    const int g = nid[j];
+    const int g = j == threadIdx.x ? g0 : nid[j];
     if (g >= 0) ln.stage(j, p.pos[g], p.m[g], p.vv[g]);
   }
   for (int k = threadIdx.x; k <= p.kmax; k += NT) joff[k] = p.off_pad[(long)b * (p.kmax + 1) + k];
   __syncthreads();
 
   EAcc ea;
-  for (int t = threadIdx.x; t < nel; t += NT) {
+  for (int t = te; lane < NQ * EW && t < nel; t += EB) {
     const int e = es + t;
-    const uint16_t *lc = p.conn_local + (long)e * NPE;
-    const uint16_t *pos = p.csr_pos + (long)e * NPE;
-    auto get = [&](int k, double xk[3], double vk[3]) { ln.get(lc[k], xk, vk); };
-    // the element's corner slots belong to this thread alone: its forces
-    // accumulate there point by point instead of in registers
-#pragma unroll
-    for (int k = 0; k < NPE; k++) {
-      R *dst = lf + 3 * pos[k];
-      dst[0] = dst[1] = dst[2] = R(0);
-    }
-    auto add = [&](int k, const R dn[3], const R s[6], R wd) {
-      R *dst = lf + 3 * pos[k];
-      R fk[3] = {dst[0], dst[1], dst[2]};
-      add_bts<R>(fk, dn, s, wd);
-      dst[0] = fk[0];
-      dst[1] = fk[1];
-      dst[2] = fk[2];
+    if (t != te) ahead(t);
+    const StateBlock<R> at = state_block<R>(p, b, NQ * t + q);
+    auto half = [](const uint32_t w[5], int k) {
+      return (int)((w[k >> 1] >> (16 * (k & 1))) & 0xffffu);
     };
-    tet10_points<RULE, R, PHYS>(p, get, dt, e, add, ea);
+    auto get = [&](int k, double xk[3], double vk[3]) { ln.get(half(lw, k), xk, vk); };
+    auto store = [&](int k, const R f[3]) {
+      if (q == NQ - 1) {
+        R *dst = lf + 3 * half(pw, k);
+#pragma unroll
+        for (int c = 0; c < 3; c++) dst[c] = f[c];
+      }
+    };
+    if constexpr (sizeof(R) == 8) {
+      auto put = [&](int k, const R fq[3]) {
+        R f[3] = {fq[0], fq[1], fq[2]};
+#pragma unroll
+        for (int s = 1; s < NQ; s++)
+#pragma unroll
+          for (int c = 0; c < 3; c++) f[c] = fq[c] + dpp_mov<kDppBefore>(f[c]);
+        store(k, f);
+      };
+      tet10_point_lane<RULE, R, PHYS, false, false>(p, at, get, dt, e, q, pre, put, ea);
+    } else {
+      auto put = [&](int k, const R g[3], R wd) {
+        R f[3];
+#pragma unroll
+        for (int c = 0; c < 3; c++) f[c] = fma(wd, g[c], R(0));
+#pragma unroll
+        for (int s = 1; s < NQ; s++)
+#pragma unroll
+          for (int c = 0; c < 3; c++) f[c] = fma(wd, g[c], dpp_mov<kDppBefore>(f[c]));
+        store(k, f);
+      };
+      tet10_point<RULE, R, PHYS, true>(p, at, get, dt, e, q, put, ea, &pre);
+      if constexpr (PHYS != PHYS_COMPAT)
+        if (q == 0) tet10_stable_dt<R>(p, get, ea);
+    }
   }
   __syncthreads();
 
   for (int j = threadIdx.x; j < ml; j += NT) {
-    const int g = nid[j];
+    const bool first = j == threadIdx.x;
+    const int g = first ? g0 : nid[j];
     if (g < 0) continue;
-    const int deg = p.deg_pad[(long)b * ml + j];
     double f[3];
-    node_force_sum<R>(lf, joff, j, deg, f);
-    const int slot = p.slot_pad[(long)b * ml + j];
+    node_force_sum<R>(lf, joff, j, first ? deg0 : p.deg_pad[o + j], f);
+    const int slot = first ? slot0 : p.slot_pad[o + j];
     if (slot < 0) {
       double x[3], v[3];
       ln.get(j, x, v);
@@ -400,8 +451,8 @@ __global__ void __launch_bounds__(NT) k_elem_block(Params p) {
 // only LDS and its registers.  Corner k's element force (summed over the
 // element's four lanes in rule order) is stored by lane k & 3 into the
 // corner's jagged-diagonal slot, off[rank] + local node; the nodes are then
-// assembled as in k_elem_block, and the point's state is stored last.  LDS
-// as k_elem_block.
+// assembled as in k_elem_block5, and the point's state is stored last.  LDS
+// as k_elem_block5.
 template <int RULE, typename R, int PHYS, bool AUX, int NT, int WPE, bool STREAM>
 __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WPE)))
 k_elem_block10(Params p) {
@@ -471,7 +522,8 @@ k_elem_block10(Params p) {
       const int h = (int)((wj >> (16 * (q & 1))) & 0xffffu);
       sl[j] = (int)joff[h >> 9] + (h & 511);
     }
-    auto put = [&](int k, const R f[3]) {
+    auto put = [&](int k, const R fq[3]) {
+      const R f[3] = {quad_sum(fq[0]), quad_sum(fq[1]), quad_sum(fq[2])};
       if ((k & 3) == q) {
         R *dst = lf + 3 * sl[k >> 2];
         dst[0] = f[0];
@@ -1090,7 +1142,8 @@ k_resident(Params p, Resident rs) {
           const uint32_t wj = (qs >> 1) ? cw[j == 2 ? 4 : 2 * j + 1] : cw[2 * j];
           sl[j] = slot_of((int)((wj >> (16 * (qs & 1))) & 0xffffu));
         }
-        auto put = [&](int k, const R f[3]) {
+        auto put = [&](int k, const R fq[3]) {
+          const R f[3] = {quad_sum(fq[0]), quad_sum(fq[1]), quad_sum(fq[2])};
           if ((k & 3) == qs) {
             R *dst = lf + 3 * sl[k >> 2];
             dst[0] = f[0];
@@ -1813,15 +1866,30 @@ static inline void timed_launch(K kern, dim3 grid, dim3 block, size_t smem, hipS
   } while (0)
 
 // threads per workgroup of the block kernels: tet4 one per element (384),
-// tet10 on a 4-point rule one per point (512 for 128 elements), tet10 on
-// the 5-point rule one per element (128)
+// tet10 one per point (512 for 128 elements; on the five-point rule, twelve
+// elements per wave, 704)
 template <int NPE, int RULE> constexpr int block_threads() {
-  return NPE == 4 ? 384 : (Quad<RULE>::n == 4 ? 512 : 128);
+  return NPE == 4 ? 384 : (Quad<RULE>::n == 4 ? 512 : 704);
 }
 // default elements per workgroup
 constexpr int block_elements(int npe) { return npe == 4 ? 384 : 128; }
 // minimum waves per SIMD of the per-point tet10 kernel
 template <typename R> constexpr int tet10_waves() { return 4; }
+
+// Threads of the 5-point tet10 kernel.  Up to one block per CU a step takes
+// as long as one block does, and 704 threads do its 128 elements in one round
+// (13k elements, FP64 compat: 9.5 us, 384 threads 12.2).  With more blocks 384
+// threads, two rounds, leave room for more workgroups per CU and one's loads
+// overlap another's arithmetic (663k elements: FP64 compat 141 us against 153,
+// FP32 114 against 139, FP32 EP 154 against 170), but FP64 EP takes 148 VGPRs,
+// three waves per SIMD, where a second 6-wave workgroup often finds no room:
+// 259 us against 230.
+constexpr int kNarrow5 = 384;
+static bool narrow5(int nblocks, bool f64_state) { return nblocks > 256 && !f64_state; }
+// its waves per SIMD: FP64 with a state takes 144 VGPRs
+template <typename R, int PHYS> constexpr int tet10_waves5() {
+  return sizeof(R) == 8 && PHYS != PHYS_COMPAT ? 3 : 4;
+}
 
 // minimum waves per SIMD the tet4 element kernels are compiled for: FP64
 // fits 96 VGPRs (three 6-wave workgroups per CU), FP32 64 (five per CU);
@@ -1847,9 +1915,12 @@ size_t elem_block_smem(int npe, int prec, int, int ml, int max_el, int kmax) {
   return (size_t)lds_node_bytes(ml) + lds_force_bytes(rsz, npe, max_el) + lds_off_bytes(kmax);
 }
 
-int elem_block_threads(int npe, int rule) {
+int elem_block_threads(int npe, int rule, int prec, int phys, int nblocks) {
   if (npe == 4) return block_threads<4, RULE_CENTROID>();
-  return rule == RULE_REF5 ? block_threads<10, RULE_REF5>() : block_threads<10, RULE_EXACT4>();
+  if (rule == RULE_REF5)
+    return narrow5(nblocks, prec != 1 && phys != PHYS_COMPAT) ? kNarrow5
+                                                              : block_threads<10, RULE_REF5>();
+  return block_threads<10, RULE_EXACT4>();
 }
 
 int elem_block_default_elements(int npe) { return block_elements(npe); }
@@ -1944,8 +2015,14 @@ static hipError_t elem_block_t(const Params &p, bool aux, int nblocks, size_t sm
     if (aux) CPI_LAUNCH((k_elem_block10<RULE, R, PHYS, true, NT, W, false>), nblocks, NT, smem, s, p);
     CPI_LAUNCH((k_elem_block10<RULE, R, PHYS, false, NT, W, false>), nblocks, NT, smem, s, p);
   } else {
-    if (aux) CPI_LAUNCH((k_elem_block<NPE, RULE, R, PHYS, true, NT>), nblocks, NT, smem, s, p);
-    CPI_LAUNCH((k_elem_block<NPE, RULE, R, PHYS, false, NT>), nblocks, NT, smem, s, p);
+    constexpr int W = tet10_waves5<R, PHYS>();
+    if (narrow5(nblocks, sizeof(R) == 8 && PHYS != PHYS_COMPAT)) {
+      constexpr int N2 = kNarrow5;
+      if (aux) CPI_LAUNCH((k_elem_block5<RULE, R, PHYS, true, N2, W>), nblocks, N2, smem, s, p);
+      CPI_LAUNCH((k_elem_block5<RULE, R, PHYS, false, N2, W>), nblocks, N2, smem, s, p);
+    }
+    if (aux) CPI_LAUNCH((k_elem_block5<RULE, R, PHYS, true, NT, W>), nblocks, NT, smem, s, p);
+    CPI_LAUNCH((k_elem_block5<RULE, R, PHYS, false, NT, W>), nblocks, NT, smem, s, p);
   }
 }
 
@@ -2023,9 +2100,12 @@ template <int NPE, int RULE, typename R, int PHYS> struct ElemBlockPrepF {
         }
         return e;
       } else {
-        hipError_t e = lds_opt_in(k_elem_block<NPE, RULE, R, PHYS, true, NT>, smem);
-        if (e != hipSuccess) return e;
-        return lds_opt_in(k_elem_block<NPE, RULE, R, PHYS, false, NT>, smem);
+        constexpr int W = tet10_waves5<R, PHYS>();
+        hipError_t e = lds_opt_in(k_elem_block5<RULE, R, PHYS, true, NT, W>, smem);
+        if (e == hipSuccess) e = lds_opt_in(k_elem_block5<RULE, R, PHYS, false, NT, W>, smem);
+        if (e == hipSuccess) e = lds_opt_in(k_elem_block5<RULE, R, PHYS, true, kNarrow5, W>, smem);
+        if (e == hipSuccess) e = lds_opt_in(k_elem_block5<RULE, R, PHYS, false, kNarrow5, W>, smem);
+        return e;
       }
     }
   }
