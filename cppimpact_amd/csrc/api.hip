@@ -641,7 +641,7 @@ static int create_impl(cpi_ctx *c, const cpi_mesh_desc *m, const cpi_material *m
     // per node)
     const long share = npe == 4 ? (c->prec == CPI_PREC_F32 ? 40960 : 54272) : 81920;
     const long budget = std::min<long>((long)prop.sharedMemPerBlock, share);
-    const long fixed = (long)elem_block_smem(npe, c->prec, c->phys, 0, me, 64);
+    const long fixed = (long)elem_block_smem(npe, c->rule, c->prec, 0, me, 64);
     long mnl = (budget - fixed - 16) / 56;
     if (mnl < 4L * npe)
       return fail(c, CPI_ERR_INVALID, "block_elements " + std::to_string(me) +
@@ -756,12 +756,12 @@ static int create_impl(cpi_ctx *c, const cpi_mesh_desc *m, const cpi_material *m
     std::vector<uint32_t> spos(ne);
     c->state_points = c->nq * (size_t)ne;
     if (c->scatter == CPI_SCATTER_BLOCK) {
-      // rows of a multiple of 32 points (five-point rule: 40); of a block
+      // rows of a multiple of 64 points (five-point rule: 80); of a block
       // smaller than that, its points to the next power of two (times five),
       // so a row is never twice its block
       const BlockPlan &B = c->plan;
       int row = c->nq;
-      while (row < 32 && row < c->nq * B.max_block_elems) row *= 2;
+      while (row < 64 && row < c->nq * B.max_block_elems) row *= 2;
       P.state_ld = (c->nq * B.max_block_elems + row - 1) / row * row;
       c->state_points = (size_t)B.nblocks * P.state_ld;
       if (c->state_points / c->nq > UINT32_MAX)
@@ -861,7 +861,15 @@ static int create_impl(cpi_ctx *c, const cpi_mesh_desc *m, const cpi_material *m
       P.mlp_rows = rows;
     }
     P.nblocks = B.nblocks;
-    c->smem = elem_block_smem(npe, c->prec, c->phys, P.ml, P.max_el, P.kmax);
+    // FP64 tet10 on a 4-point rule: the matrix units sum the corner forces
+    // while the chip is not full twice over (whose blocks may be resident).
+    // There the arithmetic counts (48k elements, resident: 13.1 -> 10.2 us a
+    // step, 48 spilled registers down to 4); a larger mesh is bound by its state's
+    // traffic, and sixteen elements a wave meet twice the LDS bank conflicts of
+    // quads (1.2M elements: 165 us with quads, 170).
+    P.matrix = npe == 10 && c->nq == 4 && c->prec != CPI_PREC_F32 &&
+               B.nblocks <= 2 * prop.multiProcessorCount;
+    c->smem = elem_block_smem(npe, c->rule, c->prec, P.ml, P.max_el, P.kmax);
     if (c->smem > (size_t)prop.sharedMemPerBlock)
       return fail(c, CPI_ERR_INVALID, "element block needs " + std::to_string(c->smem) +
                                           " bytes of LDS; lower block_elements");
@@ -870,7 +878,8 @@ static int create_impl(cpi_ctx *c, const cpi_mesh_desc *m, const cpi_material *m
       return fail(c, CPI_ERR_HIP, std::string("LDS opt-in for the element kernel: ") +
                                       hipGetErrorString(pe));
     // resident steps when every block fits the chip at once
-    if (opt->use_graph && c->phys != 2 && words && prop.cooperativeLaunch) {
+    if (opt->use_graph && c->phys != 2 && words && prop.cooperativeLaunch &&
+        (npe == 4 || c->prec == CPI_PREC_F32 || P.matrix)) {
       const MailPlan M = build_mail(B);
       const size_t n = M.dest.size(), bytes = mail_bytes(c->prec, n);
       const size_t smem = resident_smem(c->smem, c->prec, M.most);

@@ -99,6 +99,9 @@ struct Params {
   void *sig;
   void *epbar;
   int state_ld;
+  // FP64 per-point tet10 kernels: corner forces on the matrix units
+  // (tet10_wave_forces) instead of over quads of lanes
+  int matrix;
   // tet4 and per-point tet10 block kernels, exact return: one bit per
   // stress point, set once it has yielded (ep > 0), ywords 64-bit words per
   // block (the point of thread t of block b at word b*ywords + t/64, bit
@@ -274,7 +277,7 @@ __device__ __forceinline__ R inv3(const R J[9], R Ji[9]) {
 
 // quadratic basis gradients at (x,y,z), tetrahedral.h:199-250 layout
 template <typename T>
-__device__ __forceinline__ void tet10_grad(T x, T y, T z, T G[30]) {
+__host__ __device__ constexpr __forceinline__ void tet10_grad(T x, T y, T z, T G[30]) {
   G[0] = 4 * x - 1; G[1] = 0.0; G[2] = 0.0;
   G[3] = 0.0; G[4] = 4 * y - 1; G[5] = 0.0;
   G[6] = 4 * x + 4 * y + 4 * z - 3;

@@ -20,29 +20,29 @@ enum : int { RULE_REF5 = 0, RULE_REF4 = 1, RULE_EXACT4 = 2, RULE_CENTROID = 3 };
 template <int RULE> struct Quad;
 template <> struct Quad<RULE_REF5> {  // tetrahedral.h:12-40
   static constexpr int n = 5;
-  __device__ static constexpr double w(int q) { return q == 0 ? -0.13333333333 : 0.075; }
-  __device__ static constexpr double pt(int q, int c) {
+  __host__ __device__ static constexpr double w(int q) { return q == 0 ? -0.13333333333 : 0.075; }
+  __host__ __device__ static constexpr double pt(int q, int c) {
     return q == 0 ? 0.25 : (q - 1 == c ? 0.5 : 0.16666666666);
   }
 };
 template <> struct Quad<RULE_REF4> {  // tetrahedral.h:48-73
   static constexpr int n = 4;
-  __device__ static constexpr double w(int) { return 0.041666667; }
-  __device__ static constexpr double pt(int q, int c) {
+  __host__ __device__ static constexpr double w(int) { return 0.041666667; }
+  __host__ __device__ static constexpr double pt(int q, int c) {
     return (q >= 1 && q - 1 == c) ? 0.58541020 : 0.13819660;
   }
 };
 template <> struct Quad<RULE_EXACT4> {  // alpha = (5+3 sqrt5)/20, beta = (5-sqrt5)/20
   static constexpr int n = 4;
-  __device__ static constexpr double w(int) { return 1.0 / 24.0; }
-  __device__ static constexpr double pt(int q, int c) {
+  __host__ __device__ static constexpr double w(int) { return 1.0 / 24.0; }
+  __host__ __device__ static constexpr double pt(int q, int c) {
     return (q >= 1 && q - 1 == c) ? 0.58541019662496845446 : 0.13819660112501051518;
   }
 };
 template <> struct Quad<RULE_CENTROID> {
   static constexpr int n = 1;
-  __device__ static constexpr double w(int) { return 1.0 / 6.0; }
-  __device__ static constexpr double pt(int, int) { return 0.25; }
+  __host__ __device__ static constexpr double w(int) { return 1.0 / 6.0; }
+  __host__ __device__ static constexpr double pt(int, int) { return 0.25; }
 };
 
 // Where a point's stress state lies.  The kernels with a thread per point
@@ -117,7 +117,7 @@ template <typename R> struct StateBlock {
     st<STREAM>(ep, off, 0, v);
   }
 };
-// b: uniform; threads past the block's row take its last place
+// b: uniform; places past the block's row are its last one
 template <typename R>
 __device__ __forceinline__ StateBlock<R> state_block(const Params &p, int b, int t) {
   const int row = p.state_ld * (int)sizeof(R);
@@ -349,7 +349,7 @@ __device__ __forceinline__ void tet4_forces(const R Ji[9], const R s[6], R wd, c
 // the rule enters only through its weight sum (compat) and the element keeps
 // one stress point (ep).  Corner forces reach put() as soon as known.
 // STREAM: the state is read and written non-temporal.  DEFER: the updated
-// state is left in pre, as in tet10_point_lane.
+// state is left in pre, as in tet10_point_stress.
 // ---------------------------------------------------------------------------
 template <typename R, int PHYS, bool PRE, bool STREAM = false, bool DEFER = false, class At,
           class Get, class Put>
@@ -491,17 +491,17 @@ __device__ __forceinline__ void tet10_stable_dt(const Params &p, const Get &get,
 //   Lv = sum_i v_i (x) G_i, grad v = Lv J^-1, de = dt sym(grad v)
 //   M  = w detJ sigma J^-T, f_i = M G_i      (= w detJ sigma . dN_i)
 // so a node's force is one or two products per component instead of the
-// gradient dN_i = J^-T G_i and sigma . dN_i.  The point's part of corner i's
-// force goes to put(i, f), which sums it over the element's lanes.  DEFER:
-// the updated state is left in pre (ep changed
+// gradient dN_i = J^-T G_i and sigma . dN_i: tet10_point_kin gives J^-1,
+// det J and Lv, tet10_point_stress M, tet10_point_forces (a wave's at once:
+// tet10_wave_forces) the M G_i.
+// DEFER: the updated state is left in pre (ep changed
 // in pre.changed) for the caller to store after everything else it does,
 // else it is stored here (STREAM: non-temporal): registers that a store
 // reads must not be reused before the store has completed, so a store
 // issued here makes the rest of the kernel wait for it.
-template <int RULE, typename R, int PHYS, bool STREAM, bool DEFER, class At, class Get, class Put>
-__device__ __forceinline__ void tet10_point_lane(const Params &p, const At &at, const Get &get,
-                                                 double dt, int e, int q, PreState<R> &pre, const Put &put,
-                                                 EAcc &ea) {
+template <int RULE, typename R, int PHYS, class Get>
+__device__ __forceinline__ R tet10_point_kin(const Params &p, const Get &get, int q, R Ji[9],
+                                             R Lv[9], EAcc &ea) {
   using Q = Quad<RULE>;
   const double px = Q::pt(q, 0), py = Q::pt(q, 1), pz = Q::pt(q, 2);
   const R a = R(4.0 * px), b = R(4.0 * py), c = R(4.0 * pz);
@@ -591,11 +591,10 @@ __device__ __forceinline__ void tet10_point_lane(const Params &p, const At &at, 
       J[3 * r + 2] += lc() * d[r];
     }
   }
-  R Ji[9];
   const R detJ = inv3<R>(J, Ji);
-  if (!(detJ > R(0))) ea.bad += 1.0;
   // Lv[r][k] = d v_r / d xi_k
-  R Lv[9] = {R(0), R(0), R(0), R(0), R(0), R(0), R(0), R(0), R(0)};
+#pragma unroll
+  for (int k = 0; k < 9; k++) Lv[k] = R(0);
   {
     R u[3];
     vel(0, u);
@@ -654,6 +653,15 @@ __device__ __forceinline__ void tet10_point_lane(const Params &p, const At &at, 
       Lv[3 * r + 2] += lc() * u[r];
     }
   }
+  return detJ;
+}
+
+template <int RULE, typename R, int PHYS, bool STREAM, bool DEFER, class At>
+__device__ __forceinline__ void tet10_point_stress(const Params &p, const At &at, double dt, int e,
+                                                   int q, PreState<R> &pre, const R Ji[9], R detJ,
+                                                   const R Lv[9], R M[9], EAcc &ea) {
+  using Q = Quad<RULE>;
+  if (!(detJ > R(0))) ea.bad += 1.0;
   // grad v[r][s] = sum_k Lv[r][k] Ji[k][s]; engineering shear
   auto gv = [&](int r, int s) {
     return Lv[3 * r] * Ji[s] + Lv[3 * r + 1] * Ji[3 + s] + Lv[3 * r + 2] * Ji[6 + s];
@@ -667,21 +675,32 @@ __device__ __forceinline__ void tet10_point_lane(const Params &p, const At &at, 
   point_stress<R, PHYS, true, STREAM, DEFER>(p, at, e, q, de, wd, s, ea, &pre);
   // M[r][k] = sum_t (w detJ sigma)[r][t] Ji[k][t], sigma rows (s0 s3 s5),
   // (s3 s1 s4), (s5 s4 s2)
-  R M[9], S[3];
-  {
-    R w[6];
+  R w[6];
 #pragma unroll
-    for (int k = 0; k < 6; k++) w[k] = wd * s[k];
+  for (int k = 0; k < 6; k++) w[k] = wd * s[k];
 #pragma unroll
-    for (int k = 0; k < 3; k++) {
-      M[k] = w[0] * Ji[3 * k] + w[3] * Ji[3 * k + 1] + w[5] * Ji[3 * k + 2];
-      M[3 + k] = w[3] * Ji[3 * k] + w[1] * Ji[3 * k + 1] + w[4] * Ji[3 * k + 2];
-      M[6 + k] = w[5] * Ji[3 * k] + w[4] * Ji[3 * k + 1] + w[2] * Ji[3 * k + 2];
-    }
-#pragma unroll
-    for (int r = 0; r < 3; r++) S[r] = M[3 * r] + M[3 * r + 1] + M[3 * r + 2];
+  for (int k = 0; k < 3; k++) {
+    M[k] = w[0] * Ji[3 * k] + w[3] * Ji[3 * k + 1] + w[5] * Ji[3 * k + 2];
+    M[3 + k] = w[3] * Ji[3 * k] + w[1] * Ji[3 * k + 1] + w[4] * Ji[3 * k + 2];
+    M[6 + k] = w[5] * Ji[3 * k] + w[4] * Ji[3 * k + 1] + w[2] * Ji[3 * k + 2];
   }
-  // f_i = M G_i (f_5, f_6, f_9 through S = M (1, 1, 1))
+}
+
+// The forces M G_i of one point, handed to put(i, f) for the caller to sum
+// over the element's points (f_5, f_6, f_9 through S = M (1, 1, 1))
+template <int RULE, typename R, class Put>
+__device__ __forceinline__ void tet10_point_forces(int q, const R M[9], const Put &put) {
+  using Q = Quad<RULE>;
+  const double px = Q::pt(q, 0), py = Q::pt(q, 1), pz = Q::pt(q, 2);
+  const R a = R(4.0 * px), b = R(4.0 * py), c = R(4.0 * pz);
+  const R l = R(4.0 - 4.0 * px - 4.0 * py - 4.0 * pz);
+  R S[3];
+#pragma unroll
+  for (int r = 0; r < 3; r++) S[r] = M[3 * r] + M[3 * r + 1] + M[3 * r + 2];
+  auto am1 = [&]() { return a - R(1); };
+  auto bm1 = [&]() { return b - R(1); };
+  auto cm1 = [&]() { return c - R(1); };
+  auto l1 = [&]() { return R(1) - l; };
   auto emit = [&](int i, R f0, R f1, R f2) {
     const R f[3] = {f0, f1, f2};
     put(i, f);
@@ -697,6 +716,65 @@ __device__ __forceinline__ void tet10_point_lane(const Params &p, const At &at, 
   emit(8, c * M[1] + b * M[2], c * M[4] + b * M[5], c * M[7] + b * M[8]);
   emit(9, l * M[2] - c * S[0], l * M[5] - c * S[1], l * M[8] - c * S[2]);
 }
+
+// The forces of a wave of 16 elements on a 4-point rule (FP64), on the matrix
+// units.  Lane e + 16 q holds M of element e's point q, which is how
+// v_mfma_f64_4x4x4_4b reads its B operand (B[k][n] of block n' at lane
+// 16 k + 4 n' + n) and writes its result: with A[i][q] = G_{4g+i}(q)[k], the
+// same for the four blocks, the sum over k of three products leaves in lane
+// e + 16 i component r of corner 4g + i's force of element e, summed over the
+// points: 27 instructions for the 30 forces and no move between lanes, where
+// the quads below take 60 products and 180 moves and adds.  A is read from
+// LDS (Tet10Basis).  All lanes of the wave run it; what lanes without an
+// element hold stays in their own columns.  (The same for J and Lv, 54
+// instructions with four node reads a lane instead of ten, is slower: 13.8
+// us a resident step of 48k elements against 10.2, its operands spill.)
+template <int RULE> struct Tet10Basis {
+  static constexpr int n = 144;  // G_{4g+i}(q)[k] at 48 k + 16 g + 4 q + i, zero past node 9
+  double v[n];
+  __host__ __device__ constexpr Tet10Basis() : v{} {
+    for (int q = 0; q < 4; q++) {
+      double G[30] = {};
+      tet10_grad(Quad<RULE>::pt(q, 0), Quad<RULE>::pt(q, 1), Quad<RULE>::pt(q, 2), G);
+      for (int i = 0; i < 10; i++)
+        for (int k = 0; k < 3; k++) v[48 * k + 16 * (i >> 2) + 4 * q + (i & 3)] = G[3 * i + k];
+    }
+  }
+};
+template <int RULE> __device__ const Tet10Basis<RULE> tet10_basis{};
+
+template <class Put>
+__device__ __forceinline__ void tet10_wave_forces(const double *basis, int lane, const double M[9],
+                                                  const Put &put) {
+  const double *A = basis + 4 * (lane >> 4) + (lane & 3);
+#pragma unroll
+  for (int g = 0; g < 3; g++) {
+    double f[3] = {0.0, 0.0, 0.0};
+#pragma unroll
+    for (int k = 0; k < 3; k++)
+#pragma unroll
+      for (int r = 0; r < 3; r++)
+        f[r] = __builtin_amdgcn_mfma_f64_4x4x4f64(A[48 * k + 16 * g], M[3 * r + k], f[r], 0, 0, 0);
+    put(g, f);
+  }
+}
+
+// Which point a thread of the per-point kernels of the 4-point rules takes:
+// MM, as tet10_wave_forces wants it, sixteen elements per wave; else a quad
+// per element, whose sum (q0 + q1) + (q2 + q3) DPP moves inside the quad give.
+// place: the point's place in the block's state row, the thread's number; with
+// MM a row shorter than a wave holds its few elements' points a quarter of
+// the row apart.
+template <bool MM> struct PointLane {
+  int q, el;
+  __device__ __forceinline__ explicit PointLane(int t)
+      : q(MM ? (t >> 4) & 3 : t & 3), el(MM ? ((t >> 6) << 4) | (t & 15) : t >> 2) {}
+  __device__ __forceinline__ int place(const Params &p) const {
+    if (!MM) return 4 * el + q;
+    const int w = p.state_ld < 64 ? p.state_ld >> 2 : 16;
+    return 64 * (el >> 4) + q * w + ((el & 15) < w ? el & 15 : w - 1);
+  }
+};
 
 // tet10, an element's points one after another, its corner forces summed in
 // registers and handed to put() at the end

@@ -319,6 +319,9 @@ __host__ __device__ constexpr int lds_force_bytes(int rsz, int npe, int max_el) 
   return lds_round16((long)rsz * 3 * npe * max_el);
 }
 __host__ __device__ constexpr int lds_off_bytes(int kmax) { return lds_round16(2L * (kmax + 1)); }
+__host__ __device__ constexpr int lds_basis_bytes(int npe, int rsz, int points) {
+  return npe == 10 && rsz == 8 && points == 4 ? 8 * Tet10Basis<RULE_EXACT4>::n : 0;
+}
 
 // ---------------------------------------------------------------------------
 // LDS-assembled element pass, tet10 on the 5-point rule: five lanes per
@@ -326,7 +329,7 @@ __host__ __device__ constexpr int lds_off_bytes(int kmax) { return lds_round16(2
 // corner's force is the chain f = w_q detJ_q g_q + f over the points in rule
 // order, which every lane runs on the value of the lane before it: after
 // four steps the last point's lane has it, with the bits of one thread going
-// through the points.  FP64 takes tet10_point_lane's arithmetic (f_q = M G
+// through the points.  FP64 takes tet10_point_kin's arithmetic (f_q = M G
 // summed in the same order); FP32 keeps tet10_point's, whose bits the direct
 // kernels share.  VALU-bound for a full chip.  Against one thread per element
 // looping over the points (128 threads): 13k elements FP64 compat 18.9 -> 9.4
@@ -403,7 +406,10 @@ k_elem_block5(Params p) {
           for (int c = 0; c < 3; c++) f[c] = fq[c] + dpp_mov<kDppBefore>(f[c]);
         store(k, f);
       };
-      tet10_point_lane<RULE, R, PHYS, false, false>(p, at, get, dt, e, q, pre, put, ea);
+      double Ji[9], Lv[9], M[9];
+      const double detJ = tet10_point_kin<RULE, R, PHYS>(p, get, q, Ji, Lv, ea);
+      tet10_point_stress<RULE, R, PHYS, false, false>(p, at, dt, e, q, pre, Ji, detJ, Lv, M, ea);
+      tet10_point_forces<RULE, R>(q, M, put);
     } else {
       auto put = [&](int k, const R g[3], R wd) {
         R f[3];
@@ -440,31 +446,78 @@ k_elem_block5(Params p) {
   wave_flush<AUX>(p, p.epart_base + b * (NT / 64), ea, row);
 }
 
-// tet10 on a 4-point rule: four lanes per element, lane t & 3 taking
-// quadrature point t & 3, so a workgroup of NT threads holds at most NT/4
-// elements, and the plan gives it at most NT local nodes, one per thread.
+// A workgroup's elements on a 4-point tet10 rule: the corner forces into the
+// block's slots.  cw: the corner words of the thread's element e, of the
+// block's last one in threads without (has_e false); some: the wave has an
+// element.  Lane q stores corners q, q + 4 and q + 8.
+template <int RULE, typename R, int PHYS, bool STREAM, bool DEFER, bool MM, class At>
+__device__ __forceinline__ void tet10_block(const Params &p, const At &at, const LNodes &ln,
+                                            R *lf, const uint16_t *joff, const double *basis,
+                                            const uint32_t cw[5], double dt, int e, int t, int q,
+                                            bool has_e, bool some, PreState<R> &pre, EAcc &ea) {
+  auto half = [&](int k) { return (int)((cw[k >> 1] >> (16 * (k & 1))) & 0xffffu); };
+  auto get = [&](int k, double x[3], double v[3]) { ln.get(half(k) & 511, x, v); };
+  int sl[3];
+#pragma unroll
+  for (int j = 0; j < 3; j++) {
+    const uint32_t lo = cw[2 * j], hi = cw[j == 2 ? 4 : 2 * j + 1];
+    const int h = (int)(((q >> 1 ? hi : lo) >> (16 * (q & 1))) & 0xffffu);
+    sl[j] = (int)joff[h >> 9] + (h & 511);
+  }
+  auto store = [&](int j, const R f[3]) {
+    R *dst = lf + 3 * sl[j];
+    dst[0] = f[0];
+    dst[1] = f[1];
+    dst[2] = f[2];
+  };
+  R Ji[9], Lv[9], M[9] = {};
+  if (has_e) {
+    const R detJ = tet10_point_kin<RULE, R, PHYS>(p, get, q, Ji, Lv, ea);
+    tet10_point_stress<RULE, R, PHYS, STREAM, DEFER>(p, at, dt, e, q, pre, Ji, detJ, Lv, M, ea);
+  }
+  if constexpr (MM) {
+    if (!__builtin_amdgcn_readfirstlane(some)) return;
+    auto put = [&](int g, const double f[3]) {
+      if (has_e && (g < 2 || q < 2)) store(g, f);
+    };
+    tet10_wave_forces(basis, t & 63, M, put);
+  } else if (has_e) {
+    auto put = [&](int k, const R fq[3]) {
+      const R f[3] = {quad_sum(fq[0]), quad_sum(fq[1]), quad_sum(fq[2])};
+      if ((k & 3) == q) store(k >> 2, f);
+    };
+    tet10_point_forces<RULE, R>(q, M, put);
+  }
+}
+
+// tet10 on a 4-point rule: four lanes per element, one per quadrature point
+// (PointLane), so a workgroup of NT threads holds at most NT/4 elements, and
+// the plan gives it at most NT local nodes, one per thread.
 // As in the tet4 kernel every global load of the workgroup (the node's id,
 // slot and contribution count, the node records and slot offsets, the
 // element's ten corner words, the point's stress state with its ep only
 // when the point's yielded bit says it has yielded) is issued before the
 // first barrier; after it the element pass reads only LDS and the node pass
-// only LDS and its registers.  Corner k's element force (summed over the
-// element's four lanes in rule order) is stored by lane k & 3 into the
-// corner's jagged-diagonal slot, off[rank] + local node; the nodes are then
-// assembled as in k_elem_block5, and the point's state is stored last.  LDS
-// as k_elem_block5.
-template <int RULE, typename R, int PHYS, bool AUX, int NT, int WPE, bool STREAM>
+// only LDS and its registers.  Lane q of an element stores corners q, q + 4
+// and q + 8 (summed over the element's four points) into the corner's
+// jagged-diagonal slot, off[rank] + local node; the nodes are then assembled
+// as in k_elem_block5, and the point's state is stored last.  LDS as
+// k_elem_block5, then the basis gradients (MM).
+template <int RULE, typename R, int PHYS, bool AUX, int NT, int WPE, bool STREAM, bool MM>
 __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WPE)))
 k_elem_block10(Params p) {
   extern __shared__ double smem[];
   const int b = xcd_remap(blockIdx.x, gridDim.x);
-  const int t = threadIdx.x, q = t & 3;
+  const int t = threadIdx.x;
+  const PointLane<MM> pt(t);
+  const int q = pt.q;
   RowPre row = row_prefetch(p, p.epart_base + b * (NT / 64));
   const int32_t *mt = p.meta + 8 * b;
   const int es = mt[0], nel = mt[1];
   const LNodes ln{smem, p.ml};
   R *lf = (R *)((char *)smem + lds_node_bytes(p.ml));
   uint16_t *joff = (uint16_t *)((char *)lf + lds_force_bytes(sizeof(R), 10, p.max_el));
+  double *basis = (double *)((char *)joff + lds_off_bytes(p.kmax));
   double dt = p.ctl->dt;
   // yielded bits, one per lane (point) of the wave: a point's ep is read
   // only when it has yielded before
@@ -484,10 +537,13 @@ k_elem_block10(Params p) {
   const double mr = p.m[has_n && slot_o < 0 ? g_o : 0];
   const Vec3 vr = p.vv[has_n ? g_o : 0];
   const uint16_t jo = p.off_pad[(long)b * (p.kmax + 1) + (t < p.kmax ? t : p.kmax)];
+  [[maybe_unused]] double gk = 0.0;
+  if constexpr (MM)
+    gk = tet10_basis<RULE>.v[t < Tet10Basis<RULE>::n ? t : Tet10Basis<RULE>::n - 1];
   __builtin_amdgcn_sched_barrier(0);
-  const bool has_e = (t >> 2) < nel;
-  const int e = es + (t >> 2), ec = has_e ? e : es + nel - 1;
-  const StateBlock<R> at = state_block<R>(p, b, t);
+  const bool has_e = pt.el < nel;
+  const int e = es + pt.el, ec = has_e ? e : es + nel - 1;
+  const StateBlock<R> at = state_block<R>(p, b, pt.place(p));
   // the element's ten corner words (local node | rank << 9), two per word
   // (the rows of 20 bytes are 4-byte aligned)
   uint32_t cw[5];
@@ -504,6 +560,8 @@ k_elem_block10(Params p) {
   keep_here(row);
   if (has_n) ln.stage(t, xr, mr, vr);
   if (t <= p.kmax) joff[t] = jo;
+  if constexpr (MM)
+    if (t < Tet10Basis<RULE>::n) basis[t] = gk;
   __syncthreads();
 
   EAcc ea;
@@ -511,29 +569,9 @@ k_elem_block10(Params p) {
   // loaded state again, so nothing after the element pass waits for the
   // state loads (nor, by the in-order wait count, for the state stores)
   bool yielded = false;
-  if (has_e) {
-    auto half = [&](int k) { return (int)((cw[k >> 1] >> (16 * (k & 1))) & 0xffffu); };
-    auto get = [&](int k, double xk[3], double vk[3]) { ln.get(half(k) & 511, xk, vk); };
-    // lane q stores corners q, q + 4 and q + 8: their force slots
-    int sl[3];
-#pragma unroll
-    for (int j = 0; j < 3; j++) {
-      const uint32_t wj = (q >> 1) ? cw[j == 2 ? 4 : 2 * j + 1] : cw[2 * j];
-      const int h = (int)((wj >> (16 * (q & 1))) & 0xffffu);
-      sl[j] = (int)joff[h >> 9] + (h & 511);
-    }
-    auto put = [&](int k, const R fq[3]) {
-      const R f[3] = {quad_sum(fq[0]), quad_sum(fq[1]), quad_sum(fq[2])};
-      if ((k & 3) == q) {
-        R *dst = lf + 3 * sl[k >> 2];
-        dst[0] = f[0];
-        dst[1] = f[1];
-        dst[2] = f[2];
-      }
-    };
-    tet10_point_lane<RULE, R, PHYS, STREAM, !AUX>(p, at, get, dt, e, q, pre, put, ea);
-    yielded = pre.ep > R(0);
-  }
+  tet10_block<RULE, R, PHYS, STREAM, !AUX, MM>(p, at, ln, lf, joff, basis, cw, dt, e, t, q, has_e,
+                                               pt.el - (t & 15) < nel, pre, ea);
+  if (has_e) yielded = pre.ep > R(0);
   if constexpr (PHYS == PHYS_EP) {
     const unsigned long long nb = __ballot(yielded);
     if (has_word && (t & 63) == 0 && nb != yw) p.yielded[yi] = nb;
@@ -552,7 +590,7 @@ k_elem_block10(Params p) {
     }
   }
   wave_flush<AUX>(p, p.epart_base + b * (NT / 64), ea, row);
-  // the point's state last (tet10_point_lane leaves it in pre), except in
+  // the point's state last (tet10_point_stress leaves it in pre), except in
   // the once-per-batch variant, whose outputs leave no registers for it
   if constexpr (PHYS != PHYS_COMPAT && !AUX)
     if (has_e) store_state<STREAM, R>(at, pre.s, pre.ep, pre.changed);
@@ -1051,13 +1089,17 @@ k_resident(Params p, Resident rs) {
   __syncthreads();
   if (gave_up) return;
   const int b = xcd_remap(blockIdx.x, gridDim.x);
-  const int t = threadIdx.x, q = NPE == 4 ? 0 : t & 3, el = NPE == 4 ? t : t >> 2;
+  const int t = threadIdx.x;
+  constexpr bool MM = NPE == 10 && sizeof(R) == 8;
+  const PointLane<MM> pt(t);
+  const int q = NPE == 4 ? 0 : pt.q, el = NPE == 4 ? t : pt.el;
   const int32_t *mt = p.meta + 8 * b;
   const int es = mt[0], nel = mt[1];
   const LNodes ln{smem, p.ml};
   R *lf = (R *)((char *)smem + lds_node_bytes(p.ml));
   uint16_t *joff = (uint16_t *)((char *)lf + lds_force_bytes(sizeof(R), NPE, p.max_el));
-  R *lm = (R *)((char *)joff + lds_off_bytes(p.kmax));
+  double *basis = (double *)((char *)joff + lds_off_bytes(p.kmax));
+  R *lm = (R *)((char *)basis + lds_basis_bytes(NPE, sizeof(R), Quad<RULE>::n));
   int32_t *ldest = (int32_t *)((char *)lm + lds_round16(3L * sizeof(R) * rs.most));
   uint16_t *lsrc = (uint16_t *)(ldest + rs.most), *lidx = lsrc + rs.most;
   const double dt = p.ctl->dt;
@@ -1094,17 +1136,22 @@ k_resident(Params p, Resident rs) {
   }
   const __amdgpu_buffer_rsrc_t mail = mail_rsrc(rs.mail, (int)(2 * rs.messages * Rec::bytes));
   for (int k = t; k <= p.kmax; k += NT) joff[k] = p.off_pad[(long)b * (p.kmax + 1) + k];
+  if constexpr (MM)
+    for (int k = t; k < Tet10Basis<RULE>::n; k += NT) basis[k] = tet10_basis<RULE>.v[k];
   // element el: corner words and the point's state
   const bool has_e = el < nel;
   uint32_t cw[NPE / 2];
   PreState<R> pre{};
-  if (has_e) {
-    const uint32_t *cp = reinterpret_cast<const uint32_t *>(p.corner + (long)NPE * (es + el));
+  {
+    const int ec = es + (has_e ? el : nel - 1);
+    const uint32_t *cp = reinterpret_cast<const uint32_t *>(p.corner + (long)NPE * ec);
 #pragma unroll
     for (int k = 0; k < NPE / 2; k++) cw[k] = cp[k];
+  }
+  if (has_e) {
     if constexpr (PHYS == PHYS_EP) {
       const unsigned long long yw = has_word ? p.yielded[yi] : 0ull;
-      load_state<false, R>(state_block<R>(p, b, t), (yw >> (t & 63)) & 1ull, pre);
+      load_state<false, R>(state_block<R>(p, b, NPE == 4 ? t : pt.place(p)), (yw >> (t & 63)) & 1ull, pre);
     }
   }
   __syncthreads();
@@ -1126,36 +1173,21 @@ k_resident(Params p, Resident rs) {
     for (int k = 0; k < NPE / 2; k++) asm volatile("" : "+v"(cw[k]));
     Params pl = params_again(args, p);
     pl.samples = nullptr;  // the recorder's steps are not resident
-    if (has_e) {
-      if constexpr (NPE == 4) {
+    if constexpr (NPE == 4) {
+      if (has_e) {
         auto put = [&](int k, const R fk[3]) {
           R *dst = lf + 3 * slot_of(half(k));
 #pragma unroll
           for (int c = 0; c < 3; c++) dst[c] = fk[c];
         };
         tet4_core<R, PHYS, true, false, true>(pl, StatePlane<R>{}, get, dt, es + el, put, ea, &pre);
-      } else {
-        // lane q stores corners q, q + 4 and q + 8
-        int sl[3];
-#pragma unroll
-        for (int j = 0; j < 3; j++) {
-          const uint32_t wj = (qs >> 1) ? cw[j == 2 ? 4 : 2 * j + 1] : cw[2 * j];
-          sl[j] = slot_of((int)((wj >> (16 * (qs & 1))) & 0xffffu));
-        }
-        auto put = [&](int k, const R fq[3]) {
-          const R f[3] = {quad_sum(fq[0]), quad_sum(fq[1]), quad_sum(fq[2])};
-          if ((k & 3) == qs) {
-            R *dst = lf + 3 * sl[k >> 2];
-            dst[0] = f[0];
-            dst[1] = f[1];
-            dst[2] = f[2];
-          }
-        };
-        tet10_point_lane<RULE, R, PHYS, false, true>(pl, StatePlane<R>{}, get, dt, es + el, qs, pre, put,
-                                                     ea);
       }
-      if constexpr (PHYS == PHYS_EP) changed = changed || pre.changed;
+    } else {
+      tet10_block<RULE, R, PHYS, false, true, MM>(pl, StatePlane<R>{}, ln, lf, joff, basis, cw, dt,
+                                              es + el, ts, qs, has_e, el - (t & 15) < nel, pre, ea);
     }
+    if constexpr (PHYS == PHYS_EP)
+      if (has_e) changed = changed || pre.changed;
     // the emptying stores of the last step have completed
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
@@ -1245,7 +1277,7 @@ k_resident(Params p, Resident rs) {
     p.vv[n] = Vec3{v[0], v[1], v[2]};
   }
   if constexpr (PHYS == PHYS_EP) {
-    if (has_e) store_state<false, R>(state_block<R>(p, b, t), pre.s, pre.ep, changed);
+    if (has_e) store_state<false, R>(state_block<R>(p, b, NPE == 4 ? t : pt.place(p)), pre.s, pre.ep, changed);
     const unsigned long long nb = __ballot(has_e && pre.ep > R(0));
     if (has_word && (t & 63) == 0) p.yielded[yi] = nb;
   }
@@ -1778,8 +1810,17 @@ __global__ void __launch_bounds__(256) k_export_nodes(Params p, const int32_t *n
   if (o.m3) o.m3[i] = p.m[g];
 }
 
-// spos: per user element, its place in ep, in elements (nq points each, next
-// to each other) of the block layout; in the planes the device element
+// place in ep (and in a component of sig) of point q of an element.  spos, of
+// the element: in the planes (state_ld 0) the device element; in rows per
+// block its place in elements, and its points lie next to each other, or
+// (p.matrix) as PointLane<true> places them
+__device__ __forceinline__ long state_place(const Params &p, uint32_t spos, int q) {
+  if (!p.state_ld) return spos + (long)q * p.ne;
+  if (!p.matrix) return (long)spos * p.nq + q;
+  const uint32_t w = p.state_ld < 64 ? p.state_ld >> 2 : 16;
+  return (long)(spos / w) * 4 * w + q * w + spos % w;
+}
+
 template <typename R>
 __global__ void __launch_bounds__(256) k_export_elems(Params p, const uint32_t *spos, double *sig,
                                                       double *ep) {
@@ -1788,14 +1829,15 @@ __global__ void __launch_bounds__(256) k_export_elems(Params p, const uint32_t *
   if (sig && i < ne * w) {
     const long e = i / w;
     const int q = (int)(i - e * w) / 6, c = (int)(i - e * w) - 6 * q;
-    const long at = ld ? (long)spos[e] * p.nq + q : spos[e];
-    sig[i] = double(static_cast<const R *>(
-        p.sig)[ld ? (at / ld) * 6 * ld + c * ld + at % ld : (6L * q + c) * ne + at]);
+    const long at = state_place(p, spos[e], q);
+    const R *sr = static_cast<const R *>(p.sig);
+    sig[i] = double(ld ? sr[(at / ld) * 6 * ld + c * ld + at % ld]
+                       : sr[(6L * q + c) * ne + spos[e]]);
   }
   if (ep && i < ne * p.nq) {
     const long e = i / p.nq;
     const int q = (int)(i - e * p.nq);
-    ep[i] = double(static_cast<const R *>(p.epbar)[ld ? (long)spos[e] * p.nq + q : spos[e] + q * ne]);
+    ep[i] = double(static_cast<const R *>(p.epbar)[state_place(p, spos[e], q)]);
   }
 }
 
@@ -1909,10 +1951,11 @@ constexpr int kMlpQueueGrid = 2048;
 constexpr int kMlpQueueThreads = 256;
 
 // LDS of the workgroup element kernels: node records, corner forces, the
-// slot offsets
-size_t elem_block_smem(int npe, int prec, int, int ml, int max_el, int kmax) {
+// slot offsets, the basis of the FP64 per-point tet10 kernels
+size_t elem_block_smem(int npe, int rule, int prec, int ml, int max_el, int kmax) {
   const int rsz = prec == 1 ? 4 : 8;
-  return (size_t)lds_node_bytes(ml) + lds_force_bytes(rsz, npe, max_el) + lds_off_bytes(kmax);
+  return (size_t)lds_node_bytes(ml) + lds_force_bytes(rsz, npe, max_el) + lds_off_bytes(kmax) +
+         lds_basis_bytes(npe, rsz, rule == RULE_REF5 ? 5 : 4);
 }
 
 int elem_block_threads(int npe, int rule, int prec, int phys, int nblocks) {
@@ -1992,6 +2035,26 @@ static hipError_t elem_block4_t(const Params &p, bool aux, int nblocks, size_t s
   }
 }
 
+// the per-point tet10 kernel's LDS opt-in and launch, cached or streamed
+// state, quads or the matrix units (p.matrix)
+template <int RULE, typename R, int PHYS, bool STREAM, bool MM>
+static hipError_t tet10_opt_in(size_t smem) {
+  constexpr int NT = block_threads<10, RULE>();
+  constexpr int W = tet10_waves<R>();
+  hipError_t e = lds_opt_in(k_elem_block10<RULE, R, PHYS, true, NT, W, STREAM, MM>, smem);
+  if (e == hipSuccess) e = lds_opt_in(k_elem_block10<RULE, R, PHYS, false, NT, W, STREAM, MM>, smem);
+  return e;
+}
+
+template <int RULE, typename R, int PHYS, bool STREAM, bool MM>
+static hipError_t tet10_t(const Params &p, bool aux, int nblocks, size_t smem, hipStream_t s) {
+  constexpr int NT = block_threads<10, RULE>();
+  constexpr int W = tet10_waves<R>();
+  if (aux)
+    CPI_LAUNCH((k_elem_block10<RULE, R, PHYS, true, NT, W, STREAM, MM>), nblocks, NT, smem, s, p);
+  CPI_LAUNCH((k_elem_block10<RULE, R, PHYS, false, NT, W, STREAM, MM>), nblocks, NT, smem, s, p);
+}
+
 template <int NPE, int RULE, typename R, int PHYS>
 static hipError_t elem_block_t(const Params &p, bool aux, int nblocks, size_t smem, hipStream_t s,
                                int part) {
@@ -2004,16 +2067,11 @@ static hipError_t elem_block_t(const Params &p, bool aux, int nblocks, size_t sm
       if (p.stream_state) return elem_block4_t<R, PHYS, true, true>(p, aux, nblocks, smem, s, part);
     return elem_block4_t<R, PHYS, false, true>(p, aux, nblocks, smem, s, part);
   } else if constexpr (Quad<RULE>::n == 4) {
-    constexpr int W = tet10_waves<R>();
-    if constexpr (PHYS != PHYS_COMPAT) {
-      if (p.stream_state) {
-        if (aux)
-          CPI_LAUNCH((k_elem_block10<RULE, R, PHYS, true, NT, W, true>), nblocks, NT, smem, s, p);
-        CPI_LAUNCH((k_elem_block10<RULE, R, PHYS, false, NT, W, true>), nblocks, NT, smem, s, p);
-      }
-    }
-    if (aux) CPI_LAUNCH((k_elem_block10<RULE, R, PHYS, true, NT, W, false>), nblocks, NT, smem, s, p);
-    CPI_LAUNCH((k_elem_block10<RULE, R, PHYS, false, NT, W, false>), nblocks, NT, smem, s, p);
+    if constexpr (sizeof(R) == 8)
+      if (p.matrix) return tet10_t<RULE, R, PHYS, false, true>(p, aux, nblocks, smem, s);
+    if constexpr (PHYS != PHYS_COMPAT)
+      if (p.stream_state) return tet10_t<RULE, R, PHYS, true, false>(p, aux, nblocks, smem, s);
+    return tet10_t<RULE, R, PHYS, false, false>(p, aux, nblocks, smem, s);
   } else {
     constexpr int W = tet10_waves5<R, PHYS>();
     if (narrow5(nblocks, sizeof(R) == 8 && PHYS != PHYS_COMPAT)) {
@@ -2091,13 +2149,11 @@ template <int NPE, int RULE, typename R, int PHYS> struct ElemBlockPrepF {
           if (e == hipSuccess) e = tet4_opt_in<R, PHYS, true, true>(smem);
         return e;
       } else if constexpr (Quad<RULE>::n == 4) {
-        constexpr int W = tet10_waves<R>();
-        hipError_t e = lds_opt_in(k_elem_block10<RULE, R, PHYS, true, NT, W, false>, smem);
-        if (e == hipSuccess) e = lds_opt_in(k_elem_block10<RULE, R, PHYS, false, NT, W, false>, smem);
-        if constexpr (PHYS != PHYS_COMPAT) {
-          if (e == hipSuccess) e = lds_opt_in(k_elem_block10<RULE, R, PHYS, true, NT, W, true>, smem);
-          if (e == hipSuccess) e = lds_opt_in(k_elem_block10<RULE, R, PHYS, false, NT, W, true>, smem);
-        }
+        hipError_t e = tet10_opt_in<RULE, R, PHYS, false, false>(smem);
+        if constexpr (PHYS != PHYS_COMPAT)
+          if (e == hipSuccess) e = tet10_opt_in<RULE, R, PHYS, true, false>(smem);
+        if constexpr (sizeof(R) == 8)
+          if (e == hipSuccess) e = tet10_opt_in<RULE, R, PHYS, false, true>(smem);
         return e;
       } else {
         constexpr int W = tet10_waves5<R, PHYS>();
