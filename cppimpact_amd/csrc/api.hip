@@ -803,7 +803,14 @@ static int create_impl(cpi_ctx *c, const cpi_mesh_desc *m, const cpi_material *m
     int32_t *meta, *bn, *bs, *sp, *dn, *ds;
     uint16_t *cl, *ci, *cw = nullptr, *dg, *dof;
     Vec3 *part;
-    const bool words = corner_words(c);
+    // the five-point tet10 kernel reads no words, but its resident steps do:
+    // a thread per node, its elements in one round, a block per CU
+    const int nt5 = elem_block_threads(npe, c->rule, c->prec, c->phys, B.nblocks);
+    const bool five = npe == 10 && c->nq == 5 && B.nblocks <= prop.multiProcessorCount &&
+                      nt5 == elem_block_threads(npe, c->rule, c->prec, c->phys, 0) &&
+                      B.max_local_nodes <= nt5 && B.max_block_elems <= nt5 / 64 * 12 &&
+                      B.corner_fits();
+    const bool words = corner_words(c) || five;
     if ((rc = dalloc(c, &meta, B.meta.size())) || (rc = upload(c, meta, B.meta)) ||
         (rc = dalloc(c, &cl, B.conn_local.size())) || (rc = upload(c, cl, B.conn_local)) ||
         (rc = dalloc(c, &ci, B.csr_pos.size())) || (rc = upload(c, ci, B.csr_pos)) ||
@@ -879,7 +886,7 @@ static int create_impl(cpi_ctx *c, const cpi_mesh_desc *m, const cpi_material *m
                                       hipGetErrorString(pe));
     // resident steps when every block fits the chip at once
     if (opt->use_graph && c->phys != 2 && words && prop.cooperativeLaunch &&
-        (npe == 4 || c->prec == CPI_PREC_F32 || P.matrix)) {
+        (npe == 4 || five || c->prec == CPI_PREC_F32 || P.matrix)) {
       const MailPlan M = build_mail(B);
       const size_t n = M.dest.size(), bytes = mail_bytes(c->prec, n);
       const size_t smem = resident_smem(c->smem, c->prec, M.most);

@@ -406,7 +406,7 @@ __device__ __forceinline__ void tet10_dn(const R Ji[9], const G Gd[30], int i, R
 // sigma . dN_i and w detJ go to put(i, g, w detJ).  pre: the point's stress
 // state, loaded ahead (PRE).
 // ---------------------------------------------------------------------------
-template <int RULE, typename R, int PHYS, bool PRE, class At, class Get, class Put>
+template <int RULE, typename R, int PHYS, bool PRE, bool DEFER, class At, class Get, class Put>
 __device__ __forceinline__ void tet10_point(const Params &p, const At &at, const Get &get,
                                             double dt, int e, int q, const Put &put, EAcc &ea,
                                             PreState<R> *pre = nullptr) {
@@ -446,7 +446,7 @@ __device__ __forceinline__ void tet10_point(const Params &p, const At &at, const
   }
   R wd = R(Q::w(q)) * detJ;
   R s[6];
-  point_stress<R, PHYS, PRE>(p, at, e, q, de, wd, s, ea, pre);
+  point_stress<R, PHYS, PRE, false, DEFER>(p, at, e, q, de, wd, s, ea, pre);
 #pragma unroll
   for (int i = 0; i < 10; i++) {
     R dn[3], g[3];
@@ -792,7 +792,7 @@ __device__ __forceinline__ void tet10_core(const Params &p, const Get &get, doub
 #pragma unroll
       for (int c = 0; c < 3; c++) f[i][c] = fma(wd, g[c], f[i][c]);
     };
-    tet10_point<RULE, R, PHYS, false>(p, state_plane<R>(p, e, q), get, dt, e, q, add, ea);
+    tet10_point<RULE, R, PHYS, false, false>(p, state_plane<R>(p, e, q), get, dt, e, q, add, ea);
   }
   if constexpr (PHYS != PHYS_COMPAT) tet10_stable_dt<R>(p, get, ea);
 #pragma unroll

@@ -323,15 +323,59 @@ __host__ __device__ constexpr int lds_basis_bytes(int npe, int rsz, int points) 
   return npe == 10 && rsz == 8 && points == 4 ? 8 * Tet10Basis<RULE_EXACT4>::n : 0;
 }
 
+// One element on the 5-point tet10 rule by five lanes, lane q's point q:
+// slot(k) is where its force at corner k goes.  The force is the chain
+// f = w_q detJ_q g_q + f over the points in rule order, which every lane runs
+// on the value of the lane before it: after four steps the last point's lane
+// has it, with the bits of one thread going through the points.  FP64 takes
+// tet10_point_kin's arithmetic (f_q = M G summed in the same order); FP32 keeps
+// tet10_point's, whose bits the direct kernels share.
+template <int RULE, typename R, int PHYS, bool DEFER, class At, class Get, class Slot>
+__device__ __forceinline__ void tet10_five(const Params &p, const At &at, const Get &get,
+                                           const Slot &slot, R *lf, double dt, int e, int q,
+                                           PreState<R> &pre, EAcc &ea) {
+  constexpr int NQ = Quad<RULE>::n;
+  auto store = [&](int k, const R f[3]) {
+    if (q == NQ - 1) {
+      R *dst = lf + 3 * slot(k);
+#pragma unroll
+      for (int c = 0; c < 3; c++) dst[c] = f[c];
+    }
+  };
+  if constexpr (sizeof(R) == 8) {
+    auto put = [&](int k, const R fq[3]) {
+      R f[3] = {fq[0], fq[1], fq[2]};
+#pragma unroll
+      for (int s = 1; s < NQ; s++)
+#pragma unroll
+        for (int c = 0; c < 3; c++) f[c] = fq[c] + dpp_mov<kDppBefore>(f[c]);
+      store(k, f);
+    };
+    double Ji[9], Lv[9], M[9];
+    const double detJ = tet10_point_kin<RULE, R, PHYS>(p, get, q, Ji, Lv, ea);
+    tet10_point_stress<RULE, R, PHYS, false, DEFER>(p, at, dt, e, q, pre, Ji, detJ, Lv, M, ea);
+    tet10_point_forces<RULE, R>(q, M, put);
+  } else {
+    auto put = [&](int k, const R g[3], R wd) {
+      R f[3];
+#pragma unroll
+      for (int c = 0; c < 3; c++) f[c] = fma(wd, g[c], R(0));
+#pragma unroll
+      for (int s = 1; s < NQ; s++)
+#pragma unroll
+        for (int c = 0; c < 3; c++) f[c] = fma(wd, g[c], dpp_mov<kDppBefore>(f[c]));
+      store(k, f);
+    };
+    tet10_point<RULE, R, PHYS, true, DEFER>(p, at, get, dt, e, q, put, ea, &pre);
+    if constexpr (PHYS != PHYS_COMPAT)
+      if (q == 0) tet10_stable_dt<R>(p, get, ea);
+  }
+}
+
 // ---------------------------------------------------------------------------
 // LDS-assembled element pass, tet10 on the 5-point rule: five lanes per
-// element, one per point, twelve elements per wave (four lanes idle).  A
-// corner's force is the chain f = w_q detJ_q g_q + f over the points in rule
-// order, which every lane runs on the value of the lane before it: after
-// four steps the last point's lane has it, with the bits of one thread going
-// through the points.  FP64 takes tet10_point_kin's arithmetic (f_q = M G
-// summed in the same order); FP32 keeps tet10_point's, whose bits the direct
-// kernels share.  VALU-bound for a full chip.  Against one thread per element
+// element, one per point, twelve elements per wave (four lanes idle; see
+// tet10_five).  VALU-bound for a full chip.  Against one thread per element
 // looping over the points (128 threads): 13k elements FP64 compat 18.9 -> 9.4
 // us, FP32 15.6 -> 9.3, FP64 EP 23.2 -> 10.9; 663k elements 214 -> 141, FP32
 // 127 -> 114, FP64 EP 319 -> 230, FP32 EP 180 -> 154 us.
@@ -390,41 +434,8 @@ k_elem_block5(Params p) {
       return (int)((w[k >> 1] >> (16 * (k & 1))) & 0xffffu);
     };
     auto get = [&](int k, double xk[3], double vk[3]) { ln.get(half(lw, k), xk, vk); };
-    auto store = [&](int k, const R f[3]) {
-      if (q == NQ - 1) {
-        R *dst = lf + 3 * half(pw, k);
-#pragma unroll
-        for (int c = 0; c < 3; c++) dst[c] = f[c];
-      }
-    };
-    if constexpr (sizeof(R) == 8) {
-      auto put = [&](int k, const R fq[3]) {
-        R f[3] = {fq[0], fq[1], fq[2]};
-#pragma unroll
-        for (int s = 1; s < NQ; s++)
-#pragma unroll
-          for (int c = 0; c < 3; c++) f[c] = fq[c] + dpp_mov<kDppBefore>(f[c]);
-        store(k, f);
-      };
-      double Ji[9], Lv[9], M[9];
-      const double detJ = tet10_point_kin<RULE, R, PHYS>(p, get, q, Ji, Lv, ea);
-      tet10_point_stress<RULE, R, PHYS, false, false>(p, at, dt, e, q, pre, Ji, detJ, Lv, M, ea);
-      tet10_point_forces<RULE, R>(q, M, put);
-    } else {
-      auto put = [&](int k, const R g[3], R wd) {
-        R f[3];
-#pragma unroll
-        for (int c = 0; c < 3; c++) f[c] = fma(wd, g[c], R(0));
-#pragma unroll
-        for (int s = 1; s < NQ; s++)
-#pragma unroll
-          for (int c = 0; c < 3; c++) f[c] = fma(wd, g[c], dpp_mov<kDppBefore>(f[c]));
-        store(k, f);
-      };
-      tet10_point<RULE, R, PHYS, true>(p, at, get, dt, e, q, put, ea, &pre);
-      if constexpr (PHYS != PHYS_COMPAT)
-        if (q == 0) tet10_stable_dt<R>(p, get, ea);
-    }
+    auto slot = [&](int k) { return half(pw, k); };
+    tet10_five<RULE, R, PHYS, false>(p, at, get, slot, lf, dt, e, q, pre, ea);
   }
   __syncthreads();
 
@@ -980,7 +991,8 @@ __global__ void __launch_bounds__(256) k_node_bnd(Params p) {
 //
 // Per step (MI355X; before: the two launches): 6,000 tet4 8.9 -> 5.0 us
 // (FP64), 8.7 -> 4.6 (FP32); 196,608 tet4 12.2 -> 7.9, 10.6 -> 6.5; 48,000 tet10
-// 17.2 -> 13, 13.8 -> 8.5.  What is left is the element pass and node sums
+// 17.2 -> 10.3, 13.8 -> 8.7; 13,464 tet10 on the 5-point rule 12.4 -> 9.2, 12.3 ->
+// 8.5.  What is left is the element pass and node sums
 // (3.9 us for 16 blocks, 4.8 for 512) and one trip of the mail.
 // ---------------------------------------------------------------------------
 typedef unsigned mail4 __attribute__((ext_vector_type(4)));
@@ -1090,9 +1102,14 @@ k_resident(Params p, Resident rs) {
   if (gave_up) return;
   const int b = xcd_remap(blockIdx.x, gridDim.x);
   const int t = threadIdx.x;
-  constexpr bool MM = NPE == 10 && sizeof(R) == 8;
+  // the thread's element and point, as the per-step kernels take them
+  constexpr bool FIVE = NPE == 10 && Quad<RULE>::n == 5;
+  constexpr bool MM = NPE == 10 && !FIVE && sizeof(R) == 8;
   const PointLane<MM> pt(t);
-  const int q = NPE == 4 ? 0 : pt.q, el = NPE == 4 ? t : pt.el;
+  const int lane = t & 63;
+  const int q = NPE == 4 ? 0 : FIVE ? lane % 5 : pt.q;
+  const int el = NPE == 4 ? t : FIVE ? 12 * (t >> 6) + lane / 5 : pt.el;
+  auto place = [&]() { return NPE == 4 ? t : FIVE ? 5 * el + q : pt.place(p); };
   const int32_t *mt = p.meta + 8 * b;
   const int es = mt[0], nel = mt[1];
   const LNodes ln{smem, p.ml};
@@ -1139,7 +1156,7 @@ k_resident(Params p, Resident rs) {
   if constexpr (MM)
     for (int k = t; k < Tet10Basis<RULE>::n; k += NT) basis[k] = tet10_basis<RULE>.v[k];
   // element el: corner words and the point's state
-  const bool has_e = el < nel;
+  const bool has_e = el < nel && (!FIVE || lane < 60);
   uint32_t cw[NPE / 2];
   PreState<R> pre{};
   {
@@ -1150,8 +1167,8 @@ k_resident(Params p, Resident rs) {
   }
   if (has_e) {
     if constexpr (PHYS == PHYS_EP) {
-      const unsigned long long yw = has_word ? p.yielded[yi] : 0ull;
-      load_state<false, R>(state_block<R>(p, b, NPE == 4 ? t : pt.place(p)), (yw >> (t & 63)) & 1ull, pre);
+      const unsigned long long yw = has_word ? p.yielded[yi] : FIVE ? ~0ull : 0ull;
+      load_state<false, R>(state_block<R>(p, b, place()), (yw >> (t & 63)) & 1ull, pre);
     }
   }
   __syncthreads();
@@ -1182,6 +1199,10 @@ k_resident(Params p, Resident rs) {
         };
         tet4_core<R, PHYS, true, false, true>(pl, StatePlane<R>{}, get, dt, es + el, put, ea, &pre);
       }
+    } else if constexpr (FIVE) {
+      auto slot = [&](int k) { return slot_of(half(k)); };
+      if (has_e)
+        tet10_five<RULE, R, PHYS, true>(pl, StatePlane<R>{}, get, slot, lf, dt, es + el, qs, pre, ea);
     } else {
       tet10_block<RULE, R, PHYS, false, true, MM>(pl, StatePlane<R>{}, ln, lf, joff, basis, cw, dt,
                                               es + el, ts, qs, has_e, el - (t & 15) < nel, pre, ea);
@@ -1277,7 +1298,7 @@ k_resident(Params p, Resident rs) {
     p.vv[n] = Vec3{v[0], v[1], v[2]};
   }
   if constexpr (PHYS == PHYS_EP) {
-    if (has_e) store_state<false, R>(state_block<R>(p, b, NPE == 4 ? t : pt.place(p)), pre.s, pre.ep, changed);
+    if (has_e) store_state<false, R>(state_block<R>(p, b, place()), pre.s, pre.ep, changed);
     const unsigned long long nb = __ballot(has_e && pre.ep > R(0));
     if (has_word && (t & 63) == 0) p.yielded[yi] = nb;
   }
@@ -2190,13 +2211,15 @@ hipError_t launch_elem_direct(const Params &p, int rule, int prec, int phys, boo
 }
 
 // minimum waves per SIMD of the resident kernels
-template <int NPE, typename R> constexpr int resident_waves() {
-  return 4;
+// minimum waves per SIMD: the five-point tet10 kernel's eleven waves a block
+// leave a CU no second block, and get the registers
+template <int NPE, int RULE> constexpr int resident_waves() {
+  return NPE == 10 && Quad<RULE>::n == 5 ? 3 : 4;
 }
 
 template <int NPE, int RULE, typename R, int PHYS> struct ResidentF {
   static constexpr bool has() {
-    return PHYS != PHYS_EP_MLP && (NPE == 4 || Quad<RULE>::n == 4);
+    return PHYS != PHYS_EP_MLP;
   }
   // the kernel, its threads per workgroup
   static hipError_t run(const void **kernel, int *threads) {
@@ -2204,7 +2227,7 @@ template <int NPE, int RULE, typename R, int PHYS> struct ResidentF {
       return hipErrorInvalidValue;
     } else {
       *kernel = reinterpret_cast<const void *>(
-          k_resident<NPE, RULE, R, PHYS, block_threads<NPE, RULE>(), resident_waves<NPE, R>()>);
+          k_resident<NPE, RULE, R, PHYS, block_threads<NPE, RULE>(), resident_waves<NPE, RULE>()>);
       *threads = block_threads<NPE, RULE>();
       return hipSuccess;
     }
