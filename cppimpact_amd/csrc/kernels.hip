@@ -4,7 +4,7 @@
 // LDS-assembled scatter (the default):
 //   k_elem_block4 (tet4; with the surrogate the elastic pass, k_mlp_queue
 //                 and k_elem_block4_walk),
-//   k_elem_block10 (tet10, 4-point rules), k_elem_block (tet10, 5 points)
+//   k_elem_block10 (tet10, 4-point rules), k_elem_block5 (tet10, 5 points)
 //                 one workgroup per element block: stage the block's nodes
 //                 in LDS, compute element forces (and the stress update),
 //                 sum them per node in a fixed order, finish the nodes owned
