@@ -2088,8 +2088,13 @@ static hipError_t elem_block_t(const Params &p, bool aux, int nblocks, size_t sm
       if (p.stream_state) return elem_block4_t<R, PHYS, true, true>(p, aux, nblocks, smem, s, part);
     return elem_block4_t<R, PHYS, false, true>(p, aux, nblocks, smem, s, part);
   } else if constexpr (Quad<RULE>::n == 4) {
-    if constexpr (sizeof(R) == 8)
-      if (p.matrix) return tet10_t<RULE, R, PHYS, false, true>(p, aux, nblocks, smem, s);
+    if constexpr (sizeof(R) == 8) {
+      if (p.matrix) {
+        if constexpr (PHYS != PHYS_COMPAT)
+          if (p.stream_state) return tet10_t<RULE, R, PHYS, true, true>(p, aux, nblocks, smem, s);
+        return tet10_t<RULE, R, PHYS, false, true>(p, aux, nblocks, smem, s);
+      }
+    }
     if constexpr (PHYS != PHYS_COMPAT)
       if (p.stream_state) return tet10_t<RULE, R, PHYS, true, false>(p, aux, nblocks, smem, s);
     return tet10_t<RULE, R, PHYS, false, false>(p, aux, nblocks, smem, s);
@@ -2173,8 +2178,11 @@ template <int NPE, int RULE, typename R, int PHYS> struct ElemBlockPrepF {
         hipError_t e = tet10_opt_in<RULE, R, PHYS, false, false>(smem);
         if constexpr (PHYS != PHYS_COMPAT)
           if (e == hipSuccess) e = tet10_opt_in<RULE, R, PHYS, true, false>(smem);
-        if constexpr (sizeof(R) == 8)
+        if constexpr (sizeof(R) == 8) {
           if (e == hipSuccess) e = tet10_opt_in<RULE, R, PHYS, false, true>(smem);
+          if constexpr (PHYS != PHYS_COMPAT)
+            if (e == hipSuccess) e = tet10_opt_in<RULE, R, PHYS, true, true>(smem);
+        }
         return e;
       } else {
         constexpr int W = tet10_waves5<R, PHYS>();
