@@ -902,7 +902,7 @@ static int create_impl(cpi_ctx *c, const cpi_mesh_desc *m, const cpi_material *m
             (rc = dalloc(c, &ms, n)) || (rc = upload(c, ms, M.src)) || (rc = dalloc(c, &mi, n)) ||
             (rc = upload(c, mi, M.idx)))
           return rc;
-        c->res = Resident{mail, (int)n, M.most, mf, md, ms, mlo, mi, 0, 0, 0,
+        c->res = Resident{mail, (int)n, M.most, mf, md, ms, mlo, mi, (int)c->loose.size(), 0, 0, 0,
                           opt->debug_fill_nan & 2 ? 1u : 1u << 20};
         c->res_smem = smem;
         c->resident = true;

@@ -173,6 +173,7 @@ struct Resident {
   const uint16_t *src;  // per message: the local node it is of
   const int32_t *lo;    // [nblocks][ml]: start of a shared node's list in idx
   const uint16_t *idx;  // lists of the block's messages per node, in slot order
+  int loose;            // nodes of no element, the last ones
   int base, steps;      // inbox of the first step, steps to take
   unsigned launch;      // number of the launch (Ctl::decision)
   unsigned spin_limit;  // polls of one wait before it gives up

@@ -1302,6 +1302,28 @@ k_resident(Params p, Resident rs) {
     const unsigned long long nb = __ballot(has_e && pre.ep > R(0));
     if (has_word && (t & 63) == 0) p.yielded[yi] = nb;
   }
+  // nodes of no element (no block holds one): only gravity and the wall act on
+  // them, so each takes its steps here by itself
+  const Params pl = params_again(args, p);
+  for (int n = pl.nn - rs.loose + (int)blockIdx.x * NT + t; n < pl.nn; n += (int)gridDim.x * NT) {
+    const bool nheld = node_held(pl, n), ncontact = node_contact(pl, n, nheld);
+    const double f[3] = {0.0, 0.0, 0.0}, m = pl.m[n];
+    const Vec3 xr = pl.pos[n], vr = pl.vv[n];
+    double x[3] = {xr.x, xr.y, xr.z}, v[3] = {vr.x, vr.y, vr.z};
+    for (int k = 0; k < rs.steps; k++) {
+      NodeStep s;
+      EAcc en;
+      node_advance(pl, nheld, ncontact, f, x, v, m, 1.0 / m, dt, s, en);
+      ea.wgrav += en.wgrav;
+#pragma unroll
+      for (int c = 0; c < 3; c++) {
+        x[c] = s.x[c];
+        v[c] = s.v[c];
+      }
+    }
+    pl.pos[n] = Vec3{x[0], x[1], x[2]};
+    pl.vv[n] = Vec3{v[0], v[1], v[2]};
+  }
   const int row_base = p.epart_base + b * (NT / 64);
   wave_flush<false>(p, row_base, ea, row_prefetch(p, row_base));
   if (blockIdx.x == 0 && t == 0) p.ctl->step += rs.steps;
