@@ -116,6 +116,7 @@ SIGNATURES = {
     "cpi_synchronize": (C.c_int, [C.c_void_p]),
     "cpi_get_state": (C.c_int, [C.c_void_p, _dp, _dp, _dp, _dp, _dp]),
     "cpi_get_state_mass3": (C.c_int, [C.c_void_p, _dp, _dp, _dp, _dp, _dp, _dp]),
+    "cpi_get_resident_steps": (C.c_int, [C.c_void_p, C.POINTER(C.c_int64), C.POINTER(C.c_int64)]),
     "cpi_get_increment": (C.c_int, [C.c_void_p, _dp]),
     "cpi_get_element_state": (C.c_int, [C.c_void_p, _dp, _dp]),
     "cpi_get_stress_strain": (C.c_int, [C.c_void_p, _dp, _dp]),

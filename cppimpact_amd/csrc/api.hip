@@ -69,6 +69,7 @@ struct cpi_ctx {
   size_t res_smem = 0;
   bool resident = false;
   bool res_pending = false;  // launched since the control block was last read
+  int64_t redone = 0;        // steps taken one by one instead, since cpi_init
   bool mass_ready = false, inited = false;
   double dt = 0.0;
   int64_t step = 0;
@@ -462,6 +463,7 @@ int settle(cpi_ctx *c, const Ctl &h) {
   c->resident = false;
   int rc = steps_one_by_one(c, h.missed);
   if (rc) return rc;
+  c->redone += h.missed;
   // no launch reads these again; a later call must not settle twice
   HIPCHK(c, hipMemsetAsync(&c->P.ctl->decision, 0, sizeof(uint32_t), c->stream));
   HIPCHK(c, hipMemsetAsync(&c->P.ctl->missed, 0, sizeof(int64_t), c->stream));
@@ -1102,6 +1104,7 @@ extern "C" int cpi_init(cpi_ctx *c, double dt) {
   }
   c->dt = dt;
   c->step = 0;
+  c->redone = 0;
   Ctl h{};
   h.dt = dt;
   h.dt_contact = dtc;
@@ -1356,6 +1359,16 @@ extern "C" int cpi_get_info(cpi_ctx *c, cpi_info *info) {
   }
   info->dt = c->dt;
   info->step = c->step;
+  return CPI_OK;
+}
+
+extern "C" int cpi_get_resident_steps(cpi_ctx *c, int64_t *taken, int64_t *redone) {
+  if (!c) return CPI_ERR_INVALID;
+  Ctl h;
+  int rc = settled_ctl(c, &h);
+  if (rc) return rc;
+  if (taken) *taken = h.resident;
+  if (redone) *redone = c->redone;
   return CPI_OK;
 }
 

@@ -38,6 +38,7 @@ struct Ctl {
   uint32_t decision;
   uint64_t finished;
   int64_t missed;
+  int64_t resident;  // steps that resident launches took
   double e0;       // KE + Epen of the initial state
   double row[8];   // latest energy row (CPI_E_* order)
   double dt_contact;  // wall-spring limit 2 sqrt(m_min / k) (fixed: mass is)

@@ -1326,7 +1326,10 @@ k_resident(Params p, Resident rs) {
   }
   const int row_base = p.epart_base + b * (NT / 64);
   wave_flush<false>(p, row_base, ea, row_prefetch(p, row_base));
-  if (blockIdx.x == 0 && t == 0) p.ctl->step += rs.steps;
+  if (blockIdx.x == 0 && t == 0) {
+    p.ctl->step += rs.steps;
+    p.ctl->resident += rs.steps;
+  }
 }
 
 // ---------------------------------------------------------------------------

@@ -283,6 +283,13 @@ class Dynamics:
         L.check(L.lib().cpi_get_info(self.ctx, C.byref(inf)), self.ctx)
         return inf
 
+    def resident_steps(self):
+        """(steps since init that resident launches took, steps taken one by one
+        after such a launch gave up)."""
+        a, b = C.c_int64(), C.c_int64()
+        L.check(L.lib().cpi_get_resident_steps(self.ctx, C.byref(a), C.byref(b)), self.ctx)
+        return a.value, b.value
+
     def coloring(self):
         col = np.zeros(self.mesh.num_elements, dtype=np.int32)
         n = C.c_int32()

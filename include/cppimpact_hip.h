@@ -278,6 +278,12 @@ int cpi_get_energy_history(cpi_ctx *ctx, double *rows, int32_t cap,
 int cpi_get_info(cpi_ctx *ctx, cpi_info *info);
 
 /* Greedy colour of every element (user order) and the colour count. */
+/* How the steps since cpi_init were taken (diagnostics): taken of them in
+   resident launches (the plain steps of a call in one launch, small meshes),
+   redone of them one by one after such a launch gave up.  Either may be
+   NULL. */
+int cpi_get_resident_steps(cpi_ctx *ctx, int64_t *taken, int64_t *redone);
+
 int cpi_get_coloring(cpi_ctx *ctx, int32_t *color, int32_t *num_colors);
 
 /* Enqueues nsteps steps between two HIP events on the context's stream and
