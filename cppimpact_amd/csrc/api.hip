@@ -1146,6 +1146,7 @@ extern "C" int cpi_step(cpi_ctx *c, int32_t nsteps) {
     if (e == hipSuccess) {
       c->res.base ^= c->res.steps & 1;
       c->res_pending = true;
+      HIPCHK(c, launch_resident_loose(p, c->res, c->stream));
       rest = 1;
     } else {
       (void)hipGetLastError();

@@ -29,6 +29,8 @@ hipError_t launch_elem_direct(const Params &p, int rule, int prec, int phys, boo
 int resident_capacity(int npe, int rule, int prec, int phys, size_t smem, int cus);
 hipError_t launch_resident(const Params &p, int rule, int prec, int phys, const Resident &rs,
                            int nblocks, size_t smem, hipStream_t s);
+// its nodes of no element, after it
+hipError_t launch_resident_loose(const Params &p, const Resident &rs, hipStream_t s);
 hipError_t launch_mail_clear(const Resident &rs, int prec, hipStream_t s);
 // LDS of a resident workgroup and bytes of the mail records
 size_t resident_smem(size_t block_smem, int prec, int most);

@@ -1302,34 +1302,36 @@ k_resident(Params p, Resident rs) {
     const unsigned long long nb = __ballot(has_e && pre.ep > R(0));
     if (has_word && (t & 63) == 0) p.yielded[yi] = nb;
   }
-  // nodes of no element (no block holds one): only gravity and the wall act on
-  // them, so each takes its steps here by itself
-  const Params pl = params_again(args, p);
-  for (int n = pl.nn - rs.loose + (int)blockIdx.x * NT + t; n < pl.nn; n += (int)gridDim.x * NT) {
-    const bool nheld = node_held(pl, n), ncontact = node_contact(pl, n, nheld);
-    const double f[3] = {0.0, 0.0, 0.0}, m = pl.m[n];
-    const Vec3 xr = pl.pos[n], vr = pl.vv[n];
-    double x[3] = {xr.x, xr.y, xr.z}, v[3] = {vr.x, vr.y, vr.z};
-    for (int k = 0; k < rs.steps; k++) {
-      NodeStep s;
-      EAcc en;
-      node_advance(pl, nheld, ncontact, f, x, v, m, 1.0 / m, dt, s, en);
-      ea.wgrav += en.wgrav;
-#pragma unroll
-      for (int c = 0; c < 3; c++) {
-        x[c] = s.x[c];
-        v[c] = s.v[c];
-      }
-    }
-    pl.pos[n] = Vec3{x[0], x[1], x[2]};
-    pl.vv[n] = Vec3{v[0], v[1], v[2]};
-  }
   const int row_base = p.epart_base + b * (NT / 64);
   wave_flush<false>(p, row_base, ea, row_prefetch(p, row_base));
   if (blockIdx.x == 0 && t == 0) {
     p.ctl->step += rs.steps;
     p.ctl->resident += rs.steps;
   }
+}
+
+// The nodes of no element, the last ones: no block holds one, and only gravity
+// and the wall act on them, so each takes a resident launch's steps by itself,
+// once the launch counts.
+__global__ void __launch_bounds__(256) k_resident_loose(Params p, Resident rs) {
+  const int g = p.nn - rs.loose + (int)(blockIdx.x * 256 + threadIdx.x);
+  if (g >= p.nn || p.ctl->decision != 2u * rs.launch) return;
+  const bool held = node_held(p, g), contact = node_contact(p, g, held);
+  const double f[3] = {0.0, 0.0, 0.0}, m = p.m[g], dt = p.ctl->dt;
+  const Vec3 xr = p.pos[g], vr = p.vv[g];
+  double x[3] = {xr.x, xr.y, xr.z}, v[3] = {vr.x, vr.y, vr.z};
+  for (int k = 0; k < rs.steps; k++) {
+    NodeStep s;
+    EAcc ea;  // without mass there is no energy
+    node_advance(p, held, contact, f, x, v, m, 1.0 / m, dt, s, ea);
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+      x[c] = s.x[c];
+      v[c] = s.v[c];
+    }
+  }
+  p.pos[g] = Vec3{x[0], x[1], x[2]};
+  p.vv[g] = Vec3{v[0], v[1], v[2]};
 }
 
 // ---------------------------------------------------------------------------
@@ -2248,6 +2250,11 @@ hipError_t launch_elem_direct(const Params &p, int rule, int prec, int phys, boo
 // leave a CU no second block, and get the registers
 template <int NPE, int RULE> constexpr int resident_waves() {
   return NPE == 10 && Quad<RULE>::n == 5 ? 3 : 4;
+}
+
+hipError_t launch_resident_loose(const Params &p, const Resident &rs, hipStream_t s) {
+  if (rs.loose == 0) return hipSuccess;
+  CPI_LAUNCH(k_resident_loose, (rs.loose + 255) / 256, 256, 0, s, p, rs);
 }
 
 template <int NPE, int RULE, typename R, int PHYS> struct ResidentF {
