@@ -68,7 +68,10 @@ struct cpi_ctx {
   Resident res{};
   size_t res_smem = 0;
   bool resident = false;
-  bool res_pending = false;  // launched since the control block was last read
+  // launches whose outcome the host has not seen, and the step that each call
+  // since the first of them ends at (kMaxCalls at most)
+  bool res_pending = false;
+  std::vector<int64_t> calls;
   int64_t redone = 0;        // steps taken one by one instead, since cpi_init
   bool mass_ready = false, inited = false;
   double dt = 0.0;
@@ -339,6 +342,9 @@ constexpr int kGraphRuns[2] = {32, 4};
 // cooperative launch and first loads cost as much as a few steps
 constexpr int kMinResident = 4;
 
+// most calls queued on resident launches of unknown outcome (cpi_ctx::calls)
+constexpr size_t kMaxCalls = 1024;
+
 int capture(cpi_ctx *c, bool aux, hipGraphExec_t *out, int nrep = 1) {
   hipGraph_t g = nullptr;
   HIPCHK(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
@@ -454,20 +460,26 @@ int report_flags(cpi_ctx *c, const Ctl &h) {
 
 int steps_one_by_one(cpi_ctx *c, int64_t nsteps);
 
-// Steps that resident launches missed are taken now, one launch per kernel of
-// a step: the state does not depend on how its steps were launched, only on
-// their number.  h: the control block as read after the launches.
-int settle(cpi_ctx *c, const Ctl &h) {
+// The outcome of the resident launches is known: done steps were taken.  The
+// first launch to give up left out every step queued behind it; they are taken
+// now, one launch per kernel of a step and call by call, so that each call's
+// energies are those of its own last step.  Until that has succeeded the
+// launches stay pending, and the next read tries again.
+int settle(cpi_ctx *c, int64_t done, bool *missing) {
+  *missing = done < c->step;
+  if (*missing) {
+    c->resident = false;
+    HIPCHK(c, hipMemsetAsync(&c->P.ctl->decision, 0, sizeof(uint32_t), c->stream));
+    for (const int64_t end : c->calls) {
+      if (end <= done) continue;
+      int rc = steps_one_by_one(c, end - done);
+      if (rc) return rc;
+      c->redone += end - done;
+      done = end;
+    }
+  }
   c->res_pending = false;
-  if (!(h.decision & 1u)) return CPI_OK;
-  c->resident = false;
-  int rc = steps_one_by_one(c, h.missed);
-  if (rc) return rc;
-  c->redone += h.missed;
-  // no launch reads these again; a later call must not settle twice
-  HIPCHK(c, hipMemsetAsync(&c->P.ctl->decision, 0, sizeof(uint32_t), c->stream));
-  HIPCHK(c, hipMemsetAsync(&c->P.ctl->missed, 0, sizeof(int64_t), c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
+  c->calls.clear();
   return CPI_OK;
 }
 
@@ -475,9 +487,9 @@ int settle(cpi_ctx *c, const Ctl &h) {
 int settled_ctl(cpi_ctx *c, Ctl *h) {
   int rc = get_ctl(c, h);
   if (rc || !c->res_pending) return rc;
-  const bool missed = h->decision & 1u;
-  if ((rc = settle(c, *h))) return rc;
-  return missed ? get_ctl(c, h) : CPI_OK;
+  bool missing;
+  rc = settle(c, h->step, &missing);
+  return rc || !missing ? rc : get_ctl(c, h);
 }
 
 // before results are read by other ways than the control block
@@ -904,10 +916,12 @@ static int create_impl(cpi_ctx *c, const cpi_mesh_desc *m, const cpi_material *m
             (rc = dalloc(c, &ms, n)) || (rc = upload(c, ms, M.src)) || (rc = dalloc(c, &mi, n)) ||
             (rc = upload(c, mi, M.idx)))
           return rc;
-        c->res = Resident{mail, (int)n, M.most, mf, md, ms, mlo, mi, (int)c->loose.size(), 0, 0, 0,
-                          opt->debug_fill_nan & 2 ? 1u : 1u << 20};
+        c->res = Resident{mail, (int)n, M.most, mf, md, ms, mlo, mi, 0, 0, 0,
+                          opt->debug_fill_nan & 2 ? 1u : 1u << 20, (int)c->loose.size()};
         c->res_smem = smem;
+        c->calls.reserve(kMaxCalls + 1);
         c->resident = true;
+        P.resident = B.nblocks > 1;  // one block waits for nobody
       }
     }
     // one energy row per wave
@@ -1006,7 +1020,8 @@ extern "C" int cpi_set_state(cpi_ctx *c, const double *x0, const double *v0) {
   if (v0 && !all_finite(v0, n)) return fail(c, CPI_ERR_INVALID, "non-finite velocity");
   if (x0) c->mass_ready = false;
   c->inited = false;
-  c->res_pending = false;
+  c->res_pending = false;  // steps of a state that is given up
+  c->calls.clear();
   int rc = x0 ? put_nodes(c, x0, nullptr, c->P.X0) : CPI_OK;
   if (!rc && v0) rc = put_nodes(c, v0, c->d_V0, nullptr);
   return rc ? rc : reset_state(c);
@@ -1088,6 +1103,7 @@ extern "C" int cpi_init(cpi_ctx *c, double dt) {
     return fail(c, CPI_ERR_STATE, "cpi_init: CPI_RETURN_MLP needs cpi_set_surrogate first");
   c->inited = false;
   c->res_pending = false;  // steps of a state that is given up
+  c->calls.clear();
   int rc = reset_state(c);
   if (!rc) rc = compute_mass(c);
   if (rc) return rc;
@@ -1134,9 +1150,18 @@ extern "C" int cpi_step(cpi_ctx *c, int32_t nsteps) {
   if (!c->inited) return fail(c, CPI_ERR_STATE, "cpi_step before cpi_init");
   if (nsteps < 0) return fail(c, CPI_ERR_INVALID, "nsteps < 0");
   int64_t rest = nsteps;
+  int rc = CPI_OK;
+  auto may = [&]() {
+    return c->resident && c->gs.plain && !c->P.samples && nsteps - 1 >= kMinResident;
+  };
+  // plain steps launched one by one run whatever became of the launches before
+  // them: these have to be settled first
+  if (c->res_pending && ((!may() && nsteps > 1) || !c->resident || c->calls.size() >= kMaxCalls) &&
+      (rc = settled(c)))
+    return rc;
   // the plain steps in one launch (the last step of a call is the one with
   // the energies and outputs)
-  if (c->resident && c->gs.plain && !c->P.samples && nsteps - 1 >= kMinResident) {
+  if (may()) {
     c->res.steps = nsteps - 1;
     c->res.launch++;
     Params p = c->P;
@@ -1145,17 +1170,19 @@ extern "C" int cpi_step(cpi_ctx *c, int32_t nsteps) {
                                          c->res_smem, c->stream);
     if (e == hipSuccess) {
       c->res.base ^= c->res.steps & 1;
-      c->res_pending = true;
+      c->res_pending = c->P.resident;
       HIPCHK(c, launch_resident_loose(p, c->res, c->stream));
       rest = 1;
     } else {
       (void)hipGetLastError();
       c->resident = false;  // the per-step launches from here on
+      if ((rc = settled(c))) return rc;
     }
   }
-  int rc = steps_one_by_one(c, rest);
+  rc = steps_one_by_one(c, rest);
   if (rc) return rc;
   c->step += nsteps;
+  if (c->res_pending) c->calls.push_back(c->step);
   return CPI_OK;
 }
 
@@ -1221,12 +1248,14 @@ extern "C" int cpi_get_state_mass3(cpi_ctx *c, double *x, double *v, double *a, 
   o.half_dt = 0.5 * c->dt;
   HIPCHK(c, launch_export_nodes(c->P, c->d_ninv, o, c->stream));
   if ((rc = bring_back(c, p, k))) return rc;
-  if (c->res_pending && (h.decision & 1u)) {
-    if ((rc = settle(c, h))) return rc;
-    HIPCHK(c, launch_export_nodes(c->P, c->d_ninv, o, c->stream));
-    if ((rc = bring_back(c, p, k))) return rc;
+  if (c->res_pending) {
+    bool missing;
+    if ((rc = settle(c, h.step, &missing))) return rc;
+    if (missing) {
+      HIPCHK(c, launch_export_nodes(c->P, c->d_ninv, o, c->stream));
+      if ((rc = bring_back(c, p, k))) return rc;
+    }
   }
-  c->res_pending = false;
   return c->inited ? report_flags(c, h) : CPI_OK;
 }
 
@@ -1365,8 +1394,8 @@ extern "C" int cpi_get_info(cpi_ctx *c, cpi_info *info) {
 
 extern "C" int cpi_get_resident_steps(cpi_ctx *c, int64_t *taken, int64_t *redone) {
   if (!c) return CPI_ERR_INVALID;
-  Ctl h;
-  int rc = settled_ctl(c, &h);
+  Ctl h{};
+  int rc = c->inited ? settled_ctl(c, &h) : CPI_OK;
   if (rc) return rc;
   if (taken) *taken = h.resident;
   if (redone) *redone = c->redone;
@@ -1382,13 +1411,22 @@ extern "C" int cpi_get_coloring(cpi_ctx *c, int32_t *color, int32_t *ncol) {
 
 extern "C" int cpi_time_steps(cpi_ctx *c, int32_t nsteps, double *ms) {
   if (!c || !ms) return CPI_ERR_INVALID;
+  int rc = settled(c);  // the steps queued before have no part in the time
+  if (rc) return rc;
   hipEvent_t a, b;
   HIPCHK(c, hipEventCreate(&a));
   HIPCHK(c, hipEventCreate(&b));
   HIPCHK(c, hipEventRecord(a, c->stream));
-  int rc = cpi_step(c, nsteps);
+  rc = cpi_step(c, nsteps);
   HIPCHK(c, hipEventRecord(b, c->stream));
   HIPCHK(c, hipEventSynchronize(b));
+  // steps that a resident launch left out belong to the time
+  const int64_t redone = c->redone;
+  if (!rc) rc = settled(c);
+  if (c->redone != redone) {
+    HIPCHK(c, hipEventRecord(b, c->stream));
+    HIPCHK(c, hipEventSynchronize(b));
+  }
   float t = 0.f;
   HIPCHK(c, hipEventElapsedTime(&t, a, b));
   (void)hipEventDestroy(a);
@@ -1401,6 +1439,7 @@ extern "C" int cpi_profile_kernels(cpi_ctx *c, int32_t nsteps, cpi_kernel_time *
                                    int32_t *count) {
   if (!c || !out || !count) return CPI_ERR_INVALID;
   if (!c->inited) return fail(c, CPI_ERR_STATE, "cpi_profile_kernels before cpi_init");
+  if (int rc = settled(c)) return rc;
   // with the surrogate the element pass is three launches: every other step
   // times them one by one, "elem_pass" (the elastic pass), "mlp_queue" (the
   // network on the queue) and "mlp_walk" (the deferred blocks), and the

@@ -32,12 +32,11 @@ struct Ctl {
   uint32_t flags;  // bit 0: non-finite energy, bit 1: inverted element,
                    // bit 2: dt above the stable limit of the configuration
   // resident launches, numbered from 1: decision is 2 L once launch L has
-  // stored its steps, 2 L + 1 if it gave up, and then no later one runs;
-  // finished counts the workgroups that reached the end, missed the steps of
-  // the launches that did not run
+  // stored its steps, 2 L + 1 if it gave up, and then neither a later one nor
+  // a step with outputs (STEP_OUT_ASK) does anything until the host has
+  // cleared it; finished counts the workgroups that reached the end
   uint32_t decision;
   uint64_t finished;
-  int64_t missed;
   int64_t resident;  // steps that resident launches took
   double e0;       // KE + Epen of the initial state
   double row[8];   // latest energy row (CPI_E_* order)
@@ -155,6 +154,7 @@ struct Params {
   int2 *mlp_list;        // [nblocks] (block, its first queue row)
   uint16_t *mlp_rows;    // [ne + 16] rows of 32 bytes (see mlp_infer.h)
   int nblocks;           // element blocks of the block scatter
+  int resident;          // the context takes resident steps
   float *samples;        // return-mapping sample buffer (optional)
   int *sample_count;
   int sample_cap;
@@ -174,10 +174,10 @@ struct Resident {
   const uint16_t *src;  // per message: the local node it is of
   const int32_t *lo;    // [nblocks][ml]: start of a shared node's list in idx
   const uint16_t *idx;  // lists of the block's messages per node, in slot order
-  int loose;            // nodes of no element, the last ones
   int base, steps;      // inbox of the first step, steps to take
   unsigned launch;      // number of the launch (Ctl::decision)
   unsigned spin_limit;  // polls of one wait before it gives up
+  int loose;            // nodes of no element, the last ones
 };
 
 // ---------------------------------------------------------------------------

@@ -76,6 +76,16 @@ __device__ __forceinline__ RowPre row_prefetch(const Params &p, int base) {
   return RowPre{r[EP_WINT], r[EP_WPL], r[EP_BAD], r[EP_WGRAV]};
 }
 
+// Variants of the step kernels: a plain step; one with outputs; and one with
+// outputs of a context that takes resident steps, which is left out when it
+// was queued behind a launch that gave up.  It costs 0.2 to 0.7 us of a step
+// with outputs of 24 to 32 us, and is a variant of its own because the step of
+// a mesh too large to be resident lost 1-2% (1.57M tet4, FP64: 102 -> 104 us).
+enum : int { STEP_PLAIN = 0, STEP_OUT = 1, STEP_OUT_ASK = 2 };
+template <int AUX> __device__ __forceinline__ bool left_out(const Params &p) {
+  return AUX == STEP_OUT_ASK && (p.ctl->decision & 1u);
+}
+
 // Scalar loads issued at the kernel's start (the energy row, dt) must not
 // sink: the compiler moves them down to their first use, past the loads of
 // the node records, where the whole workgroup then waits for another round
@@ -382,7 +392,7 @@ __device__ __forceinline__ void tet10_five(const Params &p, const At &at, const 
 // LDS: node records (LNodes), corner forces [max_el*10][3] R in jagged-
 // diagonal slots (local node j's k-th contribution at off[k] + j), off[k].
 // ---------------------------------------------------------------------------
-template <int RULE, typename R, int PHYS, bool AUX, int NT, int WPE>
+template <int RULE, typename R, int PHYS, int AUX, int NT, int WPE>
 __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WPE)))
 k_elem_block5(Params p) {
   extern __shared__ double smem[];
@@ -397,6 +407,7 @@ k_elem_block5(Params p) {
   R *lf = (R *)((char *)smem + lds_node_bytes(ml));
   uint16_t *joff = (uint16_t *)((char *)lf + lds_force_bytes(sizeof(R), 10, p.max_el));
   const double dt = p.ctl->dt;
+  const bool leave = left_out<AUX>(p);
   const int lane = threadIdx.x & 63, q = lane % NQ, te = (threadIdx.x >> 6) * EW + lane / NQ;
 
   // a thread's element words, local ids and slots two per word (rows of 20
@@ -424,6 +435,7 @@ k_elem_block5(Params p) {
   }
   for (int k = threadIdx.x; k <= p.kmax; k += NT) joff[k] = p.off_pad[(long)b * (p.kmax + 1) + k];
   __syncthreads();
+  if (leave) return;
 
   EAcc ea;
   for (int t = te; lane < NQ * EW && t < nel; t += EB) {
@@ -449,12 +461,12 @@ k_elem_block5(Params p) {
     if (slot < 0) {
       double x[3], v[3];
       ln.get(j, x, v);
-      node_update<AUX>(p, g, f, x, v, ln.mass(j), dt, ea);
+      node_update<AUX != 0>(p, g, f, x, v, ln.mass(j), dt, ea);
     } else {
       store_partial<R>(p, slot, f);
     }
   }
-  wave_flush<AUX>(p, p.epart_base + b * (NT / 64), ea, row);
+  wave_flush<AUX != 0>(p, p.epart_base + b * (NT / 64), ea, row);
 }
 
 // A workgroup's elements on a 4-point tet10 rule: the corner forces into the
@@ -514,7 +526,7 @@ __device__ __forceinline__ void tet10_block(const Params &p, const At &at, const
 // jagged-diagonal slot, off[rank] + local node; the nodes are then assembled
 // as in k_elem_block5, and the point's state is stored last.  LDS as
 // k_elem_block5, then the basis gradients (MM).
-template <int RULE, typename R, int PHYS, bool AUX, int NT, int WPE, bool STREAM, bool MM>
+template <int RULE, typename R, int PHYS, int AUX, int NT, int WPE, bool STREAM, bool MM>
 __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WPE)))
 k_elem_block10(Params p) {
   extern __shared__ double smem[];
@@ -530,6 +542,7 @@ k_elem_block10(Params p) {
   uint16_t *joff = (uint16_t *)((char *)lf + lds_force_bytes(sizeof(R), 10, p.max_el));
   double *basis = (double *)((char *)joff + lds_off_bytes(p.kmax));
   double dt = p.ctl->dt;
+  const bool leave = left_out<AUX>(p);
   // yielded bits, one per lane (point) of the wave: a point's ep is read
   // only when it has yielded before
   const int wv = __builtin_amdgcn_readfirstlane(t >> 6);
@@ -574,6 +587,7 @@ k_elem_block10(Params p) {
   if constexpr (MM)
     if (t < Tet10Basis<RULE>::n) basis[t] = gk;
   __syncthreads();
+  if (leave) return;
 
   EAcc ea;
   // set where the point is computed: a lane without one never reads its
@@ -595,12 +609,12 @@ k_elem_block10(Params p) {
     if (slot < 0) {
       double x[3], v[3];
       ln.get(t, x, v);
-      node_update<AUX>(p, g, f, x, v, ln.mass(t), dt, ea);
+      node_update<AUX != 0>(p, g, f, x, v, ln.mass(t), dt, ea);
     } else {
       store_partial<R>(p, slot, f);
     }
   }
-  wave_flush<AUX>(p, p.epart_base + b * (NT / 64), ea, row);
+  wave_flush<AUX != 0>(p, p.epart_base + b * (NT / 64), ea, row);
   // the point's state last (tet10_point_stress leaves it in pre), except in
   // the once-per-batch variant, whose outputs leave no registers for it
   if constexpr (PHYS != PHYS_COMPAT && !AUX)
@@ -633,7 +647,7 @@ k_elem_block10(Params p) {
 // barrier; otherwise the local ids and slots as two u16 arrays (16 B), for
 // plans whose blocks exceed the words (a node in more than 128 elements of
 // one block).
-template <typename R, int PHYS, bool AUX, int NT, bool WALK, bool STREAM, bool CW>
+template <typename R, int PHYS, int AUX, int NT, bool WALK, bool STREAM, bool CW>
 __device__ __forceinline__ void block4(const Params &p, const int b, const unsigned qbase,
                                        int *wcnt, unsigned *misc) {
   extern __shared__ double smem[];
@@ -645,6 +659,10 @@ __device__ __forceinline__ void block4(const Params &p, const int b, const unsig
   R *lf = (R *)((char *)smem + lds_node_bytes(p.ml));
   uint16_t *joff = (uint16_t *)((char *)lf + lds_force_bytes(sizeof(R), 4, p.max_el));
   double dt = p.ctl->dt;
+  const bool leave = left_out<AUX>(p);
+  // the FP64 EP body has no register to hold the answer in: it leaves at once
+  constexpr bool kEarly = sizeof(R) == 8 && PHYS == PHYS_EP;
+  if (kEarly && leave) return;
 
   // yielded bits of this wave's elements: a block has ywords words, one
   // per 64 elements of the largest block, and a wave past them (a block
@@ -688,6 +706,7 @@ __device__ __forceinline__ void block4(const Params &p, const int b, const unsig
   if constexpr (WALK)
     if (t == 0) misc[0] = misc[1] = 0u;
   __syncthreads();
+  if (!kEarly && leave) return;
 
   EAcc ea;
   // corner k's 16-bit field of the two loaded words: its local id for the
@@ -829,12 +848,12 @@ __device__ __forceinline__ void block4(const Params &p, const int b, const unsig
     if (slot < 0) {
       double x[3], v[3];
       ln.get(t, x, v);
-      node_update<AUX>(p, g, f, x, v, ln.mass(t), dt, ea);
+      node_update<AUX != 0>(p, g, f, x, v, ln.mass(t), dt, ea);
     } else {
       store_partial<R>(p, slot, f);
     }
   }
-  wave_flush<AUX>(p, p.epart_base + b * (NT / 64), ea, row);
+  wave_flush<AUX != 0>(p, p.epart_base + b * (NT / 64), ea, row);
   // the walk stores the element's state last: registers that a store
   // reads must not be reused before it completes, so a store issued
   // earlier would hold up the node pass (the exact-return body stores it
@@ -844,7 +863,7 @@ __device__ __forceinline__ void block4(const Params &p, const int b, const unsig
   }
 }
 
-template <typename R, int PHYS, bool AUX, int NT, int WPE, bool STREAM, bool CW>
+template <typename R, int PHYS, int AUX, int NT, int WPE, bool STREAM, bool CW>
 __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WPE)))
 k_elem_block4(Params p) {
   __shared__ int wcnt[NT / 64];
@@ -921,13 +940,14 @@ __device__ __forceinline__ void sum_records(const PR *rec, I s, I s1, double f[3
   if (s < s1) add(rec[s]);
 }
 
-template <bool AUX, typename R>
+template <int AUX, typename R>
 __global__ void __launch_bounds__(256) k_node_bnd(Params p) {
   using PR = typename std::conditional<std::is_same<R, float>::value, Vec3f, Vec3>::type;
   const PR *part = reinterpret_cast<const PR *>(p.partial);
   const int i = xcd_remap(blockIdx.x, gridDim.x) * 256 + threadIdx.x;
   const RowPre row = row_prefetch(p, p.epart_base + blockIdx.x * 4);
   const double dt = p.ctl->dt;
+  const bool leave = left_out<AUX>(p);
   EAcc ea;
   if (i < p.n_boundary) {
     const int g = p.n_interior + i;
@@ -937,9 +957,10 @@ __global__ void __launch_bounds__(256) k_node_bnd(Params p) {
     double f[3] = {0.0, 0.0, 0.0};
     sum_records(part, p.slot_ptr[i], p.slot_ptr[i + 1], f);
     const double x[3] = {xr.x, xr.y, xr.z}, v[3] = {vv.x, vv.y, vv.z};
-    node_update<AUX>(p, g, f, x, v, m, dt, ea);
+    if (!leave) node_update<AUX != 0>(p, g, f, x, v, m, dt, ea);
   }
-  wave_flush<AUX>(p, p.epart_base + blockIdx.x * 4, ea, row);
+  if (leave) return;
+  wave_flush<AUX != 0>(p, p.epart_base + blockIdx.x * 4, ea, row);
   // the last launch of the step: the surrogate's queue and block list start
   // empty in the next one
   if (blockIdx.x == 0 && threadIdx.x == 0) {
@@ -982,8 +1003,11 @@ __global__ void __launch_bounds__(256) k_node_bnd(Params p) {
 // spin_limit polls a thread decides that the launch gives up
 // (Ctl::decision), and every block leaves without storing anything.  The
 // blocks store their state only after the last of them to finish has decided
-// that the launch counts, so a launch takes all its steps or none; the host
-// takes missed steps with the per-step kernels (settled_ctl).
+// that the launch counts, so a launch takes all its steps or none.  Until the
+// host has seen to it (settled_ctl, which takes the missing steps with the
+// per-step kernels), the later launches and the steps with outputs queued
+// behind one that gave up are left out: what they would record belongs to
+// later steps.
 //
 // Same arithmetic in the same order as the per-step kernels: same state
 // bits.  The cumulative energies are summed over the steps per lane and over
@@ -1081,9 +1105,8 @@ __device__ __forceinline__ uint32_t decision(const Params &p) {
   return __hip_atomic_load(&p.ctl->decision, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 // launch L's decision, taken once: 0 it counts, 1 it gives up
-__device__ __forceinline__ void decide(const Params &p, unsigned L, unsigned how, int steps) {
-  if (atomicCAS(&p.ctl->decision, 2u * (L - 1u), 2u * L + how) == 2u * (L - 1u) && how)
-    p.ctl->missed = steps;
+__device__ __forceinline__ void decide(const Params &p, unsigned L, unsigned how) {
+  atomicCAS(&p.ctl->decision, 2u * (L - 1u), 2u * L + how);
 }
 
 template <int NPE, int RULE, typename R, int PHYS, int NT, int WPE>
@@ -1093,11 +1116,7 @@ k_resident(Params p, Resident rs) {
   extern __shared__ double smem[];
   __shared__ int gave_up;
   // after a launch that gave up, whose mail lies about, none runs
-  if (threadIdx.x == 0) {
-    const uint32_t past = decision(p);
-    gave_up = past & 1u;
-    if (blockIdx.x == 0 && gave_up && past >> 1 != rs.launch) p.ctl->missed += rs.steps;
-  }
+  if (threadIdx.x == 0) gave_up = decision(p) & 1u;
   __syncthreads();
   if (gave_up) return;
   const int b = xcd_remap(blockIdx.x, gridDim.x);
@@ -1234,7 +1253,6 @@ k_resident(Params p, Resident rs) {
       while (!Rec::get(mail, 2 * rs.messages, inbox + m0 + m, w)) {
         if (++spins >= rs.spin_limit || ((spins & 255u) == 0u && (decision(pl) & 1u))) {
           gave_up = 1;
-          decide(pl, rs.launch, 1u, rs.steps);
           break;
         }
         asm volatile("" ::: "memory");
@@ -1244,7 +1262,7 @@ k_resident(Params p, Resident rs) {
       for (int c = 0; c < 3; c++) lm[3 * m + c] = w[c];
     }
     __syncthreads();
-    if (gave_up) return;
+    if (gave_up) break;
     if (has_n) {
       const int own = (int)(own_cnt & 0xffffu), cnt = (int)(own_cnt >> 16);
       if (cnt != (int)kNotShared) {
@@ -1276,19 +1294,21 @@ k_resident(Params p, Resident rs) {
 
   // all blocks or none
   if (gridDim.x > 1) {
-    if (t == 0) {
+    if (t == 0 && gave_up) {
+      decide(p, rs.launch, 1u);
+    } else if (t == 0) {
       const uint64_t all = (uint64_t)rs.launch * gridDim.x;
       if (atomicAdd((unsigned long long *)&p.ctl->finished, 1ull) + 1ull == all)
-        decide(p, rs.launch, 0u, 0);
+        decide(p, rs.launch, 0u);
       uint32_t d = decision(p);
       for (unsigned spins = 0; d == 2u * (rs.launch - 1u); d = decision(p))
-        if (++spins == rs.spin_limit) decide(p, rs.launch, 1u, rs.steps);
+        if (++spins == rs.spin_limit) decide(p, rs.launch, 1u);
       gave_up = d & 1u;
     }
     __syncthreads();
     if (gave_up) return;
   } else if (t == 0) {
-    decide(p, rs.launch, 0u, 0);
+    decide(p, rs.launch, 0u);
   }
   if (has_n && (own_cnt & 0xffffu) == 0u) {
     const int n = p.nid_pad[o];
@@ -1485,12 +1505,14 @@ __global__ void __launch_bounds__(256) k_energy_reduce1(Params p) {
 
 __global__ void __launch_bounds__(64) k_energy_reduce2(Params p) {
   if (threadIdx.x == 0) {
+    const bool leave = left_out<STEP_OUT_ASK>(p);  // (0 without resident steps)
     double s[EP_N] = {0, 0, 1e300, 0, 0, 0, 0, 0};
     for (int b = 0; b < kEredBlocks; b++)
       for (int k = 0; k < EP_N; k++) {
         const double o = p.ered[b * EP_N + k];
         s[k] = (k == EP_MINDT) ? fmin(s[k], o) : s[k] + o;
       }
+    if (leave) return;
     Ctl *c = p.ctl;
     double row[8];
     row[0] = s[EP_KE];
@@ -2030,8 +2052,11 @@ template <typename R, int PHYS, bool STREAM, bool CW>
 static hipError_t tet4_opt_in(size_t smem) {
   constexpr int NT = block_threads<4, RULE_CENTROID>();
   constexpr int W = tet4_waves<R, PHYS>();
-  hipError_t e = lds_opt_in(k_elem_block4<R, PHYS, true, NT, W, STREAM, CW>, smem);
-  if (e == hipSuccess) e = lds_opt_in(k_elem_block4<R, PHYS, false, NT, W, STREAM, CW>, smem);
+  hipError_t e = lds_opt_in(k_elem_block4<R, PHYS, STEP_OUT, NT, W, STREAM, CW>, smem);
+  if (e == hipSuccess) e = lds_opt_in(k_elem_block4<R, PHYS, STEP_PLAIN, NT, W, STREAM, CW>, smem);
+  if constexpr (CW && PHYS != PHYS_EP_MLP)
+    if (e == hipSuccess)
+      e = lds_opt_in(k_elem_block4<R, PHYS, STEP_OUT_ASK, NT, W, STREAM, CW>, smem);
   if constexpr (PHYS == PHYS_EP_MLP) {
     if (e == hipSuccess)
       e = lds_opt_in(k_elem_block4_walk<true, NT, kMlpWalkWaves, STREAM, CW>, smem);
@@ -2055,10 +2080,10 @@ static hipError_t elem_block4_t(const Params &p, bool aux, int nblocks, size_t s
     // deferred blocks (part 1, 2, 3 alone for per-launch timing)
     if (part == 0 || part == 1) {
       if (aux)
-        timed_launch((k_elem_block4<R, PHYS, true, NT, W, STREAM, CW>), dim3(nblocks), dim3(NT), smem,
-                     s, p);
+        timed_launch((k_elem_block4<R, PHYS, STEP_OUT, NT, W, STREAM, CW>), dim3(nblocks), dim3(NT),
+                     smem, s, p);
       else
-        timed_launch((k_elem_block4<R, PHYS, false, NT, W, STREAM, CW>), dim3(nblocks), dim3(NT),
+        timed_launch((k_elem_block4<R, PHYS, STEP_PLAIN, NT, W, STREAM, CW>), dim3(nblocks), dim3(NT),
                      smem, s, p);
     }
     if (part == 0 || part == 2) {
@@ -2078,8 +2103,11 @@ static hipError_t elem_block4_t(const Params &p, bool aux, int nblocks, size_t s
     }
     return hipGetLastError();
   } else {
-    if (aux) CPI_LAUNCH((k_elem_block4<R, PHYS, true, NT, W, STREAM, CW>), nblocks, NT, smem, s, p);
-    CPI_LAUNCH((k_elem_block4<R, PHYS, false, NT, W, STREAM, CW>), nblocks, NT, smem, s, p);
+    if constexpr (CW)
+      if (aux && p.resident)
+        CPI_LAUNCH((k_elem_block4<R, PHYS, STEP_OUT_ASK, NT, W, STREAM, CW>), nblocks, NT, smem, s, p);
+    if (aux) CPI_LAUNCH((k_elem_block4<R, PHYS, STEP_OUT, NT, W, STREAM, CW>), nblocks, NT, smem, s, p);
+    CPI_LAUNCH((k_elem_block4<R, PHYS, STEP_PLAIN, NT, W, STREAM, CW>), nblocks, NT, smem, s, p);
   }
 }
 
@@ -2089,8 +2117,12 @@ template <int RULE, typename R, int PHYS, bool STREAM, bool MM>
 static hipError_t tet10_opt_in(size_t smem) {
   constexpr int NT = block_threads<10, RULE>();
   constexpr int W = tet10_waves<R>();
-  hipError_t e = lds_opt_in(k_elem_block10<RULE, R, PHYS, true, NT, W, STREAM, MM>, smem);
-  if (e == hipSuccess) e = lds_opt_in(k_elem_block10<RULE, R, PHYS, false, NT, W, STREAM, MM>, smem);
+  hipError_t e = lds_opt_in(k_elem_block10<RULE, R, PHYS, STEP_OUT, NT, W, STREAM, MM>, smem);
+  if (e == hipSuccess)
+    e = lds_opt_in(k_elem_block10<RULE, R, PHYS, STEP_PLAIN, NT, W, STREAM, MM>, smem);
+  if constexpr (MM || sizeof(R) == 4)
+    if (e == hipSuccess)
+      e = lds_opt_in(k_elem_block10<RULE, R, PHYS, STEP_OUT_ASK, NT, W, STREAM, MM>, smem);
   return e;
 }
 
@@ -2098,9 +2130,13 @@ template <int RULE, typename R, int PHYS, bool STREAM, bool MM>
 static hipError_t tet10_t(const Params &p, bool aux, int nblocks, size_t smem, hipStream_t s) {
   constexpr int NT = block_threads<10, RULE>();
   constexpr int W = tet10_waves<R>();
+  if constexpr (MM || sizeof(R) == 4)
+    if (aux && p.resident)
+      CPI_LAUNCH((k_elem_block10<RULE, R, PHYS, STEP_OUT_ASK, NT, W, STREAM, MM>), nblocks, NT, smem, s,
+                 p);
   if (aux)
-    CPI_LAUNCH((k_elem_block10<RULE, R, PHYS, true, NT, W, STREAM, MM>), nblocks, NT, smem, s, p);
-  CPI_LAUNCH((k_elem_block10<RULE, R, PHYS, false, NT, W, STREAM, MM>), nblocks, NT, smem, s, p);
+    CPI_LAUNCH((k_elem_block10<RULE, R, PHYS, STEP_OUT, NT, W, STREAM, MM>), nblocks, NT, smem, s, p);
+  CPI_LAUNCH((k_elem_block10<RULE, R, PHYS, STEP_PLAIN, NT, W, STREAM, MM>), nblocks, NT, smem, s, p);
 }
 
 template <int NPE, int RULE, typename R, int PHYS>
@@ -2129,11 +2165,13 @@ static hipError_t elem_block_t(const Params &p, bool aux, int nblocks, size_t sm
     constexpr int W = tet10_waves5<R, PHYS>();
     if (narrow5(nblocks, sizeof(R) == 8 && PHYS != PHYS_COMPAT)) {
       constexpr int N2 = kNarrow5;
-      if (aux) CPI_LAUNCH((k_elem_block5<RULE, R, PHYS, true, N2, W>), nblocks, N2, smem, s, p);
-      CPI_LAUNCH((k_elem_block5<RULE, R, PHYS, false, N2, W>), nblocks, N2, smem, s, p);
+      if (aux) CPI_LAUNCH((k_elem_block5<RULE, R, PHYS, STEP_OUT, N2, W>), nblocks, N2, smem, s, p);
+      CPI_LAUNCH((k_elem_block5<RULE, R, PHYS, STEP_PLAIN, N2, W>), nblocks, N2, smem, s, p);
     }
-    if (aux) CPI_LAUNCH((k_elem_block5<RULE, R, PHYS, true, NT, W>), nblocks, NT, smem, s, p);
-    CPI_LAUNCH((k_elem_block5<RULE, R, PHYS, false, NT, W>), nblocks, NT, smem, s, p);
+    if (aux && p.resident)
+      CPI_LAUNCH((k_elem_block5<RULE, R, PHYS, STEP_OUT_ASK, NT, W>), nblocks, NT, smem, s, p);
+    if (aux) CPI_LAUNCH((k_elem_block5<RULE, R, PHYS, STEP_OUT, NT, W>), nblocks, NT, smem, s, p);
+    CPI_LAUNCH((k_elem_block5<RULE, R, PHYS, STEP_PLAIN, NT, W>), nblocks, NT, smem, s, p);
   }
 }
 
@@ -2213,10 +2251,11 @@ template <int NPE, int RULE, typename R, int PHYS> struct ElemBlockPrepF {
         return e;
       } else {
         constexpr int W = tet10_waves5<R, PHYS>();
-        hipError_t e = lds_opt_in(k_elem_block5<RULE, R, PHYS, true, NT, W>, smem);
-        if (e == hipSuccess) e = lds_opt_in(k_elem_block5<RULE, R, PHYS, false, NT, W>, smem);
-        if (e == hipSuccess) e = lds_opt_in(k_elem_block5<RULE, R, PHYS, true, kNarrow5, W>, smem);
-        if (e == hipSuccess) e = lds_opt_in(k_elem_block5<RULE, R, PHYS, false, kNarrow5, W>, smem);
+        hipError_t e = lds_opt_in(k_elem_block5<RULE, R, PHYS, STEP_OUT, NT, W>, smem);
+        if (e == hipSuccess) e = lds_opt_in(k_elem_block5<RULE, R, PHYS, STEP_OUT_ASK, NT, W>, smem);
+        if (e == hipSuccess) e = lds_opt_in(k_elem_block5<RULE, R, PHYS, STEP_PLAIN, NT, W>, smem);
+        if (e == hipSuccess) e = lds_opt_in(k_elem_block5<RULE, R, PHYS, STEP_OUT, kNarrow5, W>, smem);
+        if (e == hipSuccess) e = lds_opt_in(k_elem_block5<RULE, R, PHYS, STEP_PLAIN, kNarrow5, W>, smem);
         return e;
       }
     }
@@ -2322,12 +2361,16 @@ size_t mail_bytes(int prec, size_t messages) {
 
 hipError_t launch_node_bnd(const Params &p, int prec, bool aux, hipStream_t s) {
   const int grid = std::max(1, (p.n_boundary + 255) / 256);
-  if (prec == 1) {
-    if (aux) CPI_LAUNCH((k_node_bnd<true, float>), grid, 256, 0, s, p);
-    CPI_LAUNCH((k_node_bnd<false, float>), grid, 256, 0, s, p);
+  if (aux && p.resident) {
+    if (prec == 1) CPI_LAUNCH((k_node_bnd<STEP_OUT_ASK, float>), grid, 256, 0, s, p);
+    CPI_LAUNCH((k_node_bnd<STEP_OUT_ASK, double>), grid, 256, 0, s, p);
   }
-  if (aux) CPI_LAUNCH((k_node_bnd<true, double>), grid, 256, 0, s, p);
-  CPI_LAUNCH((k_node_bnd<false, double>), grid, 256, 0, s, p);
+  if (prec == 1) {
+    if (aux) CPI_LAUNCH((k_node_bnd<STEP_OUT, float>), grid, 256, 0, s, p);
+    CPI_LAUNCH((k_node_bnd<STEP_PLAIN, float>), grid, 256, 0, s, p);
+  }
+  if (aux) CPI_LAUNCH((k_node_bnd<STEP_OUT, double>), grid, 256, 0, s, p);
+  CPI_LAUNCH((k_node_bnd<STEP_PLAIN, double>), grid, 256, 0, s, p);
 }
 
 hipError_t launch_node_all(const Params &p, int prec, bool aux, hipStream_t s) {
