@@ -64,10 +64,12 @@ struct cpi_ctx {
     hipGraphExec_t plain = nullptr, aux = nullptr;
     hipGraphExec_t run[2] = {nullptr, nullptr};
   } gs;
-  // resident steps (k_resident): usable, and the steps taken that way
+  // resident steps (k_resident): the plan allows them, and none has given up or
+  // failed since cpi_init
   Resident res{};
   size_t res_smem = 0;
-  bool resident = false;
+  bool res_able = false, resident = false;
+  hipEvent_t res_done[2] = {nullptr, nullptr};  // of every kAhead-th launch of a call, in turn
   // launches whose outcome the host has not seen, and the step that each call
   // since the first of them ends at (kMaxCalls at most)
   bool res_pending = false;
@@ -342,6 +344,24 @@ constexpr int kGraphRuns[2] = {32, 4};
 // cooperative launch and first loads cost as much as a few steps
 constexpr int kMinResident = 4;
 
+// Most steps of one resident launch.  A longer call takes several: between them
+// the chip is free for other streams' kernels (another context's ten steps, one
+// launch per kernel, took 440 ms beside a call of 60,000 in one launch, 12 to 40
+// ms so; its own resident launches wait for those queued before them, as
+// cooperative launches do), and one that gives up loses the steps of one launch
+// only.  A launch's fixed cost is 30 us, of the 4.5 to 10 ms of its steps.  At
+// most 2 kAhead launches are queued, where a call of millions of steps would
+// queue thousands.
+constexpr int64_t kMaxResident = 1024;
+constexpr int kAhead = 64;
+
+// Polls after which a wait of a resident launch gives up: 6 ms, much longer than
+// another stream's kernels hold up its last blocks, and short beside the waits
+// that never end (another kernel's blocks in between left two of this one's
+// without a contiguous piece of LDS on some CU), after which the context's steps
+// are launched one by one until the next cpi_init.
+constexpr unsigned kSpinLimit = 1u << 15;
+
 // most calls queued on resident launches of unknown outcome (cpi_ctx::calls)
 constexpr size_t kMaxCalls = 1024;
 
@@ -460,23 +480,24 @@ int report_flags(cpi_ctx *c, const Ctl &h) {
 
 int steps_one_by_one(cpi_ctx *c, int64_t nsteps);
 
-// The outcome of the resident launches is known: done steps were taken.  The
-// first launch to give up left out every step queued behind it; they are taken
-// now, one launch per kernel of a step and call by call, so that each call's
-// energies are those of its own last step.  Until that has succeeded the
-// launches stay pending, and the next read tries again.
-int settle(cpi_ctx *c, int64_t done, bool *missing) {
+// The outcome of the resident launches is known (h).  The first launch to give up
+// left out every step queued behind it; they are taken now, one launch per
+// kernel of a step and call by call, so that each call's energies are those of
+// its own last step.  Until that has succeeded the launches stay pending, and
+// the next read tries again.
+int settle(cpi_ctx *c, const Ctl &h, bool *missing) {
+  int64_t done = h.step;
   *missing = done < c->step;
-  if (*missing) {
+  if (h.decision & 1u) {
     c->resident = false;
     HIPCHK(c, hipMemsetAsync(&c->P.ctl->decision, 0, sizeof(uint32_t), c->stream));
-    for (const int64_t end : c->calls) {
-      if (end <= done) continue;
-      int rc = steps_one_by_one(c, end - done);
-      if (rc) return rc;
-      c->redone += end - done;
-      done = end;
-    }
+  }
+  for (const int64_t end : c->calls) {
+    if (end <= done) continue;
+    int rc = steps_one_by_one(c, end - done);
+    if (rc) return rc;
+    c->redone += end - done;
+    done = end;
   }
   c->res_pending = false;
   c->calls.clear();
@@ -488,7 +509,7 @@ int settled_ctl(cpi_ctx *c, Ctl *h) {
   int rc = get_ctl(c, h);
   if (rc || !c->res_pending) return rc;
   bool missing;
-  rc = settle(c, h->step, &missing);
+  rc = settle(c, *h, &missing);
   return rc || !missing ? rc : get_ctl(c, h);
 }
 
@@ -544,6 +565,8 @@ extern "C" void cpi_destroy(cpi_ctx *c) {
   for (void *p : c->allocs) (void)hipFree(p);
   if (c->pin) (void)hipHostFree(c->pin);
   for (hipEvent_t e : c->ring)
+    if (e) (void)hipEventDestroy(e);
+  for (hipEvent_t e : c->res_done)
     if (e) (void)hipEventDestroy(e);
   mlp_free(c->mlp);
   if (c->stream) (void)hipStreamDestroy(c->stream);
@@ -917,10 +940,12 @@ static int create_impl(cpi_ctx *c, const cpi_mesh_desc *m, const cpi_material *m
             (rc = upload(c, mi, M.idx)))
           return rc;
         c->res = Resident{mail, (int)n, M.most, mf, md, ms, mlo, mi, 0, 0, 0,
-                          opt->debug_fill_nan & 2 ? 1u : 1u << 20, (int)c->loose.size()};
+                          opt->debug_fill_nan & 2 ? 1u : kSpinLimit, (int)c->loose.size()};
         c->res_smem = smem;
         c->calls.reserve(kMaxCalls + 1);
-        c->resident = true;
+        for (hipEvent_t &e : c->res_done)
+          HIPCHK(c, hipEventCreateWithFlags(&e, hipEventDisableTiming));
+        c->res_able = true;
         P.resident = B.nblocks > 1;  // one block waits for nobody
       }
     }
@@ -1129,6 +1154,7 @@ extern "C" int cpi_init(cpi_ctx *c, double dt) {
   if (e == hipSuccess) e = launch_energy_reduce(c->P, c->stream);
   if (e != hipSuccess) return fail(c, CPI_ERR_HIP, std::string("init kernels: ") + hipGetErrorString(e));
   HIPCHK(c, hipMemsetAsync(c->P.epart, 0, sizeof(double) * EP_N * c->n_rows, c->stream));
+  c->resident = c->res_able;
   if (c->resident) {
     c->res.base = 0;
     c->res.launch = 0;
@@ -1159,10 +1185,16 @@ extern "C" int cpi_step(cpi_ctx *c, int32_t nsteps) {
   if (c->res_pending && ((!may() && nsteps > 1) || !c->resident || c->calls.size() >= kMaxCalls) &&
       (rc = settled(c)))
     return rc;
-  // the plain steps in one launch (the last step of a call is the one with
+  // the plain steps in a few launches (the last step of a call is the one with
   // the energies and outputs)
-  if (may()) {
-    c->res.steps = nsteps - 1;
+  int k = 0;
+  for (bool go = may(); go && rest > 1; k++) {
+    if (k % kAhead == 0) {
+      const hipEvent_t e = c->res_done[(k / kAhead) & 1];
+      if (k >= 2 * kAhead) HIPCHK(c, hipEventSynchronize(e));
+      if (rest > kMaxResident) HIPCHK(c, hipEventRecord(e, c->stream));
+    }
+    c->res.steps = (int)std::min(rest - 1, kMaxResident);
     c->res.launch++;
     Params p = c->P;
     p.epart_base = 0;
@@ -1172,11 +1204,14 @@ extern "C" int cpi_step(cpi_ctx *c, int32_t nsteps) {
       c->res.base ^= c->res.steps & 1;
       c->res_pending = c->P.resident;
       HIPCHK(c, launch_resident_loose(p, c->res, c->stream));
-      rest = 1;
+      rest -= c->res.steps;
     } else {
+      // the per-step launches from here on, for all that has not been taken
       (void)hipGetLastError();
-      c->resident = false;  // the per-step launches from here on
-      if ((rc = settled(c))) return rc;
+      go = c->resident = false;
+      Ctl h;
+      if ((rc = settled_ctl(c, &h))) return rc;
+      rest = c->step + nsteps - h.step;
     }
   }
   rc = steps_one_by_one(c, rest);
@@ -1250,7 +1285,7 @@ extern "C" int cpi_get_state_mass3(cpi_ctx *c, double *x, double *v, double *a, 
   if ((rc = bring_back(c, p, k))) return rc;
   if (c->res_pending) {
     bool missing;
-    if ((rc = settle(c, h.step, &missing))) return rc;
+    if ((rc = settle(c, h, &missing))) return rc;
     if (missing) {
       HIPCHK(c, launch_export_nodes(c->P, c->d_ninv, o, c->stream));
       if ((rc = bring_back(c, p, k))) return rc;
