@@ -922,14 +922,20 @@ static int create_impl(cpi_ctx *c, const cpi_mesh_desc *m, const cpi_material *m
       return fail(c, CPI_ERR_HIP, std::string("LDS opt-in for the element kernel: ") +
                                       hipGetErrorString(pe));
     // resident steps when every block fits the chip at once
+    // (asked with no mail first: most meshes are too large, and their messages
+    // need not be counted)
+    auto fits = [&](size_t smem) {
+      return smem <= (size_t)prop.sharedMemPerBlock &&
+             B.nblocks <= resident_capacity(npe, c->rule, c->prec, c->phys, smem,
+                                            prop.multiProcessorCount);
+    };
     if (opt->use_graph && c->phys != 2 && words && prop.cooperativeLaunch &&
-        (npe == 4 || five || c->prec == CPI_PREC_F32 || P.matrix)) {
-      const MailPlan M = build_mail(B);
-      const size_t n = M.dest.size(), bytes = mail_bytes(c->prec, n);
-      const size_t smem = resident_smem(c->smem, c->prec, M.most);
-      if (bytes <= (size_t)INT32_MAX && M.most <= 65535 && smem <= (size_t)prop.sharedMemPerBlock &&
-          B.nblocks <= resident_capacity(npe, c->rule, c->prec, c->phys, smem,
-                                         prop.multiProcessorCount)) {
+        (npe == 4 || five || c->prec == CPI_PREC_F32 || P.matrix) && fits(c->smem)) {
+      const MailCount N = count_mail(B);
+      const size_t n = N.all, bytes = mail_bytes(c->prec, n);
+      const size_t smem = resident_smem(c->smem, c->prec, (int)std::min<size_t>(N.most, 65536));
+      if (bytes <= (size_t)INT32_MAX && N.most <= 65535 && fits(smem)) {
+        const MailPlan M = build_mail(B);
         char *mail = nullptr;
         int32_t *mf, *mlo, *md;
         uint16_t *ms, *mi;
@@ -1027,6 +1033,9 @@ extern "C" int cpi_create(const cpi_mesh_desc *m, const cpi_material *mat, const
     rc = create_impl(c, m, mat, wall, opt ? opt : &def);
   } catch (const std::bad_alloc &) {
     c->err = "cpi_create: out of host memory";
+    rc = CPI_ERR_ALLOC;
+  } catch (const std::exception &e) {
+    c->err = std::string("cpi_create: ") + e.what();
     rc = CPI_ERR_ALLOC;
   }
   if (rc) {

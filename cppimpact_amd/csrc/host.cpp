@@ -464,6 +464,22 @@ bool build_block_plan(int ne, int npe, const int32_t *conn, int nn,
   return true;
 }
 
+MailCount count_mail(const BlockPlan &P) {
+  MailCount N;
+  for (int b = 0; b < P.nblocks; b++) {
+    size_t n = 0;
+    for (int l = 0; l < P.max_local_nodes; l++) {
+      const size_t i = (size_t)b * P.max_local_nodes + l;
+      if (P.slot_pad[i] < 0) continue;
+      const int k = P.nid_pad[i] - P.n_interior;
+      n += P.slot_ptr[k + 1] - P.slot_ptr[k] - 1;
+    }
+    N.all += n;
+    N.most = std::max(N.most, n);
+  }
+  return N;
+}
+
 MailPlan build_mail(const BlockPlan &P) {
   MailPlan M;
   const int nb = P.nblocks, ml = P.max_local_nodes, ns = P.n_slots;

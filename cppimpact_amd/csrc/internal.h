@@ -79,6 +79,12 @@ struct MailPlan {
   int most = 0;  // messages of one block
 };
 MailPlan build_mail(const BlockPlan &plan);
+// The messages of a plan, all and the most of one block, without their tables
+// (which hold up to 2^31 of them).
+struct MailCount {
+  size_t all = 0, most = 0;
+};
+MailCount count_mail(const BlockPlan &plan);
 
 // Corner-force slots of the colour scatter: node n's slots are node_slot[n]
 // .. node_slot[n+1], one per element that holds it, in ascending colour, and
