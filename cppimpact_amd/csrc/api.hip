@@ -178,15 +178,31 @@ constexpr size_t kRing = 32;
 constexpr int kCopyThreads = 6;
 constexpr size_t kStateWords = (sizeof(Ctl) + 7) / 8;  // ahead of the exported arrays
 
-int ensure_tmp(cpi_ctx *c, size_t n);
+// Words of d_tmp.  Nodal results pass at once where the device has room, else in
+// parts of kTmpLow (16 MiB).  For an element state, which may be a third of the
+// device's memory, it grows to kTmpMost (128 MiB) at most: a part costs 0.1 ms
+// for its launch and copy threads, of the 4.6 ms its transfer takes.
+constexpr size_t kTmpLow = 2u << 20, kTmpMost = 16u << 20;
+
+// What passes through d_tmp goes in as many parts as it takes: n items of
+// words doubles each, beside head words.  The first item and the number of
+// items of each part to f.
+template <class F>
+int in_parts(cpi_ctx *c, size_t n, size_t words, size_t head, const F &f) {
+  const size_t part = words ? std::max<size_t>(1, (c->tmp_len - head) / words) : n;
+  for (size_t i = 0; i < n; i += part)
+    if (int rc = f(i, std::min(part, n - i))) return rc;
+  return CPI_OK;
+}
 
 // user-order [N][3] on the host -> nodal records in device node order
 int put_nodes(cpi_ctx *c, const double *aos, Vec3 *d3, Node4 *d4) {
-  const size_t n = 3 * (size_t)c->nn;
-  int rc = ensure_tmp(c, n);
+  int rc = in_parts(c, c->nn, 3, 0, [&](size_t i, size_t n) -> int {
+    HIPCHK(c, hipMemcpyAsync(c->d_tmp, aos + 3 * i, 24 * n, hipMemcpyHostToDevice, c->stream));
+    HIPCHK(c, launch_import_nodes(c->d_tmp, c->d_ninv + i, (int)n, d3, d4, c->stream));
+    return CPI_OK;
+  });
   if (rc) return rc;
-  HIPCHK(c, hipMemcpyAsync(c->d_tmp, aos, sizeof(double) * n, hipMemcpyHostToDevice, c->stream));
-  HIPCHK(c, launch_import_nodes(c->d_tmp, c->d_ninv, c->nn, d3, d4, c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));  // d_tmp and the caller's array are free again
   return CPI_OK;
 }
@@ -401,18 +417,23 @@ int capture_graphs(cpi_ctx *c) {
   return CPI_OK;
 }
 
+// d_tmp of n words at least, on the context's device whichever is current.  On
+// failure it is what it was.
 int ensure_tmp(cpi_ctx *c, size_t n) {
   if (c->tmp_len >= n) return CPI_OK;
+  int cur = 0;
+  HIPCHK(c, hipGetDevice(&cur));
+  if (cur != c->dev) HIPCHK(c, hipSetDevice(c->dev));
+  double *p = nullptr;
+  int rc = dalloc(c, &p, n);
+  if (rc) (void)hipGetLastError();  // not to be taken for a launch's
+  if (cur != c->dev) HIPCHK(c, hipSetDevice(cur));
+  if (rc) return rc;
   if (c->d_tmp) {
     HIPCHK(c, hipStreamSynchronize(c->stream));
     c->allocs.erase(std::find(c->allocs.begin(), c->allocs.end(), (void *)c->d_tmp));
     (void)hipFree(c->d_tmp);
-    c->d_tmp = nullptr;
-    c->tmp_len = 0;
   }
-  double *p = nullptr;
-  int rc = dalloc(c, &p, n);
-  if (rc) return rc;
   c->d_tmp = p;
   c->tmp_len = n;
   return CPI_OK;
@@ -653,12 +674,17 @@ static int create_impl(cpi_ctx *c, const cpi_mesh_desc *m, const cpi_material *m
   {
     const size_t all = 8 * (kStateWords + 16 * (size_t)c->nn);
     size_t pinned = kSmall;
-    if (all > kSmall) {
+    if (all > kSmall && !(opt->debug_fill_nan & 4)) {
       c->ring.resize(std::min(kRing, (all + kChunk - 1) / kChunk), nullptr);
       pinned = std::max(pinned, c->ring.size() * kChunk);
       for (hipEvent_t &e : c->ring) HIPCHK(c, hipEventCreateWithFlags(&e, hipEventDisableTiming));
     }
-    HIPCHK(c, hipHostMalloc((void **)&c->pin, pinned, hipHostMallocDefault));
+    if (hipHostMalloc((void **)&c->pin, pinned, hipHostMallocDefault) != hipSuccess) {
+      (void)hipGetLastError();
+      for (hipEvent_t e : c->ring) (void)hipEventDestroy(e);
+      c->ring.clear();
+      HIPCHK(c, hipHostMalloc((void **)&c->pin, kSmall, hipHostMallocDefault));
+    }
   }
   // device orders
   if (c->scatter == CPI_SCATTER_BLOCK) {
@@ -1003,8 +1029,12 @@ static int create_impl(cpi_ctx *c, const cpi_mesh_desc *m, const cpi_material *m
     P.mlp = c->mlp.d_params;
     P.mlp_stats = c->mlp.d_stats;
   }
-  // the words cpi_get_state brings back, allocated once
-  if ((rc = ensure_tmp(c, kStateWords + 16 * (size_t)nn))) return rc;
+  // the words cpi_get_state brings back, allocated once, or what there is room
+  // for
+  const size_t whole = kStateWords + 16 * (size_t)nn;
+  rc = opt->debug_fill_nan & 4 ? CPI_ERR_ALLOC : ensure_tmp(c, whole);
+  if (rc) rc = ensure_tmp(c, opt->debug_fill_nan & 4 ? kStateWords + 100 : std::min(whole, kTmpLow));
+  if (rc) return rc;
   // reference positions on the device
   if ((rc = put_nodes(c, X0u, nullptr, c->P.X0))) return rc;
   return reset_state(c);
@@ -1268,54 +1298,54 @@ extern "C" int cpi_get_state(cpi_ctx *c, double *x, double *v, double *a, double
 extern "C" int cpi_get_state_mass3(cpi_ctx *c, double *x, double *v, double *a, double *m,
                                    double *vi, double *m3) {
   if (!c) return CPI_ERR_INVALID;
-  const size_t n3 = 3 * (size_t)c->nn;
-  int rc = ensure_tmp(c, kStateWords + 5 * n3 + c->nn);
-  if (rc) return rc;
   Ctl h;
-  Piece p[7] = {{&h, sizeof(Ctl) / 8}};
-  int k = 1;
-  double *d = c->d_tmp + kStateWords;
-  auto place = [&](double *host, size_t n) -> double * {
-    if (!host) return nullptr;
-    p[k++] = Piece{host, n};
-    d += n;
-    return d - n;
+  // the nodes i .. i + n, and the control block with each part
+  auto part = [&](size_t i, size_t n) -> int {
+    Piece p[7] = {{&h, sizeof(Ctl) / 8}};
+    int k = 1;
+    double *d = c->d_tmp + kStateWords;
+    auto place = [&](double *host, size_t words) -> double * {
+      if (!host) return nullptr;
+      p[k++] = Piece{host + words * i, words * n};
+      d += words * n;
+      return d - words * n;
+    };
+    NodeExport o{};
+    o.ctl = reinterpret_cast<Ctl *>(c->d_tmp);
+    o.x = place(x, 3);
+    o.v = place(v, 3);
+    o.a = place(a, 3);
+    o.m = place(m, 1);
+    o.vi = place(vi, 3);
+    o.m3 = place(m3, 3);
+    o.half_dt = 0.5 * c->dt;
+    HIPCHK(c, launch_export_nodes(c->P, c->d_ninv + i, (int)n, o, c->stream));
+    return bring_back(c, p, k);
   };
-  NodeExport o{};
-  o.ctl = reinterpret_cast<Ctl *>(c->d_tmp);
-  o.x = place(x, n3);
-  o.v = place(v, n3);
-  o.a = place(a, n3);
-  o.m = place(m, c->nn);
-  o.vi = place(vi, n3);
-  o.m3 = place(m3, n3);
-  o.half_dt = 0.5 * c->dt;
-  HIPCHK(c, launch_export_nodes(c->P, c->d_ninv, o, c->stream));
-  if ((rc = bring_back(c, p, k))) return rc;
+  const size_t words = 3 * (!!x + !!v + !!a + !!vi + !!m3) + !!m;
+  int rc = in_parts(c, c->nn, words, kStateWords, part);
+  if (rc) return rc;
   if (c->res_pending) {
     bool missing;
     if ((rc = settle(c, h, &missing))) return rc;
-    if (missing) {
-      HIPCHK(c, launch_export_nodes(c->P, c->d_ninv, o, c->stream));
-      if ((rc = bring_back(c, p, k))) return rc;
-    }
+    if (missing && (rc = in_parts(c, c->nn, words, kStateWords, part))) return rc;
   }
   return c->inited ? report_flags(c, h) : CPI_OK;
 }
 
 extern "C" int cpi_get_increment(cpi_ctx *c, double *du) {
   if (!c || !du) return CPI_ERR_INVALID;
-  const size_t n3 = 3 * (size_t)c->nn;
   int rc = settled(c);
-  if (!rc) rc = ensure_tmp(c, n3);
   if (rc) return rc;
   Params p = c->P;
   p.acc = c->P.du;
   NodeExport o{};
   o.a = c->d_tmp;
-  HIPCHK(c, launch_export_nodes(p, c->d_ninv, o, c->stream));
-  const Piece q{du, n3};
-  return bring_back(c, &q, 1);
+  return in_parts(c, c->nn, 3, 0, [&](size_t i, size_t n) -> int {
+    HIPCHK(c, launch_export_nodes(p, c->d_ninv + i, (int)n, o, c->stream));
+    const Piece q{du + 3 * i, 3 * n};
+    return bring_back(c, &q, 1);
+  });
 }
 
 extern "C" int cpi_get_element_state(cpi_ctx *c, double *sig, double *ep) {
@@ -1327,39 +1357,45 @@ extern "C" int cpi_get_element_state(cpi_ctx *c, double *sig, double *ep) {
     return CPI_OK;
   }
   int rc = settled(c);
-  if (!rc) rc = ensure_tmp(c, (sig ? 6 * n : 0) + (ep ? n : 0));
-  if (rc) return rc;
-  Piece p[2];
-  int k = 0;
-  if (sig) p[k++] = Piece{sig, 6 * n};
-  if (ep) p[k++] = Piece{ep, n};
-  if (k)
-    HIPCHK(c, launch_export_elems(c->P, c->prec, c->d_spos, sig ? c->d_tmp : nullptr,
-                                  ep ? c->d_tmp + (sig ? 6 * n : 0) : nullptr, c->stream));
-  return bring_back(c, p, k);
+  if (rc || (!sig && !ep)) return rc;
+  // an element's words
+  const size_t ws = sig ? 6 * (size_t)c->nq : 0, we = ep ? (size_t)c->nq : 0;
+  if (!(c->opt.debug_fill_nan & 4)) (void)ensure_tmp(c, std::min((ws + we) * c->ne, kTmpMost));
+  return in_parts(c, c->ne, ws + we, 0, [&](size_t i, size_t ne) -> int {
+    Piece p[2];
+    int k = 0;
+    if (sig) p[k++] = Piece{sig + ws * i, ws * ne};
+    if (ep) p[k++] = Piece{ep + we * i, we * ne};
+    HIPCHK(c, launch_export_elems(c->P, c->prec, c->d_spos + i, (int)ne, sig ? c->d_tmp : nullptr,
+                                  ep ? c->d_tmp + ws * ne : nullptr, c->stream));
+    return bring_back(c, p, k);
+  });
 }
 
 extern "C" int cpi_get_stress_strain(cpi_ctx *c, double *strain, double *stress) {
   if (!c) return CPI_ERR_INVALID;
   if (!c->inited) return fail(c, CPI_ERR_STATE, "cpi_get_stress_strain before cpi_init");
-  const size_t n6 = 6 * (size_t)c->nn;
   int rc = settled(c);
-  if (!rc) rc = ensure_tmp(c, 2 * n6);
   if (rc) return rc;
-  hipError_t e = launch_stress_node(c->P, c->d_last, strain ? c->d_tmp : nullptr,
-                                    stress ? c->d_tmp + (strain ? n6 : 0) : nullptr, c->stream);
-  if (e != hipSuccess) return fail(c, CPI_ERR_HIP, hipGetErrorString(e));
   // nodes of no element keep what the caller's arrays hold
   double *out[2] = {strain, stress};
   std::vector<double> keep;
-  for (double *o : out)
-    if (o)
-      for (int32_t n : c->loose) keep.insert(keep.end(), o + 6L * n, o + 6L * n + 6);
-  Piece p[2];
-  int k = 0;
-  if (strain) p[k++] = Piece{strain, n6};
-  if (stress) p[k++] = Piece{stress, n6};
-  if ((rc = bring_back(c, p, k))) return rc;
+  try {
+    for (double *o : out)
+      if (o)
+        for (int32_t n : c->loose) keep.insert(keep.end(), o + 6L * n, o + 6L * n + 6);
+  } catch (const std::bad_alloc &) {
+    return fail(c, CPI_ERR_ALLOC, "cpi_get_stress_strain: out of host memory");
+  }
+  rc = in_parts(c, c->nn, 6 * (!!strain + !!stress), 0, [&](size_t i, size_t n) -> int {
+    Piece p[2];
+    int k = 0;
+    if (strain) p[k++] = Piece{strain + 6 * i, 6 * n};
+    if (stress) p[k++] = Piece{stress + 6 * i, 6 * n};
+    HIPCHK(c, launch_stress_node(c->P, c->d_last + i, (int)n, strain ? c->d_tmp : nullptr,
+                                 stress ? c->d_tmp + (strain ? 6 * n : 0) : nullptr, c->stream));
+    return bring_back(c, p, k);
+  });
   const double *was = keep.data();
   for (double *o : out)
     if (o)
@@ -1367,7 +1403,7 @@ extern "C" int cpi_get_stress_strain(cpi_ctx *c, double *strain, double *stress)
         std::memcpy(o + 6L * n, was, 6 * sizeof(double));
         was += 6;
       }
-  return CPI_OK;
+  return rc;
 }
 
 extern "C" int cpi_get_energy(cpi_ctx *c, double *row, int64_t *step) {

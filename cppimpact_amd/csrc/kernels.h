@@ -48,29 +48,30 @@ hipError_t launch_mass(const Params &p, int rule, int scatter, int kind, double 
 hipError_t launch_elem_dt(const Params &p, double *out, hipStream_t s);
 // user-order host layouts (ninv: user node -> device id; spos: see
 // k_export_elems).
-// Import: [nn][3] into Vec3 and / or Node4 records (w = 0), null skipped.
-hipError_t launch_import_nodes(const double *src, const int32_t *ninv, int nn, Vec3 *d3, Node4 *d4,
+// Parts: n nodes (elements), ninv, spos and last from the first of them on.
+// Import: [n][3] into Vec3 and / or Node4 records (w = 0), null skipped.
+hipError_t launch_import_nodes(const double *src, const int32_t *ninv, int n, Vec3 *d3, Node4 *d4,
                                hipStream_t s);
 // Export: the arrays that are not null, vi = v - half_dt a
 struct NodeExport {
-  double *x, *v, *a, *vi;  // [nn][3]
-  double *m;               // [nn]
-  double *m3;              // [nn][3], the mass in each component
+  double *x, *v, *a, *vi;  // [n][3]
+  double *m;               // [n]
+  double *m3;              // [n][3], the mass in each component
   Ctl *ctl;                // a copy of the control block
   double half_dt;
 };
-hipError_t launch_export_nodes(const Params &p, const int32_t *ninv, const NodeExport &o,
+hipError_t launch_export_nodes(const Params &p, const int32_t *ninv, int n, const NodeExport &o,
                                hipStream_t s);
-// sig [ne][nq][6], ep [ne][nq] as doubles (null skipped)
-hipError_t launch_export_elems(const Params &p, int prec, const uint32_t *spos, double *sig,
+// sig [n][nq][6], ep [n][nq] as doubles (null skipped)
+hipError_t launch_export_elems(const Params &p, int prec, const uint32_t *spos, int n, double *sig,
                                double *ep, hipStream_t s);
 // positions X0, velocities v0 (device order), forces, a and du zeroed
 hipError_t launch_reset_nodes(const Params &p, const Vec3 *v0, hipStream_t s);
 // smallest positive mass, one minimum per workgroup into out[blocks]
 hipError_t launch_mass_min(const Params &p, double *out, int blocks, hipStream_t s);
-// strain and stress [nn][6] in user node order; last: per user node, the
+// strain and stress [n][6] in user node order; last: per user node, the
 // device id of the highest-numbered element holding it (-1: none, not written)
-hipError_t launch_stress_node(const Params &p, const int32_t *last, double *strain,
+hipError_t launch_stress_node(const Params &p, const int32_t *last, int n, double *strain,
                               double *stress, hipStream_t s);
 hipError_t launch_debug_strain(const Params &p, int rule, double alpha, int dcase, double nu,
                                double *out, hipStream_t s);

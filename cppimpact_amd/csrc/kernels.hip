@@ -1689,10 +1689,10 @@ __global__ void __launch_bounds__(256) k_elem_dt(Params p, double *out) {
 // of 196,608 tet4 (100 FP32 steps, nodal state, strain and stress) took 11.8
 // ms, now 1.9 ms.  Bound by the copy to the caller's pages.
 template <int NPE>
-__global__ void __launch_bounds__(256) k_stress_node(Params p, const int32_t *last,
+__global__ void __launch_bounds__(256) k_stress_node(Params p, const int32_t *last, int count,
                                                      double *strain, double *stress) {
   const int node = blockIdx.x * 256 + threadIdx.x;
-  if (node >= p.nn) return;
+  if (node >= count) return;
   const int e = last[node];
   if (e < 0) return;
   double xs[NPE][3], u[NPE][3];
@@ -1842,11 +1842,11 @@ __global__ void __launch_bounds__(256) k_debug_strain(Params p, double alpha, in
 // the host cost several passes over fresh host pages per array.
 // ---------------------------------------------------------------------------
 __global__ void __launch_bounds__(256) k_import_nodes(const double *src, const int32_t *ninv,
-                                                      int nn, Vec3 *d3, Node4 *d4) {
+                                                      int n, Vec3 *d3, Node4 *d4) {
   const long i = (long)blockIdx.x * 256 + threadIdx.x;
-  if (i >= 3L * nn) return;
-  const int n = (int)(i / 3), c = (int)(i - 3L * n);
-  const long g = ninv[n];
+  if (i >= 3L * n) return;
+  const int k = (int)(i / 3), c = (int)(i - 3L * k);
+  const long g = ninv[k];
   const double v = src[i];
   if (d3) reinterpret_cast<double *>(d3)[3 * g + c] = v;
   if (d4) {
@@ -1856,15 +1856,16 @@ __global__ void __launch_bounds__(256) k_import_nodes(const double *src, const i
 }
 
 // ctl: a copy of the control block, so one transfer brings it along
-__global__ void __launch_bounds__(256) k_export_nodes(Params p, const int32_t *ninv, NodeExport o) {
+__global__ void __launch_bounds__(256) k_export_nodes(Params p, const int32_t *ninv, int n,
+                                                      NodeExport o) {
   const long i = (long)blockIdx.x * 256 + threadIdx.x;
   constexpr int words = sizeof(Ctl) / 8;
   if (blockIdx.x == 0 && threadIdx.x < words && o.ctl)
     reinterpret_cast<uint64_t *>(o.ctl)[threadIdx.x] =
         reinterpret_cast<const uint64_t *>(p.ctl)[threadIdx.x];
-  if (i >= 3L * p.nn) return;
-  const int n = (int)(i / 3), c = (int)(i - 3L * n);
-  const long g = ninv[n];
+  if (i >= 3L * n) return;
+  const int k = (int)(i / 3), c = (int)(i - 3L * k);
+  const long g = ninv[k];
   if (o.x) o.x[i] = reinterpret_cast<const double *>(p.pos)[3 * g + c];
   double v = 0.0, a = 0.0;
   if (o.v || o.vi) v = reinterpret_cast<const double *>(p.vv)[3 * g + c];
@@ -1876,7 +1877,7 @@ __global__ void __launch_bounds__(256) k_export_nodes(Params p, const int32_t *n
     const double h = o.half_dt * a;
     o.vi[i] = v - h;
   }
-  if (o.m && c == 0) o.m[n] = p.m[g];
+  if (o.m && c == 0) o.m[k] = p.m[g];
   if (o.m3) o.m3[i] = p.m[g];
 }
 
@@ -1892,11 +1893,11 @@ __device__ __forceinline__ long state_place(const Params &p, uint32_t spos, int 
 }
 
 template <typename R>
-__global__ void __launch_bounds__(256) k_export_elems(Params p, const uint32_t *spos, double *sig,
-                                                      double *ep) {
+__global__ void __launch_bounds__(256) k_export_elems(Params p, const uint32_t *spos, int n,
+                                                      double *sig, double *ep) {
   const long i = (long)blockIdx.x * 256 + threadIdx.x, ne = p.ne, ld = p.state_ld;
   const int w = 6 * p.nq;
-  if (sig && i < ne * w) {
+  if (sig && i < (long)n * w) {
     const long e = i / w;
     const int q = (int)(i - e * w) / 6, c = (int)(i - e * w) - 6 * q;
     const long at = state_place(p, spos[e], q);
@@ -1904,7 +1905,7 @@ __global__ void __launch_bounds__(256) k_export_elems(Params p, const uint32_t *
     sig[i] = double(ld ? sr[(at / ld) * 6 * ld + c * ld + at % ld]
                        : sr[(6L * q + c) * ne + spos[e]]);
   }
-  if (ep && i < ne * p.nq) {
+  if (ep && i < (long)n * p.nq) {
     const long e = i / p.nq;
     const int q = (int)(i - e * p.nq);
     ep[i] = double(static_cast<const R *>(p.epbar)[state_place(p, spos[e], q)]);
@@ -2444,21 +2445,21 @@ hipError_t launch_elem_dt(const Params &p, double *out, hipStream_t s) {
   CPI_LAUNCH(k_elem_dt<10>, grid, 256, 0, s, p, out);
 }
 
-hipError_t launch_import_nodes(const double *src, const int32_t *ninv, int nn, Vec3 *d3, Node4 *d4,
+hipError_t launch_import_nodes(const double *src, const int32_t *ninv, int n, Vec3 *d3, Node4 *d4,
                                hipStream_t s) {
-  CPI_LAUNCH(k_import_nodes, (unsigned)((3L * nn + 255) / 256), 256, 0, s, src, ninv, nn, d3, d4);
+  CPI_LAUNCH(k_import_nodes, (unsigned)((3L * n + 255) / 256), 256, 0, s, src, ninv, n, d3, d4);
 }
 
-hipError_t launch_export_nodes(const Params &p, const int32_t *ninv, const NodeExport &o,
+hipError_t launch_export_nodes(const Params &p, const int32_t *ninv, int n, const NodeExport &o,
                                hipStream_t s) {
-  CPI_LAUNCH(k_export_nodes, (unsigned)((3L * p.nn + 255) / 256), 256, 0, s, p, ninv, o);
+  CPI_LAUNCH(k_export_nodes, (unsigned)((3L * n + 255) / 256), 256, 0, s, p, ninv, n, o);
 }
 
-hipError_t launch_export_elems(const Params &p, int prec, const uint32_t *spos, double *sig,
+hipError_t launch_export_elems(const Params &p, int prec, const uint32_t *spos, int n, double *sig,
                                double *ep, hipStream_t s) {
-  const unsigned grid = (unsigned)(((long)p.ne * p.nq * (sig ? 6 : 1) + 255) / 256);
-  if (prec == 1) CPI_LAUNCH(k_export_elems<float>, grid, 256, 0, s, p, spos, sig, ep);
-  CPI_LAUNCH(k_export_elems<double>, grid, 256, 0, s, p, spos, sig, ep);
+  const unsigned grid = (unsigned)(((long)n * p.nq * (sig ? 6 : 1) + 255) / 256);
+  if (prec == 1) CPI_LAUNCH(k_export_elems<float>, grid, 256, 0, s, p, spos, n, sig, ep);
+  CPI_LAUNCH(k_export_elems<double>, grid, 256, 0, s, p, spos, n, sig, ep);
 }
 
 hipError_t launch_reset_nodes(const Params &p, const Vec3 *v0, hipStream_t s) {
@@ -2469,11 +2470,11 @@ hipError_t launch_mass_min(const Params &p, double *out, int blocks, hipStream_t
   CPI_LAUNCH(k_mass_min, blocks, 256, 0, s, (const double *)p.m, p.nn, out);
 }
 
-hipError_t launch_stress_node(const Params &p, const int32_t *last, double *strain,
+hipError_t launch_stress_node(const Params &p, const int32_t *last, int n, double *strain,
                               double *stress, hipStream_t s) {
-  const int grid = (p.nn + 255) / 256;
-  if (p.npe == 4) CPI_LAUNCH(k_stress_node<4>, grid, 256, 0, s, p, last, strain, stress);
-  CPI_LAUNCH(k_stress_node<10>, grid, 256, 0, s, p, last, strain, stress);
+  const int grid = (n + 255) / 256;
+  if (p.npe == 4) CPI_LAUNCH(k_stress_node<4>, grid, 256, 0, s, p, last, n, strain, stress);
+  CPI_LAUNCH(k_stress_node<10>, grid, 256, 0, s, p, last, n, strain, stress);
 }
 
 hipError_t launch_debug_strain(const Params &p, int rule, double alpha, int dcase, double nu,

@@ -152,7 +152,10 @@ typedef struct cpi_options {
                                non-finite state (diagnostics; default 0).
                                  3: also every wait of a resident step gives
                                  up at once, so the steps are taken one by
-                                 one */
+                                 one.
+                                 4 added to these: the context behaves as if
+                                 the device had no room for what it allocates
+                                 only to be faster */
   int32_t stream_state;     /* the block kernels' stress-state accesses
                                (tet4 and the 4-point tet10 kernel):
                                0 = non-temporal when a step's working set
