@@ -155,6 +155,14 @@ int upload(cpi_ctx *c, T *d, const std::vector<T> &h) {
   return CPI_OK;
 }
 
+// the assembled forces that element kernels add to (the other scatters sum
+// records of their own: 24 bytes a node saved, and their clearing at init)
+int alloc_forces(cpi_ctx *c) {
+  int rc = CPI_OK;
+  for (int k = 0; k < 3 && !rc; k++) rc = dalloc(c, &c->P.f[k], c->nn);
+  return rc;
+}
+
 int default_rule(int npe, int phys, int q) {
   if (q >= 0) return q;
   if (phys == CPI_PHYSICS_COMPAT) return CPI_QUAD_REF5;
@@ -757,9 +765,7 @@ static int create_impl(cpi_ctx *c, const cpi_mesh_desc *m, const cpi_material *m
   P.wsum = rule_weight_sum(c->rule);
   int rc = CPI_OK;
   const int nn = c->nn, ne = c->ne;
-  for (int kk = 0; kk < 3 && !rc; kk++) {
-    rc = dalloc(c, &P.f[kk], nn);
-  }
+  if (c->scatter == CPI_SCATTER_ATOMIC) rc = alloc_forces(c);
   if (!rc) rc = dalloc(c, &P.pos, nn);
   if (!rc) rc = dalloc(c, &P.vv, nn);
   if (!rc) rc = dalloc(c, &P.acc, nn);

@@ -79,7 +79,7 @@ struct Params {
   Vec3 *pos;             // x
   Vec3 *vv;              // v_{n+1/2}
   double *m;             // lumped mass (read by the node's owner only)
-  double *f[3];          // assembled force (atomic scatter)
+  double *f[3];          // assembled force (atomic scatter; null: another)
   // colour scatter: one corner force (Vec3, Vec3f in FP32) per node and
   // element in cforce, a node's slots node_slot[n] .. node_slot[n+1] in
   // ascending colour; corner k of element e at fslot[k * ne + e].

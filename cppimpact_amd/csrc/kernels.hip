@@ -1912,7 +1912,7 @@ __global__ void __launch_bounds__(256) k_export_elems(Params p, const uint32_t *
   }
 }
 
-// x = X0, v = v0, forces, du and a zeroed
+// x = X0, v = v0, du, a and the assembled forces (atomic scatter) zeroed
 __global__ void __launch_bounds__(256) k_reset_nodes(Params p, const Vec3 *v0) {
   const int g = blockIdx.x * 256 + threadIdx.x;
   if (g >= p.nn) return;
@@ -1922,6 +1922,7 @@ __global__ void __launch_bounds__(256) k_reset_nodes(Params p, const Vec3 *v0) {
   p.xprev[g] = Node4{x.x, x.y, x.z, 0.0};
   p.acc[g] = Node4{0.0, 0.0, 0.0, 0.0};
   p.du[g] = Node4{0.0, 0.0, 0.0, 0.0};
+  if (p.f[0] == nullptr) return;
 #pragma unroll
   for (int c = 0; c < 3; c++) p.f[c][g] = 0.0;
 }
