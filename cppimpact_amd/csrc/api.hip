@@ -41,6 +41,8 @@ struct cpi_ctx {
   std::vector<int32_t> conn_u, color, slave_u;
   int ncol = 0;
   std::vector<int32_t> eperm, nperm, ninv;  // device->user elem, device->user node, user->device
+  std::vector<int32_t> color_off;           // the colours' elements in d_by_color
+  int32_t *d_by_color = nullptr;            // (null: the colour scatter has its slots)
   std::vector<int32_t> loose;               // user nodes of no element
   int32_t *d_last = nullptr;                // per user node: last element holding it (device id)
   int32_t *d_ninv = nullptr;                // user node -> device id
@@ -143,6 +145,19 @@ int dalloc(cpi_ctx *c, T **p, size_t n) {
   if (c->opt.debug_fill_nan && c->stream)
     HIPCHK(c, hipMemsetAsync(q, 0xFF, std::max<size_t>(n, 1) * sizeof(T), c->stream));
   return CPI_OK;
+}
+
+void dfree(cpi_ctx *c, void *p) {
+  const auto i = std::find(c->allocs.begin(), c->allocs.end(), p);
+  if (p == nullptr || i == c->allocs.end()) return;
+  c->allocs.erase(i);
+  (void)hipFree(p);
+}
+
+// energy rows of a k_elem_direct launch on n elements, one per wave
+int elem_direct_rows(int npe, int n) {
+  const int nt = elem_direct_threads(npe);
+  return nt / 64 * ((n + nt - 1) / nt);
 }
 
 template <typename T>
@@ -335,6 +350,22 @@ bool all_finite(const double *v, size_t n) {
   return s[0] + s[1] + s[2] + s[3] == 0.0;
 }
 
+// The element pass of the colour and atomic scatters: one launch, or, when the
+// colour scatter's slots found no room, one per colour.
+hipError_t elem_direct(cpi_ctx *c, Params p, int64_t *launches) {
+  const int32_t *list = c->d_by_color;
+  hipError_t e = hipSuccess;
+  p.epart_base = 0;
+  for (int k = 0; e == hipSuccess && k < (list ? c->ncol : 1); k++) {
+    const int first = list ? c->color_off[k] : 0, n = (list ? c->color_off[k + 1] : c->ne) - first;
+    e = launch_elem_direct(p, c->rule, c->prec, c->phys, list || c->scatter == CPI_SCATTER_ATOMIC,
+                           list ? list + first : nullptr, n, c->stream);
+    p.epart_base += elem_direct_rows(c->npe, n);
+    if (launches) ++*launches;
+  }
+  return e;
+}
+
 int enqueue_step(cpi_ctx *c, bool aux) {
   Params p = c->P;
   p.store_aux = aux ? 1 : 0;
@@ -347,8 +378,7 @@ int enqueue_step(cpi_ctx *c, bool aux) {
       e = launch_node_bnd(p, c->prec, aux, c->stream);
     }
   } else {
-    p.epart_base = 0;
-    e = launch_elem_direct(p, c->rule, c->prec, c->phys, c->scatter == CPI_SCATTER_ATOMIC, c->stream);
+    e = elem_direct(c, p, nullptr);
     if (e == hipSuccess) {
       p.epart_base = c->n_elem_rows;
       e = launch_node_all(p, c->prec, aux, c->stream);
@@ -439,8 +469,7 @@ int ensure_tmp(cpi_ctx *c, size_t n) {
   if (rc) return rc;
   if (c->d_tmp) {
     HIPCHK(c, hipStreamSynchronize(c->stream));
-    c->allocs.erase(std::find(c->allocs.begin(), c->allocs.end(), (void *)c->d_tmp));
-    (void)hipFree(c->d_tmp);
+    dfree(c, c->d_tmp);
   }
   c->d_tmp = p;
   c->tmp_len = n;
@@ -452,8 +481,13 @@ int compute_mass(cpi_ctx *c) {
   HIPCHK(c, hipMemsetAsync((void *)p.m, 0, sizeof(double) * c->nn, c->stream));
   const double rho = c->mat.rho;
   hipError_t e = hipSuccess;
-  // CPI_SCATTER_* in launch_mass's numbering
-  e = launch_mass(p, c->rule, c->scatter, c->mass_kind, rho, c->nblocks, c->stream);
+  // CPI_SCATTER_* in launch_mass's numbering; colour by colour as elem_direct
+  const int32_t *list = c->d_by_color;
+  for (int k = 0; e == hipSuccess && k < (list ? c->ncol : 1); k++) {
+    const int first = list ? c->color_off[k] : 0, n = (list ? c->color_off[k + 1] : c->ne) - first;
+    e = launch_mass(p, c->rule, list ? CPI_SCATTER_ATOMIC : c->scatter, c->mass_kind, rho, c->nblocks,
+                    list ? list + first : nullptr, n, c->stream);
+  }
   if (e != hipSuccess) return fail(c, CPI_ERR_HIP, std::string("mass kernel: ") + hipGetErrorString(e));
   HIPCHK(c, hipStreamSynchronize(c->stream));
   c->mass_ready = true;
@@ -991,28 +1025,44 @@ static int create_impl(cpi_ctx *c, const cpi_mesh_desc *m, const cpi_material *m
     c->n_elem_rows = c->nblocks * (elem_block_threads(npe, c->rule, c->prec, c->phys, c->nblocks) / 64);
     c->n_node_rows = 4 * std::max(1, (B.n_boundary + 255) / 256);
   } else {
-    const int nt = elem_direct_threads(npe);
-    const int rows = (nt / 64) * ((ne + nt - 1) / nt);
+    c->n_elem_rows = elem_direct_rows(npe, ne);
     if (c->scatter == CPI_SCATTER_COLOR) {
-      if ((size_t)npe * ne > UINT32_MAX)
-        return fail(c, CPI_ERR_INVALID, "the colour scatter holds at most 2^32 element corners");
-      std::vector<uint32_t> slot, ptr;
-      std::vector<int32_t> order;
-      color_slots(ne, npe, c->conn_u.data(), nn, c->color.data(), c->ncol, slot, ptr, order);
-      uint32_t *ds, *dp;
+      std::vector<int32_t> order, by_color;
+      color_order(ne, c->color.data(), c->ncol, order, by_color, c->color_off);
       int32_t *dor;
-      char *cf;  // the records; before the first step, FP64 corner masses
-      if ((rc = dalloc(c, &ds, slot.size())) || (rc = upload(c, ds, slot)) ||
-          (rc = dalloc(c, &dp, ptr.size())) || (rc = upload(c, dp, ptr)) ||
-          (rc = dalloc(c, &dor, order.size())) || (rc = upload(c, dor, order)) ||
-          (rc = dalloc(c, &cf, slot.size() * (c->prec == CPI_PREC_F32 ? sizeof(Vec3f) : sizeof(Vec3)))))
-        return rc;
-      P.fslot = ds;
-      P.node_slot = dp;
+      if ((rc = dalloc(c, &dor, order.size())) || (rc = upload(c, dor, order))) return rc;
       P.sample_id = dor;
-      P.cforce = cf;
+      // a record per corner, of 2^32 at most; before the first step, FP64 corner
+      // masses
+      const size_t corners = (size_t)npe * ne;
+      uint32_t *ds = nullptr, *dp = nullptr;
+      char *cf = nullptr;
+      if (corners > UINT32_MAX || (opt->debug_fill_nan & 4))
+        rc = CPI_ERR_ALLOC;
+      else if (!(rc = dalloc(c, &ds, corners)) && !(rc = dalloc(c, &dp, (size_t)nn + 1)))
+        rc = dalloc(c, &cf, corners * (c->prec == CPI_PREC_F32 ? sizeof(Vec3f) : sizeof(Vec3)));
+      if (rc == CPI_OK) {
+        std::vector<uint32_t> slot, ptr;
+        color_slots(ne, npe, c->conn_u.data(), nn, c->color.data(), c->ncol, slot, ptr, order);
+        if ((rc = upload(c, ds, slot)) || (rc = upload(c, dp, ptr))) return rc;
+        P.fslot = ds;
+        P.node_slot = dp;
+        P.cforce = cf;
+      } else if (rc == CPI_ERR_ALLOC) {
+        // no room: the forces are added up colour by colour, a launch each
+        (void)hipGetLastError();
+        dfree(c, ds);
+        dfree(c, dp);
+        if ((rc = alloc_forces(c)) || (rc = dalloc(c, &c->d_by_color, by_color.size())) ||
+            (rc = upload(c, c->d_by_color, by_color)))
+          return rc;
+        c->n_elem_rows = 0;
+        for (int k = 0; k < c->ncol; k++)
+          c->n_elem_rows += elem_direct_rows(npe, c->color_off[k + 1] - c->color_off[k]);
+      } else {
+        return rc;
+      }
     }
-    c->n_elem_rows = rows;
     c->n_node_rows = 4 * ((nn + 255) / 256);
   }
   c->n_rows = std::max(c->n_elem_rows + c->n_node_rows, 4 * ((nn + 255) / 256));
@@ -1584,9 +1634,7 @@ extern "C" int cpi_profile_kernels(cpi_ctx *c, int32_t nsteps, cpi_kernel_time *
       launches[0] += 1;
     } else {
       HIPCHK(c, hipEventRecord(ev[0], c->stream));
-      e = launch_elem_direct(p, c->rule, c->prec, c->phys, c->scatter == CPI_SCATTER_ATOMIC,
-                             c->stream);
-      launches[0] += 1;
+      e = elem_direct(c, p, &launches[0]);
       HIPCHK(c, hipEventRecord(ev[1], c->stream));
     }
     p.epart_base = c->n_elem_rows;

@@ -61,18 +61,25 @@ int greedy_coloring(int ne, int npe, const int32_t *conn, int nn,
   return ncol;
 }
 
+void color_order(int ne, const int32_t *color, int ncol, std::vector<int32_t> &order,
+                 std::vector<int32_t> &by_color, std::vector<int32_t> &off) {
+  off.assign(ncol + 1, 0);
+  for (int e = 0; e < ne; e++) off[color[e] + 1]++;
+  for (int c = 0; c < ncol; c++) off[c + 1] += off[c];
+  std::vector<int32_t> next(off.begin(), off.end() - 1);
+  order.assign(ne, 0);
+  by_color.assign(ne, 0);
+  for (int e = 0; e < ne; e++) {
+    order[e] = next[color[e]]++;
+    by_color[order[e]] = e;
+  }
+}
+
 void color_slots(int ne, int npe, const int32_t *conn, int nn, const int32_t *color, int ncol,
                  std::vector<uint32_t> &slot, std::vector<uint32_t> &node_slot,
                  std::vector<int32_t> &order) {
-  std::vector<int32_t> off(ncol + 1, 0);
-  for (int e = 0; e < ne; e++) off[color[e] + 1]++;
-  for (int c = 0; c < ncol; c++) off[c + 1] += off[c];
-  std::vector<int32_t> by_color(ne);
-  order.assign(ne, 0);
-  for (int e = 0; e < ne; e++) {
-    order[e] = off[color[e]]++;
-    by_color[order[e]] = e;
-  }
+  std::vector<int32_t> by_color, off;
+  color_order(ne, color, ncol, order, by_color, off);
   node_slot.assign((size_t)nn + 1, 0);
   for (size_t i = 0; i < (size_t)ne * npe; i++) node_slot[conn[i] + 1]++;
   for (int n = 0; n < nn; n++) node_slot[n + 1] += node_slot[n];

@@ -86,10 +86,14 @@ struct MailCount {
 };
 MailCount count_mail(const BlockPlan &plan);
 
+// The elements sorted by colour (stable): order[e] is element e's place among
+// them, by_color the elements in that order, colour c's at off[c] .. off[c+1].
+void color_order(int ne, const int32_t *color, int ncol, std::vector<int32_t> &order,
+                 std::vector<int32_t> &by_color, std::vector<int32_t> &off);
+
 // Corner-force slots of the colour scatter: node n's slots are node_slot[n]
 // .. node_slot[n+1], one per element that holds it, in ascending colour, and
-// corner k of element e writes slot[k * ne + e].  order[e]: the element's
-// place in the elements sorted by colour (stable).
+// corner k of element e writes slot[k * ne + e].  order as color_order.
 void color_slots(int ne, int npe, const int32_t *conn, int nn, const int32_t *color, int ncol,
                  std::vector<uint32_t> &slot, std::vector<uint32_t> &node_slot,
                  std::vector<int32_t> &order);

@@ -22,8 +22,10 @@ hipError_t prepare_elem_block(int npe, int rule, int prec, int phys, size_t smem
 // kernel's own start and end (hipExtLaunchKernel); (null, null) restores
 // plain launches.  For per-kernel timing outside graph capture.
 void set_launch_events(hipEvent_t start, hipEvent_t stop);
+// atomic: on n elements, those of list (device ids) if it is given; else n all
+// of them
 hipError_t launch_elem_direct(const Params &p, int rule, int prec, int phys, bool atomic,
-                              hipStream_t s);
+                              const int32_t *list, int n, hipStream_t s);
 // workgroups of the resident kernel the device can hold at once (0: there is
 // none for this combination)
 int resident_capacity(int npe, int rule, int prec, int phys, size_t smem, int cus);
@@ -42,9 +44,10 @@ hipError_t launch_node_all(const Params &p, int prec, bool aux, hipStream_t s);
 hipError_t launch_node_init(const Params &p, hipStream_t s);
 hipError_t launch_energy_reduce(const Params &p, hipStream_t s);
 int energy_reduce_blocks();  // rows of p.ered (EP_N doubles each)
-// lumped mass into p.m (scatter: 0 block, 1 colour, 2 atomic)
+// lumped mass into p.m (scatter: 0 block, 1 colour, 2 atomic; list, n as
+// launch_elem_direct)
 hipError_t launch_mass(const Params &p, int rule, int scatter, int kind, double rho,
-                       int nblocks, hipStream_t s);
+                       int nblocks, const int32_t *list, int n, hipStream_t s);
 hipError_t launch_elem_dt(const Params &p, double *out, hipStream_t s);
 // user-order host layouts (ninv: user node -> device id; spos: see
 // k_export_elems).

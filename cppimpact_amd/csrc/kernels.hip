@@ -1365,14 +1365,18 @@ __global__ void __launch_bounds__(256) k_resident_loose(Params p, Resident rs) {
 // Per step: 6,000 tet4 148 -> 10.0 us, 48,000 tet10 684 -> 35 us, 1.57M
 // tet4 484 -> 204 us (there bound by the scattered 24-byte records).
 // ---------------------------------------------------------------------------
+// Atomic: on n elements, those of list if it is given.  One launch per colour
+// is the colour scatter of a mesh whose slots found no room: each node takes at
+// most one sum per launch, so the order and the bits are the same.
 template <int NPE, int RULE, typename R, int PHYS, bool ATOMIC, int NT>
-__global__ void __launch_bounds__(NT) k_elem_direct(Params p) {
+__global__ void __launch_bounds__(NT) k_elem_direct(Params p, const int32_t *list, int n) {
   using FR = typename std::conditional<std::is_same<R, float>::value, Vec3f, Vec3>::type;
-  const int e = blockIdx.x * NT + threadIdx.x;
+  const int t = blockIdx.x * NT + threadIdx.x;
   const RowPre row = row_prefetch(p, p.epart_base + blockIdx.x * (NT / 64));
   const double dt = p.ctl->dt;
   EAcc ea;
-  if (e < p.ne) {
+  if (t < n) {
+    const int e = ATOMIC && list ? list[t] : t;
     int nd[NPE];
 #pragma unroll
     for (int k = 0; k < NPE; k++) nd[k] = p.conn[(long)k * p.ne + e];
@@ -1607,10 +1611,13 @@ __global__ void __launch_bounds__(256) k_mass_bnd(Params p) {
 
 // colour scatter: corner masses into the x of the corner-force slots (FP64
 // words, whatever the slots' record), summed in colour order by k_mass_slots
+// (atomic: on n elements, those of list if it is given, as k_elem_direct)
 template <int NPE, int RULE, bool ATOMIC>
-__global__ void __launch_bounds__(256) k_mass_direct(Params p, int kind, double rho) {
-  const int e = blockIdx.x * 256 + threadIdx.x;
-  if (e >= p.ne) return;
+__global__ void __launch_bounds__(256) k_mass_direct(Params p, int kind, double rho,
+                                                      const int32_t *list, int n) {
+  const int t = blockIdx.x * 256 + threadIdx.x;
+  if (t >= n) return;
+  const int e = ATOMIC && list ? list[t] : t;
   int nd[NPE];
   double xs[NPE][3], me[NPE];
 #pragma unroll
@@ -2178,11 +2185,12 @@ static hipError_t elem_block_t(const Params &p, bool aux, int nblocks, size_t sm
 }
 
 template <int NPE, int RULE, typename R, int PHYS>
-static hipError_t elem_direct_t(const Params &p, bool atomic, hipStream_t s) {
+static hipError_t elem_direct_t(const Params &p, bool atomic, const int32_t *list, int n,
+                                hipStream_t s) {
   constexpr int NT = NPE == 4 ? 256 : 128;
-  const int grid = (p.ne + NT - 1) / NT;
-  if (atomic) CPI_LAUNCH((k_elem_direct<NPE, RULE, R, PHYS, true, NT>), grid, NT, 0, s, p);
-  CPI_LAUNCH((k_elem_direct<NPE, RULE, R, PHYS, false, NT>), grid, NT, 0, s, p);
+  const int grid = (n + NT - 1) / NT;
+  if (atomic) CPI_LAUNCH((k_elem_direct<NPE, RULE, R, PHYS, true, NT>), grid, NT, 0, s, p, list, n);
+  CPI_LAUNCH((k_elem_direct<NPE, RULE, R, PHYS, false, NT>), grid, NT, 0, s, p, list, n);
 }
 
 int elem_direct_threads(int npe) { return npe == 4 ? 256 : 128; }
@@ -2264,11 +2272,11 @@ template <int NPE, int RULE, typename R, int PHYS> struct ElemBlockPrepF {
   }
 };
 template <int NPE, int RULE, typename R, int PHYS> struct ElemDirectF {
-  static hipError_t run(const Params &p, bool atomic, hipStream_t s) {
+  static hipError_t run(const Params &p, bool atomic, const int32_t *list, int n, hipStream_t s) {
     if constexpr (PHYS == PHYS_EP_MLP)
       return hipErrorInvalidValue;
     else
-      return elem_direct_t<NPE, RULE, R, PHYS>(p, atomic, s);
+      return elem_direct_t<NPE, RULE, R, PHYS>(p, atomic, list, n, s);
   }
 };
 
@@ -2282,8 +2290,8 @@ hipError_t prepare_elem_block(int npe, int rule, int prec, int phys, size_t smem
 }
 
 hipError_t launch_elem_direct(const Params &p, int rule, int prec, int phys, bool atomic,
-                              hipStream_t s) {
-  return dispatch<ElemDirectF>(p.npe, rule, prec, phys, p, atomic, s);
+                              const int32_t *list, int n, hipStream_t s) {
+  return dispatch<ElemDirectF>(p.npe, rule, prec, phys, p, atomic, list, n, s);
 }
 
 // minimum waves per SIMD of the resident kernels
@@ -2404,7 +2412,7 @@ int energy_reduce_blocks() { return kEredBlocks; }
 
 template <int NPE, int RULE>
 static hipError_t mass_rule_t(const Params &p, int scatter, int kind, double rho, int nblocks,
-                              hipStream_t s) {
+                              const int32_t *list, int n, hipStream_t s) {
   if (scatter == 0) {
     constexpr int NT = NPE == 4 ? 512 : 128;
     const size_t smem = 8 * (3 * (size_t)p.ml + (size_t)p.max_el * NPE) + lds_off_bytes(p.kmax);
@@ -2415,28 +2423,30 @@ static hipError_t mass_rule_t(const Params &p, int scatter, int kind, double rho
     if (e != hipSuccess || p.n_boundary == 0) return e;
     CPI_LAUNCH(k_mass_bnd, (p.n_boundary + 255) / 256, 256, 0, s, p);
   }
-  const int grid = (p.ne + 255) / 256;
-  if (scatter == 2) CPI_LAUNCH((k_mass_direct<NPE, RULE, true>), grid, 256, 0, s, p, kind, rho);
-  hipLaunchKernelGGL((k_mass_direct<NPE, RULE, false>), dim3(grid), dim3(256), 0, s, p, kind, rho);
+  const int grid = (n + 255) / 256;
+  if (scatter == 2)
+    CPI_LAUNCH((k_mass_direct<NPE, RULE, true>), grid, 256, 0, s, p, kind, rho, list, n);
+  hipLaunchKernelGGL((k_mass_direct<NPE, RULE, false>), dim3(grid), dim3(256), 0, s, p, kind, rho,
+                     list, n);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   CPI_LAUNCH(k_mass_slots, (p.nn + 255) / 256, 256, 0, s, p);
 }
 
 hipError_t launch_mass(const Params &p, int rule, int scatter, int kind, double rho, int nblocks,
-                       hipStream_t s) {
+                       const int32_t *list, int n, hipStream_t s) {
   if (p.npe == 4) {
     switch (rule) {
-      case RULE_REF4: return mass_rule_t<4, RULE_REF4>(p, scatter, kind, rho, nblocks, s);
-      case RULE_EXACT4: return mass_rule_t<4, RULE_EXACT4>(p, scatter, kind, rho, nblocks, s);
-      case RULE_CENTROID: return mass_rule_t<4, RULE_CENTROID>(p, scatter, kind, rho, nblocks, s);
-      default: return mass_rule_t<4, RULE_REF5>(p, scatter, kind, rho, nblocks, s);
+      case RULE_REF4: return mass_rule_t<4, RULE_REF4>(p, scatter, kind, rho, nblocks, list, n, s);
+      case RULE_EXACT4: return mass_rule_t<4, RULE_EXACT4>(p, scatter, kind, rho, nblocks, list, n, s);
+      case RULE_CENTROID: return mass_rule_t<4, RULE_CENTROID>(p, scatter, kind, rho, nblocks, list, n, s);
+      default: return mass_rule_t<4, RULE_REF5>(p, scatter, kind, rho, nblocks, list, n, s);
     }
   }
   switch (rule) {
-    case RULE_REF4: return mass_rule_t<10, RULE_REF4>(p, scatter, kind, rho, nblocks, s);
-    case RULE_EXACT4: return mass_rule_t<10, RULE_EXACT4>(p, scatter, kind, rho, nblocks, s);
-    default: return mass_rule_t<10, RULE_REF5>(p, scatter, kind, rho, nblocks, s);
+    case RULE_REF4: return mass_rule_t<10, RULE_REF4>(p, scatter, kind, rho, nblocks, list, n, s);
+    case RULE_EXACT4: return mass_rule_t<10, RULE_EXACT4>(p, scatter, kind, rho, nblocks, list, n, s);
+    default: return mass_rule_t<10, RULE_REF5>(p, scatter, kind, rho, nblocks, list, n, s);
   }
 }
 
