@@ -71,6 +71,7 @@ struct cpi_ctx {
   Resident res{};
   size_t res_smem = 0;
   bool res_able = false, resident = false;
+  int res_min = 0;  // fewest plain steps of a call (kMinResident)
   hipEvent_t res_done[2] = {nullptr, nullptr};  // of every kAhead-th launch of a call, in turn
   // launches whose outcome the host has not seen, and the step that each call
   // since the first of them ends at (kMaxCalls at most)
@@ -394,9 +395,14 @@ int enqueue_step(cpi_ctx *c, bool aux) {
 // steps (measured at c2: ≈ 4 µs less per step than one graph per step)
 constexpr int kGraphRuns[2] = {32, 4};
 
-// fewest plain steps of a call that go through the resident kernel: its
-// cooperative launch and first loads cost as much as a few steps
-constexpr int kMinResident = 4;
+// Fewest plain steps of a call that go through the resident kernel: its launch
+// and first loads cost as much as some steps.  With up to a block per CU calls
+// of 5 steps take as long either way (energies read after each: 72-93 us, one
+// launch per kernel 75-89), of 6 steps 4-12% less in the resident kernel.  With
+// more blocks a call of 5 or 6 takes longer in it (196,608 tet4, FP32: 101 us
+// against 87, 110 against 103; 48,000 tet10: 128 against 114, 139 against 135),
+// one of 7 less (117 against 118; 148 against 155).
+constexpr int kMinResident = 4, kMinResidentMany = 6;
 
 // Most steps of one resident launch.  A longer call takes several: between them
 // the chip is free for other streams' kernels (another context's ten steps, one
@@ -1018,6 +1024,7 @@ static int create_impl(cpi_ctx *c, const cpi_mesh_desc *m, const cpi_material *m
         for (hipEvent_t &e : c->res_done)
           HIPCHK(c, hipEventCreateWithFlags(&e, hipEventDisableTiming));
         c->res_able = true;
+        c->res_min = B.nblocks <= prop.multiProcessorCount ? kMinResident : kMinResidentMany;
         P.resident = B.nblocks > 1;  // one block waits for nobody
       }
     }
@@ -1273,7 +1280,7 @@ extern "C" int cpi_step(cpi_ctx *c, int32_t nsteps) {
   int64_t rest = nsteps;
   int rc = CPI_OK;
   auto may = [&]() {
-    return c->resident && c->gs.plain && !c->P.samples && nsteps - 1 >= kMinResident;
+    return c->resident && c->gs.plain && !c->P.samples && nsteps - 1 >= c->res_min;
   };
   // plain steps launched one by one run whatever became of the launches before
   // them: these have to be settled first

@@ -41,7 +41,7 @@ def run(quad, rule, calls, read, **opts):
 @pytest.mark.parametrize("calls,read", [
     ((25, 25, 25, 25), ()),
     ((30, 1, 6, 3, 17, 2, 1), ()),       # short calls between them
-    ((5, 1, 1, 1, 1, 1, 1, 1), ()),      # more queued calls than steps of the first
+    ((7, 1, 1, 1, 1, 1, 1, 1, 1), ()),    # more queued calls than steps of the first
     ((12, 7, 9), (1,)),                  # read half way
 ])
 def test_every_call_has_the_energies_of_its_own_last_step(quad, rule, calls, read):
@@ -59,7 +59,7 @@ def test_every_call_has_the_energies_of_its_own_last_step(quad, rule, calls, rea
 
 @pytest.mark.parametrize("more", [dict(debug_fill_nan=3), {}])
 def test_more_queued_calls_than_the_context_remembers(more):
-    calls = (5,) * 1100
+    calls = (7,) * 1100
     a = run(False, -1, calls, (), **more)
     b = run(False, -1, calls, (), use_graph=0)
     assert len(a[0]) == len(b[0]) == len(calls) + 1

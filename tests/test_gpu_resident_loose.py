@@ -29,7 +29,7 @@ def run(cells, quad, rule, loose, **opts):
     d.vel[:] = v0
     d.init(2e-7)
     out = []
-    for k in (5, 1, 26):
+    for k in (7, 1, 24):
         d.step(k)
         out += list(d.fetch()) + [d.energy()[0]]
     d.close()

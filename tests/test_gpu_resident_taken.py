@@ -1,7 +1,8 @@
 """Which steps the resident kernel takes: the plain steps of a call of five or
-more where every block fits the chip, none elsewhere.  A resident path that is
-silently off gives the same results as the per-step kernels, so the tests that
-compare the two say nothing without this one."""
+more (seven, with more blocks than CUs) where every block fits the chip, none
+elsewhere.  A resident path that is silently off gives the same results as the
+per-step kernels, so the tests that compare the two say nothing without this
+one."""
 import pytest
 
 import cppimpact_amd as ci
@@ -11,8 +12,8 @@ from common import E, H, NU, RHO, SY
 
 pytestmark = pytest.mark.gpu
 
-CALLS = (5, 6, 1, 40)
-PLAIN = 4 + 5 + 39
+CALLS = (7, 8, 1, 4, 40)
+PLAIN = 6 + 7 + 39
 
 
 def counts(cells, quad, calls=CALLS, **opts):
@@ -64,11 +65,13 @@ def test_other_meshes_are_not(cells, quad, more):
 
 def test_short_calls_are_not():
     assert counts((4, 4, 5), False, calls=(1, 2, 3, 4), physics=L.PHYSICS_EP) == (0, 0)
+    assert counts((4, 4, 5), False, calls=(5, 6), physics=L.PHYSICS_EP) == (9, 0)
+    assert counts((32, 32, 32), False, calls=(5, 6), physics=L.PHYSICS_EP) == (0, 0)
 
 
 @pytest.mark.parametrize("quad,rule", [(False, -1), (True, L.QUAD_EXACT4), (True, L.QUAD_REF5)])
 def test_a_launch_that_gives_up_takes_none(quad, rule):
     """Every wait gives up at its first poll."""
-    taken, redone = counts((5, 6, 7), quad, calls=(30, 6, 17), physics=L.PHYSICS_EP,
+    taken, redone = counts((5, 6, 7), quad, calls=(30, 7, 17), physics=L.PHYSICS_EP,
                            debug_fill_nan=3, **(dict(quadrature=rule) if quad else {}))
-    assert taken == 0 and redone >= 29 + 5 + 16
+    assert taken == 0 and redone >= 29 + 6 + 16
