@@ -416,10 +416,11 @@ constexpr int64_t kMaxResident = 1024;
 constexpr int kAhead = 64;
 
 // Polls after which a wait of a resident launch gives up: 6 ms, much longer than
-// another stream's kernels hold up its last blocks, and short beside the waits
-// that never end (another kernel's blocks in between left two of this one's
-// without a contiguous piece of LDS on some CU), after which the context's steps
-// are launched one by one until the next cpi_init.
+// another stream's kernels hold up its last blocks.  Some waits never end: 512
+// blocks, two on every CU, that were launched while another context's step ran
+// did not all get to run (some CU's room for the second is not the room it has
+// when it starts empty).  The context's steps are then launched one by one until
+// the next cpi_init.
 constexpr unsigned kSpinLimit = 1u << 15;
 
 // most calls queued on resident launches of unknown outcome (cpi_ctx::calls)
@@ -718,6 +719,7 @@ static int create_impl(cpi_ctx *c, const cpi_mesh_desc *m, const cpi_material *m
     return fail(c, CPI_ERR_NO_DEVICE, std::string("device is ") + prop.gcnArchName +
                                           ", this library is built for gfx950 only");
   c->dev = opt->device;
+  const int cus = prop.multiProcessorCount;
   HIPCHK(c, hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
   {
     const size_t all = 8 * (kStateWords + 16 * (size_t)c->nn);
@@ -736,7 +738,7 @@ static int create_impl(cpi_ctx *c, const cpi_mesh_desc *m, const cpi_material *m
   }
   // device orders
   if (c->scatter == CPI_SCATTER_BLOCK) {
-    const int nt = elem_block_threads(npe, c->rule, c->prec, c->phys, 0);
+    const int nt = elem_block_threads(npe, c->rule, c->prec, c->phys, 0, cus);
     const int dflt = elem_block_default_elements(npe);
     int me = opt->block_elements > 0 ? opt->block_elements : dflt;
     // the tet4 kernel gives each thread one element and at most one node,
@@ -905,18 +907,17 @@ static int create_impl(cpi_ctx *c, const cpi_mesh_desc *m, const cpi_material *m
   }
   if (c->scatter == CPI_SCATTER_BLOCK) {
     BlockPlan &B = c->plan;
-    if (npe == 4 && B.max_local_nodes > elem_block_threads(4, c->rule, c->prec, c->phys, B.nblocks))
+    if (npe == 4 && B.max_local_nodes > elem_block_threads(4, c->rule, c->prec, c->phys, B.nblocks, cus))
       return fail(c, CPI_ERR_INVALID, "partition: a tet4 block has more nodes than threads");
-    if (npe == 10 && c->nq == 4 && 4 * B.max_block_elems > elem_block_threads(10, c->rule, c->prec, c->phys, B.nblocks))
+    if (npe == 10 && c->nq == 4 && 4 * B.max_block_elems > elem_block_threads(10, c->rule, c->prec, c->phys, B.nblocks, cus))
       return fail(c, CPI_ERR_INVALID, "partition: a tet10 block has more points than threads");
     int32_t *meta, *bn, *bs, *sp, *dn, *ds;
     uint16_t *cl, *ci, *cw = nullptr, *dg, *dof;
     Vec3 *part;
     // the five-point tet10 kernel reads no words, but its resident steps do:
     // a thread per node, its elements in one round, a block per CU
-    const int nt5 = elem_block_threads(npe, c->rule, c->prec, c->phys, B.nblocks);
-    const bool five = npe == 10 && c->nq == 5 && B.nblocks <= prop.multiProcessorCount &&
-                      nt5 == elem_block_threads(npe, c->rule, c->prec, c->phys, 0) &&
+    const int nt5 = elem_block_threads(npe, c->rule, c->prec, c->phys, B.nblocks, cus);
+    const bool five = npe == 10 && c->nq == 5 && B.nblocks <= cus &&
                       B.max_local_nodes <= nt5 && B.max_block_elems <= nt5 / 64 * 12 &&
                       B.corner_fits();
     const bool words = corner_words(c) || five;
@@ -977,6 +978,7 @@ static int create_impl(cpi_ctx *c, const cpi_mesh_desc *m, const cpi_material *m
       P.mlp_rows = rows;
     }
     P.nblocks = B.nblocks;
+    P.narrow5 = npe == 10 && c->nq == 5 && nt5 != elem_block_threads(npe, c->rule, c->prec, c->phys, 0, cus);
     // FP64 tet10 on a 4-point rule: the matrix units sum the corner forces
     // while the chip is not full twice over (whose blocks may be resident).
     // There the arithmetic counts (48k elements, resident: 13.1 -> 10.2 us a
@@ -984,7 +986,7 @@ static int create_impl(cpi_ctx *c, const cpi_mesh_desc *m, const cpi_material *m
     // traffic, and sixteen elements a wave meet twice the LDS bank conflicts of
     // quads (1.2M elements: 165 us with quads, 170).
     P.matrix = npe == 10 && c->nq == 4 && c->prec != CPI_PREC_F32 &&
-               B.nblocks <= 2 * prop.multiProcessorCount;
+               B.nblocks <= 2 * cus;
     c->smem = elem_block_smem(npe, c->rule, c->prec, P.ml, P.max_el, P.kmax);
     if (c->smem > (size_t)prop.sharedMemPerBlock)
       return fail(c, CPI_ERR_INVALID, "element block needs " + std::to_string(c->smem) +
@@ -999,7 +1001,7 @@ static int create_impl(cpi_ctx *c, const cpi_mesh_desc *m, const cpi_material *m
     auto fits = [&](size_t smem) {
       return smem <= (size_t)prop.sharedMemPerBlock &&
              B.nblocks <= resident_capacity(npe, c->rule, c->prec, c->phys, smem,
-                                            prop.multiProcessorCount);
+                                            cus);
     };
     if (opt->use_graph && c->phys != 2 && words && prop.cooperativeLaunch &&
         (npe == 4 || five || c->prec == CPI_PREC_F32 || P.matrix) && fits(c->smem)) {
@@ -1024,12 +1026,12 @@ static int create_impl(cpi_ctx *c, const cpi_mesh_desc *m, const cpi_material *m
         for (hipEvent_t &e : c->res_done)
           HIPCHK(c, hipEventCreateWithFlags(&e, hipEventDisableTiming));
         c->res_able = true;
-        c->res_min = B.nblocks <= prop.multiProcessorCount ? kMinResident : kMinResidentMany;
+        c->res_min = B.nblocks <= cus ? kMinResident : kMinResidentMany;
         P.resident = B.nblocks > 1;  // one block waits for nobody
       }
     }
     // one energy row per wave
-    c->n_elem_rows = c->nblocks * (elem_block_threads(npe, c->rule, c->prec, c->phys, c->nblocks) / 64);
+    c->n_elem_rows = c->nblocks * (elem_block_threads(npe, c->rule, c->prec, c->phys, c->nblocks, cus) / 64);
     c->n_node_rows = 4 * std::max(1, (B.n_boundary + 255) / 256);
   } else {
     c->n_elem_rows = elem_direct_rows(npe, ne);

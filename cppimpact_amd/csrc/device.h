@@ -65,7 +65,8 @@ struct Params {
   // c44 = (1-2nu)/2 k with k = E/((1+nu)(1-2nu)))
   double c11, c12, c44, mu, sy0, H, wave_speed;
   // wall (wall.h:37-44)
-  int wall_on, wall_dim, wall_normal, pad0;
+  int wall_on, wall_dim, wall_normal;
+  int narrow5;           // the five-point tet10 kernel in 384 threads (narrow5())
   double wall_loc, wall_k, wall_nk;
   const uint8_t *contact_mask;  // slave-only contact, or null for all nodes
   const uint8_t *fixed_mask;    // held nodes (fixed set), or null for none

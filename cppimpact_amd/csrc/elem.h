@@ -46,8 +46,10 @@ template <> struct Quad<RULE_CENTROID> {
 };
 
 // Where a point's stress state lies.  The kernels with a thread per point
-// (k_elem_block4, k_elem_block10, the resident steps) keep a block's state
-// together, [block][6][state_ld] with thread t's point at t (StateBlock): a
+// (k_elem_block4, k_elem_block10, k_elem_block5, the resident steps) keep a
+// block's state together, [block][6][state_ld] (StateBlock), with thread t's point
+// at t (tet10 on a 4-point rule: PointLane::place; on the five-point rule point q
+// of the block's element k at 5 k + q): a
 // wave reads whole aligned lines, and a block one contiguous piece of memory
 // per step, through a buffer descriptor with one 32-bit offset per thread
 // (64-bit addresses, shared by a component's load and store, stay live across

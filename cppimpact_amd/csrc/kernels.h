@@ -8,7 +8,7 @@
 namespace cpi {
 
 size_t elem_block_smem(int npe, int rule, int prec, int ml, int max_el, int kmax);
-int elem_block_threads(int npe, int rule, int prec, int phys, int nblocks);
+int elem_block_threads(int npe, int rule, int prec, int phys, int nblocks, int cus);
 int elem_block_default_elements(int npe);
 int elem_direct_threads(int npe);
 

@@ -1099,8 +1099,6 @@ __host__ __device__ constexpr int lds_mail_bytes(int rsz, int most) {
   return lds_round16(3L * rsz * most) + lds_round16(8L * most);
 }
 
-// NPE 4: thread t has element t and node t of the block, as k_elem_block4.
-// NPE 10: thread t has point t & 3 of element t / 4, as k_elem_block10.
 __device__ __forceinline__ uint32_t decision(const Params &p) {
   return __hip_atomic_load(&p.ctl->decision, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
@@ -1109,6 +1107,10 @@ __device__ __forceinline__ void decide(const Params &p, unsigned L, unsigned how
   atomicCAS(&p.ctl->decision, 2u * (L - 1u), 2u * L + how);
 }
 
+// Thread t has node t of the block, and the element and point that it has in the
+// per-step kernels: tet4, element t (k_elem_block4); tet10 on a 4-point rule,
+// PointLane's (k_elem_block10); on the five-point rule, point lane % 5 of the
+// wave's element lane / 5, twelve of them (k_elem_block5).
 template <int NPE, int RULE, typename R, int PHYS, int NT, int WPE>
 __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WPE)))
 k_resident(Params p, Resident rs) {
@@ -1997,7 +1999,7 @@ constexpr int block_elements(int npe) { return npe == 4 ? 384 : 128; }
 // minimum waves per SIMD of the per-point tet10 kernel
 template <typename R> constexpr int tet10_waves() { return 4; }
 
-// Threads of the 5-point tet10 kernel.  Up to one block per CU a step takes
+// Threads of the 5-point tet10 kernel (cus: the device's CUs).  Up to one block per CU a step takes
 // as long as one block does, and 704 threads do its 128 elements in one round
 // (13k elements, FP64 compat: 9.5 us, 384 threads 12.2).  With more blocks 384
 // threads, two rounds, leave room for more workgroups per CU and one's loads
@@ -2006,8 +2008,11 @@ template <typename R> constexpr int tet10_waves() { return 4; }
 // three waves per SIMD, where a second 6-wave workgroup often finds no room:
 // 259 us against 230.
 constexpr int kNarrow5 = 384;
-static bool narrow5(int nblocks, bool f64_state) { return nblocks > 256 && !f64_state; }
-// its waves per SIMD: FP64 with a state takes 144 VGPRs
+template <typename R, int PHYS> constexpr bool may_narrow5() {
+  return sizeof(R) == 4 || PHYS == PHYS_COMPAT;
+}
+static bool narrow5(int nblocks, int cus, bool f64_state) { return nblocks > cus && !f64_state; }
+// its waves per SIMD: FP64 with a state takes 148 VGPRs
 template <typename R, int PHYS> constexpr int tet10_waves5() {
   return sizeof(R) == 8 && PHYS != PHYS_COMPAT ? 3 : 4;
 }
@@ -2037,11 +2042,11 @@ size_t elem_block_smem(int npe, int rule, int prec, int ml, int max_el, int kmax
          lds_basis_bytes(npe, rsz, rule == RULE_REF5 ? 5 : 4);
 }
 
-int elem_block_threads(int npe, int rule, int prec, int phys, int nblocks) {
+int elem_block_threads(int npe, int rule, int prec, int phys, int nblocks, int cus) {
   if (npe == 4) return block_threads<4, RULE_CENTROID>();
   if (rule == RULE_REF5)
-    return narrow5(nblocks, prec != 1 && phys != PHYS_COMPAT) ? kNarrow5
-                                                              : block_threads<10, RULE_REF5>();
+    return narrow5(nblocks, cus, prec != 1 && phys != PHYS_COMPAT) ? kNarrow5
+                                                                   : block_threads<10, RULE_REF5>();
   return block_threads<10, RULE_EXACT4>();
 }
 
@@ -2172,10 +2177,12 @@ static hipError_t elem_block_t(const Params &p, bool aux, int nblocks, size_t sm
     return tet10_t<RULE, R, PHYS, false, false>(p, aux, nblocks, smem, s);
   } else {
     constexpr int W = tet10_waves5<R, PHYS>();
-    if (narrow5(nblocks, sizeof(R) == 8 && PHYS != PHYS_COMPAT)) {
+    if constexpr (may_narrow5<R, PHYS>()) {
       constexpr int N2 = kNarrow5;
-      if (aux) CPI_LAUNCH((k_elem_block5<RULE, R, PHYS, STEP_OUT, N2, W>), nblocks, N2, smem, s, p);
-      CPI_LAUNCH((k_elem_block5<RULE, R, PHYS, STEP_PLAIN, N2, W>), nblocks, N2, smem, s, p);
+      if (p.narrow5) {
+        if (aux) CPI_LAUNCH((k_elem_block5<RULE, R, PHYS, STEP_OUT, N2, W>), nblocks, N2, smem, s, p);
+        CPI_LAUNCH((k_elem_block5<RULE, R, PHYS, STEP_PLAIN, N2, W>), nblocks, N2, smem, s, p);
+      }
     }
     if (aux && p.resident)
       CPI_LAUNCH((k_elem_block5<RULE, R, PHYS, STEP_OUT_ASK, NT, W>), nblocks, NT, smem, s, p);
@@ -2264,8 +2271,12 @@ template <int NPE, int RULE, typename R, int PHYS> struct ElemBlockPrepF {
         hipError_t e = lds_opt_in(k_elem_block5<RULE, R, PHYS, STEP_OUT, NT, W>, smem);
         if (e == hipSuccess) e = lds_opt_in(k_elem_block5<RULE, R, PHYS, STEP_OUT_ASK, NT, W>, smem);
         if (e == hipSuccess) e = lds_opt_in(k_elem_block5<RULE, R, PHYS, STEP_PLAIN, NT, W>, smem);
-        if (e == hipSuccess) e = lds_opt_in(k_elem_block5<RULE, R, PHYS, STEP_OUT, kNarrow5, W>, smem);
-        if (e == hipSuccess) e = lds_opt_in(k_elem_block5<RULE, R, PHYS, STEP_PLAIN, kNarrow5, W>, smem);
+        if constexpr (may_narrow5<R, PHYS>()) {
+          if (e == hipSuccess)
+            e = lds_opt_in(k_elem_block5<RULE, R, PHYS, STEP_OUT, kNarrow5, W>, smem);
+          if (e == hipSuccess)
+            e = lds_opt_in(k_elem_block5<RULE, R, PHYS, STEP_PLAIN, kNarrow5, W>, smem);
+        }
         return e;
       }
     }
@@ -2294,8 +2305,7 @@ hipError_t launch_elem_direct(const Params &p, int rule, int prec, int phys, boo
   return dispatch<ElemDirectF>(p.npe, rule, prec, phys, p, atomic, list, n, s);
 }
 
-// minimum waves per SIMD of the resident kernels
-// minimum waves per SIMD: the five-point tet10 kernel's eleven waves a block
+// minimum waves per SIMD of the resident kernels: the five-point tet10 kernel's eleven waves a block
 // leave a CU no second block, and get the registers
 template <int NPE, int RULE> constexpr int resident_waves() {
   return NPE == 10 && Quad<RULE>::n == 5 ? 3 : 4;
