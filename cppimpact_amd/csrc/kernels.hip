@@ -1252,8 +1252,10 @@ k_resident(Params p, Resident rs) {
     for (int m = ts; m < nm; m += NT) {
       R w[3];
       unsigned spins = 0;
+      // (decision by p: pl's pointer would be loaded again ahead of every wait,
+      // 3% of a step of 3,072 tet4 in FP32)
       while (!Rec::get(mail, 2 * rs.messages, inbox + m0 + m, w)) {
-        if (++spins >= rs.spin_limit || ((spins & 255u) == 0u && (decision(pl) & 1u))) {
+        if (++spins >= rs.spin_limit || ((spins & 255u) == 0u && (decision(p) & 1u))) {
           gave_up = 1;
           break;
         }
