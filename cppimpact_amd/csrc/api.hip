@@ -410,7 +410,7 @@ constexpr int kMinResident = 4, kMinResidentMany = 6;
 // ms so; its own resident launches wait for those queued before them, as
 // cooperative launches do), and one that gives up loses the steps of one launch
 // only.  The further launches of a call cost nothing that shows (3,000 steps of
-// 512 elements in one launch or three: 13.74 and 13.73 ms).  At most 2 kAhead
+// 3,072 tet4 in one launch or three: 13.74 and 13.73 ms).  At most 2 kAhead
 // launches are queued, where a call of millions of steps would queue thousands.
 constexpr int64_t kMaxResident = 1024;
 constexpr int kAhead = 64;
