@@ -406,22 +406,23 @@ constexpr int kMinResident = 4, kMinResidentMany = 6;
 
 // Most steps of one resident launch.  A longer call takes several: between them
 // the chip is free for other streams' kernels (another context's ten steps, one
-// launch per kernel, took 440 ms beside a call of 60,000 in one launch, 12 to 40
+// launch per kernel, took 440 ms beside a call of 60,000 in one launch, 29 to 40
 // ms so; its own resident launches wait for those queued before them, as
 // cooperative launches do), and one that gives up loses the steps of one launch
-// only.  The further launches of a call cost nothing that shows (3,000 steps of
-// 3,072 tet4 in one launch or three: 13.74 and 13.73 ms).  At most 2 kAhead
-// launches are queued, where a call of millions of steps would queue thousands.
+// only.  A further launch takes 25 to 40 us: calls of 3,000 steps took 3-4%
+// longer in launches of 128 steps, 1-2% in 256, 0.5% in 512, and in 1,024 no
+// longer than in one.  At most 2 kAhead launches are queued, where a call of
+// millions of steps would queue thousands.
 constexpr int64_t kMaxResident = 1024;
 constexpr int kAhead = 64;
 
-// Polls after which a wait of a resident launch gives up: 6 ms, much longer than
-// another stream's kernels hold up its last blocks.  Some waits never end: 512
+// Polls after which a wait of a resident launch gives up: 24 ms (the last blocks
+// may have to wait for another stream's kernels).  Some waits never end: 512
 // blocks, two on every CU, that were launched while another context's step ran
 // did not all get to run (some CU's room for the second is not the room it has
 // when it starts empty).  The context's steps are then launched one by one until
 // the next cpi_init.
-constexpr unsigned kSpinLimit = 1u << 15;
+constexpr unsigned kSpinLimit = 1u << 17;
 
 // most calls queued on resident launches of unknown outcome (cpi_ctx::calls)
 constexpr size_t kMaxCalls = 1024;

@@ -235,7 +235,10 @@ int cpi_init(cpi_ctx *ctx, double dt);
 
 /* nsteps iterations of the loop body of Dynamics::solve
    (dynamics.h:471-511, dynamics.cuh:450-517): du = dt v; update(); x += du;
-   v += dt a; v_i = v - dt/2 a.  Asynchronous: returns after enqueueing. */
+   v += dt a; v_i = v - dt/2 a.  Asynchronous: returns after enqueueing.  (On a
+   mesh small enough for resident launches, a call of 2 to 6 steps waits for
+   longer calls queued before it, and one of more than 131,072 steps for all
+   but its last 65,536.) */
 int cpi_step(cpi_ctx *ctx, int32_t nsteps);
 
 /* Waits for queued work; reports CPI_ERR_NUMERIC if a NaN/Inf or an inverted
