@@ -57,8 +57,8 @@ template <> struct Quad<RULE_CENTROID> {
 // kernels keep planes of the whole mesh, [nq][6][ne] (StatePlane), as all did:
 // the 1.2M-tet10 kernel's waves then read four short runs of each of 24 planes,
 // and its traffic alone (no arithmetic) took 204 of its 217 us in FP64.  With
-// the block layout the whole kernel takes 165 us on the same box (FP32 137 ->
-// 117; over the boxes 165-187 and 115-128), the 64^3
+// the block layout the whole kernel takes 165 us on the same card (FP32 137 ->
+// 117; over several cards 165-187 and 115-128), the 64^3
 // tet4 kernel 41 -> 39 (FP32 27.5 -> 26.5).
 //
 // State words are read and written once per step.  STREAM = true marks those
